@@ -279,8 +279,6 @@ struct kc_graph {
   Arena arena;
   KernelTimer timer;
   std::vector<LevelRec> levels;
-  bool base_case_used = false;
-  uint64_t base_case_rounds = 0;
   hipEvent_t ev_begin = nullptr, ev_end = nullptr;
   uint32_t components = 0;
   bool have_labels = false;
@@ -471,25 +469,24 @@ Bins make_bins(kc_graph *g, uint64_t n, const uint64_t *off, const BinCfg &cfg, 
   return b;
 }
 
-uint64_t sweep_bytes(uint64_t n, uint64_t m2, bool count) {
-  // offsets, neighbour ids, neighbour keys, own key read + write, inter count
-  return 8 * (n + 1) + 12 * m2 + 16 * n + (count ? 4 * n : 0);
+uint64_t sweep_bytes(uint64_t n, uint64_t m2) {
+  // offsets, neighbour ids, neighbour keys, own key read + write
+  return 8 * (n + 1) + 12 * m2 + 16 * n;
 }
 
-// Runs in-place sweeps (and optionally pointer jumps) until no key changes.
+// Runs in-place sweeps until no key changes.
 // Sweeps are launched in speculative batches; a sweep whose predecessor
 // changed nothing returns at once.  Returns the number of sweeps that did work
 // (the last of them found no change).
-// packed (non-null: plain in-place sweeps without counts or jumps): the
-// sweeps run over these packed keys (pack_keys) instead of key.
+// packed (non-null): the sweeps run over these packed keys (pack_keys)
+// instead of key.
 uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t *off, const uint32_t *col,
-                           uint64_t *key, uint64_t hop, const Bins &b, bool count, bool with_jump,
-                           uint32_t &flag_base, bool book_bytes = true, uint64_t block = 0,
+                           uint64_t *key, uint64_t hop, const Bins &b, uint32_t &flag_base, bool book_bytes = true,
                            uint32_t *packed = nullptr) {
   uint64_t done = 0;
   const uint32_t batch = n < (1u << 16) ? 8u : 3u;
   // (packed: 4-byte keys for the neighbours and the row's own)
-  const uint64_t bytes = !book_bytes ? 0 : packed ? 8 * (n + 1) + 8 * m2 + 8 * n : sweep_bytes(n, m2, count);
+  const uint64_t bytes = !book_bytes ? 0 : packed ? 8 * (n + 1) + 8 * m2 + 8 * n : sweep_bytes(n, m2);
   while (true) {
     if (flag_base + batch + 2 >= kMaxFlags) {
       fill_u32(reinterpret_cast<uint32_t *>(g->flags), kMaxFlags, 0, g->stream);
@@ -507,13 +504,9 @@ uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t 
       if (packed)
         sweep_packed(off, col, packed, b, &g->flags[f], prev, g->stream, true);
       else
-        sweep(block ? kSweepBlock : kSweepInPlace, count, off, col, key, key, hop, b, g->deg_inter, g->hub_inter,
-              &g->flags[f], prev, g->stream, block, true);
+        sweep(kSweepInPlace, false, off, col, key, key, hop, b, g->deg_inter, g->hub_inter, &g->flags[f], prev,
+              g->stream, true);
       g->timer.stop(slots[i], bytes);
-      if (with_jump) {
-        TimedScope js(g->timer, KC_K_JUMP, 16 * n);
-        jump(n, key, &g->flags[f], g->stream);
-      }
     }
     d2h(g, g->h_flags, &g->flags[flag_base], batch * sizeof(int));
     sync(g);
@@ -721,7 +714,7 @@ uint64_t rounds_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t
         // reach the same fixed point in as many sweeps as the longest chain
         // of improvements among them, instead of one round per distance left.
         // (The rounds' booked bytes already cover one read of every row.)
-        done += sweep_to_fixpoint(g, n, m2, off, col, key, kOneHop, b, false, false, flag_base, false);
+        done += sweep_to_fixpoint(g, n, m2, off, col, key, kOneHop, b, flag_base, false);
         break;
       }
     }
@@ -958,8 +951,6 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out) {
   int pp = 0;
   fill_u32(reinterpret_cast<uint32_t *>(g->flags), kMaxFlags, 0, g->stream);
   g->levels.clear();
-  g->base_case_used = false;
-  g->base_case_rounds = 0;
   const int max_levels = o->max_levels > 0 ? o->max_levels : 4096;
   DeviateArgs da{o->seed, 0, g->non_isolated, o->deviate_fma, o->deviate_stream, g->d_table, g->table_k};
   bool top_from_keys = false;  // top rep computed by the base case into rep of that level
@@ -978,22 +969,20 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out) {
     const bool pre = pre_left > 0 && m2_l > 0;
     if (pre) --pre_left;
     if (!pre && (m2_l == 0 || (o->seq_limit > 0 && m2_l / 2 <= o->seq_limit))) {
-      // Base case (RunSequentialCC, exponential_contraction.h:908-922): min-label
-      // propagation with pointer jumping on the remaining graph.
-      if (!bins_valid) b = make_bins(g, n_l, off_l, cfg);
+      // Base case (RunSequentialCC, exponential_contraction.h:908-922): the
+      // components of the remaining graph.
+      // (one pass of union-find over the edges, cid holding the forest; 30 us
+      // against 150 for the min-label sweeps and their bins on a level of
+      // 2283 vertices)
       {
-        TimedScope ts(g->timer, KC_K_DEVIATES, 8 * n_l);
-        init_keys_index(n_l, g->key, g->stream);
+        TimedScope ts(g->timer, KC_K_JUMP, 8 * (n_l + 1) + 4 * m2_l + 4 * n_l);
+        union_components(n_l, m2_l, off_l, col_l, 0, g->cid, g->stream);
       }
-      uint64_t r = 0;
-      if (m2_l > 0) r = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, 0, b, false, true, flag_base);
-      g->base_case_used = m2_l > 0;
-      g->base_case_rounds = r;
-      out.sweeps += r;
+      out.sweeps += m2_l > 0;
       top_rep = g->rep_a;
       {
-        TimedScope ts(g->timer, KC_K_UNDO, 16 * n_l);
-        rep_from_keys(n_l, g->key, gid_l, top_rep, g->stream);
+        TimedScope ts(g->timer, KC_K_UNDO, 12 * n_l);
+        union_reps(n_l, g->cid, gid_l, top_rep, g->stream);
       }
       top_from_keys = true;
       break;
@@ -1007,15 +996,13 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out) {
     }
     uint64_t sweeps = 0;
     if (pre) {
-      // components inside the blocks: min-label propagation over the edges
-      // inside a block, with pointer jumping, to the fixpoint
+      // components inside the blocks: union-find over the edges inside a block
       const uint64_t bsize = ceil_div(n_l, static_cast<uint64_t>(o->pre_blocks));
       {
-        TimedScope ts(g->timer, KC_K_DEVIATES, 8 * n_l);
-        init_keys_index(n_l, g->key, g->stream);
+        TimedScope ts(g->timer, KC_K_JUMP, 8 * (n_l + 1) + 4 * m2_l + 12 * n_l);
+        union_components(n_l, m2_l, off_l, col_l, bsize, g->cid, g->stream);
+        union_keys(n_l, g->cid, g->key, g->stream);
       }
-      // (sweeps over the edges inside the blocks, with pointer jumping, in batches)
-      sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, 0, b, false, true, flag_base, true, bsize);
       if (o->pre_contract == KC_PRE_LOCAL) {
         TimedScope ts(g->timer, KC_K_SWEEP, 8 * (n_l + 1) + 4 * m2_l + 8 * n_l);
         block_interface(off_l, col_l, n_l, bsize, g->key, g->stream);
@@ -1062,7 +1049,7 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out) {
           uint64_t *kin = pass == 0 ? g->key : g->key2;
           uint64_t *kout = pass == 0 ? g->key2 : g->key;
           KC_HIP(hipMemcpyAsync(kout, kin, n_l * 8, hipMemcpyDeviceToDevice, g->stream));
-          TimedScope ts(g->timer, KC_K_SWEEP, sweep_bytes(n_l, m2_l, false));
+          TimedScope ts(g->timer, KC_K_SWEEP, sweep_bytes(n_l, m2_l));
           sweep(kSweepJacobi, false, off_l, col_l, kin, kout, 0, b, g->deg_inter, g->hub_inter,
                 &g->flags[kMaxFlags - 1], nullptr, g->stream);
         }
@@ -1085,8 +1072,7 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out) {
           sync(g);
           if (g->h_small[7]) pk = nullptr;
         }
-        sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, kOneHop, b, false, false, flag_base, true, 0,
-                                   pk);
+        sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, kOneHop, b, flag_base, true, pk);
         if (pk) unpack_keys(n_l, pk, g->key, g->stream);
       }
     }
@@ -1329,22 +1315,33 @@ void ensure_learned_buffers(kc_graph *g, uint64_t n) {
   g->learned_cap = n;
 }
 
-// Min-label propagation (labels) or propagation + pointer jumping (shortcuts).
+// Min-label propagation (labels), or the shortcuts variant: the same labels by
+// union-find, whose pointer shortening is its pointer jumping (one pass over
+// the edges counts as its one sweep).
 void run_propagation(kc_graph *g, const kc_options *o, RunOut &out) {
-  const BinCfg cfg = bin_cfg(g, o);
+  g->levels.clear();
+  out.levels = 0;
+  uint32_t *partial = reinterpret_cast<uint32_t *>(g->scan_scratch);
+  if (o->variant == KC_VARIANT_SHORTCUT) {
+    out.sweeps = g->n > 0;
+    {
+      TimedScope ts(g->timer, KC_K_JUMP, 8 * (g->n + 1) + 4 * g->m2 + 4 * g->n);
+      union_components(g->n, g->m2, g->off0, g->col0, 0, g->cid, g->stream);
+    }
+    TimedScope ts(g->timer, KC_K_CANON, 8 * g->n);
+    union_labels(g->n, g->cid, g->labels, g->small + 5, partial, g->stream);
+    return;
+  }
   uint32_t flag_base = 0;
   fill_u32(reinterpret_cast<uint32_t *>(g->flags), kMaxFlags, 0, g->stream);
-  g->levels.clear();
-  Bins b = make_bins(g, g->n, g->off0, cfg);
+  Bins b = make_bins(g, g->n, g->off0, bin_cfg(g, o));
   {
     TimedScope ts(g->timer, KC_K_DEVIATES, 8 * g->n);
     init_keys_index(g->n, g->key, g->stream);
   }
-  out.sweeps = sweep_to_fixpoint(g, g->n, g->m2, g->off0, g->col0, g->key, 0, b, false,
-                                 o->variant == KC_VARIANT_SHORTCUT, flag_base);
-  out.levels = 0;
+  out.sweeps = sweep_to_fixpoint(g, g->n, g->m2, g->off0, g->col0, g->key, 0, b, flag_base);
   TimedScope ts(g->timer, KC_K_CANON, 12 * g->n);
-  labels_from_keys(g->n, g->key, g->labels, g->small + 5, reinterpret_cast<uint32_t *>(g->scan_scratch), g->stream);
+  labels_from_keys(g->n, g->key, g->labels, g->small + 5, partial, g->stream);
 }
 
 }  // namespace

@@ -58,8 +58,7 @@ struct Bins {
 enum SweepMode : int {
   kSweepInPlace = 0,  // key[v] <- min(key[v], key[w] + hop), updates visible at once
   kSweepJacobi = 1,   // kout[v] <- min over closed neighbourhood of kin (kout pre-copied)
-  kSweepCountOnly = 2, // no update: count neighbours with a different label
-  kSweepBlock = 3      // in place, hop 0, over the neighbours in the row's block of consecutive indices
+  kSweepCountOnly = 2  // no update: count neighbours with a different label
 };
 
 struct DeviateArgs {
@@ -109,7 +108,7 @@ uint64_t bin_scratch_words(uint64_t n);
 // null): when it reads 0 the launch returns at once (converged earlier).
 void sweep(int mode, bool count, const uint64_t *off, const uint32_t *col, const uint64_t *kin,
            uint64_t *kout, uint64_t hop, const Bins &b, uint32_t *deg_inter, uint32_t *hub_inter,
-           int *flag, const int *prev_flag, hipStream_t s, uint64_t block = 0, bool hubs_first = false);
+           int *flag, const int *prev_flag, hipStream_t s, bool hubs_first = false);
 // Packed keys (distance << 24 | label) for the pull sweeps of levels below
 // 2^24 vertices: pack_keys writes them and sets *bad (zeroed first) when a
 // distance exceeds kPackedMaxDist - 1 or a label 24 bits; sweep_packed is
@@ -135,8 +134,18 @@ void push_round(const uint64_t *off, const uint32_t *col, uint64_t *key, uint64_
 void hub_fold(const Bins &b, const uint32_t *hub_inter, uint32_t *deg_inter, uint32_t *hub_pos, uint64_t *prefix,
               uint64_t *scratch, hipStream_t s);
 
-// Pointer jumping on keys: key[v] <- min(key[v], key[label(v)]).
-void jump(uint64_t n, uint64_t *key, int *flag, hipStream_t s);
+// Connected components by union-find (union.hip): parent (n) becomes a forest
+// whose roots are the components' smallest indices; with block > 0, the
+// components of the edges inside blocks of that many consecutive indices.
+// Then the root of every vertex: as a representative gid[root] (null gid: the
+// root), as a key of distance 0, or as its label with the number of roots
+// (partial: min(ceil(n / 256), 2048) words).
+void union_components(uint64_t n, uint64_t m2, const uint64_t *off, const uint32_t *col, uint64_t block,
+                      uint32_t *parent, hipStream_t s);
+void union_reps(uint64_t n, const uint32_t *parent, const uint32_t *gid, uint32_t *rep, hipStream_t s);
+void union_keys(uint64_t n, const uint32_t *parent, uint64_t *key, hipStream_t s);
+void union_labels(uint64_t n, const uint32_t *parent, uint32_t *labels, uint32_t *roots, uint32_t *partial,
+                  hipStream_t s);
 
 // Interface vertices of blocks of bsize consecutive indices (a neighbour in
 // another block) get their own index back as key: key[v] = v.
@@ -289,8 +298,8 @@ int radix_sort_pairs(uint64_t n, int bits, uint32_t *keys, uint32_t *vals, uint3
 
 void undo(uint64_t n, const uint32_t *lab, const uint32_t *newidx, const uint32_t *gid,
           const uint32_t *rep_up, uint32_t *rep_out, hipStream_t s);
-// rep of a base-case level: rep[v] = gid[low(key[v])].
-void rep_from_keys(uint64_t n, const uint64_t *key, const uint32_t *gid, uint32_t *rep, hipStream_t s);
+// *out = sum of partial[0 .. count).
+void sum_partials_u32(const uint32_t *partial, uint64_t count, uint32_t *out, hipStream_t s);
 // minid[rep[v]] = min over v of gid[v] (identity gid when null).
 void canon_min(uint64_t n, const uint32_t *rep, const uint32_t *gid, uint32_t *minid, hipStream_t s);
 // roots (device) = number of vertices that are their own label; partial needs

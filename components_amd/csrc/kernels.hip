@@ -204,7 +204,6 @@ struct SweepArgs {
   uint32_t *hub_inter;
   int *flag;
   const int *prev_flag;
-  uint64_t block = 0;  // kSweepBlock: indices per block
   int hubs_first = 0;  // k_sweep: sections dispatched from the hub chunks down (as k_round's)
 };
 
@@ -220,9 +219,6 @@ __device__ __forceinline__ bool sweep_group(const SweepArgs &a, bool active, uin
   uint32_t cnt = 0;
   if (active) {
     const uint32_t lv = static_cast<uint32_t>(kv);
-    // kSweepBlock reads the keys of the neighbours in v's block only
-    const uint64_t lo = MODE == kSweepBlock ? v / a.block * a.block : 0;
-    const uint64_t hi = MODE == kSweepBlock ? lo + a.block : ~0ull;
     uint64_t e = e0 + gl;
     // kGather edges per lane per step: their neighbour ids, then their keys,
     // are all in flight together
@@ -232,7 +228,7 @@ __device__ __forceinline__ bool sweep_group(const SweepArgs &a, bool active, uin
 #pragma unroll
       for (int j = 0; j < kGather; ++j) c[j] = a.col[e + j * W];
 #pragma unroll
-      for (int j = 0; j < kGather; ++j) k[j] = c[j] >= lo && c[j] < hi ? a.kin[c[j]] : ~0ull;
+      for (int j = 0; j < kGather; ++j) k[j] = a.kin[c[j]];
 #pragma unroll
       for (int j = 0; j < kGather; ++j) {
         best = min_u64(best, k[j] + a.hop);
@@ -240,8 +236,7 @@ __device__ __forceinline__ bool sweep_group(const SweepArgs &a, bool active, uin
       }
     }
     for (; e < e1; e += W) {
-      const uint32_t c = a.col[e];
-      const uint64_t kw = c >= lo && c < hi ? a.kin[c] : ~0ull;
+      const uint64_t kw = a.kin[a.col[e]];
       best = min_u64(best, kw + a.hop);
       if (COUNT) cnt += static_cast<uint32_t>(kw) != lv;
     }
@@ -849,24 +844,10 @@ __global__ void k_hub_fold(const HubChunk *hubs, uint32_t nH, const uint64_t *pr
   if (c + 1 == nH || hubs[c + 1].k == 0) deg_inter[h.v] = static_cast<uint32_t>(prefix[c + 1] - first);
 }
 
-__global__ void k_jump(uint64_t n, uint64_t *key, int *flag) {
-  uint64_t v = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
-  bool changed = false;
-  if (v < n) {
-    const uint64_t k = key[v];
-    const uint64_t k2 = key[static_cast<uint32_t>(k)];
-    if (k2 < k) {
-      key[v] = k2;
-      changed = true;
-    }
-  }
-  if (__ballot(changed) != 0 && lane_id() == 0) *flag = 1;
-}
-
 // ---------------------------------------------------------------------------
 // Blocks of consecutive level indices (block b holds [b*bsize, (b+1)*bsize)),
 // the PEs of a vertex-block distribution; their components come from
-// kSweepBlock sweeps with pointer jumping.
+// union_components.
 // Interface vertices (a neighbour outside the block) keep their own index as
 // label: key[v] = v.
 __global__ __launch_bounds__(kBlock) void k_block_interface(const uint64_t *off, const uint32_t *col, uint64_t n,
@@ -1880,13 +1861,6 @@ __global__ __launch_bounds__(kBlock) void k_undo(uint64_t n, const uint32_t *lab
   }
 }
 
-__global__ void k_rep_from_keys(uint64_t n, const uint64_t *key, const uint32_t *gid, uint32_t *rep) {
-  uint64_t v = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
-  if (v >= n) return;
-  const uint32_t a = static_cast<uint32_t>(key[v]);
-  rep[v] = gid ? gid[a] : a;
-}
-
 // minid[rep[v]] = min over v of the input id.  Grid-stride: each wave merges
 // the lanes sharing its first lane's representative and carries that minimum
 // while the next steps keep the same representative (the giant component's),
@@ -2289,9 +2263,9 @@ void finish_bins(Bins &b) {
 
 void sweep(int mode, bool count, const uint64_t *off, const uint32_t *col, const uint64_t *kin, uint64_t *kout,
            uint64_t hop, const Bins &b, uint32_t *deg_inter, uint32_t *hub_inter, int *flag, const int *prev_flag,
-           hipStream_t s, uint64_t block, bool hubs_first) {
+           hipStream_t s, bool hubs_first) {
   if (b.blocks == 0) return;
-  SweepArgs a{off, col, kin, kout, hop, b, deg_inter, hub_inter, flag, prev_flag, block, hubs_first ? 1 : 0};
+  SweepArgs a{off, col, kin, kout, hop, b, deg_inter, hub_inter, flag, prev_flag, hubs_first ? 1 : 0};
   dim3 g(b.blocks), t(kBlock);
   if (mode == kSweepInPlace && count)
     hipLaunchKernelGGL((k_sweep<kSweepInPlace, true>), g, t, 0, s, a);
@@ -2299,8 +2273,6 @@ void sweep(int mode, bool count, const uint64_t *off, const uint32_t *col, const
     hipLaunchKernelGGL((k_sweep<kSweepInPlace, false>), g, t, 0, s, a);
   else if (mode == kSweepJacobi)
     hipLaunchKernelGGL((k_sweep<kSweepJacobi, false>), g, t, 0, s, a);
-  else if (mode == kSweepBlock)
-    hipLaunchKernelGGL((k_sweep<kSweepBlock, false>), g, t, 0, s, a);
   else
     hipLaunchKernelGGL((k_sweep<kSweepCountOnly, true>), g, t, 0, s, a);
   KC_LAUNCH_CHECK();
@@ -2357,12 +2329,6 @@ void block_interface(const uint64_t *off, const uint32_t *col, uint64_t n, uint6
                      hipStream_t s) {
   if (n == 0) return;
   hipLaunchKernelGGL(k_block_interface, dim3(row_wave_grid(n)), dim3(kBlock), 0, s, off, col, n, bsize, key);
-  KC_LAUNCH_CHECK();
-}
-
-void jump(uint64_t n, uint64_t *key, int *flag, hipStream_t s) {
-  if (!n) return;
-  hipLaunchKernelGGL(k_jump, dim3(grid_for(n)), dim3(kBlock), 0, s, n, key, flag);
   KC_LAUNCH_CHECK();
 }
 
@@ -2747,9 +2713,8 @@ void undo(uint64_t n, const uint32_t *lab, const uint32_t *newidx, const uint32_
   KC_LAUNCH_CHECK();
 }
 
-void rep_from_keys(uint64_t n, const uint64_t *key, const uint32_t *gid, uint32_t *rep, hipStream_t s) {
-  if (!n) return;
-  hipLaunchKernelGGL(k_rep_from_keys, dim3(grid_for(n)), dim3(kBlock), 0, s, n, key, gid, rep);
+void sum_partials_u32(const uint32_t *partial, uint64_t count, uint32_t *out, hipStream_t s) {
+  hipLaunchKernelGGL(k_reduce_sum, dim3(1), dim3(kBlock), 0, s, partial, count, out);
   KC_LAUNCH_CHECK();
 }
 
@@ -2766,8 +2731,7 @@ void canon_label(uint64_t n, const uint32_t *rep, const uint32_t *gid, const uin
   const unsigned g = static_cast<unsigned>(std::min<uint64_t>(grid_for(n), kCountBlocks));
   hipLaunchKernelGGL(k_canon_label, dim3(g), dim3(kBlock), 0, s, n, rep, gid, minid, labels, partial);
   KC_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_reduce_sum, dim3(1), dim3(kBlock), 0, s, partial, static_cast<uint64_t>(g), roots);
-  KC_LAUNCH_CHECK();
+  sum_partials_u32(partial, g, roots, s);
 }
 
 void drop_isolated(uint64_t n, const uint64_t *off, const uint32_t *col, uint64_t m2, uint32_t *newid, uint32_t *gid0,
@@ -2927,8 +2891,7 @@ void labels_from_keys(uint64_t n, const uint64_t *key, uint32_t *labels, uint32_
   const unsigned g = static_cast<unsigned>(std::min<uint64_t>(grid_for(n), kCountBlocks));
   hipLaunchKernelGGL(k_labels_from_keys, dim3(g), dim3(kBlock), 0, s, n, key, labels, partial);
   KC_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_reduce_sum, dim3(1), dim3(kBlock), 0, s, partial, static_cast<uint64_t>(g), roots);
-  KC_LAUNCH_CHECK();
+  sum_partials_u32(partial, g, roots, s);
 }
 
 

@@ -81,6 +81,65 @@ T *region(uint8_t *base, uint64_t at) {
   return reinterpret_cast<T *>(base + at);
 }
 
+// Min-label propagation in place, as kc_find_components runs KC_VARIANT_LABELS;
+// small + 4 receives the number of roots.  Returns the sweeps.
+uint64_t propagate(uint64_t n, const uint64_t *offsets, const uint32_t *targets, const kc_options &o, uint8_t *base,
+                   uint32_t *labels, hipStream_t s) {
+  uint64_t *key = region<uint64_t>(base, kKeyAt);
+  uint32_t *lists = region<uint32_t>(base, kListsAt);
+  uint32_t *deg_inter = region<uint32_t>(base, kDegAt);
+  HubChunk *hubs = region<HubChunk>(base, kHubsAt);
+  uint32_t *hub_inter = region<uint32_t>(base, kHubInterAt);
+  int *flags = region<int>(base, kFlagsAt);
+  uint32_t *small = region<uint32_t>(base, kSmallAt);
+  // degree bins of the graph (as make_bins does for this variant)
+  const BinCfg cfg = bin_config(o.sweep_group_small, o.sweep_group_mid, o.sweep_group_large);
+  Bins b;
+  b.listT = lists;
+  b.listS = lists + n;
+  b.listW = lists + 2 * n;
+  b.hubs = hubs;
+  bin_vertices(n, offsets, cfg, b.listT, b.listS, b.listW, b.hubs, small, deg_inter,
+               region<uint64_t>(base, kBinScratchAt), s);
+  uint32_t counts[4];
+  KC_HIP(hipMemcpyAsync(counts, small, sizeof(counts), hipMemcpyDeviceToHost, s));
+  KC_HIP(hipStreamSynchronize(s));
+  b.nT = counts[0];
+  b.nS = counts[1];
+  b.nW = counts[2];
+  b.nH = counts[3];
+  if (b.nH > kHubCap) fail(KC_ERR_INVALID, "internal: hub chunk overflow (%u)", b.nH);
+  finish_bins(b);
+  init_keys_index(n, key, s);
+  // sweeps to the fixed point in speculative batches: a sweep whose
+  // predecessor changed nothing returns at once
+  const uint32_t batch = n < (1u << 16) ? 8u : 3u;
+  uint32_t flag_base = 0;
+  uint64_t sweeps = 0;
+  fill_u32(reinterpret_cast<uint32_t *>(flags), kFlagSlots, 0, s);
+  while (true) {
+    if (flag_base + batch + 2 >= kFlagSlots) {
+      fill_u32(reinterpret_cast<uint32_t *>(flags), kFlagSlots, 0, s);
+      flag_base = 0;
+    }
+    for (uint32_t i = 0; i < batch; ++i) {
+      const uint32_t f = flag_base + i;
+      const int *prev = i == 0 ? nullptr : &flags[f - 1];
+      sweep(kSweepInPlace, false, offsets, targets, key, key, 0, b, deg_inter, hub_inter, &flags[f], prev, s);
+    }
+    int h_flags[8];
+    KC_HIP(hipMemcpyAsync(h_flags, &flags[flag_base], batch * sizeof(int), hipMemcpyDeviceToHost, s));
+    KC_HIP(hipStreamSynchronize(s));
+    uint32_t i = 0;
+    while (i < batch && h_flags[i] != 0) ++i;
+    sweeps += i < batch ? i + 1 : batch;
+    flag_base += batch;
+    if (i < batch) break;
+  }
+  labels_from_keys(n, key, labels, small + 4, region<uint32_t>(base, kPartialAt), s);
+  return sweeps;
+}
+
 }  // namespace
 }  // namespace kc
 
@@ -121,59 +180,17 @@ extern "C" int kc_find_components_noalloc(uint64_t n, const uint64_t *offsets, c
     if (n) {
       uint8_t *base = device_scratch();
       uint64_t *key = region<uint64_t>(base, kKeyAt);
-      uint32_t *lists = region<uint32_t>(base, kListsAt);
-      uint32_t *deg_inter = region<uint32_t>(base, kDegAt);
-      HubChunk *hubs = region<HubChunk>(base, kHubsAt);
-      uint32_t *hub_inter = region<uint32_t>(base, kHubInterAt);
-      int *flags = region<int>(base, kFlagsAt);
       uint32_t *small = region<uint32_t>(base, kSmallAt);
       uint32_t *partial = region<uint32_t>(base, kPartialAt);
-      uint64_t *bin_scratch = region<uint64_t>(base, kBinScratchAt);
-      // degree bins of the graph (as make_bins does for these variants)
-      const BinCfg cfg = bin_config(o.sweep_group_small, o.sweep_group_mid, o.sweep_group_large);
-      Bins b;
-      b.listT = lists;
-      b.listS = lists + n;
-      b.listW = lists + 2 * n;
-      b.hubs = hubs;
-      bin_vertices(n, offsets, cfg, b.listT, b.listS, b.listW, b.hubs, small, deg_inter, bin_scratch, s);
-      uint32_t counts[4];
-      KC_HIP(hipMemcpyAsync(counts, small, sizeof(counts), hipMemcpyDeviceToHost, s));
-      KC_HIP(hipStreamSynchronize(s));
-      b.nT = counts[0];
-      b.nS = counts[1];
-      b.nW = counts[2];
-      b.nH = counts[3];
-      if (b.nH > kHubCap) fail(KC_ERR_INVALID, "internal: hub chunk overflow (%u)", b.nH);
-      finish_bins(b);
-      init_keys_index(n, key, s);
-      // sweeps to the fixed point in speculative batches, as kc_find_components
-      // runs them: a sweep whose predecessor changed nothing returns at once
-      const bool with_jump = o.variant == KC_VARIANT_SHORTCUT;
-      const uint32_t batch = n < (1u << 16) ? 8u : 3u;
-      uint32_t flag_base = 0;
-      fill_u32(reinterpret_cast<uint32_t *>(flags), kFlagSlots, 0, s);
-      while (true) {
-        if (flag_base + batch + 2 >= kFlagSlots) {
-          fill_u32(reinterpret_cast<uint32_t *>(flags), kFlagSlots, 0, s);
-          flag_base = 0;
-        }
-        for (uint32_t i = 0; i < batch; ++i) {
-          const uint32_t f = flag_base + i;
-          const int *prev = i == 0 ? nullptr : &flags[f - 1];
-          sweep(kSweepInPlace, false, offsets, targets, key, key, 0, b, deg_inter, hub_inter, &flags[f], prev, s);
-          if (with_jump) jump(n, key, &flags[f], s);
-        }
-        int h_flags[8];
-        KC_HIP(hipMemcpyAsync(h_flags, &flags[flag_base], batch * sizeof(int), hipMemcpyDeviceToHost, s));
-        KC_HIP(hipStreamSynchronize(s));
-        uint32_t i = 0;
-        while (i < batch && h_flags[i] != 0) ++i;
-        sweeps += i < batch ? i + 1 : batch;
-        flag_base += batch;
-        if (i < batch) break;
+      if (o.variant == KC_VARIANT_SHORTCUT) {
+        // union-find, as kc_find_components runs this variant (the forest in the keys' place)
+        uint32_t *parent = reinterpret_cast<uint32_t *>(key);
+        union_components(n, m2, offsets, targets, 0, parent, s);
+        union_labels(n, parent, labels, small + 4, partial, s);
+        sweeps = 1;
+      } else {
+        sweeps = propagate(n, offsets, targets, o, base, labels, s);
       }
-      labels_from_keys(n, key, labels, small + 4, partial, s);
       KC_HIP(hipMemcpyAsync(&components, small + 4, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
       KC_HIP(hipStreamSynchronize(s));
     }

@@ -1,0 +1,300 @@
+// Connected components by lock-free union-find: the base case of the
+// contraction (RunSequentialCC, lib/components/exponential_contraction.h:
+// 908-922), the shortcuts variant and the components inside the blocks of the
+// pre-contraction.
+//
+// parent[v] <= v always; a root is its own parent, and only roots are hooked,
+// under a smaller root, by compare-and-swap.  So the forest has no cycles and
+// a finished tree's root is its component's smallest index.  Any parent value
+// ever read stays an ancestor, so loads may be stale (the chiplets' L2s are
+// not coherent within a launch): a hook with a stale root fails and returns
+// the current parent, from which the search goes on downward.
+//
+// A few passes over the edges replace min-label sweeps with a pointer jump
+// after each, whose number grows with the diameter (2D grid 1500 x 1100, p =
+// 0.6: 62 sweeps and jumps, 2.0 ms; now 0.21 ms).  What bounds it: the random
+// parent reads and one device atomic per successful hook.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "kc_common.h"
+#include "kernels.h"
+
+namespace kc {
+
+namespace {
+
+constexpr int kLinkSlots = 512;    // edge slots of one wave: every wave the same work, whatever the rows' lengths
+constexpr uint32_t kFirstNeighbours = 4;
+constexpr int kShortenHops = 32;
+constexpr uint64_t kShortenTwiceMin = 1u << 16;
+constexpr uint32_t kUnionCountBlocks = 2048;
+
+// Indices [lo, hi) whose edges count for v: its block of consecutive indices,
+// or everything.
+__device__ __forceinline__ bool same_block(uint32_t u, uint32_t v, uint64_t block) {
+  return block == 0 || u / block == v / block;
+}
+
+// parent[v] = the smallest of v and its first few neighbours: no cycle (every
+// parent is at most its child) and no atomic, and it leaves far fewer trees.
+__global__ __launch_bounds__(kBlock) void k_union_init(uint64_t n, const uint64_t *off, const uint32_t *col,
+                                                      uint64_t block, uint32_t *parent) {
+  const uint64_t v = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
+  if (v >= n) return;
+  const uint32_t self = static_cast<uint32_t>(v);
+  const uint64_t e0 = off[v], len = off[v + 1] - e0;
+  uint32_t p = self;
+  uint32_t c[kFirstNeighbours];
+#pragma unroll
+  for (uint32_t j = 0; j < kFirstNeighbours; ++j) c[j] = j < len ? col[e0 + j] : self;
+#pragma unroll
+  for (uint32_t j = 0; j < kFirstNeighbours; ++j)
+    if (c[j] < p && same_block(c[j], self, block)) p = c[j];
+  parent[v] = p;
+}
+
+// Every vertex jumps up to kShortenHops ancestors: a chain of d edges shrinks
+// to about d / kShortenHops, or less where other vertices' jumps are seen.
+__global__ __launch_bounds__(kBlock) void k_union_shorten(uint64_t n, uint32_t *parent) {
+  const uint64_t v = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
+  if (v >= n) return;
+  const uint32_t first = parent[v];
+  uint32_t p = first;
+  for (int h = 0; h < kShortenHops; ++h) {
+    const uint32_t q = parent[p];
+    if (q == p) break;
+    p = q;
+  }
+  if (p != first) parent[v] = p;
+}
+
+// Root of v; every vertex passed is pointed at its grandparent.
+__device__ __forceinline__ uint32_t find_root(uint32_t *parent, uint32_t v) {
+  uint32_t cur = parent[v];
+  if (cur == v) return cur;
+  uint32_t prev = v, next;
+  while (cur > (next = parent[cur])) {
+    parent[prev] = next;
+    prev = cur;
+    cur = next;
+  }
+  return cur;
+}
+
+__device__ __forceinline__ void link(uint32_t *parent, uint32_t u, uint32_t w) {
+  uint32_t a = find_root(parent, u), b = find_root(parent, w);
+  while (a != b) {
+    const uint32_t hi = a > b ? a : b, lo = a > b ? b : a;
+    const uint32_t old = atomicCAS(&parent[hi], hi, lo);
+    if (old == hi) break;
+    a = find_root(parent, old);  // hi was hooked meanwhile: old < hi
+    b = lo;
+  }
+}
+
+// The last row r with off[r] <= e (off[0] <= e < off[n]), 64 probes a step.
+__device__ __forceinline__ uint64_t row_of_slot(const uint64_t *off, uint64_t n, uint64_t e) {
+  uint64_t lo = 0, hi = n;
+  while (hi - lo > 1) {
+    const uint64_t step = (hi - lo + kWave - 1) / kWave;
+    const uint64_t p = lo + (lane_id() + 1) * step;
+    const uint64_t below = __popcll(__ballot(p < hi && off[p] <= e));
+    lo += below * step;
+    hi = lo + step < hi ? lo + step : hi;
+  }
+  return lo;
+}
+
+// Hooks the larger of the two ends' parents under the smaller one without a
+// search: trees that are stars (or nearly) merge in one step each.  Where the
+// larger is no root any more its link is replaced; every edge is linked again
+// by the last pass, so nothing is lost.
+__device__ __forceinline__ void hook(uint32_t *parent, uint32_t u, uint32_t w) {
+  const uint32_t a = parent[u], b = parent[w];
+  if (a == b) return;
+  const uint32_t hi = a > b ? a : b, lo = a > b ? b : a;
+  if (parent[hi] > lo) atomicMin(&parent[hi], lo);
+}
+
+// Links (or, with kHook, hooks) the two ends of every edge, from its larger
+// end's row.  A wave takes
+// kLinkSlots consecutive slots: it searches its first and last row, marks the
+// rows' first slots in LDS and spreads the marks by a running maximum; where
+// the range spans many empty rows, each lane searches its slot's row instead.
+template <bool kHook>
+__global__ __launch_bounds__(kBlock) void k_union_link(uint64_t n, uint64_t m2, const uint64_t *off,
+                                                      const uint32_t *col, uint64_t block, uint32_t *parent) {
+  __shared__ uint32_t row_lds[kBlock / kWave][kLinkSlots];
+  uint32_t *row = row_lds[threadIdx.x / kWave];
+  const uint32_t ln = lane_id();
+  const uint64_t c0 = (blockIdx.x * static_cast<uint64_t>(kBlock / kWave) + threadIdx.x / kWave) * kLinkSlots;
+  if (c0 >= m2) return;
+  const uint64_t c1 = c0 + kLinkSlots < m2 ? c0 + kLinkSlots : m2;
+  const uint64_t r0 = row_of_slot(off, n, c0), r1 = row_of_slot(off, n, c1 - 1);
+  constexpr uint32_t kPerLane = kLinkSlots / kWave;
+  const bool marked = r1 - r0 <= 4 * kLinkSlots;
+  if (marked) {
+    for (uint32_t j = ln; j < kLinkSlots; j += kWave) row[j] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (uint64_t r = r0 + 1 + ln; r <= r1; r += kWave) {  // non-empty rows start at distinct slots
+      const uint64_t s = off[r];
+      if (off[r + 1] > s) row[s - c0] = static_cast<uint32_t>(r - r0);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    uint32_t m[kPerLane], run = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kPerLane; ++j) {
+      const uint32_t x = row[ln * kPerLane + j];
+      run = x > run ? x : run;
+      m[j] = run;
+    }
+    uint32_t inc = run;
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t t = static_cast<uint32_t>(__shfl_up(static_cast<int>(inc), o));
+      if (ln >= static_cast<uint32_t>(o) && t > inc) inc = t;
+    }
+    uint32_t before = static_cast<uint32_t>(__shfl_up(static_cast<int>(inc), 1));
+    if (ln == 0) before = 0;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (uint32_t j = 0; j < kPerLane; ++j) row[ln * kPerLane + j] = m[j] > before ? m[j] : before;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  uint32_t w[kPerLane];
+#pragma unroll
+  for (uint32_t j = 0; j < kPerLane; ++j) {
+    const uint64_t e = c0 + j * kWave + ln;
+    w[j] = e < c1 ? col[e] : kNone;
+  }
+#pragma unroll
+  for (uint32_t j = 0; j < kPerLane; ++j) {
+    const uint64_t e = c0 + j * kWave + ln;
+    if (e >= c1) continue;
+    uint64_t u;
+    if (marked) {
+      u = r0 + row[j * kWave + ln];
+    } else {
+      uint64_t lo = r0, hi = r1 + 1;
+      while (hi - lo > 1) {
+        const uint64_t mid = lo + (hi - lo) / 2;
+        if (off[mid] <= e)
+          lo = mid;
+        else
+          hi = mid;
+      }
+      u = lo;
+    }
+    const uint32_t v = static_cast<uint32_t>(u);
+    if (w[j] < v && same_block(w[j], v, block)) {
+      if (kHook)
+        hook(parent, v, w[j]);
+      else
+        link(parent, v, w[j]);
+    }
+  }
+}
+
+__device__ __forceinline__ uint32_t root_of(const uint32_t *parent, uint64_t v) {
+  uint32_t p = parent[v], q;
+  while ((q = parent[p]) != p) p = q;
+  return p;
+}
+
+__global__ __launch_bounds__(kBlock) void k_union_reps(uint64_t n, const uint32_t *parent, const uint32_t *gid,
+                                                      uint32_t *rep) {
+  const uint64_t v = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
+  if (v >= n) return;
+  const uint32_t r = root_of(parent, v);
+  rep[v] = gid ? gid[r] : r;
+}
+
+__global__ __launch_bounds__(kBlock) void k_union_keys(uint64_t n, const uint32_t *parent, uint64_t *key) {
+  const uint64_t v = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
+  if (v < n) key[v] = root_of(parent, v);
+}
+
+__global__ __launch_bounds__(kBlock) void k_union_labels(uint64_t n, const uint32_t *parent, uint32_t *labels,
+                                                        uint32_t *partial) {
+  __shared__ uint32_t wc[kBlock / kWave];
+  uint32_t roots = 0;
+  for (uint64_t v = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x; v < n;
+       v += static_cast<uint64_t>(gridDim.x) * kBlock) {
+    const uint32_t r = root_of(parent, v);
+    labels[v] = r;
+    roots += r == static_cast<uint32_t>(v);
+  }
+  roots = group_sum_u32(roots, kWave);
+  if (lane_id() == 0) wc[threadIdx.x / kWave] = roots;
+  __syncthreads();
+  if (threadIdx.x == 0) partial[blockIdx.x] = wc[0] + wc[1] + wc[2] + wc[3];
+}
+
+unsigned blocks_for(uint64_t n) { return static_cast<unsigned>(ceil_div(n, static_cast<uint64_t>(kBlock))); }
+
+void shorten(uint64_t n, uint32_t *parent, hipStream_t s) {
+  // (a path of 2^20 vertices in index order is the worst case: two passes
+  // before the links and two after leave about a thousand hops to the search)
+  for (int pass = 0; pass < (n >= kShortenTwiceMin ? 2 : 1); ++pass) {
+    hipLaunchKernelGGL(k_union_shorten, dim3(blocks_for(n)), dim3(kBlock), 0, s, n, parent);
+    KC_LAUNCH_CHECK();
+  }
+}
+
+// Rounds of hooks before the links.  The links of many neighbouring trees wait
+// for one another along chains of roots (2D grid 1500 x 1100, p = 0.6: 940 us
+// in all with no hooks, 641, 692, 214 and 236 with 1 to 4 rounds; G(n, 3n) of
+// 200 K vertices: 787, 970, 143, 156); small graphs are done sooner without
+// (10 K vertices: 56 against 63 us), and on dense ones the first neighbours'
+// minima have left few trees (R-MAT 20, 30 slots a vertex: 330, 392, 516 us).
+int hook_rounds(uint64_t n, uint64_t m2) {
+  if (n < (1u << 14) || m2 > 16 * n) return 0;
+  return n < (1u << 20) ? 2 : 3;
+}
+
+}  // namespace
+
+void union_components(uint64_t n, uint64_t m2, const uint64_t *off, const uint32_t *col, uint64_t block,
+                      uint32_t *parent, hipStream_t s) {
+  if (!n) return;
+  hipLaunchKernelGGL(k_union_init, dim3(blocks_for(n)), dim3(kBlock), 0, s, n, off, col, block, parent);
+  KC_LAUNCH_CHECK();
+  if (!m2) return;
+  const unsigned g = static_cast<unsigned>(ceil_div(m2, static_cast<uint64_t>(kLinkSlots) * (kBlock / kWave)));
+  shorten(n, parent, s);
+  for (int r = 0; r < hook_rounds(n, m2); ++r) {
+    hipLaunchKernelGGL(k_union_link<true>, dim3(g), dim3(kBlock), 0, s, n, m2, off, col, block, parent);
+    KC_LAUNCH_CHECK();
+    shorten(n, parent, s);
+  }
+  hipLaunchKernelGGL(k_union_link<false>, dim3(g), dim3(kBlock), 0, s, n, m2, off, col, block, parent);
+  KC_LAUNCH_CHECK();
+  shorten(n, parent, s);
+}
+
+void union_reps(uint64_t n, const uint32_t *parent, const uint32_t *gid, uint32_t *rep, hipStream_t s) {
+  if (!n) return;
+  hipLaunchKernelGGL(k_union_reps, dim3(blocks_for(n)), dim3(kBlock), 0, s, n, parent, gid, rep);
+  KC_LAUNCH_CHECK();
+}
+
+void union_keys(uint64_t n, const uint32_t *parent, uint64_t *key, hipStream_t s) {
+  if (!n) return;
+  hipLaunchKernelGGL(k_union_keys, dim3(blocks_for(n)), dim3(kBlock), 0, s, n, parent, key);
+  KC_LAUNCH_CHECK();
+}
+
+void union_labels(uint64_t n, const uint32_t *parent, uint32_t *labels, uint32_t *roots, uint32_t *partial,
+                  hipStream_t s) {
+  if (!n) return;
+  const unsigned g = std::min(blocks_for(n), kUnionCountBlocks);
+  hipLaunchKernelGGL(k_union_labels, dim3(g), dim3(kBlock), 0, s, n, parent, labels, partial);
+  KC_LAUNCH_CHECK();
+  sum_partials_u32(partial, g, roots, s);
+}
+
+}  // namespace kc
