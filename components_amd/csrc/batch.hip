@@ -415,6 +415,283 @@ __global__ __launch_bounds__(B) void k_batch(BatchDev d) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Graphs whose keys and edges fit one workgroup's LDS: the whole level loop
+// runs there, one workgroup per graph; HBM is read once (rows) and written
+// once (labels).  The edges are a list of index pairs, each undirected edge
+// once, so a pass over them has no rows, no offsets and no long-row case:
+// lane i takes edge i, reads both keys from LDS and lowers the larger by an
+// LDS atomic.  Keys are packed (distance << LB | label, LB = log2 CapN) in 32
+// bits.  Contraction rewrites the pairs in place with the clusters' new
+// indices; repeats are dropped only where a direct-mapped filter meets them
+// (a repeated edge changes no key, label or level).  What bounds it: LDS
+// accesses and the barriers between the phases; the general kernel above pays
+// a chain of L2 or HBM round trips per phase instead (4096 graphs of 2^8 to
+// 2^12 vertices: 4.53 ms, here 0.81).
+template <int B, uint32_t CapN, uint32_t CapE>
+struct LdsGraph {
+  uint32_t key[CapN];  // packed keys; the filter while the edges contract
+  uint32_t edge[CapE ? CapE : 1];
+  uint16_t cur[CapN];   // per input vertex: its level index, or kLdsDone | its last centre's input id
+  uint16_t gid[CapN];   // per level index: the input id
+  uint16_t nidx[CapN];  // per level index: the next level's index of its cluster (kLdsNone: none)
+  uint64_t wave[B / 64];
+  uint64_t carry;
+  uint32_t count, radius;
+};
+constexpr uint16_t kLdsDone = 0x8000, kLdsNone = 0xFFFF;
+constexpr uint32_t kLdsLongRow = 64;  // longer rows are read by the whole workgroup
+
+constexpr uint32_t log2_of(uint32_t x) { return x <= 1 ? 0 : 1 + log2_of(x / 2); }
+
+template <int B, uint32_t CapN, uint32_t CapE>
+__global__ __launch_bounds__(B) void k_batch_lds(BatchDev d, const uint32_t *order) {
+  constexpr uint32_t LB = log2_of(CapN), kMask = CapN - 1, kHop = 1u << LB;
+  constexpr int kPer = CapN / B;  // level indices per thread
+  constexpr int kTile = 8;        // edges per thread and compaction step
+  static_assert((CapN & kMask) == 0 && CapN <= kLdsDone && CapN % B == 0, "16-bit ids");
+  __shared__ LdsGraph<B, CapN, CapE> s;
+  const BatchParams p = *d.params;
+  const uint32_t tid = threadIdx.x, g = order[blockIdx.x];
+  uint32_t *edge = s.edge;
+  if (CapE == 0) edge = d.lcol[0] + d.edge_off[g];
+  const uint64_t v0 = d.vtx_off[g];
+  const uint32_t n0 = static_cast<uint32_t>(d.vtx_off[g + 1] - v0);
+  const uint32_t rng_offset = d.nonisolated[g];
+  uint32_t *labels = d.labels + v0;
+  if (rng_offset == 0) {  // no edge: every vertex is its own component, no level runs
+    for (uint32_t v = tid; v < n0; v += B) labels[v] = v;
+    if (tid == 0) {
+      d.glevels[g] = 0;
+      d.gsweeps[g] = 0;
+      d.gradius[g] = 0;
+      d.gstatus[g] = 0;
+      d.gcomp[g] = n0;
+    }
+    return;
+  }
+  // edges (v, w) with v < w, in no particular order
+  {
+    const uint64_t *off = d.off + v0;
+    const uint32_t *col = d.col;
+    if (tid == 0) s.count = s.radius = 0;
+    __syncthreads();
+    uint64_t e0[kPer];
+    uint32_t len[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const uint32_t v = tid + j * B;
+      e0[j] = v < n0 ? off[v] : 0;
+      len[j] = v < n0 ? static_cast<uint32_t>(off[v + 1] - e0[j]) : 0u;
+    }
+    uint32_t longest = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      if (len[j] > kLdsLongRow) {
+        s.nidx[atomicAdd(&s.radius, 1u)] = static_cast<uint16_t>(tid + j * B);
+        len[j] = 0;
+      }
+      longest = len[j] > longest ? len[j] : longest;
+    }
+    for (uint32_t i = 0; i < longest; i += 4) {
+      uint32_t w[kPer][4];
+#pragma unroll
+      for (int j = 0; j < kPer; ++j)
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) w[j][u] = i + u < len[j] ? col[e0[j] + i + u] : 0u;
+#pragma unroll
+      for (int j = 0; j < kPer; ++j) {
+        const uint32_t v = tid + j * B;
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u)
+          if (w[j][u] > v && i + u < len[j]) edge[atomicAdd(&s.count, 1u)] = v | (w[j][u] << 16);
+      }
+    }
+    __syncthreads();
+    const uint32_t n_long = s.radius;
+    for (uint32_t r = 0; r < n_long; ++r) {
+      const uint32_t v = s.nidx[r];
+      const uint64_t a = off[v];
+      const uint32_t n = static_cast<uint32_t>(off[v + 1] - a);
+      for (uint32_t i = tid; i < n; i += B) {
+        const uint32_t w = col[a + i];
+        if (w > v) edge[atomicAdd(&s.count, 1u)] = v | (w << 16);
+      }
+    }
+    for (uint32_t v = tid; v < n0; v += B) {
+      s.cur[v] = static_cast<uint16_t>(v);
+      s.gid[v] = static_cast<uint16_t>(v);
+    }
+    __syncthreads();
+  }
+  uint32_t nl = n0, ne = s.count;
+  uint32_t iteration = 1, levels = 0, sweeps = 0, radius_sum = 0, status = 0;
+  bool level0 = true;
+  while (true) {
+    if (levels >= p.max_levels) {
+      status = kStatusLevels;
+      break;
+    }
+    if (tid == 0) s.radius = 0;
+    for (uint32_t v = tid; v < nl; v += B) {
+      const uint32_t dev =
+          exp_deviate(s.gid[v], p.seed, iteration, rng_offset, p.fused != 0, p.stream, p.table, p.k_max);
+      s.key[v] = (dev << LB) | v;
+    }
+    __syncthreads();
+    bool first_change = false;
+    for (uint32_t pass = 0;; ++pass) {
+      bool changed = false;
+      for (uint32_t i0 = tid; i0 < ne; i0 += 4 * B) {
+        uint32_t e[4], ku[4], kw[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) e[j] = i0 + j * B < ne ? edge[i0 + j * B] : 0u;  // (0, 0): no change
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          ku[j] = s.key[e[j] & 0xFFFFu];
+          kw[j] = s.key[e[j] >> 16];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (ku[j] + kHop < kw[j]) {
+            atomicMin(&s.key[e[j] >> 16], ku[j] + kHop);
+            changed = true;
+          } else if (kw[j] + kHop < ku[j]) {
+            atomicMin(&s.key[e[j] & 0xFFFFu], kw[j] + kHop);
+            changed = true;
+          }
+        }
+      }
+      ++sweeps;
+      const bool any = __syncthreads_or(changed) != 0;
+      if (pass == 0) first_change = any;
+      if (!any) break;
+    }
+    ++levels;
+    if (!first_change && (!level0 || rng_offset == n0)) {  // stall, as in contract_graph
+      ++iteration;
+      continue;
+    }
+    uint32_t r = 0;
+    for (uint32_t v = tid; v < nl; v += B) {
+      const uint32_t k = s.key[v];
+      const uint32_t h = (k >> LB) - (s.key[k & kMask] >> LB);
+      r = h > r ? h : r;
+      s.nidx[v] = 0;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      const uint32_t t = static_cast<uint32_t>(__shfl_xor(static_cast<int>(r), o));
+      r = t > r ? t : r;
+    }
+    if ((tid & 63) == 0 && r) atomicMax(&s.radius, r);
+    __syncthreads();
+    radius_sum += s.radius;
+    // edges between clusters, as label pairs (smaller label first); their centres marked
+    for (uint32_t i = tid; i < ne; i += B) {
+      const uint32_t e = edge[i];
+      const uint32_t a = s.key[e & 0xFFFFu] & kMask, b = s.key[e >> 16] & kMask;
+      if (a != b) {
+        s.nidx[a] = 1;
+        s.nidx[b] = 1;
+      }
+      edge[i] = a == b ? kNone : a < b ? a | (b << 16) : b | (a << 16);
+    }
+    __syncthreads();
+    // next-level indices in label order: each thread numbers kPer consecutive labels
+    uint32_t used = 0, moved[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const uint32_t a = tid * kPer + j;
+      moved[j] = a < nl && s.nidx[a] ? s.gid[a] : kNone;
+      used += moved[j] != kNone;
+    }
+    if (tid == 0) s.carry = 0;
+    uint64_t n_next64 = 0;
+    __syncthreads();
+    uint32_t next = static_cast<uint32_t>(block_scan<B>(used, s.wave, s.carry, n_next64));
+    const uint32_t first = next;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const uint32_t a = tid * kPer + j;
+      if (a < nl) s.nidx[a] = moved[j] != kNone ? static_cast<uint16_t>(next++) : kLdsNone;
+    }
+    __syncthreads();
+    for (uint32_t v = tid; v < n0; v += B) {
+      const uint32_t c = s.cur[v];
+      if (c & kLdsDone) continue;
+      const uint32_t a = s.key[c] & kMask;
+      const uint16_t ni = s.nidx[a];
+      s.cur[v] = ni != kLdsNone ? ni : static_cast<uint16_t>(kLdsDone | s.gid[a]);
+    }
+    __syncthreads();
+    const uint32_t n_next = static_cast<uint32_t>(n_next64);
+    if (n_next == 0) break;
+    next = first;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j)
+      if (moved[j] != kNone) s.gid[next++] = static_cast<uint16_t>(moved[j]);
+    // the pairs renumbered and moved to the front, a step's edges in registers
+    // before any is written (a step never writes past its own last edge)
+    for (uint32_t j = tid; j < CapN; j += B) s.key[j] = kNone;
+    if (tid == 0) s.carry = 0;
+    __syncthreads();
+    for (uint32_t base = 0; base < ne; base += kTile * B) {
+      uint32_t x[kTile], kept = 0;
+#pragma unroll
+      for (int j = 0; j < kTile; ++j) {
+        const uint32_t i = base + j * B + tid;
+        x[j] = i < ne ? edge[i] : kNone;
+      }
+#pragma unroll
+      for (int j = 0; j < kTile; ++j) {
+        if (x[j] == kNone) continue;
+        x[j] = s.nidx[x[j] & 0xFFFFu] | (static_cast<uint32_t>(s.nidx[x[j] >> 16]) << 16);
+        uint32_t *slot = &s.key[(x[j] * 0x9E3779B1u) >> (32 - LB)];
+        const uint32_t seen = *slot;
+        // the slot's last claimant keeps its edge: of equal edges one always does
+        if (seen == x[j] || atomicCAS(slot, seen, x[j]) == x[j]) x[j] = kNone;
+        kept += x[j] != kNone;
+      }
+      uint64_t total = 0;
+      uint32_t at = static_cast<uint32_t>(block_scan<B>(kept, s.wave, s.carry, total));
+#pragma unroll
+      for (int j = 0; j < kTile; ++j)
+        if (x[j] != kNone) edge[at++] = x[j];
+      __syncthreads();  // s.carry is read by the next step
+    }
+    ne = static_cast<uint32_t>(s.carry);
+    nl = n_next;
+    level0 = false;
+    ++iteration;
+    __syncthreads();
+  }
+  if (status) {
+    for (uint32_t v = tid; v < n0; v += B) labels[v] = kNone;
+  } else {
+    // canonical: minimum input id per final centre
+    for (uint32_t v = tid; v < n0; v += B) s.key[v] = kNone;
+    if (tid == 0) s.count = 0;
+    __syncthreads();
+    for (uint32_t v = tid; v < n0; v += B) atomicMin(&s.key[s.cur[v] & (kLdsDone - 1)], v);
+    __syncthreads();
+    uint32_t roots = 0;
+    for (uint32_t v = tid; v < n0; v += B) {
+      const uint32_t l = s.key[s.cur[v] & (kLdsDone - 1)];
+      labels[v] = l;
+      roots += l == v;
+    }
+    if (roots) atomicAdd(&s.count, roots);
+    __syncthreads();
+  }
+  if (tid == 0) {
+    d.gcomp[g] = status ? 0 : s.count;
+    d.glevels[g] = levels;
+    d.gsweeps[g] = sweeps;
+    d.gradius[g] = radius_sum;
+    d.gstatus[g] = status;
+  }
+}
+
 // Clears the hash sets of graphs that stopped early (their tables may hold
 // entries) -- launched only after a run reported a non-zero status.
 __global__ void k_table_clear(uint64_t n, uint64_t *tab) {
@@ -533,6 +810,30 @@ void batch_launch(int block, uint32_t grid, const BatchDev &d, hipStream_t s) {
   KC_LAUNCH_CHECK();
 }
 
+// Size classes of the LDS kernel: (threads, vertices, undirected edges).  The
+// LDS of one class is what bounds its workgroups per CU: 6, 2, 1 and 2
+// (the last streams its edges: any number).
+struct LdsClass {
+  uint32_t n, edges;
+};
+constexpr int kLdsClasses = 4;
+constexpr LdsClass kLdsClass[kLdsClasses] = {{1024, 4096}, {2048, 12288}, {4096, 30592}, {8192, ~0u}};
+// packed keys: the distances (at most k_max + 1) and 13 label bits share 32
+constexpr uint32_t kLdsMaxDeviate = (1u << 19) - 2;
+
+void batch_lds_launch(int cls, uint32_t count, const uint32_t *order, const BatchDev &d, hipStream_t s) {
+  if (!count) return;
+  if (cls == 0)
+    hipLaunchKernelGGL((k_batch_lds<256, kLdsClass[0].n, kLdsClass[0].edges>), dim3(count), dim3(256), 0, s, d, order);
+  else if (cls == 1)
+    hipLaunchKernelGGL((k_batch_lds<512, kLdsClass[1].n, kLdsClass[1].edges>), dim3(count), dim3(512), 0, s, d, order);
+  else if (cls == 2)
+    hipLaunchKernelGGL((k_batch_lds<1024, kLdsClass[2].n, kLdsClass[2].edges>), dim3(count), dim3(1024), 0, s, d, order);
+  else
+    hipLaunchKernelGGL((k_batch_lds<1024, kLdsClass[3].n, 0>), dim3(count), dim3(1024), 0, s, d, order);
+  KC_LAUNCH_CHECK();
+}
+
 void batch_table_clear(uint64_t n, uint64_t *tab, hipStream_t s) {
   if (!n) return;
   const uint64_t g = std::min<uint64_t>(ceil_div(n, kBlock), 65536);
@@ -553,11 +854,15 @@ struct kc_batch {
   uint64_t n = 0, m2 = 0;
   int cus = 0;
   std::vector<uint64_t> h_vtx_off, h_edge_off;
+  std::vector<uint64_t> h_up;  // per graph: slots whose target is above their row (its edges, once each)
   std::vector<void *> owned;
   uint32_t *order_d = nullptr;
   // graphs above the split size go through the device-wide path as one union
   bool split_valid = false;
   uint32_t split_built = 0;
+  bool lds_built = false;
+  // order_d: the general kernel's queue, then each LDS class's graphs
+  uint32_t lds_at[kLdsClasses] = {}, lds_count[kLdsClasses] = {};
   kc_graph *big = nullptr;
   uint32_t n_big = 0;
   uint64_t n_union = 0, m2_union = 0;
@@ -634,22 +939,38 @@ void batch_params(kc_batch *b, const kc_options &o) {
 }
 
 // Routes the graphs with more than `split` vertices (none when 0) to the
-// device-wide path: the persistent kernel's queue gets the others, largest
-// first, and the large ones are copied into one union handle.
+// device-wide path; of the others, those that fit an LDS class go to the
+// smallest one (4096 graphs of 2^8 to 2^12 vertices: 4.5 -> 0.81 ms),
+// the rest to the persistent kernel's queue, each list largest first.  The
+// large ones are copied into one union handle.
 void prepare_split(kc_batch *b, uint32_t split) {
-  if (b->split_valid && b->split_built == split) return;
+  const bool lds = b->table_k <= kLdsMaxDeviate;
+  if (b->split_valid && b->split_built == split && b->lds_built == lds) return;
   b->split_valid = false;
-  std::vector<uint32_t> small, bigs;
+  std::vector<uint32_t> small, bigs, fits[kLdsClasses];
   for (uint32_t g = 0; g < b->graphs; ++g) {
     const uint64_t ng = b->h_vtx_off[g + 1] - b->h_vtx_off[g];
-    (split && ng > split ? bigs : small).push_back(g);
+    int cls = 0;
+    while (cls < kLdsClasses && (ng > kLdsClass[cls].n || b->h_up[g] > kLdsClass[cls].edges)) ++cls;
+    (split && ng > split ? bigs : lds && cls < kLdsClasses ? fits[cls] : small).push_back(g);
   }
-  std::stable_sort(small.begin(), small.end(), [&](uint32_t x, uint32_t y) {
+  const auto larger = [&](uint32_t x, uint32_t y) {
     return b->h_edge_off[x + 1] - b->h_edge_off[x] > b->h_edge_off[y + 1] - b->h_edge_off[y];
-  });
+  };
+  std::stable_sort(small.begin(), small.end(), larger);
+  b->dev.queued = static_cast<uint32_t>(small.size());
+  for (int cls = 0; cls < kLdsClasses; ++cls) {
+    std::stable_sort(fits[cls].begin(), fits[cls].end(), larger);
+    b->lds_at[cls] = static_cast<uint32_t>(small.size());
+    b->lds_count[cls] = static_cast<uint32_t>(fits[cls].size());
+    small.insert(small.end(), fits[cls].begin(), fits[cls].end());
+  }
   KC_HIP(hipStreamSynchronize(b->stream));  // the old queue order may still be read
   if (!small.empty()) KC_HIP(hipMemcpy(b->order_d, small.data(), 4ull * small.size(), hipMemcpyHostToDevice));
-  b->dev.queued = static_cast<uint32_t>(small.size());
+  if (b->exec) {  // its launches hold the old counts
+    KC_HIP(hipGraphExecDestroy(b->exec));
+    b->exec = nullptr;
+  }
   if (b->big) {
     (void)kc_graph_destroy(b->big);
     b->big = nullptr;
@@ -685,19 +1006,25 @@ void prepare_split(kc_batch *b, uint32_t split) {
     graph_device_finish(b->big);
   }
   b->split_built = split;
+  b->lds_built = lds;
   b->split_valid = true;
 }
 
 void enqueue(kc_batch *b, const kc_batch_tuning &t) {
-  fill_u32(b->queue, 1, 0, b->stream);
-  const uint32_t grid = static_cast<uint32_t>(b->cus) * static_cast<uint32_t>(t.groups_per_cu);
-  batch_launch(t.block, grid, b->dev, b->stream);
+  if (b->dev.queued) {
+    fill_u32(b->queue, 1, 0, b->stream);
+    const uint32_t grid = static_cast<uint32_t>(b->cus) * static_cast<uint32_t>(t.groups_per_cu);
+    batch_launch(t.block, grid, b->dev, b->stream);
+  }
+  for (int cls = kLdsClasses - 1; cls >= 0; --cls)
+    batch_lds_launch(cls, b->lds_count[cls], b->order_d + b->lds_at[cls], b->dev, b->stream);
 }
 
 // One run on the current parameters: eager launches, or the captured graph
 // (captured again when the launch shape changed).
 void launch(kc_batch *b) {
   const kc_batch_tuning &t = b->tuning;
+  if (b->n_big == b->graphs) return;  // nothing but the union
   if (!t.use_graph) {
     enqueue(b, t);
     return;
@@ -790,6 +1117,7 @@ int kc_batch_create(const kc_batch_host *h, kc_batch **out) {
     if (m2 && !h->targets) fail(KC_ERR_INVALID, "null batch targets");
     if (n >= (1ull << 40)) fail(KC_ERR_INVALID, "batch too large");
     std::vector<uint32_t> noniso(G);
+    std::vector<uint64_t> up(G, 0);
     std::vector<uint64_t> toff(G + 1, 0);
     for (uint32_t g = 0; g < G; ++g) {
       const uint64_t a = h->vtx_off[g], z = h->vtx_off[g + 1];
@@ -801,14 +1129,18 @@ int kc_batch_create(const kc_batch_host *h, kc_batch **out) {
       if (h->edge_off[g + 1] < h->edge_off[g] || slots >= (1ull << 31))
         fail(KC_ERR_INVALID, "batch: graph %u needs fewer than 2^31 edge slots", g);
       uint32_t ni = 0;
+      uint64_t nu = 0;
       for (uint64_t v = a; v < z; ++v) {
         if (h->offsets[v + 1] < h->offsets[v]) fail(KC_ERR_INVALID, "batch: offsets not monotone at vertex %llu", (unsigned long long)v);
         ni += h->offsets[v + 1] > h->offsets[v];
-        for (uint64_t e = h->offsets[v]; e < h->offsets[v + 1]; ++e)
+        for (uint64_t e = h->offsets[v]; e < h->offsets[v + 1]; ++e) {
           if (h->targets[e] >= z - a)
             fail(KC_ERR_INVALID, "batch: target %u out of range in graph %u", h->targets[e], g);
+          nu += h->targets[e] > v - a;
+        }
       }
       noniso[g] = ni;
+      up[g] = nu;
       uint64_t tw = 64;
       while (tw < 2 * slots) tw <<= 1;
       toff[g + 1] = toff[g] + tw;
@@ -837,6 +1169,7 @@ int kc_batch_create(const kc_batch_host *h, kc_batch **out) {
     b->m2 = m2;
     b->h_vtx_off.assign(h->vtx_off, h->vtx_off + G + 1);
     b->h_edge_off.assign(h->edge_off, h->edge_off + G + 1);
+    b->h_up = std::move(up);
     BatchDev &d = b->dev;
     d.graphs = G;
     uint32_t *order_d = b->dalloc<uint32_t>(G);

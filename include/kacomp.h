@@ -382,9 +382,11 @@ typedef struct kc_batch_gen_params {
 
 /* Launch shape of the persistent kernel: threads per workgroup (256, 512 or
  * 1024), workgroups per compute unit, and whether the launch sequence replays
- * a captured HIP graph.  Every row of a graph is processed by one lane, so the
- * batched form suits bounded-degree graphs; heavy-tailed graphs belong on the
- * plain path (kc_find_components), whose degree bins split long rows. */
+ * a captured HIP graph.  Graphs of up to 8192 vertices run in workgroups of
+ * their own size class instead, with their keys in LDS, whatever the shape.
+ * In the persistent kernel every row of a graph is processed by one lane, so it
+ * suits bounded-degree graphs; large heavy-tailed graphs belong on the plain
+ * path (kc_find_components), whose degree bins split long rows. */
 typedef struct kc_batch_tuning {
   int32_t block;
   int32_t groups_per_cu;
