@@ -264,7 +264,9 @@ struct kc_graph {
   uint64_t *d_huge_info = nullptr;
   uint64_t huge_info_cap = 0;
   int *flags = nullptr;
-  uint32_t *small = nullptr;  // [0..3] bin counters, [4] radius, [5] roots, [6] hubs found, [7] packed keys do not fit
+  // [0..3] bin counters, [4] radius, [5] roots, [6] hubs found, [7] packed keys do not fit, [8] edges of
+  // the tail, [9..12] its status, levels, sweeps, radius sum
+  uint32_t *small = nullptr;
   uint64_t *sizes = nullptr;  // [0] n_next [1] P [2] m2_next [3..5] dedup counters [8] N [9] clusters
   // pinned host mirrors
   uint64_t *h_sizes = nullptr;
@@ -779,6 +781,7 @@ struct RunOut {
   uint32_t levels = 0;
   uint64_t replicas = 0;
   uint32_t hubs = 0;
+  bool tail = false;  // the last levels ran in one workgroup: their figures come with the final word
 };
 
 // Level 0 with its hubs split into proxies (kc_options.replicate): the
@@ -900,13 +903,26 @@ bool build_replicated(kc_graph *g, const kc_options *o, uint64_t n0, uint64_t m2
 }
 
 // Exponential (or local) contraction down to an edgeless graph or the base case.
-void run_contraction(kc_graph *g, const kc_options *o, RunOut &out) {
+// Levels whose rest runs in one workgroup.  A pass over the edges takes one CU
+// about 0.14 us per thousand, the general path some 0.3 ms per level whatever
+// its size.  Whole calls, default schedule / rounds, general path and this (us):
+// G(n,m) 5000, 10 K edges 514 -> 105 / 636 -> 103; 16 K, 32 K 1039 -> 251 /
+// 914 -> 206; 16 K, 120 K 1180 -> 453 / 838 -> 384; 16 K, 240 K 1428 -> 771 /
+// 638 -> 599; 32 K, 40 K 1556 -> 439 / 1104 -> 356; 32 K, 125 K 2392 -> 903 /
+// 910 -> 624.  With 250 K edges at 32 K vertices the rounds lost (1065 -> 1148).
+bool tail_fits(uint64_t n, uint64_t m2, bool local) {
+  if (n <= kTailSmall) return m2 <= kTailSlots;
+  return !local && n <= kTailVertices && m2 <= kTailBigSlots;
+}
+
+// use_tail: the last levels, where small enough, in one workgroup.
+void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tail) {
   const bool local = o->variant == KC_VARIANT_LOCAL;
   const BinCfg cfg = bin_cfg(g, o);
   // degree-0 vertices are their own components and take no part in the
   // contraction (the reference sets them inactive at load, graph_io.h:380)
   identity_u32(g->n, g->labels, g->stream);
-  fill_u32(g->small + 5, 1, 0, g->stream);
+  fill_u32(g->small + 5, 4, 0, g->stream);
   uint64_t n_l = g->n0, m2_l = g->m2;
   const uint64_t *off_l = g->off0c;
   const uint32_t *col_l = g->col0c;
@@ -984,6 +1000,36 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out) {
         TimedScope ts(g->timer, KC_K_UNDO, 12 * n_l);
         union_reps(n_l, g->cid, gid_l, top_rep, g->stream);
       }
+      top_from_keys = true;
+      break;
+    }
+    if (use_tail && !pre && pre_left == 0 && !idx_l && tail_fits(n_l, m2_l, local) &&
+        (local || g->table_k <= kTailMaxDeviate)) {
+      TailArgs t{};
+      t.n = static_cast<uint32_t>(n_l);
+      t.m = m2_l / 2;
+      t.seq_limit = o->seq_limit;
+      t.iteration = iteration;
+      t.max_levels = static_cast<uint32_t>(std::max<int64_t>(0, static_cast<int64_t>(max_levels) -
+                                                                    static_cast<int64_t>(g->levels.size())));
+      t.local = local;
+      t.stall_rule = !local && !o->use_bfs;
+      t.d = da;
+      t.gid_in = gid_l;
+      t.edge = g->slots;
+      t.cur = g->crank;
+      t.gid = g->seg_of_cid;
+      t.key0 = g->uniq;
+      t.nidx = reinterpret_cast<uint16_t *>(g->pos_of);
+      t.rep = g->rep_a;
+      t.count = g->small + 8;
+      t.info = g->small + 9;
+      {
+        TimedScope ts(g->timer, KC_K_JUMP, 8 * (n_l + 1) + 4 * m2_l + 8 * n_l);
+        tail_levels(t, m2_l, off_l, col_l, g->stream);
+      }
+      out.tail = true;
+      top_rep = g->rep_a;
       top_from_keys = true;
       break;
     }
@@ -2113,13 +2159,32 @@ int kc_find_components(kc_graph *g, const kc_options *opt, uint32_t *labels_out,
     g->timer.begin_run(o.time_kernels != 0, g->stream, o.time_class - 1);
     KC_HIP(hipEventRecord(g->ev_begin, g->stream));
     RunOut out;
-    if (o.variant == KC_VARIANT_EXP || o.variant == KC_VARIANT_LOCAL)
-      run_contraction(g, &o, out);
-    else
-      run_propagation(g, &o, out);
-    KC_HIP(hipEventRecord(g->ev_end, g->stream));
-    d2h(g, g->h_small + 5, g->small + 5, sizeof(uint32_t));
-    sync(g);
+    const bool contraction = o.variant == KC_VARIANT_EXP || o.variant == KC_VARIANT_LOCAL;
+    // (a trace or a dataset wants every level's keys, a model its features)
+    bool use_tail = !o.record_trace && !o.learned && !g->collect;
+    while (true) {
+      if (contraction)
+        run_contraction(g, &o, out, use_tail);
+      else
+        run_propagation(g, &o, out);
+      KC_HIP(hipEventRecord(g->ev_end, g->stream));
+      d2h(g, g->h_small + 5, g->small + 5, 8 * sizeof(uint32_t));
+      sync(g);
+      if (!out.tail) break;
+      const uint32_t *info = g->h_small + 9;
+      if (info[0] == kTailFull) {  // (not seen: a hash part of the tail outgrew its table) every level the general way
+        use_tail = false;
+        out = RunOut();
+        g->arena.reset();
+        continue;
+      }
+      if (info[0] == kTailLevels)
+        fail(KC_ERR_INVALID, "contraction did not finish within %d levels", o.max_levels > 0 ? o.max_levels : 4096);
+      out.levels += info[1];
+      out.sweeps += info[2];
+      out.radius_sum += info[3];
+      break;
+    }
     g->components = g->n ? g->h_small[5] : 0;
     if (o.variant == KC_VARIANT_EXP || o.variant == KC_VARIANT_LOCAL)
       g->components += static_cast<uint32_t>(g->n - g->n0);  // degree-0 vertices

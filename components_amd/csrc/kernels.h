@@ -147,6 +147,31 @@ void union_keys(uint64_t n, const uint32_t *parent, uint64_t *key, hipStream_t s
 void union_labels(uint64_t n, const uint32_t *parent, uint32_t *labels, uint32_t *roots, uint32_t *partial,
                   hipStream_t s);
 
+// The remaining levels of a contraction in one workgroup (tail.hip): from the
+// level CSR (off, col: m2 slots) of n vertices at `iteration` down to an
+// edgeless graph or the base case, rep[v] = the id (gid_in; null: identity) of
+// v's last centre.  m: the level's undirected edges as the cut-off counts
+// them; stall_rule: the default schedule's rule for levels that change no key.
+// cur, gid, key0: n words of scratch each, nidx: n half-words, edge: m2 words,
+// count: a zeroed word; info = {status, levels, sweeps, radius sum}.
+constexpr uint64_t kTailVertices = 32768;     // 128 KB of LDS: a key per vertex
+constexpr uint64_t kTailSmall = 16128;        // ... two keys and a 16-bit index per vertex in 160 KB
+constexpr uint64_t kTailSlots = 1u << 19;     // edge slots of up to kTailSmall vertices
+constexpr uint64_t kTailBigSlots = 1u << 18;  // ... of more
+constexpr uint32_t kTailMaxDeviate = (1u << 17) - 3;  // distances share a word with 15 label bits
+constexpr uint32_t kTailDone = 0, kTailLevels = 1, kTailFull = 2;
+struct TailArgs {
+  uint32_t n;
+  uint64_t m, seq_limit;
+  uint32_t iteration, max_levels;
+  int local, stall_rule;
+  DeviateArgs d;
+  const uint32_t *gid_in;
+  uint32_t *edge, *cur, *gid, *key0, *rep, *count, *info;
+  uint16_t *nidx;
+};
+void tail_levels(const TailArgs &a, uint64_t m2, const uint64_t *off, const uint32_t *col, hipStream_t s);
+
 // Interface vertices of blocks of bsize consecutive indices (a neighbour in
 // another block) get their own index back as key: key[v] = v.
 void block_interface(const uint64_t *off, const uint32_t *col, uint64_t n, uint64_t bsize, uint64_t *key,

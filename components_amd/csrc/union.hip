@@ -20,12 +20,12 @@
 
 #include "kc_common.h"
 #include "kernels.h"
+#include "slot_rows.h"
 
 namespace kc {
 
 namespace {
 
-constexpr int kLinkSlots = 512;    // edge slots of one wave: every wave the same work, whatever the rows' lengths
 constexpr uint32_t kFirstNeighbours = 4;
 constexpr int kShortenHops = 32;
 constexpr uint64_t kShortenTwiceMin = 1u << 16;
@@ -94,19 +94,6 @@ __device__ __forceinline__ void link(uint32_t *parent, uint32_t u, uint32_t w) {
   }
 }
 
-// The last row r with off[r] <= e (off[0] <= e < off[n]), 64 probes a step.
-__device__ __forceinline__ uint64_t row_of_slot(const uint64_t *off, uint64_t n, uint64_t e) {
-  uint64_t lo = 0, hi = n;
-  while (hi - lo > 1) {
-    const uint64_t step = (hi - lo + kWave - 1) / kWave;
-    const uint64_t p = lo + (lane_id() + 1) * step;
-    const uint64_t below = __popcll(__ballot(p < hi && off[p] <= e));
-    lo += below * step;
-    hi = lo + step < hi ? lo + step : hi;
-  }
-  return lo;
-}
-
 // Hooks the larger of the two ends' parents under the smaller one without a
 // search: trees that are stars (or nearly) merge in one step each.  Where the
 // larger is no root any more its link is replaced; every edge is linked again
@@ -119,84 +106,22 @@ __device__ __forceinline__ void hook(uint32_t *parent, uint32_t u, uint32_t w) {
 }
 
 // Links (or, with kHook, hooks) the two ends of every edge, from its larger
-// end's row.  A wave takes
-// kLinkSlots consecutive slots: it searches its first and last row, marks the
-// rows' first slots in LDS and spreads the marks by a running maximum; where
-// the range spans many empty rows, each lane searches its slot's row instead.
+// end's row.
 template <bool kHook>
 __global__ __launch_bounds__(kBlock) void k_union_link(uint64_t n, uint64_t m2, const uint64_t *off,
                                                       const uint32_t *col, uint64_t block, uint32_t *parent) {
-  __shared__ uint32_t row_lds[kBlock / kWave][kLinkSlots];
-  uint32_t *row = row_lds[threadIdx.x / kWave];
-  const uint32_t ln = lane_id();
-  const uint64_t c0 = (blockIdx.x * static_cast<uint64_t>(kBlock / kWave) + threadIdx.x / kWave) * kLinkSlots;
+  __shared__ uint32_t row_lds[kBlock / kWave][kWaveSlots];
+  const uint64_t c0 = (blockIdx.x * static_cast<uint64_t>(kBlock / kWave) + threadIdx.x / kWave) * kWaveSlots;
   if (c0 >= m2) return;
-  const uint64_t c1 = c0 + kLinkSlots < m2 ? c0 + kLinkSlots : m2;
-  const uint64_t r0 = row_of_slot(off, n, c0), r1 = row_of_slot(off, n, c1 - 1);
-  constexpr uint32_t kPerLane = kLinkSlots / kWave;
-  const bool marked = r1 - r0 <= 4 * kLinkSlots;
-  if (marked) {
-    for (uint32_t j = ln; j < kLinkSlots; j += kWave) row[j] = 0;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    for (uint64_t r = r0 + 1 + ln; r <= r1; r += kWave) {  // non-empty rows start at distinct slots
-      const uint64_t s = off[r];
-      if (off[r + 1] > s) row[s - c0] = static_cast<uint32_t>(r - r0);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    uint32_t m[kPerLane], run = 0;
-#pragma unroll
-    for (uint32_t j = 0; j < kPerLane; ++j) {
-      const uint32_t x = row[ln * kPerLane + j];
-      run = x > run ? x : run;
-      m[j] = run;
-    }
-    uint32_t inc = run;
-    for (int o = 1; o < kWave; o <<= 1) {
-      const uint32_t t = static_cast<uint32_t>(__shfl_up(static_cast<int>(inc), o));
-      if (ln >= static_cast<uint32_t>(o) && t > inc) inc = t;
-    }
-    uint32_t before = static_cast<uint32_t>(__shfl_up(static_cast<int>(inc), 1));
-    if (ln == 0) before = 0;
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (uint32_t j = 0; j < kPerLane; ++j) row[ln * kPerLane + j] = m[j] > before ? m[j] : before;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  }
-  uint32_t w[kPerLane];
-#pragma unroll
-  for (uint32_t j = 0; j < kPerLane; ++j) {
-    const uint64_t e = c0 + j * kWave + ln;
-    w[j] = e < c1 ? col[e] : kNone;
-  }
-#pragma unroll
-  for (uint32_t j = 0; j < kPerLane; ++j) {
-    const uint64_t e = c0 + j * kWave + ln;
-    if (e >= c1) continue;
-    uint64_t u;
-    if (marked) {
-      u = r0 + row[j * kWave + ln];
-    } else {
-      uint64_t lo = r0, hi = r1 + 1;
-      while (hi - lo > 1) {
-        const uint64_t mid = lo + (hi - lo) / 2;
-        if (off[mid] <= e)
-          lo = mid;
-        else
-          hi = mid;
-      }
-      u = lo;
-    }
-    const uint32_t v = static_cast<uint32_t>(u);
-    if (w[j] < v && same_block(w[j], v, block)) {
+  const uint64_t c1 = c0 + kWaveSlots < m2 ? c0 + kWaveSlots : m2;
+  for_wave_slots(n, off, col, c0, c1, row_lds[threadIdx.x / kWave], [&](uint32_t, uint32_t v, uint32_t w) {
+    if (w < v && same_block(w, v, block)) {
       if (kHook)
-        hook(parent, v, w[j]);
+        hook(parent, v, w);
       else
-        link(parent, v, w[j]);
+        link(parent, v, w);
     }
-  }
+  });
 }
 
 __device__ __forceinline__ uint32_t root_of(const uint32_t *parent, uint64_t v) {
@@ -264,7 +189,7 @@ void union_components(uint64_t n, uint64_t m2, const uint64_t *off, const uint32
   hipLaunchKernelGGL(k_union_init, dim3(blocks_for(n)), dim3(kBlock), 0, s, n, off, col, block, parent);
   KC_LAUNCH_CHECK();
   if (!m2) return;
-  const unsigned g = static_cast<unsigned>(ceil_div(m2, static_cast<uint64_t>(kLinkSlots) * (kBlock / kWave)));
+  const unsigned g = static_cast<unsigned>(ceil_div(m2, static_cast<uint64_t>(kWaveSlots) * (kBlock / kWave)));
   shorten(n, parent, s);
   for (int r = 0; r < hook_rounds(n, m2); ++r) {
     hipLaunchKernelGGL(k_union_link<true>, dim3(g), dim3(kBlock), 0, s, n, m2, off, col, block, parent);

@@ -202,7 +202,7 @@ typedef struct kc_options {
 #define KC_K_CSR 7       /* next-level CSR compaction */
 #define KC_K_UNDO 8      /* undo gather */
 #define KC_K_CANON 9     /* canonical min-id labels */
-#define KC_K_JUMP 10     /* pointer jumping */
+#define KC_K_JUMP 10     /* union-find (base case, shortcuts); the last levels in one workgroup */
 #define KC_K_OTHER 11
 #define KC_K_SORT 12     /* radix sort of (label, vertex) pairs */
 #define KC_K_RELABEL 13  /* edge slots relabelled with their far end's cluster */
@@ -304,7 +304,8 @@ int kc_copy_labels(kc_graph *g, uint32_t *labels_out);
  * to query *num_pairs. */
 int kc_component_histogram(kc_graph *g, uint64_t *pairs, uint64_t capacity, uint64_t *num_pairs);
 
-/* Per-level trace of the last kc_find_components call with record_trace=1.
+/* Per-level trace of the last kc_find_components call with record_trace=1
+ * (without it the last, small levels run in one workgroup and leave no record).
  * level_sizes: n_l, m_l (undirected), sweeps_l, radius_l for level l. */
 int kc_trace_levels(const kc_graph *g, uint32_t *levels);
 int kc_trace_level_info(const kc_graph *g, uint32_t level, uint64_t info[4]);
