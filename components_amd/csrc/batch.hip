@@ -25,6 +25,7 @@
 #include <memory>
 #include <vector>
 
+#include "copy_out.h"
 #include "csr_build.h"
 #include "deviates.h"
 #include "kc_common.h"
@@ -870,6 +871,7 @@ struct kc_batch {
   uint64_t *d_uoff = nullptr, *d_ueoff = nullptr;
   BatchDev dev{};
   BatchParams *d_params = nullptr, *h_params = nullptr;
+  uint32_t *h_figures = nullptr;  // pinned: the last run's gstatus, glevels, gsweeps, gradius, gcomp (graphs each)
   uint64_t *table = nullptr;
   uint64_t table_words = 0;
   uint32_t *queue = nullptr;
@@ -891,12 +893,15 @@ struct kc_batch {
     owned.push_back(p);
     return static_cast<T *>(p);
   }
+  kc_batch() { copy_out_retain(); }
   ~kc_batch() {
+    copy_out_release();
     if (stream) (void)hipStreamSynchronize(stream);
     if (big) (void)kc_graph_destroy(big);
     if (exec) (void)hipGraphExecDestroy(exec);
     for (void *p : owned) (void)hipFree(p);
     if (h_params) (void)hipHostFree(h_params);
+    if (h_figures) (void)hipHostFree(h_figures);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (stream) (void)hipStreamDestroy(stream);
@@ -1082,11 +1087,12 @@ float run_once(kc_batch *b, const kc_options &o) {
     }
   }
   KC_HIP(hipEventRecord(b->ev1, b->stream));
+  // every graph's figures in one copy ahead of the synchronisation
+  if (b->graphs) KC_HIP(hipMemcpyAsync(b->h_figures, b->dev.gstatus, 20ull * b->graphs, hipMemcpyDeviceToHost, b->stream));
   KC_HIP(hipStreamSynchronize(b->stream));
   float ms = 0.f;
   KC_HIP(hipEventElapsedTime(&ms, b->ev0, b->ev1));
-  std::vector<uint32_t> st(b->graphs);
-  if (b->graphs) KC_HIP(hipMemcpy(st.data(), b->dev.gstatus, 4ull * b->graphs, hipMemcpyDeviceToHost));
+  const uint32_t *st = b->h_figures;
   for (uint32_t g = 0; g < b->graphs; ++g)
     if (st[g]) {
       // a graph that stopped early may have left entries in its hash set
@@ -1208,11 +1214,12 @@ int kc_batch_create(const kc_batch_host *h, kc_batch **out) {
     b->table = b->dalloc<uint64_t>(b->table_words);
     d.table = b->table;
     d.stack = b->dalloc<uint32_t>(static_cast<uint64_t>(kStackPerVertex) * n);
-    d.glevels = b->dalloc<uint32_t>(G);
-    d.gsweeps = b->dalloc<uint32_t>(G);
-    d.gradius = b->dalloc<uint32_t>(G);
-    d.gstatus = b->dalloc<uint32_t>(G);
-    d.gcomp = b->dalloc<uint32_t>(G);
+    d.gstatus = b->dalloc<uint32_t>(5ull * G);
+    d.glevels = d.gstatus + G;
+    d.gsweeps = d.glevels + G;
+    d.gradius = d.gsweeps + G;
+    d.gcomp = d.gradius + G;
+    KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&b->h_figures), 20ull * G + 64, hipHostMallocDefault));
     b->queue = b->dalloc<uint32_t>(1);
     d.queue = b->queue;
     b->d_params = b->dalloc<BatchParams>(1);
@@ -1245,9 +1252,10 @@ int kc_batch_run(kc_batch *b, const kc_options *opt, uint32_t *labels_out, kc_ba
     else
       kc_options_init(&o);
     const auto t0 = std::chrono::steady_clock::now();
+    CopyOut labels(labels_out, 4ull * b->n, b->device);
     batch_params(b, o);
     const float ms = run_once(b, o);
-    if (labels_out && b->n) KC_HIP(hipMemcpy(labels_out, b->dev.labels, 4ull * b->n, hipMemcpyDeviceToHost));
+    labels.finish(b->dev.labels, b->stream);
     const auto t1 = std::chrono::steady_clock::now();
     if (stats) {
       std::memset(stats, 0, sizeof(*stats));
@@ -1257,13 +1265,7 @@ int kc_batch_run(kc_batch *b, const kc_options *opt, uint32_t *labels_out, kc_ba
       stats->m = b->m2 / 2;
       stats->graphs = b->graphs;
       stats->tuning = b->tuning;
-      std::vector<uint32_t> lv(b->graphs), sw(b->graphs), rd(b->graphs), cc(b->graphs);
-      if (b->graphs) {
-        KC_HIP(hipMemcpy(lv.data(), b->dev.glevels, 4ull * b->graphs, hipMemcpyDeviceToHost));
-        KC_HIP(hipMemcpy(sw.data(), b->dev.gsweeps, 4ull * b->graphs, hipMemcpyDeviceToHost));
-        KC_HIP(hipMemcpy(rd.data(), b->dev.gradius, 4ull * b->graphs, hipMemcpyDeviceToHost));
-        KC_HIP(hipMemcpy(cc.data(), b->dev.gcomp, 4ull * b->graphs, hipMemcpyDeviceToHost));
-      }
+      const uint32_t *lv = b->h_figures + b->graphs, *sw = lv + b->graphs, *rd = sw + b->graphs, *cc = rd + b->graphs;
       for (uint32_t g = 0; g < b->graphs; ++g) {
         stats->levels_sum += lv[g];
         stats->sweeps_sum += sw[g];

@@ -25,6 +25,7 @@
 #include <string>
 #include <vector>
 
+#include "copy_out.h"
 #include "csr_build.h"
 #include "deviates.h"
 #include "kc_common.h"
@@ -355,7 +356,9 @@ struct kc_graph {
     for (void *p : work_owned) (void)hipFree(p);
     work_owned.clear();
   }
+  kc_graph() { copy_out_retain(); }
   ~kc_graph() {
+    copy_out_release();
     if (stream) (void)hipStreamSynchronize(stream);
     for (void *p : work_owned) (void)hipFree(p);
     for (void *p : owned) (void)hipFree(p);
@@ -2154,6 +2157,7 @@ int kc_find_components(kc_graph *g, const kc_options *opt, uint32_t *labels_out,
     }
     const auto t0 = std::chrono::steady_clock::now();
     g->have_labels = false;
+    CopyOut labels(labels_out, g->n * 4, g->device);
     if (o.variant == KC_VARIANT_EXP) ensure_table(g, o.beta);
     g->arena.reset();
     g->timer.begin_run(o.time_kernels != 0, g->stream, o.time_class - 1);
@@ -2169,6 +2173,7 @@ int kc_find_components(kc_graph *g, const kc_options *opt, uint32_t *labels_out,
         run_propagation(g, &o, out);
       KC_HIP(hipEventRecord(g->ev_end, g->stream));
       d2h(g, g->h_small + 5, g->small + 5, 8 * sizeof(uint32_t));
+      labels.enqueue(g->labels, g->stream);
       sync(g);
       if (!out.tail) break;
       const uint32_t *info = g->h_small + 9;
@@ -2191,7 +2196,7 @@ int kc_find_components(kc_graph *g, const kc_options *opt, uint32_t *labels_out,
     g->have_labels = true;
     float ms = 0.f;
     KC_HIP(hipEventElapsedTime(&ms, g->ev_begin, g->ev_end));
-    if (labels_out && g->n) KC_HIP(hipMemcpy(labels_out, g->labels, g->n * 4, hipMemcpyDeviceToHost));
+    labels.finish(g->labels, g->stream);
     const auto t1 = std::chrono::steady_clock::now();
     if (stats) {
       std::memset(stats, 0, sizeof(*stats));
@@ -2363,7 +2368,7 @@ int kc_copy_labels(kc_graph *g, uint32_t *labels_out) {
   return guarded([&] {
     if (!g || !labels_out) fail(KC_ERR_INVALID, "null argument");
     if (!g->have_labels) fail(KC_ERR_INVALID, "no labels: kc_find_components has not completed");
-    if (g->n) KC_HIP(hipMemcpy(labels_out, g->labels, g->n * 4, hipMemcpyDeviceToHost));
+    CopyOut(labels_out, g->n * 4, g->device).finish(g->labels, g->stream);
   });
 }
 
