@@ -8,12 +8,13 @@
 namespace kc {
 
 // One copy of `bytes` from device memory to the caller's `dst` at the end of a
-// call.  The constructor (at the call's start; dst may be null: nothing to do)
-// lets helper threads fault in dst's pages while the GPU works, without
-// changing what they hold.  enqueue() may put a small copy into the stream
-// ahead of a synchronisation the caller makes anyway; finish() copies, src
-// final in stream order, and returns when dst is written.  Destroying it
-// without finish() leaves dst as it was.  Throws Failure.
+// call; bytes are whole words and src is aligned to 16 bytes.  The constructor
+// (at the call's start; dst may be null: nothing to do) lets helper threads
+// fault in dst's pages while the GPU works, without changing what they hold.
+// enqueue() may put a small copy into the stream ahead of a synchronisation the
+// caller makes anyway; finish() copies, src final in stream order, and returns
+// when dst is written.  Destroying it without finish() leaves dst as it was.
+// Throws Failure.
 class CopyOut {
  public:
   CopyOut(void *dst, size_t bytes, int device);

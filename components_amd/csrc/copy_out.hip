@@ -2,7 +2,7 @@
 // runtime's staging buffer on one thread, which also took the page faults of
 // a fresh buffer: 10 GB/s (16.8 M labels: 6.4 ms beside 7 to 9 ms of GPU work),
 // against 56 GB/s into pinned memory.  Here a ring of pinned slots takes the
-// copies while helper threads move finished slots on, and the pages are faulted
+// transfers while helper threads move finished slots on, and the pages are faulted
 // in while the GPU still works.
 #include "copy_out.h"
 
@@ -29,8 +29,8 @@ namespace kc {
 
 namespace {
 
-// (a transfer costs the queue about 16 us beside its bytes: 64 of 1 MB took 2.3
-// ms where 16 of 4 MB take 1.6)
+// (short transfers leave gaps between them: 64 of 1 MB took 2.3 ms where 16 of
+// 4 MB take 1.6)
 constexpr size_t kSlotBytes = 4 << 20;
 constexpr int kSlots = 4;
 constexpr size_t kPieceBytes = 512 << 10;  // moved on by one helper
@@ -71,7 +71,7 @@ char *ring_borrow(int device) {
   if (g_ring.lent) return nullptr;
   if (!g_ring.mem) {
     void *p = nullptr;
-    if (hipHostMalloc(&p, kSlotBytes * kSlots, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(&p, kSlotBytes * kSlots, hipHostMallocPortable) != hipSuccess) {
       (void)hipGetLastError();
       return nullptr;
     }
@@ -97,6 +97,28 @@ void ring_return() {
   if (g_ring.handles == 0) ring_drop();
 }
 
+// A transfer by stores from the CUs: 50 GB/s always, where the copy engine that
+// hipMemcpyAsync picks runs at 57 or, for long stretches on some streams, at
+// 20 (67 MB: 3.6 instead of 1.6 ms).  What bounds it is the host link; 64
+// workgroups fill it (16: 5% slower).
+constexpr unsigned kTransferBlocks = 64;
+
+__global__ __launch_bounds__(kBlock) void k_transfer(uint32_t *dst, const uint32_t *src, uint64_t words) {
+  const uint64_t quads = words / 4, stride = static_cast<uint64_t>(gridDim.x) * kBlock;
+  const uint64_t first = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
+  for (uint64_t i = first; i < quads; i += stride)
+    reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+  if (first < words % 4) dst[4 * quads + first] = src[4 * quads + first];
+}
+
+// src and bytes: whole words, src aligned to 16 (device arrays and their
+// multiples of a piece).
+void transfer(void *slot, const void *src, size_t bytes, hipStream_t s) {
+  hipLaunchKernelGGL(k_transfer, dim3(kTransferBlocks), dim3(kBlock), 0, s, static_cast<uint32_t *>(slot),
+                     static_cast<const uint32_t *>(src), bytes / 4);
+  KC_LAUNCH_CHECK();
+}
+
 // Faults in the whole pages inside [p, p + bytes) for writing (their contents
 // stay); where the kernel cannot, the copy takes the faults.
 void fault_in(char *p, size_t bytes) {
@@ -113,7 +135,7 @@ void fault_in(char *p, size_t bytes) {
 struct CopyOut::Job {
   char *dst = nullptr;
   size_t bytes = 0;
-  int device = 0, helpers = 0;
+  int helpers = 0;
   std::thread first;                // starts the other helpers and joins them
   std::mutex m;
   std::condition_variable changed;  // some of the following moved on
@@ -121,14 +143,13 @@ struct CopyOut::Job {
   // once the copy begins: transfers of `chunk` bytes, one ring slot each, moved
   // on in pieces
   size_t chunk = 0;
-  size_t ready = 0;                 // bytes whose transfer and event are in the stream
+  size_t ready = 0;                 // bytes that have reached their slots
   size_t claimed = 0, done = 0;     // bytes taken and moved by helpers
   std::vector<size_t> left;         // per transfer: bytes still in its slot
-  bool stop = false, failed = false;
+  bool stop = false;
   const char *ring = nullptr;
 
   void help() {
-    bool set = false;
     std::unique_lock<std::mutex> lock(m);
     while (!stop) {
       if (claimed < ready) {
@@ -136,14 +157,10 @@ struct CopyOut::Job {
         const size_t n = std::min({kPieceBytes, (c + 1) * chunk - at, bytes - at});
         claimed += n;
         lock.unlock();
-        if (!set) (void)hipSetDevice(device);
-        set = true;
-        const bool ok = hipEventSynchronize(g_ring.events[c % kSlots]) == hipSuccess;
-        if (ok) std::memcpy(dst + at, ring + (c % kSlots) * kSlotBytes + (at - c * chunk), n);
+        std::memcpy(dst + at, ring + (c % kSlots) * kSlotBytes + (at - c * chunk), n);
         lock.lock();
         left[c] -= n;
         done += n;
-        failed = failed || !ok;
         if (left[c] == 0) changed.notify_all();
       } else if (claimed >= bytes) {
         return;
@@ -185,7 +202,6 @@ CopyOut::CopyOut(void *dst, size_t bytes, int device) : dst_(dst), bytes_(dst ? 
   std::unique_ptr<Job> j(new Job);
   j->dst = static_cast<char *>(dst);
   j->bytes = bytes;
-  j->device = device;
   const int cpus = static_cast<int>(std::thread::hardware_concurrency());
   j->helpers = std::max(1, std::min({kMaxHelpers, cpus / 2, static_cast<int>(bytes_ / kThreadsMin)}));
   try {
@@ -206,7 +222,7 @@ void CopyOut::enqueue(const void *src, hipStream_t stream) {
   if (!bytes_ || bytes_ > kThreadsMin) return;
   if (!ring_) ring_ = ring_borrow(device_);
   if (!ring_) return;
-  KC_HIP(hipMemcpyAsync(ring_, src, bytes_, hipMemcpyDeviceToHost, stream));
+  transfer(ring_, src, bytes_, stream);
   queued_ = true;
   stream_ = stream;
 }
@@ -250,24 +266,31 @@ void CopyOut::finish(const void *src, hipStream_t stream) {
       (void)hipStreamSynchronize(s);
     }
   } drain{j, stream};
-  for (size_t c = 0; c < chunks; ++c) {
-    if (c >= kSlots) {
-      std::unique_lock<std::mutex> lock(j.m);
-      j.changed.wait(lock, [&] { return j.left[c - kSlots] == 0; });
+  // (only this thread talks to the runtime)
+  size_t issued = 0, arrived = 0;
+  while (arrived < chunks) {
+    while (issued < chunks && issued < arrived + kSlots) {
+      if (issued >= kSlots) {  // its slot's last transfer has to be moved on first
+        std::unique_lock<std::mutex> lock(j.m);
+        if (j.left[issued - kSlots] != 0) {
+          if (issued > arrived) break;
+          j.changed.wait(lock, [&] { return j.left[issued - kSlots] == 0; });
+        }
+      }
+      const size_t off = issued * chunk;
+      transfer(ring_ + (issued % kSlots) * kSlotBytes, static_cast<const char *>(src) + off,
+               std::min(chunk, bytes_ - off), stream);
+      KC_HIP(hipEventRecord(g_ring.events[issued % kSlots], stream));
+      ++issued;
     }
-    const size_t off = c * chunk, n = std::min(chunk, bytes_ - off);
-    KC_HIP(hipMemcpyAsync(ring_ + (c % kSlots) * kSlotBytes, static_cast<const char *>(src) + off, n,
-                          hipMemcpyDeviceToHost, stream));
-    KC_HIP(hipEventRecord(g_ring.events[c % kSlots], stream));
+    KC_HIP(hipEventSynchronize(g_ring.events[arrived % kSlots]));
+    ++arrived;
     std::lock_guard<std::mutex> lock(j.m);
-    j.ready = off + n;
+    j.ready = std::min(arrived * chunk, bytes_);
     j.changed.notify_all();
   }
   std::unique_lock<std::mutex> lock(j.m);
   j.changed.wait(lock, [&] { return j.done == bytes_; });
-  const bool failed = j.failed;
-  lock.unlock();
-  if (failed) fail(KC_ERR_HIP, "copy of the labels to the host failed");
 }
 
 void copy_out_retain() {
