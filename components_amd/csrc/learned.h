@@ -26,10 +26,13 @@ struct MlpMaster {
 };
 constexpr int kMlpMasterFloats = static_cast<int>(sizeof(MlpMaster) / sizeof(float));
 
-// bf16 copies of the weight matrices read by the kernels (biases stay f32).
+// bf16 copies of the weight matrices read by the kernels (biases stay f32), in
+// the orders in which a fragment's four values lie together: one load of 8
+// bytes each, where the kernels of a step would spend their start on single ones.
 struct MlpBf16 {
-  uint16_t W1[kMlpInPad * kMlpHid];
-  uint16_t W2[kMlpHid * kMlpHid];
+  uint16_t W1t[kMlpHid * kMlpInPad];  // [hidden][input]
+  uint16_t W2t[kMlpHid * kMlpHid];    // [hidden 2][hidden 1]
+  uint16_t W2[kMlpHid * kMlpHid];     // [hidden 1][hidden 2]
   uint16_t w3[kMlpHid];
 };
 
@@ -51,15 +54,13 @@ struct kc_mlp {
   kc::MlpMaster *master = nullptr;  // f32 parameters
   kc::MlpBf16 *bf = nullptr;        // bf16 weights
   float *adam_m = nullptr, *adam_v = nullptr, *grad = nullptr, *loss = nullptr;
-  float *partials = nullptr;  // per-wave gradient partials of one training pass
-  uint64_t partial_waves = 0;
+  float *partials = nullptr;  // per-chain gradient partials of one training pass
+  uint64_t partial_chains = 0;
   uint64_t adam_t = 0;
   uint64_t version = 1;  // bumped by every parameter change
   // trace dataset: features [cap x 6] and targets [cap]
   float *X = nullptr, *y = nullptr;
   uint64_t count = 0, cap = 0;
-  uint32_t *idx = nullptr;
-  uint64_t idx_cap = 0;
   std::vector<void *> owned;
   template <class T>
   T *dalloc(uint64_t n);

@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <cstddef>
 #include <cstring>
 #include <memory>
 
@@ -52,7 +53,7 @@ typedef short v4s __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int kRowPad = 72;  // LDS row stride of a 16 x 64 bf16 tile (breaks bank aliasing)
-constexpr uint64_t kPartialStride = kMlpMasterFloats + 3;  // floats per wave partial (parameters, loss)
+constexpr uint64_t kPartialStride = kMlpMasterFloats + 3;  // floats per chain's partial (parameters, loss)
 constexpr int kXPad = 20;    // LDS row stride of a 16 x 16 bf16 input tile
 
 __device__ __forceinline__ v4f mfma(v4s a, v4s b, v4f c) {
@@ -192,13 +193,9 @@ __global__ __launch_bounds__(256) void k_mlp_infer(uint64_t n, const float *X, c
   float b1v[4][4], b2v[4][4], w3v[4][4];
   for (int nb = 0; nb < 4; ++nb) {
     const int h = nb * 16 + r;
-    a1[nb] = frag(wb->W1[(4 * g) * kMlpHid + h], wb->W1[(4 * g + 1) * kMlpHid + h], wb->W1[(4 * g + 2) * kMlpHid + h],
-                  wb->W1[(4 * g + 3) * kMlpHid + h]);
-    for (int kb = 0; kb < 4; ++kb) {
-      const int k = kb * 16 + 4 * g;
-      a2[kb][nb] = frag(wb->W2[k * kMlpHid + h], wb->W2[(k + 1) * kMlpHid + h], wb->W2[(k + 2) * kMlpHid + h],
-                        wb->W2[(k + 3) * kMlpHid + h]);
-    }
+    a1[nb] = *reinterpret_cast<const v4s *>(wb->W1t + h * kMlpInPad + 4 * g);
+    for (int kb = 0; kb < 4; ++kb)
+      a2[kb][nb] = *reinterpret_cast<const v4s *>(wb->W2t + h * kMlpHid + kb * 16 + 4 * g);
     for (int j = 0; j < 4; ++j) {
       const int c = nb * 16 + 4 * g + j;
       b1v[nb][j] = wm->b1[c];
@@ -263,30 +260,87 @@ __global__ void k_delays(uint64_t n, const float *score, float alpha, uint8_t *d
 
 // ---------------------------------------------------------------------------
 // Training: forward, loss 0.5 * mean((s - y)^2) over the batch, backward.
-// Every wave accumulates its gradient tiles in registers over its sample
-// tiles and adds them to grad (MlpMaster layout) once at the end.
-__global__ __launch_bounds__(256) void k_mlp_train(uint64_t bt, const uint32_t *idx, const float *X, const float *y,
-                                                  const MlpBf16 *wb, const MlpMaster *wm, float *partials) {
-  __shared__ uint16_t xs_all[4][16 * kXPad];
-  __shared__ uint16_t h1_all[4][16 * kRowPad];
-  __shared__ uint16_t dz2_all[4][16 * kRowPad];
-  __shared__ uint16_t dz1_all[4][16 * kRowPad];
+//
+// The tiles of 16 samples are dealt to `chains` (tile t to chain t % chains)
+// and every chain adds its tiles' gradients in order, so that a training is
+// reproducible bit for bit whatever runs at the same time.  One workgroup takes
+// a chain, eight tiles at once: each wave runs one tile forward and backward
+// and leaves its activations in LDS as the fragments the weight gradients
+// need; then every wave adds the eight tiles, in order, into the gradient
+// blocks it owns (two of the sixteen blocks of W2, and a block of W1 or the
+// bias columns of one block).  Bound by latency: the forward and backward of
+// one tile is a chain of four dependent products, and 64 chains (8192 samples)
+// leave most CUs idle whatever the kernel does.  With a wave per chain, which
+// ran its eight tiles one after the other on 16 workgroups, 8192 samples took
+// 41 us; so they take 14 us (a step of the training 64 -> 18 us; of 16 samples
+// 19 -> 13.5, of 2^20 1295 -> 335).
+constexpr int kTrainWaves = 8;
+
+// The batch's rows of the dataset: listed, or drawn uniformly over [0, count)
+// from a counter-based stream.
+struct BatchRows {
+  const uint32_t *idx;
+  GenStream draw;
+  uint64_t first, count;
+};
+
+__device__ __forceinline__ uint64_t batch_row(const BatchRows &b, uint64_t q) {
+  return b.idx ? b.idx[q] : gen_bounded(gen_value(b.draw, b.first + q), b.count);
+}
+
+// Orders a wave's LDS accesses across its lanes (they are served in program
+// order; this keeps the compiler to it).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__global__ __launch_bounds__(64 * kTrainWaves) void k_mlp_train(uint64_t bt, BatchRows rows, const float *X,
+                                                               const float *y, const MlpBf16 *wb,
+                                                               const MlpMaster *wm, float *partials) {
+  __shared__ uint16_t xs[kTrainWaves][16 * kXPad];    // inputs, row-major
+  __shared__ uint16_t act[kTrainWaves][16 * kRowPad];  // a wave's H1, then dZ2, from the D to the A layout
+  __shared__ v4s h1s[kTrainWaves][4][64], dz2s[kTrainWaves][4][64];
+  __shared__ v4f h2s[kTrainWaves][4][64], d1s[kTrainWaves][4][64];
+  __shared__ v4f dss[kTrainWaves][4], dfs[kTrainWaves][4];  // per sample: d loss / d score, score - target
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 15, g = lane >> 4;
-  uint16_t *xs = xs_all[wave], *h1 = h1_all[wave], *dz2s = dz2_all[wave], *dz1s = dz1_all[wave];
+  const uint64_t tiles = (bt + 15) / 16, chains = gridDim.x, chain = blockIdx.x;
+  // the four chains of a group take equally many tiles (those past the last are empty)
+  const uint64_t count = (tiles - (chain & ~3ull) + chains - 1) / chains;
+
+  float xf[4], yv;
+  auto load = [&](uint64_t i) {
+    const uint64_t q = (chain + i * chains) * 16 + r;
+    xf[0] = xf[1] = xf[2] = xf[3] = yv = 0.f;
+    if (i < count && q < bt) {
+      const uint64_t row = batch_row(rows, q);
+      const float2 *x = reinterpret_cast<const float2 *>(X + row * kMlpIn);
+      static_assert(kMlpIn == 6, "three pairs of inputs a row");
+      if (g < 2) {
+        const float2 a = x[2 * g];
+        xf[0] = a.x;
+        xf[1] = a.y;
+      }
+      if (g == 0) {
+        const float2 b = x[1];
+        xf[2] = b.x;
+        xf[3] = b.y;
+      }
+      yv = y[row];
+    }
+  };
+  load(wave);
   v4s b1f[4], b2f[4][4], b2t[4][4];
   float b1v[4], b2v[4], w3v[4];
   for (int nb = 0; nb < 4; ++nb) {
     const int c = nb * 16 + r;
-    b1f[nb] = frag(wb->W1[(4 * g) * kMlpHid + c], wb->W1[(4 * g + 1) * kMlpHid + c], wb->W1[(4 * g + 2) * kMlpHid + c],
-                   wb->W1[(4 * g + 3) * kMlpHid + c]);
+    b1f[nb] = *reinterpret_cast<const v4s *>(wb->W1t + c * kMlpInPad + 4 * g);
     for (int kb = 0; kb < 4; ++kb) {
-      const int k = kb * 16 + 4 * g;
-      b2f[kb][nb] = frag(wb->W2[k * kMlpHid + c], wb->W2[(k + 1) * kMlpHid + c], wb->W2[(k + 2) * kMlpHid + c],
-                         wb->W2[(k + 3) * kMlpHid + c]);
+      const int at = c * kMlpHid + kb * 16 + 4 * g;
+      b2f[kb][nb] = *reinterpret_cast<const v4s *>(wb->W2t + at);
       // W2 transposed: B[k = hidden 2][col = hidden 1] = W2[hidden 1][hidden 2]
-      const uint16_t *row = wb->W2 + c * kMlpHid + k;
-      b2t[kb][nb] = frag(row[0], row[1], row[2], row[3]);
+      b2t[kb][nb] = *reinterpret_cast<const v4s *>(wb->W2 + at);
     }
     b1v[nb] = wm->b1[c];
     b2v[nb] = wm->b2[c];
@@ -295,170 +349,206 @@ __global__ __launch_bounds__(256) void k_mlp_train(uint64_t bt, const uint32_t *
   const float b3 = wm->b3;
   const float inv_bt = 1.f / static_cast<float>(bt);
   const v4f zero = {0.f, 0.f, 0.f, 0.f};
-  v4f gW1[4] = {zero, zero, zero, zero};
-  v4f gW2[4][4];
-  for (int a = 0; a < 4; ++a)
-    for (int b = 0; b < 4; ++b) gW2[a][b] = zero;
-  float gb1[4] = {0, 0, 0, 0}, gb2[4] = {0, 0, 0, 0}, gw3[4] = {0, 0, 0, 0}, gb3 = 0.f, lsum = 0.f;
+  // what this wave adds up: blocks (mb, n0) and (mb, n0 + 1) of W2, block ob of
+  // W1 (waves 0..3) or of the biases and w3 (waves 4..7); wave 0 the loss
+  const int mb = wave >> 1, n0 = (wave & 1) * 2, ob = wave & 3;
+  const float w3o = bf16_to_f32(wb->w3[ob * 16 + r]);
+  v4f gW2a = zero, gW2b = zero, gW1 = zero;
+  float gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, lsum = 0.f;
 
-  const uint64_t tiles = (bt + 15) / 16;
-  for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * 4; base < tiles; base += static_cast<uint64_t>(gridDim.x) * 4) {
-    const uint64_t tile = base + wave;
-    // input tile (row r of this lane's A fragment) and its copy in LDS
-    uint16_t xa[4] = {0, 0, 0, 0};
-    const uint64_t q = tile * 16 + r;
-    if (q < bt) {
-      const uint64_t sidx = idx[q];
-      for (int j = 0; j < 4; ++j) {
-        const int k = 4 * g + j;
-        if (k < kMlpIn) xa[j] = f32_to_bf16(X[sidx * kMlpIn + k]);
-      }
-    }
-    for (int j = 0; j < 4; ++j) xs[r * kXPad + 4 * g + j] = xa[j];
-    const v4s a1 = frag(xa[0], xa[1], xa[2], xa[3]);
-    bool m1[4][4];
-    for (int nb = 0; nb < 4; ++nb) {
-      const v4f z = mfma(a1, b1f[nb], zero);
-      for (int j = 0; j < 4; ++j) {
-        const float h = z[j] + b1v[nb];
-        m1[nb][j] = h > 0.f;
-        h1[(4 * g + j) * kRowPad + nb * 16 + r] = f32_to_bf16(h > 0.f ? h : 0.f);
-      }
-    }
-    __syncthreads();
-    v4f z2[4] = {zero, zero, zero, zero};
-    for (int kb = 0; kb < 4; ++kb) {
-      const uint16_t *src = h1 + r * kRowPad + kb * 16 + 4 * g;
-      const v4s a2 = frag(src[0], src[1], src[2], src[3]);
-      for (int nb = 0; nb < 4; ++nb) z2[nb] = mfma(a2, b2f[kb][nb], z2[nb]);
-    }
-    float h2[4][4];
-    float ds[4];
-    for (int j = 0; j < 4; ++j) {
-      float acc = 0.f;
+  for (uint64_t base = 0; base < count; base += kTrainWaves) {
+    const uint64_t left = count - base;
+    const int live = left < kTrainWaves ? static_cast<int>(left) : kTrainWaves;
+    if (wave < live) {
+      const uint64_t tile = chain + (base + wave) * chains;
+      const v4s a1 = frag(f32_to_bf16(xf[0]), f32_to_bf16(xf[1]), f32_to_bf16(xf[2]), f32_to_bf16(xf[3]));
+      *reinterpret_cast<v4s *>(&xs[wave][r * kXPad + 4 * g]) = a1;
+      uint16_t *row = act[wave];
+      bool m1[4][4];
       for (int nb = 0; nb < 4; ++nb) {
-        const float h = z2[nb][j] + b2v[nb];
-        h2[nb][j] = h > 0.f ? h : 0.f;
-        acc += h2[nb][j] * w3v[nb];
+        const v4f z = mfma(a1, b1f[nb], zero);
+        uint16_t hv[4];
+        for (int j = 0; j < 4; ++j) {
+          const float h = z[j] + b1v[nb];
+          m1[nb][j] = h > 0.f;
+          hv[j] = f32_to_bf16(h > 0.f ? h : 0.f);
+          row[(4 * g + j) * kRowPad + nb * 16 + r] = hv[j];
+        }
+        h1s[wave][nb][lane] = frag(hv[0], hv[1], hv[2], hv[3]);
       }
-      const float s = sum16(acc) + b3;
-      const uint64_t qq = tile * 16 + 4 * g + j;
-      const bool valid = qq < bt;
-      const float diff = valid ? s - y[idx[qq]] : 0.f;
-      ds[j] = diff * inv_bt;
+      wave_lds_sync();
+      v4f z2[4] = {zero, zero, zero, zero};
+      for (int kb = 0; kb < 4; ++kb) {
+        const v4s a2 = *reinterpret_cast<const v4s *>(row + r * kRowPad + kb * 16 + 4 * g);
+        for (int nb = 0; nb < 4; ++nb) z2[nb] = mfma(a2, b2f[kb][nb], z2[nb]);
+      }
+      wave_lds_sync();
+      v4f h2[4], ds, df;
+      for (int j = 0; j < 4; ++j) {
+        float acc = 0.f;
+        for (int nb = 0; nb < 4; ++nb) {
+          const float h = z2[nb][j] + b2v[nb];
+          h2[nb][j] = h > 0.f ? h : 0.f;
+          acc += h2[nb][j] * w3v[nb];
+        }
+        const float s = sum16(acc) + b3;
+        const bool valid = tile * 16 + 4 * g + j < bt;
+        const float target = __shfl(yv, 4 * g + j);
+        df[j] = valid ? s - target : 0.f;
+        ds[j] = df[j] * inv_bt;
+      }
       if (r == 0) {
-        lsum += 0.5f * diff * diff * inv_bt;
-        gb3 += ds[j];
+        dss[wave][g] = ds;
+        dfs[wave][g] = df;
+      }
+      for (int nb = 0; nb < 4; ++nb) {
+        uint16_t dv[4];
+        for (int j = 0; j < 4; ++j) {
+          const float d2 = h2[nb][j] > 0.f ? ds[j] * w3v[nb] : 0.f;
+          dv[j] = f32_to_bf16(d2);
+          row[(4 * g + j) * kRowPad + nb * 16 + r] = dv[j];
+        }
+        dz2s[wave][nb][lane] = frag(dv[0], dv[1], dv[2], dv[3]);
+        h2s[wave][nb][lane] = h2[nb];
+      }
+      wave_lds_sync();
+      // dH1 = dZ2 W2^T
+      v4f dh1[4] = {zero, zero, zero, zero};
+      for (int kb = 0; kb < 4; ++kb) {
+        const v4s ad = *reinterpret_cast<const v4s *>(row + r * kRowPad + kb * 16 + 4 * g);
+        for (int nb = 0; nb < 4; ++nb) dh1[nb] = mfma(ad, b2t[kb][nb], dh1[nb]);
+      }
+      for (int nb = 0; nb < 4; ++nb) {
+        v4f d1;
+        for (int j = 0; j < 4; ++j) d1[j] = m1[nb][j] ? dh1[nb][j] : 0.f;
+        d1s[wave][nb][lane] = d1;
       }
     }
-    for (int nb = 0; nb < 4; ++nb)
-      for (int j = 0; j < 4; ++j) {
-        gw3[nb] += h2[nb][j] * ds[j];
-        const float d2 = h2[nb][j] > 0.f ? ds[j] * w3v[nb] : 0.f;
-        gb2[nb] += d2;
-        dz2s[(4 * g + j) * kRowPad + nb * 16 + r] = f32_to_bf16(d2);
-      }
     __syncthreads();
-    // dW2 += H1^T dZ2 ; dH1 = dZ2 W2^T
-    v4s bd[4];
-    for (int nb = 0; nb < 4; ++nb) {
-      const uint16_t *c0 = dz2s + (4 * g) * kRowPad + nb * 16 + r;
-      bd[nb] = frag(c0[0], c0[kRowPad], c0[2 * kRowPad], c0[3 * kRowPad]);
+    load(base + kTrainWaves + wave);  // the next tiles' rows, while these are added up
+    // dW2 += H1^T dZ2: a D fragment is the A fragment of its transpose
+    for (int i = 0; i < live; ++i) {
+      const v4s at = h1s[i][mb][lane];
+      gW2a = mfma(at, dz2s[i][n0][lane], gW2a);
+      gW2b = mfma(at, dz2s[i][n0 + 1][lane], gW2b);
     }
-    for (int mb = 0; mb < 4; ++mb) {
-      const uint16_t *c0 = h1 + (4 * g) * kRowPad + mb * 16 + r;
-      const v4s at = frag(c0[0], c0[kRowPad], c0[2 * kRowPad], c0[3 * kRowPad]);
-      for (int nb = 0; nb < 4; ++nb) gW2[mb][nb] = mfma(at, bd[nb], gW2[mb][nb]);
-    }
-    v4f dh1[4] = {zero, zero, zero, zero};
-    for (int kb = 0; kb < 4; ++kb) {
-      const uint16_t *src = dz2s + r * kRowPad + kb * 16 + 4 * g;
-      const v4s ad = frag(src[0], src[1], src[2], src[3]);
-      for (int nb = 0; nb < 4; ++nb) dh1[nb] = mfma(ad, b2t[kb][nb], dh1[nb]);
-    }
-    for (int nb = 0; nb < 4; ++nb)
-      for (int j = 0; j < 4; ++j) {
-        const float d1 = m1[nb][j] ? dh1[nb][j] : 0.f;
-        gb1[nb] += d1;
-        dz1s[(4 * g + j) * kRowPad + nb * 16 + r] = f32_to_bf16(d1);
+    if (wave < 4) {
+      // dW1 += X^T dZ1
+      for (int i = 0; i < live; ++i) {
+        const uint16_t *xc = xs[i] + (4 * g) * kXPad + r;
+        const v4f d1 = d1s[i][ob][lane];
+        gW1 = mfma(frag(xc[0], xc[kXPad], xc[2 * kXPad], xc[3 * kXPad]),
+                   frag(f32_to_bf16(d1[0]), f32_to_bf16(d1[1]), f32_to_bf16(d1[2]), f32_to_bf16(d1[3])), gW1);
       }
-    __syncthreads();
-    // dW1 += X^T dZ1
-    const uint16_t *xc = xs + (4 * g) * kXPad + r;
-    const v4s ax = frag(xc[0], xc[kXPad], xc[2 * kXPad], xc[3 * kXPad]);
-    for (int nb = 0; nb < 4; ++nb) {
-      const uint16_t *c0 = dz1s + (4 * g) * kRowPad + nb * 16 + r;
-      const v4s bz = frag(c0[0], c0[kRowPad], c0[2 * kRowPad], c0[3 * kRowPad]);
-      gW1[nb] = mfma(ax, bz, gW1[nb]);
+      if (wave == 0)
+        for (int i = 0; i < live; ++i) {
+          const v4f df = dfs[i][g];
+          for (int j = 0; j < 4; ++j) {
+            const float diff = df[j];
+            lsum += 0.5f * diff * diff * inv_bt;
+            gb3 += diff * inv_bt;
+          }
+        }
+    } else {
+      for (int i = 0; i < live; ++i) {
+        const v4f h2 = h2s[i][ob][lane], d1 = d1s[i][ob][lane], ds = dss[i][g];
+        for (int j = 0; j < 4; ++j) {
+          gw3 += h2[j] * ds[j];
+          const float d2 = h2[j] > 0.f ? ds[j] * w3o : 0.f;
+          gb2 += d2;
+          gb1 += d1[j];
+        }
+      }
     }
     __syncthreads();
   }
-  // this wave's partial gradient (every entry written once; summed in a fixed
-  // order by k_sum_partials, so training is reproducible run to run)
-  MlpMaster *grad = reinterpret_cast<MlpMaster *>(partials + static_cast<uint64_t>(blockIdx.x * 4 + wave) *
-                                                                  kPartialStride);
-  for (int nb = 0; nb < 4; ++nb) {
-    const int c = nb * 16 + r;
-    for (int j = 0; j < 4; ++j) {
-      const int k1 = 4 * g + j;
-      grad->W1[k1 * kMlpHid + c] = gW1[nb][j];
-      for (int mb = 0; mb < 4; ++mb) grad->W2[(mb * 16 + k1) * kMlpHid + c] = gW2[mb][nb][j];
+  // this chain's partial gradient (every entry written once; summed in a fixed
+  // order by k_mlp_update)
+  float *out = partials + chain * kPartialStride;
+  MlpMaster *grad = reinterpret_cast<MlpMaster *>(out);
+  for (int j = 0; j < 4; ++j) {
+    float *w2 = grad->W2 + (mb * 16 + 4 * g + j) * kMlpHid + r;
+    w2[n0 * 16] = gW2a[j];
+    w2[(n0 + 1) * 16] = gW2b[j];
+  }
+  const int c = ob * 16 + r;
+  if (wave < 4) {
+    for (int j = 0; j < 4; ++j) grad->W1[(4 * g + j) * kMlpHid + c] = gW1[j];
+    const float t3 = sum_groups(gb3), tl = sum_groups(lsum);
+    if (wave == 0 && lane == 0) {
+      grad->b3 = t3;
+      out[kMlpMasterFloats] = tl;
     }
-    const float v1 = sum_groups(gb1[nb]), v2 = sum_groups(gb2[nb]), v3 = sum_groups(gw3[nb]);
+  } else {
+    const float v1 = sum_groups(gb1), v2 = sum_groups(gb2), v3 = sum_groups(gw3);
     if (g == 0) {
       grad->b1[c] = v1;
       grad->b2[c] = v2;
       grad->w3[c] = v3;
     }
   }
-  // gb3 and the loss live on lanes r == 0 (one per row group)
-  const float t3 = sum_groups(gb3), tl = sum_groups(lsum);
-  if (lane == 0) {
-    grad->b3 = t3;
-    partials[static_cast<uint64_t>(blockIdx.x * 4 + wave) * kPartialStride + kMlpMasterFloats] = tl;
-  }
 }
 
-// grad[i] = sum over waves of partials[w][i] (i < kMlpMasterFloats), loss
-// likewise from the slot after the parameters.
-__global__ void k_sum_partials(uint32_t waves, const float *partials, float *grad, float *loss) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i <= static_cast<uint32_t>(kMlpMasterFloats);
-       i += gridDim.x * blockDim.x) {
-    float s = 0.f;
-    for (uint32_t w = 0; w < waves; ++w) s += partials[static_cast<uint64_t>(w) * kPartialStride + i];
-    if (i < static_cast<uint32_t>(kMlpMasterFloats))
-      grad[i] = s;
-    else
-      *loss = s;
-  }
-}
-
-// Adam on the f32 parameters, then the bf16 copies.
-__global__ void k_adam(uint32_t count, float *p, float *m, float *v, const float *gr, float lr, float b1, float b2,
-                       float eps, float bc1, float bc2) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < count; i += gridDim.x * blockDim.x) {
-    const float gi = gr[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    p[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
+// The bf16 copies of parameter i, value p (parameters in MlpMaster's order).
+__device__ __forceinline__ void quantize(uint32_t i, float p, MlpBf16 *b) {
+  const uint16_t h = f32_to_bf16(p);
+  constexpr uint32_t w1 = kMlpInPad * kMlpHid, w2 = w1 + kMlpHid, w3 = w2 + kMlpHid * kMlpHid + kMlpHid;
+  static_assert(w2 == offsetof(MlpMaster, W2) / 4 && w3 == offsetof(MlpMaster, w3) / 4, "order of the parameters");
+  if (i < w1) {
+    b->W1t[(i % kMlpHid) * kMlpInPad + i / kMlpHid] = h;
+  } else if (i >= w2 && i < w2 + kMlpHid * kMlpHid) {
+    const uint32_t at = i - w2;
+    b->W2[at] = h;
+    b->W2t[(at % kMlpHid) * kMlpHid + at / kMlpHid] = h;
+  } else if (i >= w3 && i < w3 + kMlpHid) {
+    b->w3[i - w3] = h;
   }
 }
 
 __global__ void k_quantize(const MlpMaster *w, MlpBf16 *b) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < kMlpInPad * kMlpHid; i += gridDim.x * blockDim.x)
-    b->W1[i] = f32_to_bf16(w->W1[i]);
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < kMlpHid * kMlpHid; i += gridDim.x * blockDim.x)
-    b->W2[i] = f32_to_bf16(w->W2[i]);
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < kMlpHid; i += gridDim.x * blockDim.x)
-    b->w3[i] = f32_to_bf16(w->w3[i]);
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < static_cast<uint32_t>(kMlpMasterFloats)) quantize(i, reinterpret_cast<const float *>(w)[i], b);
 }
 
-// Mini-batch indices: uniform over [0, count) from a counter-based stream.
-__global__ void k_batch_idx(uint32_t bt, uint64_t count, GenStream s, uint64_t step, uint32_t *idx) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < bt; i += gridDim.x * blockDim.x)
-    idx[i] = static_cast<uint32_t>(gen_bounded(gen_value(s, step * bt + i), count));
+struct AdamStep {
+  float lr, b1, b2, eps, bc1, bc2;
+};
+
+// The batch's gradient and loss, the chains' partials added in their order:
+// 32 loads in flight a lane, since the sum of 64 partials is one chain of 64
+// additions behind them.  Then, in the same pass, Adam on the f32 parameters
+// and their bf16 copies (kApply), or the gradient alone.  Sum, Adam and copies
+// as three launches: 15 + 2 x 2.5 us at 64 chains; as one 4.1 us.
+template <bool kApply>
+__global__ __launch_bounds__(64) void k_mlp_update(uint32_t chains, const float *partials, float *grad, float *loss,
+                                                   AdamStep a, float *p, float *m, float *v, MlpBf16 *b) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i > static_cast<uint32_t>(kMlpMasterFloats)) return;
+  const float *src = partials + i;
+  float s = 0.f;
+  uint32_t w = 0;
+  for (; w + 32 <= chains; w += 32) {
+    float t[32];
+#pragma unroll
+    for (int k = 0; k < 32; ++k) t[k] = src[static_cast<uint64_t>(w + k) * kPartialStride];
+#pragma unroll
+    for (int k = 0; k < 32; ++k) s += t[k];
+  }
+#pragma unroll 4
+  for (; w < chains; ++w) s += src[static_cast<uint64_t>(w) * kPartialStride];
+  if (i == static_cast<uint32_t>(kMlpMasterFloats)) {
+    *loss = s;
+  } else if (kApply) {
+    const float mi = a.b1 * m[i] + (1.f - a.b1) * s;
+    const float vi = a.b2 * v[i] + (1.f - a.b2) * s * s;
+    m[i] = mi;
+    v[i] = vi;
+    const float pi = p[i] - a.lr * (mi / a.bc1) / (sqrtf(vi / a.bc2) + a.eps);
+    p[i] = pi;
+    quantize(i, pi, b);
+  } else {
+    grad[i] = s;
+  }
 }
 
 __global__ void k_append(uint64_t n, uint64_t stride, const float *X, const float *y, float *dX, float *dy) {
@@ -503,28 +593,37 @@ void from_public(const float *in, MlpMaster &w) {
 
 void upload(kc_mlp *m, const MlpMaster &w) {
   KC_HIP(hipMemcpyAsync(m->master, &w, sizeof(w), hipMemcpyHostToDevice, m->stream));
-  hipLaunchKernelGGL(k_quantize, dim3(16), dim3(kBlock), 0, m->stream, m->master, m->bf);
+  hipLaunchKernelGGL(k_quantize, dim3(grid_of(kMlpMasterFloats)), dim3(kBlock), 0, m->stream, m->master, m->bf);
   KC_LAUNCH_CHECK();
   KC_HIP(hipStreamSynchronize(m->stream));
   ++m->version;
 }
 
-// One pass of k_mlp_train over bt rows of idx: per-wave partials, then their
-// fixed-order sum into m->grad and m->loss.
-void train_pass(kc_mlp *m, uint64_t bt, const uint32_t *idx, const float *X, const float *y, hipStream_t s) {
+// One pass of k_mlp_train over bt rows, into `chains` partials; returns chains.
+uint32_t train_pass(kc_mlp *m, uint64_t bt, const BatchRows &rows, const float *X, const float *y, hipStream_t s) {
   const uint64_t tiles = (bt + 15) / 16;
-  // about 8 tiles per wave
-  const uint64_t blocks = std::max<uint64_t>(1, std::min<uint64_t>(1024, (tiles + 31) / 32));
-  const uint64_t waves = blocks * 4;
-  if (waves > m->partial_waves) {
-    m->partials = m->dalloc<float>(waves * kPartialStride);
-    m->partial_waves = waves;
+  // groups of four chains, about 8 tiles a chain
+  const uint64_t chains = 4 * std::max<uint64_t>(1, std::min<uint64_t>(1024, (tiles + 31) / 32));
+  if (chains > m->partial_chains) {
+    m->partials = m->dalloc<float>(chains * kPartialStride);
+    m->partial_chains = chains;
   }
-  hipLaunchKernelGGL(k_mlp_train, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, bt, idx, X, y, m->bf, m->master,
-                     m->partials);
+  hipLaunchKernelGGL(k_mlp_train, dim3(static_cast<unsigned>(chains)), dim3(64 * kTrainWaves), 0, s, bt, rows, X, y,
+                     m->bf, m->master, m->partials);
   KC_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_sum_partials, dim3(grid_of(kMlpMasterFloats + 1)), dim3(kBlock), 0, s,
-                     static_cast<uint32_t>(waves), m->partials, m->grad, m->loss);
+  return static_cast<uint32_t>(chains);
+}
+
+// The partials' sum: one Adam step (the loss to m->loss[slot]), or m->grad.
+void train_update(kc_mlp *m, uint32_t chains, const AdamStep *step, int slot, hipStream_t s) {
+  const dim3 grid(grid_of(kMlpMasterFloats + 1, 64)), block(64);
+  float *p = reinterpret_cast<float *>(m->master);
+  if (step)
+    hipLaunchKernelGGL(k_mlp_update<true>, grid, block, 0, s, chains, m->partials, m->grad, m->loss + slot, *step, p,
+                       m->adam_m, m->adam_v, m->bf);
+  else
+    hipLaunchKernelGGL(k_mlp_update<false>, grid, block, 0, s, chains, m->partials, m->grad, m->loss + slot,
+                       AdamStep{}, p, m->adam_m, m->adam_v, m->bf);
   KC_LAUNCH_CHECK();
 }
 
@@ -615,7 +714,7 @@ int kc_mlp_create(int32_t seed, kc_mlp **out) {
     m->adam_m = m->dalloc<float>(kMlpMasterFloats);
     m->adam_v = m->dalloc<float>(kMlpMasterFloats);
     m->grad = m->dalloc<float>(kMlpMasterFloats);
-    m->loss = m->dalloc<float>(1);
+    m->loss = m->dalloc<float>(2);
     fill_u32(reinterpret_cast<uint32_t *>(m->adam_m), kMlpMasterFloats, 0u, m->stream);
     fill_u32(reinterpret_cast<uint32_t *>(m->adam_v), kMlpMasterFloats, 0u, m->stream);
     // He-uniform initialisation from a counter-based stream
@@ -686,7 +785,7 @@ int kc_mlp_gradients(kc_mlp *m, const float *features, const float *targets, uin
     KC_HIP(hipMemcpyAsync(dX, features, n * kMlpIn * sizeof(float), hipMemcpyHostToDevice, m->stream));
     KC_HIP(hipMemcpyAsync(dy, targets, n * sizeof(float), hipMemcpyHostToDevice, m->stream));
     KC_HIP(hipMemcpyAsync(di, id.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, m->stream));
-    train_pass(m, n, di, dX, dy, m->stream);
+    train_update(m, train_pass(m, n, BatchRows{di, {}, 0, n}, dX, dy, m->stream), nullptr, 0, m->stream);
     MlpMaster g;
     KC_HIP(hipMemcpyAsync(&g, m->grad, sizeof(g), hipMemcpyDeviceToHost, m->stream));
     float l = 0.f;
@@ -761,36 +860,21 @@ int kc_mlp_train(kc_mlp *m, const kc_train_params *pp, kc_train_stats *st) {
     if (m->count == 0) fail(KC_ERR_INVALID, "mlp: empty dataset (collect traces first)");
     if (p.steps < 0 || p.batch < 16 || !(p.lr > 0.f)) fail(KC_ERR_INVALID, "mlp: bad training parameters");
     const uint32_t bt = static_cast<uint32_t>(p.batch);
-    if (bt > m->idx_cap) {
-      m->idx = m->dalloc<uint32_t>(bt);
-      m->idx_cap = bt;
-    }
     const GenStream rs = gen_stream(p.seed, 12);
     const auto t0 = std::chrono::steady_clock::now();
-    float first = -1.f, last = -1.f;
     for (int32_t step = 0; step < p.steps; ++step) {
-      hipLaunchKernelGGL(k_batch_idx, dim3(grid_of(bt)), dim3(kBlock), 0, m->stream, bt, m->count, rs,
-                         static_cast<uint64_t>(step), m->idx);
-      KC_LAUNCH_CHECK();
-      train_pass(m, bt, m->idx, m->X, m->y, m->stream);
+      const BatchRows rows{nullptr, rs, static_cast<uint64_t>(step) * bt, m->count};
+      const uint32_t chains = train_pass(m, bt, rows, m->X, m->y, m->stream);
       ++m->adam_t;
       const float bc1 = 1.f - std::pow(p.beta1, static_cast<float>(m->adam_t));
       const float bc2 = 1.f - std::pow(p.beta2, static_cast<float>(m->adam_t));
-      hipLaunchKernelGGL(k_adam, dim3(grid_of(kMlpMasterFloats)), dim3(kBlock), 0, m->stream,
-                         static_cast<uint32_t>(kMlpMasterFloats), reinterpret_cast<float *>(m->master), m->adam_m,
-                         m->adam_v, m->grad, p.lr, p.beta1, p.beta2, p.eps, bc1, bc2);
-      KC_LAUNCH_CHECK();
-      hipLaunchKernelGGL(k_quantize, dim3(16), dim3(kBlock), 0, m->stream, m->master, m->bf);
-      KC_LAUNCH_CHECK();
-      if (step == 0 || step == p.steps - 1) {
-        float l = 0.f;
-        KC_HIP(hipMemcpyAsync(&l, m->loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
-        KC_HIP(hipStreamSynchronize(m->stream));
-        if (step == 0) first = l;
-        last = l;
-      }
+      const AdamStep adam{p.lr, p.beta1, p.beta2, p.eps, bc1, bc2};
+      train_update(m, chains, &adam, step == 0 ? 0 : 1, m->stream);
     }
+    float loss[2] = {-1.f, -1.f};  // of the first and of the last step
+    if (p.steps > 0) KC_HIP(hipMemcpyAsync(loss, m->loss, sizeof(loss), hipMemcpyDeviceToHost, m->stream));
     KC_HIP(hipStreamSynchronize(m->stream));
+    const float first = loss[0], last = loss[p.steps == 1 ? 0 : 1];
     ++m->version;
     if (st) {
       std::memset(st, 0, sizeof(*st));
