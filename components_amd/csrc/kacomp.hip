@@ -265,10 +265,10 @@ struct kc_graph {
   uint64_t *d_huge_info = nullptr;
   uint64_t huge_info_cap = 0;
   int *flags = nullptr;
-  // [0..3] bin counters, [4] radius, [5] roots, [6] hubs found, [7] packed keys do not fit, [8] edges of
+  // [4] radius, [5] roots, [6] hubs found, [7] packed keys do not fit, [8] edges of
   // the tail, [9..12] its status, levels, sweeps, radius sum
   uint32_t *small = nullptr;
-  uint64_t *sizes = nullptr;  // [0] n_next [1] P [2] m2_next [3..5] dedup counters [8] N [9] clusters
+  uint64_t *sizes = nullptr;  // [0] n_next [1] P [2] m2_next [3..5] dedup counters [9] clusters
   // pinned host mirrors
   uint64_t *h_sizes = nullptr;
   uint32_t *h_small = nullptr;
@@ -397,6 +397,8 @@ constexpr uint64_t kDirectionMinDegree = 8;     // ... on levels of this average
 constexpr uint64_t kHugeBitmapBytes = 2ull << 30;  // above this the huge buckets use hash tables
 constexpr uint64_t kHugeMapBytes = 8ull << 30;     // byte maps of the largest huge buckets
 constexpr uint64_t kMapMinShare = 32;              // byte maps from C / 32 elements on
+constexpr uint64_t kDenseVertices = 1ull << 20;    // dense cluster ids above this many vertices ...
+constexpr uint64_t kDenseDegree = 8;               // ... at this average degree or more
 constexpr uint64_t kHubPullMin = 65536;            // smallest degree of a hub that pulls round 0
 
 
@@ -428,6 +430,28 @@ BinCfg bin_cfg(const kc_graph *g, const kc_options *o) {
   return bin_config(o->sweep_group_small, o->sweep_group_mid, o->sweep_group_large);
 }
 
+// The launches of make_bins into the given lists; after a synchronisation
+// read_bins has their sizes.
+void enqueue_bins(kc_graph *g, uint64_t n, const uint64_t *off, const BinCfg &cfg, Bins &b, uint32_t *lists,
+                  HubChunk *hubs, const uint64_t *key, uint32_t tmin, HostWords words = {}) {
+  b.listT = lists;
+  b.listS = lists + g->cap_n;
+  b.listW = lists + 2 * g->cap_n;
+  b.hubs = hubs;
+  TimedScope ts(g->timer, KC_K_BIN, (key ? 24 : 16) * n + 8);
+  bin_vertices(n, off, cfg, b.listT, b.listS, b.listW, b.hubs, g->h_small, key ? nullptr : g->deg_inter,
+               g->scan_scratch, g->stream, key, tmin, words);
+}
+
+void read_bins(kc_graph *g, Bins &b) {
+  b.nT = g->h_small[0];
+  b.nS = g->h_small[1];
+  b.nW = g->h_small[2];
+  b.nH = g->h_small[3];
+  if (b.nH > g->hubs_cap) fail(KC_ERR_INVALID, "hub chunk overflow (%u > %llu)", b.nH, (unsigned long long)g->hubs_cap);
+  finish_bins(b);
+}
+
 // Bins of the level CSR (one sync to size the binned launches).  With key,
 // only the vertices at key distance >= tmin, into the second set of lists.
 // Level 0's full bins go to their own lists and are reused by later calls
@@ -448,24 +472,10 @@ Bins make_bins(kc_graph *g, uint64_t n, const uint64_t *off, const BinCfg &cfg, 
   if (n > g->cap_n) fail(KC_ERR_INVALID, "internal: level of %llu vertices above the work set's %llu",
                          static_cast<unsigned long long>(n), static_cast<unsigned long long>(g->cap_n));
   Bins b;
-  uint32_t *lists = key ? g->flists : level0 ? g->l0_lists : g->lists;
-  b.listT = lists;
-  b.listS = lists + g->cap_n;
-  b.listW = lists + 2 * g->cap_n;
-  b.hubs = key ? g->fhubs : level0 ? g->l0_hubs : g->hubs;
-  {
-    TimedScope ts(g->timer, KC_K_BIN, (key ? 24 : 16) * n + 8);
-    bin_vertices(n, off, cfg, b.listT, b.listS, b.listW, b.hubs, g->small, key ? nullptr : g->deg_inter,
-                 g->scan_scratch, g->stream, key, tmin);
-  }
-  d2h(g, g->h_small, g->small, 4 * sizeof(uint32_t));
+  enqueue_bins(g, n, off, cfg, b, key ? g->flists : level0 ? g->l0_lists : g->lists,
+               key ? g->fhubs : level0 ? g->l0_hubs : g->hubs, key, tmin);
   sync(g);
-  b.nT = g->h_small[0];
-  b.nS = g->h_small[1];
-  b.nW = g->h_small[2];
-  b.nH = g->h_small[3];
-  if (b.nH > g->hubs_cap) fail(KC_ERR_INVALID, "hub chunk overflow (%u > %llu)", b.nH, (unsigned long long)g->hubs_cap);
-  finish_bins(b);
+  read_bins(g, b);
   if (level0) {
     g->l0_bins = b;
     g->l0_cfg = cfg;
@@ -533,7 +543,7 @@ uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t 
 // bitmaps over the label space (mode KC_DEDUP_AUTO: byte maps while they fit
 // their cap, then bitmaps) or in global tables processed in fixed-size chunks
 // planned on the host.  The medium and huge lists (n_medium, n_huge) come
-// from classify_buckets; total = elements of all buckets.  Returns the timer
+// from sum_segments or classify_buckets; total = elements of all buckets.  Returns the timer
 // slot of the first dedup launch (its algorithmic bytes are booked by the
 // caller).  `scratch` serves the scans (the handle's own scan scratch does not
 // exist yet while a generated graph's CSR is built).
@@ -1160,13 +1170,22 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
       KC_HIP(hipMemcpyAsync(rec.keys_copy, g->key, n_l * 8, hipMemcpyDeviceToDevice, g->stream));
     }
     fill_u32(g->small + 4, 1, 0, g->stream);
-    // dense cluster ids in label order: the buckets below hold them, so the
-    // dedup works over the C clusters instead of the n_l labels; the labels'
-    // pass marks the used ones
-    fill_u32(g->cid, n_l, 0, g->stream);  // the used-label flags, then the ids
+    // on a degree-ordered level 0 whose first kHotClusters positions hold a
+    // large share of the edge slots, the clusters of those positions take the
+    // ids below 65536, so the relabel keeps those positions' ids in LDS at 16
+    // bits (twice as many as at 32)
+    const bool hot_ids = pos_l != nullptr && g->l0_hot_skewed;
+    // The buckets hold labels; on large levels with long rows dense cluster ids
+    // in label order, so that the dedup's maps cover the C clusters instead of
+    // the n_l labels (marked by the labels' pass): R-MAT 24 in input order 12.17
+    // -> 11.11 ms a call, G(2^22, 2^24) 5.55 -> 5.45; with shorter rows the
+    // ranks cost more (the 256^3 grid 7.41 -> 7.76, G(2^22, 2^23) 4.22 -> 4.30).
+    const bool dense = hot_ids || (n_l > kDenseVertices && m2_l >= kDenseDegree * n_l);
+    uint32_t *sum = g->sk;
+    if (dense) fill_u32(g->cid, n_l, 0, g->stream);  // the used-label flags, then the ids
     {
       TimedScope ts(g->timer, KC_K_COUNT, 8 * n_l + 4 * n_l + 4 * n_l + (local ? 0 : 8 * n_l));
-      labels_radius(n_l, g->key, pos_l, rec.lab, g->small + 4, !local && !pre, g->stream, g->cid);
+      labels_radius(n_l, g->key, pos_l, rec.lab, g->small + 4, !local && !pre, g->stream, dense ? g->cid : nullptr, sum);
     }
     if (g->collect && !pre) {
       // trace of the plain method: features and the log2 size of each vertex's cluster
@@ -1175,22 +1194,19 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
       cluster_targets(n_l, rec.lab, g->csize, g->target, g->stream);
       mlp_append(g->collect, n_l, g->feat, g->target, g->collect_stride, g->stream);
     }
-    // on a degree-ordered level 0 whose first kHotClusters positions hold a
-    // large share of the edge slots, the clusters of those positions take the
-    // ids below 65536, so the relabel keeps those positions' ids in LDS at 16
-    // bits (twice as many as at 32)
-    const bool hot_ids = pos_l != nullptr && g->l0_hot_skewed;
-    {
-      TimedScope ts(g->timer, KC_K_COUNT, 8 * n_l);
-      if (hot_ids)
-        cluster_ranks_hot(n_l, std::min<uint64_t>(n_l, kHotClusters), rec.lab, g->cid, g->crank, g->sizes + 9,
-                          g->scan_scratch, g->stream);
-      else
-        cluster_ranks(n_l, g->cid, g->crank, g->sizes + 9, g->scan_scratch, g->stream);
-    }
-    {
+    const uint32_t *cid = rec.lab;  // what the buckets hold: labels, or cluster ids
+    if (dense) {
+      {
+        TimedScope ts(g->timer, KC_K_COUNT, 8 * n_l);
+        if (hot_ids)
+          cluster_ranks_hot(n_l, std::min<uint64_t>(n_l, kHotClusters), rec.lab, g->cid, g->crank, g->sizes + 9,
+                            g->scan_scratch, g->stream);
+        else
+          cluster_ranks(n_l, g->cid, g->crank, g->sizes + 9, g->scan_scratch, g->stream);
+      }
       TimedScope ts(g->timer, KC_K_COUNT, 12 * n_l);
       cluster_ids(n_l, rec.lab, g->crank, g->cid, g->stream);
+      cid = g->cid;
     }
     // relabel: every row packs the cluster ids of its far ends outside its
     // cluster at the start of its slots; the slot buffer later takes the unique
@@ -1221,53 +1237,30 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
       relabel_slot = ts.slot;
       // the hot-label launch pays off on the degree-ordered level 0
       if (split)
-        relabel_split(off_l, col_l, g->cid, n_l, b, g->l0_pieces, g->l0_part_list, g->l0_part_at, relab,
+        relabel_split(off_l, col_l, cid, n_l, b, g->l0_pieces, g->l0_part_list, g->l0_part_at, relab,
                       g->deg_inter, r_inter, n_l, g->stream);
       else
-        relabel(off_l, col_l, g->cid, b, relab, g->deg_inter, g->hub_inter, pos_l || level_hot ? n_l : 0,
+        relabel(off_l, col_l, cid, b, relab, g->deg_inter, g->hub_inter, pos_l || level_hot ? n_l : 0,
                 g->stream, hot_ids);
     }
     if (rb.nH) {
       TimedScope ts(g->timer, KC_K_COUNT, 12ull * rb.nH + 4ull * rb.nH);
       hub_fold(rb, r_inter, g->deg_inter, r_pos, r_prefix, g->scan_scratch, g->stream);
     }
-    // clusters as segments of the (label, vertex) list sorted by label
     {
-      TimedScope ts(g->timer, KC_K_SCAN, 2 * 4 * n_l + 8 * n_l + 8 * n_l);
-      select_inter(n_l, g->key, g->deg_inter, g->sk, g->sv, g->sizes + 8, g->scan_scratch, g->stream);
+      TimedScope ts(g->timer, KC_K_SCAN, 4 * n_l + 4 * n_l + 4 * n_l);
+      cluster_sums(n_l, rec.lab, g->deg_inter, sum, g->pos_of, g->stream);
     }
-    d2h(g, g->h_sizes + 8, g->sizes + 8, 2 * sizeof(uint64_t));
+    {
+      TimedScope ts(g->timer, KC_K_SCAN, 2 * 4 * n_l + 4 * n_l);
+      sum_segments(n_l, sum, gid_l, dense ? g->crank : nullptr, rec.newidx, g->seg_of_cid, gid_next, g->seg_off,
+                   g->dl_medium, g->dl_huge, g->small + 4, dense ? g->sizes + 9 : nullptr, g->h_sizes, g->h_small + 4,
+                   g->scan_scratch, g->stream);
+    }
     sync(g);
-    const uint64_t N = g->h_sizes[8];
-    const uint64_t clusters = g->h_sizes[9];
-    int bits = 1;
-    while (bits < 32 && (1ull << bits) < n_l) ++bits;
-    int which = 0;
-    {
-      TimedScope ts(g->timer, KC_K_SORT, 24 * N * static_cast<uint64_t>((bits + 7) / 8));
-      which = radix_sort_pairs(N, bits, g->sk, g->sv, g->sk2, g->sv2, g->sort_scratch, g->stream);
-    }
-    const uint32_t *sk = which ? g->sk2 : g->sk, *sv = which ? g->sv2 : g->sv;
-    fill_u32(rec.newidx, n_l, kNone, g->stream);
-    {
-      TimedScope ts(g->timer, KC_K_SCAN, 2 * (8 * N + 4 * N) + 4 * N + 20 * n_l / 8);
-      // the sort's other buffer pair is free: it caches the gathered counts
-      segments(N, sk, sv, g->deg_inter, gid_l, g->crank, g->pos_of, rec.newidx, g->seg_of_cid, gid_next, g->seg_off,
-               g->sizes, which ? g->sk : g->sk2, g->scan_scratch, g->stream);
-    }
-    // medium and huge buckets listed before the sizes come back (the
-    // clusters bound n_next)
-    {
-      TimedScope ts(g->timer, KC_K_SCAN, 16 * clusters + 4 * clusters / 8);
-      classify_buckets(std::min(N, clusters), g->sizes, g->seg_off, g->dl_medium, g->dl_huge, g->sizes + 3,
-                       g->scan_scratch, g->stream);
-    }
-    d2h(g, g->h_sizes, g->sizes, 5 * sizeof(uint64_t));
-    d2h(g, g->h_small + 4, g->small + 4, sizeof(uint32_t));
-    sync(g);
-    const uint64_t n_next = N ? g->h_sizes[0] : 0;
-    const uint64_t P = N ? g->h_sizes[1] : 0;
-    const uint64_t n_medium = N ? g->h_sizes[3] : 0, n_huge = N ? g->h_sizes[4] : 0;
+    const uint64_t label_space = dense ? g->h_sizes[9] : n_l;
+    const uint64_t n_next = g->h_sizes[0], P = g->h_sizes[1];
+    const uint64_t n_medium = g->h_sizes[3], n_huge = g->h_sizes[4];
     rec.radius = local || pre ? 0 : g->h_small[4];
     if (!pre) out.sweeps += sweeps;  // the block passes are not decomposition sweeps
     out.radius_sum += rec.radius;
@@ -1283,31 +1276,41 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
     {
       g->timer.retag(relabel_slot, KC_K_RELABEL, 8 * (n_l + 1) + 8 * m2_l + 8 * n_l + 4 * P);
       TimedScope ts(g->timer, KC_K_SCATTER, 8 * (n_l + 1) + 8 * n_l + 8 * P);
-      scatter(off_l, relab, rb, g->deg_inter, r_inter, r_pos, g->pos_of, bucket, g->stream);
+      scatter(off_l, relab, rb, g->deg_inter, r_inter, r_pos, g->pos_of, rec.lab, sum, bucket, g->stream);
     }
     const int dedup_slot = dedup_buckets(g, n_next, g->seg_off, bucket, g->slots, g->uniq, g->dl_medium, g->dl_huge,
-                                         n_medium, n_huge, P, clusters, g->scan_scratch, o->dedup_huge);
+                                         n_medium, n_huge, P, label_space, g->scan_scratch, o->dedup_huge);
     // next-level CSR
+    int csr_slot;
     {
       TimedScope ts(g->timer, KC_K_SCAN, 4 * n_next + 8 * (n_next + 1));
       csr_offsets(n_next, g->uniq, off_next, g->sizes, g->scan_scratch, g->stream);
     }
-    d2h(g, g->h_sizes + 2, g->sizes + 2, sizeof(uint64_t));
+    {
+      // unique runs read, mapped to next-level indices, written
+      TimedScope ts(g->timer, KC_K_CSR, 0);
+      csr_slot = ts.slot;
+      gather_uniques(n_next, off_next, g->seg_off, g->slots, dense ? g->seg_of_cid : rec.newidx, g->dl_medium, n_medium,
+                     g->dl_huge, n_huge, g->row_cstart, g->scan_scratch, col_next, g->stream);
+    }
+    // the next level's bins, unless it may be one that needs none, go in
+    // before its size comes back: one synchronisation for both
     const uint64_t hot_rows = std::min<uint64_t>(n_next, kLevelHotRows);
-    d2h(g, g->h_sizes + 15, off_next + hot_rows, sizeof(uint64_t));
+    const HostWords words{{g->sizes + 2, off_next + hot_rows}, {g->h_sizes + 2, g->h_sizes + 15}};
+    bins_valid = !(use_tail && n_next <= kTailVertices);
+    if (bins_valid)
+      enqueue_bins(g, n_next, off_next, cfg, b, g->lists, g->hubs, nullptr, 0, words);
+    else
+      publish_words(words, g->stream);
     sync(g);
+    if (bins_valid) read_bins(g, b);
     const uint64_t m2_next = g->h_sizes[2];
     level_hot = m2_next > 0 && static_cast<double>(g->h_sizes[15]) * n_next >=
                                    kHotShareFactor * static_cast<double>(hot_rows) * m2_next;
     // dedup: every bucket slot read once, the unique ones written, per
     // cluster its bucket bounds and its unique count
     g->timer.retag(dedup_slot, KC_K_DEDUP, 4 * P + 4 * m2_next + 8 * (n_next + 1) + 4 * n_next);
-    {
-      // unique runs read, mapped to next-level indices, written
-      TimedScope ts(g->timer, KC_K_CSR, 4 * m2_next + 4 * m2_next + 4 * m2_next);
-      gather_uniques(n_next, off_next, g->seg_off, g->slots, g->seg_of_cid, g->dl_medium, n_medium, g->dl_huge, n_huge,
-                     g->row_cstart, g->scan_scratch, col_next, g->stream);
-    }
+    g->timer.retag(csr_slot, KC_K_CSR, 4 * m2_next + 4 * m2_next + 4 * m2_next);
     n_l = n_next;
     m2_l = m2_next;
     off_l = off_next;
@@ -1317,7 +1320,6 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
     idx_l = nullptr;
     pos_l = nullptr;
     pp ^= 1;
-    bins_valid = false;
     input_level0 = false;
     if (!pre) ++iteration;
   }
@@ -1659,7 +1661,7 @@ void build_device_csr(kc_graph *g, uint64_t n, const uint32_t *src, const uint32
   uint32_t *medium = lists.as<uint32_t>();
   uint32_t *huge = medium + n + 2;
   DevTemp runs(P * 4 + 64);
-  classify_buckets(n, nullptr, off_tmp.as<uint64_t>(), medium, huge, g->sizes + 3, scratch.as<uint64_t>(), s);
+  classify_buckets(n, off_tmp.as<uint64_t>(), medium, huge, g->sizes + 3, scratch.as<uint64_t>(), s);
   KC_HIP(hipMemcpyAsync(g->h_sizes + 3, g->sizes + 3, 16, hipMemcpyDeviceToHost, s));
   KC_HIP(hipStreamSynchronize(s));
   const uint64_t n_medium = g->h_sizes[3], n_huge = g->h_sizes[4];

@@ -92,6 +92,13 @@ void init_keys_uniform(uint64_t n, const uint32_t *gid, const uint32_t *idx, int
                        hipStream_t s);
 void deviates_only(uint32_t gid0, uint32_t count, DeviateArgs d, uint32_t *out, hipStream_t s);
 
+// Up to two words of device memory to the host's pinned memory.
+struct HostWords {
+  const uint64_t *from[2];
+  uint64_t *to[2];
+};
+void publish_words(HostWords words, hipStream_t s);
+
 // Bins vertices of a CSR by degree (stable, no global atomics); counters[0..3]
 // receive nT, nS, nW, nH.  deg_inter of degree-0 vertices is cleared.
 // scratch: bin_scratch_words(n) words.
@@ -100,7 +107,7 @@ void deviates_only(uint32_t gid0, uint32_t count, DeviateArgs d, uint32_t *out, 
 void round_volumes(uint64_t n, const uint64_t *off, const uint64_t *key, uint32_t t, uint64_t *out, hipStream_t s);
 void bin_vertices(uint64_t n, const uint64_t *off, BinCfg cfg, uint32_t *listT, uint32_t *listS,
                   uint32_t *listW, HubChunk *hubs, uint32_t *counters, uint32_t *deg_inter, uint64_t *scratch,
-                  hipStream_t s, const uint64_t *key = nullptr, uint32_t tmin = 0);
+                  hipStream_t s, const uint64_t *key = nullptr, uint32_t tmin = 0, HostWords words = {});
 void finish_bins(Bins &b);  // computes block offsets from the counts
 uint64_t bin_scratch_words(uint64_t n);
 
@@ -181,7 +188,7 @@ void block_interface(const uint64_t *off, const uint32_t *col, uint64_t n, uint6
 // used (may be null, pre-zeroed): used[lab[v]] = 1, the used-label flags of
 // cluster_ranks.
 void labels_radius(uint64_t n, const uint64_t *key, const uint32_t *pos, uint32_t *lab, uint32_t *radius,
-                   bool with_radius, hipStream_t s, uint32_t *used = nullptr);
+                   bool with_radius, hipStream_t s, uint32_t *used = nullptr, uint32_t *zero = nullptr);
 // Dense cluster ids in label order from the used-label flags (labels_radius):
 // rank[a] = number of used labels below a, written for the used ones, and
 // *count (device) = number of clusters C; then cid[v] = rank[lab[v]] in [0, C).
@@ -198,17 +205,20 @@ constexpr uint64_t kHotClusters = 57344;
 // the relabel depends on it.
 void cluster_ranks_hot(uint64_t n, uint64_t k, const uint32_t *lab, uint32_t *used, uint32_t *rank, uint64_t *count,
                        uint64_t *scratch, hipStream_t s);
-// (label, vertex) of every vertex with a cluster edge; *count (device) = N.
-void select_inter(uint64_t n, const uint64_t *key, const uint32_t *deg_inter, uint32_t *sk, uint32_t *sv,
-                  uint64_t *count, uint64_t *scratch, hipStream_t s);
-// Over the label-sorted list: pos_of[v] = write position of v's cluster edges,
-// newidx[a] = next-level index of label a (caller pre-fills kNone),
-// seg_of_cid[rank[a]] = the same index by dense cluster id, gid_next by
-// next-level index, seg_off[0..n_next] bucket offsets; sizes[0] = n_next,
-// sizes[1] = P (cluster edges).  cache: N words of scratch.
-void segments(uint64_t N, const uint32_t *sk, const uint32_t *sv, const uint32_t *deg_inter, const uint32_t *gid,
-              const uint32_t *rank, uint32_t *pos_of, uint32_t *newidx, uint32_t *seg_of_cid, uint32_t *gid_next,
-              uint64_t *seg_off, uint64_t *sizes, uint32_t *cache, uint64_t *scratch, hipStream_t s);
+// Clusters and their buckets: sum (zeroed, one word per label) takes every
+// cluster's edge count, pos_of[v] the place of v's edges in its cluster's
+// bucket; sum_segments then writes newidx[a] = next-level index of label a
+// (kNone: no cluster edge), seg_of_cid[rank[a]] = the same by dense cluster id
+// (rank null: not), gid_next by next-level index, seg_off[0..n_next] bucket
+// offsets, in sum every bucket's start and the lists of medium and huge
+// buckets; and to the host (pinned) host_sizes[0] = n_next, [1] = cluster edges,
+// [3], [4] = medium, huge buckets, [9] = *ids (ids null: not) and the radius.
+void cluster_sums(uint64_t n, const uint32_t *lab, const uint32_t *deg_inter, uint32_t *sum, uint32_t *pos_of,
+                  hipStream_t s);
+void sum_segments(uint64_t n, uint32_t *sum, const uint32_t *gid, const uint32_t *rank, uint32_t *newidx,
+                  uint32_t *seg_of_cid, uint32_t *gid_next, uint64_t *seg_off, uint32_t *medium, uint32_t *huge,
+                  const uint32_t *radius, const uint64_t *ids, uint64_t *host_sizes, uint32_t *host_radius,
+                  uint64_t *scratch, hipStream_t s);
 
 // The labels lab[col[e]] of row v that differ from lab[v] (after a best-effort
 // LDS filter of repeats), packed at relab[off[v] ...] (hub chunks: at the
@@ -251,13 +261,13 @@ void write_pieces(uint64_t n, const uint64_t *off, const uint32_t *col, uint32_t
 // Copies the deg_inter[v] packed relab slots of every row (hub chunks:
 // hub_inter) to bucket[pos_of[v] + ...].
 void scatter(const uint64_t *off, const uint32_t *relab, const Bins &b, const uint32_t *deg_inter,
-             const uint32_t *hub_inter, const uint32_t *hub_pos, const uint32_t *pos_of, uint32_t *bucket,
-             hipStream_t s);
+             const uint32_t *hub_inter, const uint32_t *hub_pos, const uint32_t *pos_of, const uint32_t *lab,
+             const uint32_t *start, uint32_t *bucket, hipStream_t s);
 
 // Dedup of every bucket a2 (elements [seg_off[a2], seg_off[a2+1]) of bucket):
 // its uniq[a2] distinct values go to out[seg_off[a2] ...] in any order.  Small
 // buckets in wave LDS tables (dedup_small, which skips the others); medium
-// and huge ones are listed first by classify_buckets.
+// and huge ones are listed first (sum_segments, classify_buckets).
 constexpr uint32_t kDedupWaveCap = 512;
 constexpr uint32_t kDedupBlockCap = 8192;
 constexpr uint64_t kHugeChunk = 16384;  // elements (or table slots) per huge-bucket chunk (tables)
@@ -272,11 +282,10 @@ struct HugeChunk {
   uint32_t a2;        // bucket (next-level vertex)
   uint32_t pad;
 };
-// Medium (wave cap < size <= block cap) and huge (above) buckets among the
-// first *n_dev (or n when n_dev is null; n bounds *n_dev), listed in
+// Medium (wave cap < size <= block cap) and huge (above) buckets of n, listed in
 // increasing order: counts[0] = medium, counts[1] = huge.  scratch: scan scratch.
-void classify_buckets(uint64_t n, const uint64_t *n_dev, const uint64_t *seg_off, uint32_t *medium, uint32_t *huge,
-                      uint64_t *counts, uint64_t *scratch, hipStream_t s);
+void classify_buckets(uint64_t n, const uint64_t *seg_off, uint32_t *medium, uint32_t *huge, uint64_t *counts,
+                      uint64_t *scratch, hipStream_t s);
 void dedup_small(uint64_t n_next, const uint64_t *seg_off, const uint32_t *bucket, uint32_t *out, uint32_t *uniq,
                  hipStream_t s);
 void dedup_medium(uint32_t n_medium, const uint32_t *medium, const uint64_t *seg_off, const uint32_t *bucket,
@@ -306,7 +315,7 @@ void csr_offsets(uint64_t n_next, const uint32_t *uniq, uint64_t *off_next, uint
                  uint64_t *scratch, hipStream_t s);
 // col_next[off_next[a2] + i] = map[vals[seg_off[a2] + i]] for i < uniq[a2]
 // (map null: the value itself): the unique runs of the dedup, concatenated.
-// medium/huge: the listed buckets (classify_buckets); cstart: n_medium +
+// medium/huge: the listed buckets; cstart: n_medium +
 // n_huge + 1 words for their chunk plan; scratch: scan scratch.
 void gather_uniques(uint64_t n_next, const uint64_t *off_next, const uint64_t *seg_off, const uint32_t *vals,
                     const uint32_t *map, const uint32_t *medium, uint64_t n_medium, const uint32_t *huge,

@@ -182,11 +182,18 @@ __global__ __launch_bounds__(kBlock) void k_bin_write(uint64_t n, const uint64_t
   }
 }
 
-__global__ void k_bin_totals(const uint64_t *prefix, const uint64_t *total, uint32_t nblocks, uint32_t *counters) {
+// The bins' sizes (to device memory or the host's pinned memory) and up to two
+// words more to the host: one launch ahead of a synchronisation in place of a
+// copy for each.
+__global__ void k_bin_totals(const uint64_t *prefix, const uint64_t *total, uint32_t nblocks, uint32_t *counters,
+                             HostWords words) {
   const int r = threadIdx.x;
-  if (r >= 4) return;
-  const uint64_t hi = r < 3 ? prefix[static_cast<uint64_t>(r + 1) * nblocks] : *total;
-  counters[r] = static_cast<uint32_t>(hi - prefix[static_cast<uint64_t>(r) * nblocks]);
+  if (r < 4 && prefix) {
+    const uint64_t hi = r < 3 ? prefix[static_cast<uint64_t>(r + 1) * nblocks] : *total;
+    counters[r] = static_cast<uint32_t>(hi - prefix[static_cast<uint64_t>(r) * nblocks]);
+  } else if (r >= 4 && r < 6 && words.from[r - 4]) {
+    words.to[r - 4][0] = *words.from[r - 4];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -872,8 +879,8 @@ __global__ __launch_bounds__(kBlock) void k_block_interface(const uint64_t *off,
 // Grid-stride, with one atomic per workgroup: atomics on one address are
 // serialised by the device, so one per wave cost more than the pass itself.
 __global__ __launch_bounds__(kBlock) void k_labels_radius(uint64_t n, const uint64_t *key, const uint32_t *pos,
-                                                         uint32_t *lab, uint32_t *used, uint32_t *radius,
-                                                         int with_radius) {
+                                                         uint32_t *lab, uint32_t *used, uint32_t *zero,
+                                                         uint32_t *radius, int with_radius) {
   __shared__ uint32_t wave_max[kBlock / kWave];
   uint32_t r = 0;
   // four vertices per lane per step, so that their chains of dependent loads
@@ -892,6 +899,7 @@ __global__ __launch_bounds__(kBlock) void k_labels_radius(uint64_t n, const uint
       const uint32_t l = static_cast<uint32_t>(k[u]);
       lab[v] = l;
       if (used) used[l] = 1;
+      if (zero) zero[v] = 0;
     }
     if (with_radius) {
 #pragma unroll
@@ -1089,71 +1097,111 @@ void scan_exclusive(uint64_t n, Load load, Store store, T *total, uint64_t *scra
   KC_LAUNCH_CHECK();
 }
 
-// ---------------------------------------------------------------------------
-// Clusters from the (label, vertex) list sorted by label: every vertex with a
-// cluster edge is selected, the list is sorted, and one scan over the sorted
-// list yields each cluster's next-level index (segment number), its bucket
-// offset and every vertex's write position -- no atomics.
-struct SelectLoad {
-  const uint32_t *deg_inter;
-  __device__ uint64_t operator()(uint64_t i) const { return deg_inter[i] != 0 ? 1ull : 0ull; }
-};
-struct SelectStore {
-  const uint64_t *key;
-  uint32_t *sk, *sv;
-  __device__ void operator()(uint64_t i, uint64_t prefix, uint64_t v) const {
-    if (v) {
-      sk[prefix] = static_cast<uint32_t>(key[i]);
-      sv[prefix] = static_cast<uint32_t>(i);
-    }
-  }
-};
-
-// (segment head, cluster-edge count) of item i.  The first pass of the scan
-// gathers the count by vertex and keeps it in `cache` in item order; the
-// second pass reads it from there instead of gathering again.
-struct SegLoad {
-  const uint32_t *sk, *sv, *deg_inter;
-  uint32_t *cache;
-  __device__ Pair64 operator()(uint64_t i) const {
-    const uint32_t a = sk[i];
-    const bool head = i == 0 || sk[i - 1] != a;
-    const uint32_t d = deg_inter[sv[i]];
-    cache[i] = d;
-    return {head ? 1ull : 0ull, d};
-  }
-};
-struct SegLoadCached {
-  const uint32_t *sk, *cache;
-  __device__ Pair64 operator()(uint64_t i) const {
-    const uint32_t a = sk[i];
-    const bool head = i == 0 || sk[i - 1] != a;
-    return {head ? 1ull : 0ull, cache[i]};
-  }
-};
-struct SegStore {
-  const uint32_t *sk, *sv, *gid, *rank;
-  uint32_t *pos_of, *newidx, *seg_of_cid, *gid_next;
-  uint64_t *seg_off;
-  __device__ void operator()(uint64_t i, Pair64 prefix, Pair64 v) const {
-    pos_of[sv[i]] = static_cast<uint32_t>(prefix.b);
-    if (v.a) {
-      const uint32_t a = sk[i];
-      const uint32_t seg = static_cast<uint32_t>(prefix.a);
-      newidx[a] = seg;
-      seg_of_cid[rank[a]] = seg;
-      gid_next[seg] = gid ? gid[a] : a;
-      seg_off[seg] = prefix.b;
-    }
-  }
-};
-
-__global__ void k_seg_finish(const Pair64 *total, uint64_t *seg_off, uint64_t *sizes) {
-  seg_off[total->a] = total->b;
-  sizes[0] = total->a;
-  sizes[1] = total->b;
-}
 __global__ void k_copy_total(const uint64_t *t, uint64_t *dst) { *dst = *t; }
+
+// ---------------------------------------------------------------------------
+// Clusters and their buckets.  Every vertex with a cluster edge takes its place
+// in its cluster's bucket from the cluster's running sum, and one scan over the
+// labels then numbers the clusters (in label order), places their buckets and
+// lists the medium and huge ones.  The order inside a bucket is free: its dedup
+// does not see it.
+//
+// The running sums are atomics, about 8.5 a ns over distinct words but one
+// after another on one word, and a few clusters can hold most of the vertices.
+// So a workgroup first adds up its 4096 vertices by cluster in an LDS table,
+// with one device atomic for every cluster it meets: R-MAT 24's level 1 takes as
+// long as by a radix sort of the (label, vertex) pairs (whole call 10.8 ms both;
+// 12.1 with an atomic per vertex, merged over a wave only for the first lane's
+// cluster, 11.1 merged for eight), and the sort's 18 launches and a
+// synchronisation a level are gone: G(2^20, 2^22) 2.21 -> 1.85 ms a call, the
+// 256^3 grid 8.23 -> 7.42, random geometric 2 M vertices 2.34 -> 1.9, R-MAT 22
+// 3.75 -> 3.64, local contraction of 700 k vertices 1.23 -> 0.99.
+constexpr int kSumBlock = 1024, kSumPer = 4;  // 64 KB of LDS: two workgroups a CU
+__global__ __launch_bounds__(kSumBlock) void k_cluster_sums(uint64_t n, const uint32_t *lab, const uint32_t *deg_inter,
+                                                           uint32_t *sum, uint32_t *pos_of) {
+  constexpr int B = kSumBlock, kPer = kSumPer;
+  constexpr uint32_t kSlots = 2 * B * kPer;  // a power of two, twice the vertices of a block
+  __shared__ uint32_t key[kSlots], part[kSlots];
+  for (uint32_t i = threadIdx.x; i < kSlots; i += B) {
+    key[i] = kNone;
+    part[i] = 0;
+  }
+  const uint64_t v0 = blockIdx.x * static_cast<uint64_t>(B * kPer) + threadIdx.x;
+  uint32_t l[kPer], d[kPer], slot[kPer], at[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const uint64_t v = v0 + u * B;
+    d[u] = v < n ? deg_inter[v] : 0u;
+    l[u] = v < n ? lab[v] : 0u;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    if (!d[u]) continue;
+    uint32_t h = hash32(l[u]) & (kSlots - 1);
+    while (true) {
+      uint32_t cur = key[h];
+      if (cur == kNone) cur = atomicCAS(&key[h], kNone, l[u]);
+      if (cur == kNone || cur == l[u]) break;
+      h = (h + 1) & (kSlots - 1);
+    }
+    slot[u] = h;
+    at[u] = atomicAdd(&part[h], d[u]);
+  }
+  __syncthreads();
+  uint32_t base[kSlots / B];
+#pragma unroll
+  for (uint32_t u = 0; u < kSlots / B; ++u) {
+    const uint32_t i = u * B + threadIdx.x;
+    base[u] = key[i] != kNone ? atomicAdd(&sum[key[i]], part[i]) : 0u;
+  }
+#pragma unroll
+  for (uint32_t u = 0; u < kSlots / B; ++u) part[u * B + threadIdx.x] = base[u];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kPer; ++u)
+    if (d[u]) pos_of[v0 + u * B] = part[slot[u]] + at[u];
+}
+
+// (clusters, medium buckets in the upper half; cluster edges, huge buckets above
+// kSumHuge)
+constexpr int kSumHuge = 40;  // a level has fewer than 2^32 edge slots: at most 2^19 huge buckets
+struct SumLoad {
+  const uint32_t *sum;
+  __device__ Pair64 operator()(uint64_t l) const {
+    const uint64_t d = sum[l];
+    const uint64_t medium = d > kDedupWaveCap && d <= kDedupBlockCap, huge = d > kDedupBlockCap;
+    return {(d != 0) | medium << 32, d | huge << kSumHuge};
+  }
+};
+__device__ __forceinline__ uint64_t sum_edges(uint64_t b) { return b & ((1ull << kSumHuge) - 1); }
+struct SumStore {
+  uint32_t *sum, *newidx, *seg_of_cid, *gid_next, *medium, *huge;
+  const uint32_t *gid, *rank;  // rank null: the buckets hold labels
+  uint64_t *seg_off;
+  __device__ void operator()(uint64_t l, Pair64 prefix, Pair64 v) const {
+    const uint32_t at = static_cast<uint32_t>(prefix.a);
+    newidx[l] = v.a ? at : kNone;
+    if (!v.a) return;
+    sum[l] = static_cast<uint32_t>(prefix.b);
+    if (rank) seg_of_cid[rank[l]] = at;
+    gid_next[at] = gid ? gid[l] : static_cast<uint32_t>(l);
+    seg_off[at] = sum_edges(prefix.b);
+    if (v.a >> 32) medium[prefix.a >> 32] = at;
+    if (v.b >> kSumHuge) huge[prefix.b >> kSumHuge] = at;
+  }
+};
+__global__ void k_sum_finish(const Pair64 *total, uint64_t *seg_off, const uint32_t *radius, uint64_t *host_sizes,
+                             uint32_t *host_radius, const uint64_t *ids) {
+  const uint64_t clusters = static_cast<uint32_t>(total->a), edges = sum_edges(total->b);
+  if (ids) host_sizes[9] = *ids;
+  seg_off[clusters] = edges;
+  host_sizes[0] = clusters;
+  host_sizes[1] = edges;
+  host_sizes[3] = total->a >> 32;
+  host_sizes[4] = total->b >> kSumHuge;
+  *host_radius = *radius;
+}
 
 // ---------------------------------------------------------------------------
 // Scatter of cluster edges into buckets (binned like the sweep).
@@ -1168,8 +1216,13 @@ struct ScatterArgs {
   const uint32_t *hub_inter;
   const uint32_t *hub_pos;
   const uint32_t *pos_of;
+  const uint32_t *lab, *start;  // pos_of counts from start[lab[v]]
   uint32_t *bucket;
 };
+
+__device__ __forceinline__ uint64_t bucket_pos(const ScatterArgs &a, uint32_t v) {
+  return static_cast<uint64_t>(a.pos_of[v]) + a.start[a.lab[v]];
+}
 
 template <int W>
 __device__ __forceinline__ void scatter_group(const ScatterArgs &a, bool active, uint32_t v, uint64_t e0,
@@ -1179,7 +1232,7 @@ __device__ __forceinline__ void scatter_group(const ScatterArgs &a, bool active,
   const int gbase = static_cast<int>(lane_id()) & ~(W - 1);
   uint64_t pos = 0;
   active = active && d > 0;
-  if (active && gl == 0) pos = static_cast<uint64_t>(a.pos_of[v]) + extra;
+  if (active && gl == 0) pos = bucket_pos(a, v) + extra;
   if (W > 1) pos = static_cast<uint64_t>(__shfl(static_cast<unsigned long long>(pos), gbase, 64));
   if (!active) return;
   // the row's (chunk's) d cluster edges sit at its start: a straight copy,
@@ -1209,7 +1262,7 @@ __device__ __forceinline__ void scatter_small_rows(const ScatterArgs &a, bool ac
     scatter_group<1>(a, active, v, e0, 0, 0, d, 0);
     return;
   }
-  const uint64_t pos = d ? static_cast<uint64_t>(a.pos_of[v]) : 0;
+  const uint64_t pos = d ? bucket_pos(a, v) : 0;
   uint32_t val[kSteps];
 #pragma unroll
   for (int p = 0; p < kSteps; ++p) {
@@ -1278,11 +1331,8 @@ __device__ __forceinline__ bool lds_insert(uint32_t *tab, uint32_t mask, uint32_
 // Medium and huge buckets listed by a scan (positions from the prefix, no
 // atomics: appends through one shared counter are serialised by the device).
 struct ClassLoad {
-  const uint64_t *n_dev;
-  uint64_t n;
   const uint64_t *seg_off;
   __device__ Pair64 operator()(uint64_t i) const {
-    if (i >= (n_dev ? *n_dev : n)) return Pair64{0, 0};
     const uint64_t s = seg_off[i + 1] - seg_off[i];
     return s <= kDedupWaveCap ? Pair64{0, 0} : s <= kDedupBlockCap ? Pair64{1, 0} : Pair64{0, 1};
   }
@@ -2230,9 +2280,10 @@ void round_volumes(uint64_t n, const uint64_t *off, const uint64_t *key, uint32_
 
 void bin_vertices(uint64_t n, const uint64_t *off, BinCfg cfg, uint32_t *listT, uint32_t *listS, uint32_t *listW,
                   HubChunk *hubs, uint32_t *counters, uint32_t *deg_inter, uint64_t *scratch, hipStream_t s,
-                  const uint64_t *key, uint32_t tmin) {
+                  const uint64_t *key, uint32_t tmin, HostWords words) {
   if (!n) {
     fill_u32(counters, 4, 0, s);
+    publish_words(words, s);
     return;
   }
   const uint32_t nb = static_cast<uint32_t>(ceil_div(n, kBlock));
@@ -2246,7 +2297,14 @@ void bin_vertices(uint64_t n, const uint64_t *off, BinCfg cfg, uint32_t *listT, 
   hipLaunchKernelGGL(k_bin_write, dim3(nb), dim3(kBlock), 0, s, n, off, cfg, prefix, nb, listT, listS, listW, hubs,
                      deg_inter, key, tmin);
   KC_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_bin_totals, dim3(1), dim3(64), 0, s, prefix, total, nb, counters);
+  hipLaunchKernelGGL(k_bin_totals, dim3(1), dim3(64), 0, s, prefix, total, nb, counters, words);
+  KC_LAUNCH_CHECK();
+}
+
+void publish_words(HostWords words, hipStream_t s) {
+  if (!words.from[0] && !words.from[1]) return;
+  hipLaunchKernelGGL(k_bin_totals, dim3(1), dim3(64), 0, s, static_cast<const uint64_t *>(nullptr),
+                     static_cast<const uint64_t *>(nullptr), 0u, static_cast<uint32_t *>(nullptr), words);
   KC_LAUNCH_CHECK();
 }
 
@@ -2345,10 +2403,10 @@ void huge_sizes(uint32_t n_huge, const uint32_t *huge, const uint64_t *seg_off, 
 }
 
 void labels_radius(uint64_t n, const uint64_t *key, const uint32_t *pos, uint32_t *lab, uint32_t *radius,
-                   bool with_radius, hipStream_t s, uint32_t *used) {
+                   bool with_radius, hipStream_t s, uint32_t *used, uint32_t *zero) {
   if (!n) return;
   const unsigned g = static_cast<unsigned>(std::min<uint64_t>(ceil_div(n, kBlock), 2048));
-  hipLaunchKernelGGL(k_labels_radius, dim3(g), dim3(kBlock), 0, s, n, key, pos, lab, used, radius,
+  hipLaunchKernelGGL(k_labels_radius, dim3(g), dim3(kBlock), 0, s, n, key, pos, lab, used, zero, radius,
                      with_radius ? 1 : 0);
   KC_LAUNCH_CHECK();
 }
@@ -2436,39 +2494,23 @@ void cluster_ids(uint64_t n, const uint32_t *lab, const uint32_t *rank, uint32_t
   KC_LAUNCH_CHECK();
 }
 
-void select_inter(uint64_t n, const uint64_t *key, const uint32_t *deg_inter, uint32_t *sk, uint32_t *sv,
-                  uint64_t *count, uint64_t *scratch, hipStream_t s) {
-  scan_exclusive<uint64_t>(n, SelectLoad{deg_inter}, SelectStore{key, sk, sv}, count, scratch, s);
+void cluster_sums(uint64_t n, const uint32_t *lab, const uint32_t *deg_inter, uint32_t *sum, uint32_t *pos_of,
+                  hipStream_t s) {
+  if (!n) return;
+  hipLaunchKernelGGL(k_cluster_sums, dim3(static_cast<unsigned>(ceil_div(n, kSumBlock * kSumPer))), dim3(kSumBlock), 0,
+                     s, n, lab, deg_inter, sum, pos_of);
+  KC_LAUNCH_CHECK();
 }
 
-void segments(uint64_t N, const uint32_t *sk, const uint32_t *sv, const uint32_t *deg_inter, const uint32_t *gid,
-              const uint32_t *rank, uint32_t *pos_of, uint32_t *newidx, uint32_t *seg_of_cid, uint32_t *gid_next,
-              uint64_t *seg_off, uint64_t *sizes, uint32_t *cache, uint64_t *scratch, hipStream_t s) {
+void sum_segments(uint64_t n, uint32_t *sum, const uint32_t *gid, const uint32_t *rank, uint32_t *newidx,
+                  uint32_t *seg_of_cid, uint32_t *gid_next, uint64_t *seg_off, uint32_t *medium, uint32_t *huge,
+                  const uint32_t *radius, const uint64_t *ids, uint64_t *host_sizes, uint32_t *host_radius,
+                  uint64_t *scratch, hipStream_t s) {
   Pair64 *total = reinterpret_cast<Pair64 *>(scratch);
-  const SegStore store{sk, sv, gid, rank, pos_of, newidx, seg_of_cid, gid_next, seg_off};
-  if (ceil_div(N, kScanTile) <= 1) {  // one pass: nothing to cache
-    scan_exclusive<Pair64>(N, SegLoad{sk, sv, deg_inter, cache}, store, total, scratch + 4, s);
-  } else {
-    const uint64_t blocks = ceil_div(N, kScanTile);
-    Pair64 *sums = reinterpret_cast<Pair64 *>(scratch + 4);
-    Pair64 *prefix = sums + blocks;
-    uint64_t *rest = reinterpret_cast<uint64_t *>(prefix + blocks) + 4;
-    hipLaunchKernelGGL((k_scan_reduce<Pair64, SegLoad>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, s, N,
-                       SegLoad{sk, sv, deg_inter, cache}, sums);
-    KC_LAUNCH_CHECK();
-    if (blocks <= kScanFusedBlocks) {
-      hipLaunchKernelGGL((k_scan_down<Pair64, SegLoadCached, SegStore>), dim3(static_cast<unsigned>(blocks)),
-                         dim3(kBlock), 0, s, N, SegLoadCached{sk, cache}, store, static_cast<const Pair64 *>(nullptr),
-                         total, static_cast<const Pair64 *>(sums));
-    } else {
-      scan_exclusive<Pair64>(blocks, ArrayLoad<Pair64>{sums}, ArrayStore<Pair64>{prefix}, total, rest, s);
-      hipLaunchKernelGGL((k_scan_down<Pair64, SegLoadCached, SegStore>), dim3(static_cast<unsigned>(blocks)),
-                         dim3(kBlock), 0, s, N, SegLoadCached{sk, cache}, store, static_cast<const Pair64 *>(prefix),
-                         static_cast<Pair64 *>(nullptr));
-    }
-    KC_LAUNCH_CHECK();
-  }
-  hipLaunchKernelGGL(k_seg_finish, dim3(1), dim3(1), 0, s, total, seg_off, sizes);
+  scan_exclusive<Pair64>(n, SumLoad{sum}, SumStore{sum, newidx, seg_of_cid, gid_next, medium, huge, gid, rank, seg_off}, total,
+                         scratch + 4, s);
+  hipLaunchKernelGGL(k_sum_finish, dim3(1), dim3(1), 0, s, total, seg_off, radius, host_sizes, host_radius,
+                     ids);
   KC_LAUNCH_CHECK();
 }
 
@@ -2582,17 +2624,17 @@ void write_pieces(uint64_t n, const uint64_t *off, const uint32_t *col, uint32_t
 }
 
 void scatter(const uint64_t *off, const uint32_t *relab, const Bins &b, const uint32_t *deg_inter,
-             const uint32_t *hub_inter, const uint32_t *hub_pos, const uint32_t *pos_of, uint32_t *bucket,
-             hipStream_t s) {
+             const uint32_t *hub_inter, const uint32_t *hub_pos, const uint32_t *pos_of, const uint32_t *lab,
+             const uint32_t *start, uint32_t *bucket, hipStream_t s) {
   if (b.blocks == 0) return;
-  ScatterArgs a{off, relab, b, deg_inter, hub_inter, hub_pos, pos_of, bucket};
+  ScatterArgs a{off, relab, b, deg_inter, hub_inter, hub_pos, pos_of, lab, start, bucket};
   hipLaunchKernelGGL(k_scatter, dim3(b.blocks), dim3(kBlock), 0, s, a);
   KC_LAUNCH_CHECK();
 }
 
-void classify_buckets(uint64_t n, const uint64_t *n_dev, const uint64_t *seg_off, uint32_t *medium, uint32_t *huge,
-                      uint64_t *counts, uint64_t *scratch, hipStream_t s) {
-  scan_exclusive<Pair64>(n, ClassLoad{n_dev, n, seg_off}, ClassStore{medium, huge}, reinterpret_cast<Pair64 *>(counts),
+void classify_buckets(uint64_t n, const uint64_t *seg_off, uint32_t *medium, uint32_t *huge, uint64_t *counts,
+                      uint64_t *scratch, hipStream_t s) {
+  scan_exclusive<Pair64>(n, ClassLoad{seg_off}, ClassStore{medium, huge}, reinterpret_cast<Pair64 *>(counts),
                          scratch, s);
 }
 
@@ -2680,10 +2722,7 @@ void csr_offsets(uint64_t n_next, const uint32_t *uniq, uint64_t *off_next, uint
     fill_u64(sizes + 2, 1, 0, s);
     return;
   }
-  uint64_t *total = scratch;
-  scan_exclusive<uint64_t>(n_next, UniqLoad{uniq}, OffStore{off_next, n_next}, total, scratch + 4, s);
-  hipLaunchKernelGGL(k_copy_total, dim3(1), dim3(1), 0, s, total, sizes + 2);
-  KC_LAUNCH_CHECK();
+  scan_exclusive<uint64_t>(n_next, UniqLoad{uniq}, OffStore{off_next, n_next}, sizes + 2, scratch + 4, s);
 }
 
 void gather_uniques(uint64_t n_next, const uint64_t *off_next, const uint64_t *seg_off, const uint32_t *vals,

@@ -196,7 +196,7 @@ typedef struct kc_options {
 #define KC_K_SWEEP 1     /* pull sweep (decomposition, base case) */
 #define KC_K_BIN 2       /* degree binning */
 #define KC_K_COUNT 3     /* cluster labels, radius, hub chunk folding */
-#define KC_K_SCAN 4      /* prefix sums: selection and cluster segments */
+#define KC_K_SCAN 4      /* cluster sums and prefix sums: cluster numbers, buckets, offsets */
 #define KC_K_SCATTER 5   /* gather of cluster edges into their cluster's bucket */
 #define KC_K_DEDUP 6     /* LDS-staged bucket dedup */
 #define KC_K_CSR 7       /* next-level CSR compaction */
@@ -204,7 +204,7 @@ typedef struct kc_options {
 #define KC_K_CANON 9     /* canonical min-id labels */
 #define KC_K_JUMP 10     /* union-find (base case, shortcuts); the last levels in one workgroup */
 #define KC_K_OTHER 11
-#define KC_K_SORT 12     /* radix sort of (label, vertex) pairs */
+#define KC_K_SORT 12     /* radix sort (no launches of it in a contraction) */
 #define KC_K_RELABEL 13  /* edge slots relabelled with their far end's cluster */
 #define KC_K_ROUND 14    /* time-stepped push round (decomposition) */
 #define KC_K_LEARNED 15  /* features and MLP scores of learned centre proposals */
