@@ -1911,36 +1911,80 @@ __global__ __launch_bounds__(kBlock) void k_undo(uint64_t n, const uint32_t *lab
   }
 }
 
-// minid[rep[v]] = min over v of the input id.  Grid-stride: each wave merges
-// the lanes sharing its first lane's representative and carries that minimum
-// while the next steps keep the same representative (the giant component's),
-// so one atomic per wave serves it instead of one per step; atomics on one
-// address are serialised by the device.  Other lanes take their own atomic
-// (skipped when minid is already smaller).
+// minid[rep[v]] = min over v of the input id.  Grid-stride: each wave carries
+// one component's minimum while the next steps keep meeting it (the giant
+// component's), merges the lanes of one other component a step, and skips an
+// atomic whose minid is already smaller; the waves of a block merge what they
+// carry at the end.  Atomics on one address are serialised by the device, and at
+// the start every wave still reads an unset minimum, so what counts is the
+// number of waves and of lanes beside the carried component.  With one group a
+// step (the first lane's) and an atomic per wave of 2048 blocks: R-MAT 20 92 us,
+// G(2^20, 2^22) 44, random geometric 2 M 66, 256^3 grid 210; now 10, 9, 11, 140.
 __global__ __launch_bounds__(kBlock) void k_canon_min(uint64_t n, const uint32_t *rep, const uint32_t *gid,
                                                      uint32_t *minid) {
+  constexpr int kU = 4;  // vertices whose loads a lane keeps in flight
+  __shared__ uint32_t wave_key[kBlock / kWave], wave_min[kBlock / kWave];
   uint32_t carry_key = kNone, carry_min = kNone;  // wave-uniform
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
-  const uint64_t v0 = blockIdx.x * static_cast<uint64_t>(kBlock) + (threadIdx.x & ~(kWave - 1));
-  for (uint64_t w = v0; w < n; w += stride) {  // w: the wave's first vertex this step
-    const uint64_t v = w + lane_id();
-    const bool live = v < n;
-    const uint32_t key = live ? rep[v] : 0u;
-    const uint32_t id = live ? (gid ? gid[v] : static_cast<uint32_t>(v)) : 0u;
-    const uint32_t lk = __shfl(key, 0);  // lane 0 is live whenever the wave has a step
-    const bool same = live && key == lk;
-    uint32_t mn = same ? id : kNone;
+  const uint64_t v0 = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
+  auto wave_min_of = [](bool in, uint32_t id) {
+    uint32_t mn = in ? id : kNone;
     for (int o = 32; o > 0; o >>= 1) mn = min(mn, static_cast<uint32_t>(__shfl_xor(mn, o)));
-    if (lk == carry_key) {
-      carry_min = min(carry_min, mn);
-    } else {
-      if (carry_key != kNone && lane_id() == 0 && carry_min < minid[carry_key]) atomicMin(&minid[carry_key], carry_min);
-      carry_key = lk;
-      carry_min = mn;
+    return mn;
+  };
+  for (uint64_t w = v0 - lane_id(); w < n; w += kU * stride) {  // w: the wave's first vertex this step
+    uint32_t key[kU], id[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const uint64_t v = w + u * stride + lane_id();
+      key[u] = v < n ? rep[v] : kNone;
+      id[u] = v < n && gid ? gid[v] : static_cast<uint32_t>(v);
     }
-    if (live && !same && id < minid[key]) atomicMin(&minid[key], id);
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const bool live = w + u * stride + lane_id() < n;
+      bool rest = live;
+      // the carried component first, then the first other one of the step
+      if (__ballot(live && key[u] == carry_key)) {
+        const bool same = live && key[u] == carry_key;
+        carry_min = min(carry_min, wave_min_of(same, id[u]));
+        rest = rest && !same;
+      }
+      const uint64_t others = __ballot(rest);
+      if (!others) continue;
+      const uint32_t lk = __shfl(key[u], __ffsll(static_cast<unsigned long long>(others)) - 1);
+      const bool same = rest && key[u] == lk;
+      const uint64_t group = __ballot(same);
+      const uint32_t mn = wave_min_of(same, id[u]);
+      if (__popcll(group) >= kWave / 2 || carry_key == kNone) {
+        if (carry_key != kNone && lane_id() == 0 && carry_min < minid[carry_key])
+          atomicMin(&minid[carry_key], carry_min);
+        carry_key = lk;
+        carry_min = mn;
+      } else if (same && id[u] == mn && mn < minid[lk]) {
+        atomicMin(&minid[lk], mn);
+      }
+      rest = rest && !same;
+      if (rest && id[u] < minid[key[u]]) atomicMin(&minid[key[u]], id[u]);
+    }
   }
-  if (carry_key != kNone && lane_id() == 0 && carry_min < minid[carry_key]) atomicMin(&minid[carry_key], carry_min);
+  // one atomic for every component the block's waves still carry
+  if (lane_id() == 0) {
+    wave_key[threadIdx.x / kWave] = carry_key;
+    wave_min[threadIdx.x / kWave] = carry_min;
+  }
+  __syncthreads();
+  if (threadIdx.x < kBlock / kWave) {
+    const uint32_t k = wave_key[threadIdx.x];
+    bool first = k != kNone;
+    uint32_t mn = kNone;
+    for (uint32_t x = 0; x < kBlock / kWave; ++x)
+      if (wave_key[x] == k) {
+        mn = min(mn, wave_min[x]);
+        first = first && x >= threadIdx.x;
+      }
+    if (first && mn < minid[k]) atomicMin(&minid[k], mn);
+  }
 }
 
 // Block sum of the threads' counts c, written to partial[blockIdx.x].
@@ -2759,7 +2803,8 @@ void sum_partials_u32(const uint32_t *partial, uint64_t count, uint32_t *out, hi
 
 void canon_min(uint64_t n, const uint32_t *rep, const uint32_t *gid, uint32_t *minid, hipStream_t s) {
   if (!n) return;
-  const unsigned g = static_cast<unsigned>(std::min<uint64_t>(ceil_div(n, kBlock), 2048));
+  // about two steps a wave, at most 16 blocks a CU (512 blocks for 15 M vertices: 205 us)
+  const unsigned g = static_cast<unsigned>(std::max<uint64_t>(1, std::min<uint64_t>(ceil_div(n, 8 * kBlock), 4096)));
   hipLaunchKernelGGL(k_canon_min, dim3(g), dim3(kBlock), 0, s, n, rep, gid, minid);
   KC_LAUNCH_CHECK();
 }
