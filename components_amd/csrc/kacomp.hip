@@ -1235,12 +1235,12 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
     {
       TimedScope ts(g->timer, KC_K_RELABEL, 0);
       relabel_slot = ts.slot;
-      // the hot-label launch pays off on the degree-ordered level 0
+      // (the LDS copy of the hot labels pays off on skewed levels)
       if (split)
         relabel_split(off_l, col_l, cid, n_l, b, g->l0_pieces, g->l0_part_list, g->l0_part_at, relab,
                       g->deg_inter, r_inter, n_l, g->stream);
       else
-        relabel(off_l, col_l, cid, b, relab, g->deg_inter, g->hub_inter, pos_l || level_hot ? n_l : 0,
+        relabel(off_l, col_l, cid, b, relab, g->deg_inter, g->hub_inter, hot_ids || level_hot ? n_l : 0,
                 g->stream, hot_ids);
     }
     if (rb.nH) {

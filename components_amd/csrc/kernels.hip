@@ -541,6 +541,12 @@ struct LabHot {
   __device__ __forceinline__ uint32_t row(uint32_t v) const { return (*this)(v); }
 };
 
+struct LabArr {
+  const uint32_t *__restrict__ lab;
+  __device__ __forceinline__ uint32_t operator()(uint32_t c) const { return lab[c]; }
+  __device__ __forceinline__ uint32_t row(uint32_t v) const { return lab[v]; }
+};
+
 // The same with 16-bit entries: the first n_hot (up to 2 kRelabelHot)
 // positions of a degree-ordered level 0, whose clusters were numbered first
 // (cluster_ranks_hot), so that their ids fit 16 bits.
@@ -663,6 +669,14 @@ __device__ __forceinline__ void relabel_block(const SweepArgs &a, const Lab &lab
 // quarter with its own LDS filter (the quarters are whole waves and need no
 // barrier between them).
 constexpr int kRelabelQuarters = 4;
+
+__global__ __launch_bounds__(kBlock) void k_relabel_plain(SweepArgs a, const uint32_t *lab, uint32_t *relab) {
+  __shared__ uint32_t filt[kFilterWords];
+  const LabArr lk{lab};
+  relabel_block(a, lk, relab, blockIdx.x, threadIdx.x, filt);
+}
+
+constexpr uint32_t kRelabelPlainBlocks = 1024;  // one launch block per virtual block from here on (n_hot = 0)
 
 // H16: 16-bit entries for twice the positions (their cluster ids fit 16 bits).
 template <bool H16>
@@ -2572,7 +2586,14 @@ void relabel(const uint64_t *off, const uint32_t *col, const uint32_t *lab, cons
   KC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   const uint32_t blocks = static_cast<uint32_t>(ceil_div(b.blocks, kRelabelQuarters));
   const uint32_t grid = std::min<uint32_t>(blocks, static_cast<uint32_t>(cus > 0 ? cus : 1));
-  if (hot16)
+  // Where no LDS copy pays, a block per virtual block and twice the waves a CU:
+  // 256^3 grid 300 -> 240 us, G(2^20, 2^22) 97 -> 72 and 60 -> 50, random
+  // geometric 2 M 90 -> 73, mixed batch 733 -> 599.  Below about four blocks a CU
+  // the persistent launch is as good or better (1417 blocks 34 -> 35 us, 254
+  // blocks 26 -> 36).
+  if (n_hot == 0 && b.blocks >= kRelabelPlainBlocks)
+    hipLaunchKernelGGL(k_relabel_plain, dim3(b.blocks), dim3(kBlock), 0, s, a, lab, relab);
+  else if (hot16)
     hipLaunchKernelGGL(k_relabel_hot<true>, dim3(grid), dim3(kBlock * kRelabelQuarters), 0, s, a, lab, relab,
                        static_cast<uint32_t>(std::min<uint64_t>(n_hot, kRelabelHot16)));
   else
