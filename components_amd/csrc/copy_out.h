@@ -11,10 +11,10 @@ namespace kc {
 // call; bytes are whole words and src is aligned to 16 bytes.  The constructor
 // (at the call's start; dst may be null: nothing to do) lets helper threads
 // fault in dst's pages while the GPU works, without changing what they hold.
-// enqueue() may put a small copy into the stream ahead of a synchronisation the
-// caller makes anyway; finish() copies, src final in stream order, and returns
-// when dst is written.  Destroying it without finish() leaves dst as it was.
-// Throws Failure.
+// enqueue() may put a small copy into the stream ahead of a wait the caller
+// makes anyway (waited: that is over); finish() copies, src final in stream
+// order, and returns when dst is written.  Destroying it without finish()
+// leaves dst as it was.  Throws Failure.
 class CopyOut {
  public:
   CopyOut(void *dst, size_t bytes, int device);
@@ -22,7 +22,7 @@ class CopyOut {
   CopyOut(const CopyOut &) = delete;
   CopyOut &operator=(const CopyOut &) = delete;
   void enqueue(const void *src, hipStream_t stream);
-  void finish(const void *src, hipStream_t stream);
+  void finish(const void *src, hipStream_t stream, bool waited = false);
 
  private:
   struct Job;

@@ -71,7 +71,7 @@ char *ring_borrow(int device) {
   if (g_ring.lent) return nullptr;
   if (!g_ring.mem) {
     void *p = nullptr;
-    if (hipHostMalloc(&p, kSlotBytes * kSlots, hipHostMallocPortable) != hipSuccess) {
+    if (hipHostMalloc(&p, kSlotBytes * kSlots, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
       (void)hipGetLastError();
       return nullptr;
     }
@@ -227,12 +227,13 @@ void CopyOut::enqueue(const void *src, hipStream_t stream) {
   stream_ = stream;
 }
 
-void CopyOut::finish(const void *src, hipStream_t stream) {
+void CopyOut::finish(const void *src, hipStream_t stream, bool waited) {
   if (!bytes_) return;
   if (bytes_ <= kThreadsMin) {
+    waited = waited && queued_;
     if (!queued_) enqueue(src, stream);
     if (queued_) {
-      KC_HIP(hipStreamSynchronize(stream));
+      if (!waited) KC_HIP(hipStreamSynchronize(stream));
       queued_ = false;
       std::memcpy(dst_, ring_, bytes_);
       return;

@@ -272,6 +272,8 @@ struct kc_graph {
   // pinned host mirrors
   uint64_t *h_sizes = nullptr;
   uint32_t *h_small = nullptr;
+  uint32_t *h_signal = nullptr;  // the last signal that arrived (next_signal, await)
+  uint32_t signals = 0;
   int *h_flags = nullptr;
   // deviate table
   double *d_table = nullptr;
@@ -364,6 +366,7 @@ struct kc_graph {
     for (void *p : owned) (void)hipFree(p);
     if (h_sizes) (void)hipHostFree(h_sizes);
     if (h_small) (void)hipHostFree(h_small);
+    if (h_signal) (void)hipHostFree(h_signal);
     if (h_flags) (void)hipHostFree(h_flags);
     if (ev_begin) (void)hipEventDestroy(ev_begin);
     if (ev_end) (void)hipEventDestroy(ev_end);
@@ -403,6 +406,38 @@ constexpr uint64_t kHubPullMin = 65536;            // smallest degree of a hub t
 
 
 void sync(kc_graph *g) { KC_HIP(hipStreamSynchronize(g->stream)); }
+
+// The host's waits inside a contraction.  The last launch ahead of one carries
+// `next_signal` in its words; await polls for that value, which takes 9 us from
+// a launch's enqueueing where a copy and a stream synchronisation take 15.  A
+// wait of more than a millisecond, or a fault, ends in the synchronisation.
+HostWords next_signal(kc_graph *g) {
+  HostWords w;
+  w.signal = g->h_signal;
+  w.value = ++g->signals;
+  return w;
+}
+
+void await(kc_graph *g) {
+  const auto arrived = [&] { return __atomic_load_n(g->h_signal, __ATOMIC_ACQUIRE) == g->signals; };
+  const auto limit = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+  while (!arrived()) {
+    for (int i = 0; i < 64; ++i) {
+      if (arrived()) return;
+      __builtin_ia32_pause();
+    }
+    if (std::chrono::steady_clock::now() > limit) return sync(g);
+  }
+}
+
+// 32-bit words to pinned memory, then the wait.
+void fetch32(kc_graph *g, void *dst, const void *src, uint32_t count, HostWords w) {
+  w.from32 = static_cast<const uint32_t *>(src);
+  w.to32 = static_cast<uint32_t *>(dst);
+  w.count32 = count;
+  publish_words(w, g->stream);
+  await(g);
+}
 
 void d2h(kc_graph *g, void *dst, const void *src, size_t bytes) {
   KC_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g->stream));
@@ -473,8 +508,8 @@ Bins make_bins(kc_graph *g, uint64_t n, const uint64_t *off, const BinCfg &cfg, 
                          static_cast<unsigned long long>(n), static_cast<unsigned long long>(g->cap_n));
   Bins b;
   enqueue_bins(g, n, off, cfg, b, key ? g->flists : level0 ? g->l0_lists : g->lists,
-               key ? g->fhubs : level0 ? g->l0_hubs : g->hubs, key, tmin);
-  sync(g);
+               key ? g->fhubs : level0 ? g->l0_hubs : g->hubs, key, tmin, next_signal(g));
+  await(g);
   read_bins(g, b);
   if (level0) {
     g->l0_bins = b;
@@ -523,8 +558,7 @@ uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t 
               g->stream, true);
       g->timer.stop(slots[i], bytes);
     }
-    d2h(g, g->h_flags, &g->flags[flag_base], batch * sizeof(int));
-    sync(g);
+    fetch32(g, g->h_flags, &g->flags[flag_base], batch, next_signal(g));
     uint32_t i = 0;
     while (i < batch && g->h_flags[i] != 0) ++i;
     const uint32_t worked = i < batch ? i + 1 : batch;
@@ -763,12 +797,15 @@ uint64_t rounds_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t
       g->timer.stop(slots[i], 0);
       if (first_slot < 0) first_slot = slots[i];
     }
-    d2h(g, g->h_flags, &g->flags[flag_base], batch * sizeof(int));
+    HostWords w = next_signal(g);
     if (deciding) {  // edge slots at and above the next round's distance, for its direction
       round_volumes(n, off, key, t + batch, g->sizes + 12, g->stream);
-      d2h(g, g->h_sizes + 12, g->sizes + 12, 2 * sizeof(uint64_t));
+      for (int i = 0; i < 2; ++i) {
+        w.from[i] = g->sizes + 12 + i;
+        w.to[i] = g->h_sizes + 12 + i;
+      }
     }
-    sync(g);
+    fetch32(g, g->h_flags, &g->flags[flag_base], batch, w);
     uint32_t i = 0;
     while (i < batch && g->h_flags[i] != 0) ++i;
     const uint32_t worked = i < batch ? i + 1 : batch;
@@ -1127,8 +1164,7 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
         uint32_t *pk = n_l >= kPackedSweepsMin && n_l <= (1ull << kPackedLabelBits) ? g->crank : nullptr;
         if (pk) {
           pack_keys(n_l, g->key, pk, g->small + 7, g->stream);
-          d2h(g, g->h_small + 7, g->small + 7, sizeof(uint32_t));
-          sync(g);
+          fetch32(g, g->h_small + 7, g->small + 7, 1, next_signal(g));
           if (g->h_small[7]) pk = nullptr;
         }
         sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, kOneHop, b, flag_base, true, pk);
@@ -1253,11 +1289,14 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
     }
     {
       TimedScope ts(g->timer, KC_K_SCAN, 2 * 4 * n_l + 4 * n_l);
+      HostWords w = next_signal(g);
+      w.from32 = g->small + 4;  // the radius
+      w.to32 = g->h_small + 4;
+      w.count32 = 1;
       sum_segments(n_l, sum, gid_l, dense ? g->crank : nullptr, rec.newidx, g->seg_of_cid, gid_next, g->seg_off,
-                   g->dl_medium, g->dl_huge, g->small + 4, dense ? g->sizes + 9 : nullptr, g->h_sizes, g->h_small + 4,
-                   g->scan_scratch, g->stream);
+                   g->dl_medium, g->dl_huge, dense ? g->sizes + 9 : nullptr, g->h_sizes, w, g->scan_scratch, g->stream);
     }
-    sync(g);
+    await(g);
     const uint64_t label_space = dense ? g->h_sizes[9] : n_l;
     const uint64_t n_next = g->h_sizes[0], P = g->h_sizes[1];
     const uint64_t n_medium = g->h_sizes[3], n_huge = g->h_sizes[4];
@@ -1296,13 +1335,17 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
     // the next level's bins, unless it may be one that needs none, go in
     // before its size comes back: one synchronisation for both
     const uint64_t hot_rows = std::min<uint64_t>(n_next, kLevelHotRows);
-    const HostWords words{{g->sizes + 2, off_next + hot_rows}, {g->h_sizes + 2, g->h_sizes + 15}};
+    HostWords words = next_signal(g);
+    words.from[0] = g->sizes + 2;
+    words.to[0] = g->h_sizes + 2;
+    words.from[1] = off_next + hot_rows;
+    words.to[1] = g->h_sizes + 15;
     bins_valid = !(use_tail && n_next <= kTailVertices);
     if (bins_valid)
       enqueue_bins(g, n_next, off_next, cfg, b, g->lists, g->hubs, nullptr, 0, words);
     else
       publish_words(words, g->stream);
-    sync(g);
+    await(g);
     if (bins_valid) read_bins(g, b);
     const uint64_t m2_next = g->h_sizes[2];
     level_hot = m2_next > 0 && static_cast<double>(g->h_sizes[15]) * n_next >=
@@ -1430,9 +1473,11 @@ std::unique_ptr<kc_graph> new_handle() {
   KC_HIP(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
   KC_HIP(hipEventCreate(&g->ev_begin));
   KC_HIP(hipEventCreate(&g->ev_end));
-  KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_sizes), 16 * sizeof(uint64_t), hipHostMallocDefault));
-  KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_small), 16 * sizeof(uint32_t), hipHostMallocDefault));
-  KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_flags), 64 * sizeof(int), hipHostMallocDefault));
+  KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_sizes), 16 * sizeof(uint64_t), hipHostMallocCoherent));
+  KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_small), 16 * sizeof(uint32_t), hipHostMallocCoherent));
+  KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_signal), sizeof(uint32_t), hipHostMallocCoherent));
+  *g->h_signal = 0;
+  KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_flags), 64 * sizeof(int), hipHostMallocCoherent));
   g->small = g->dalloc<uint32_t>(16);
   g->sizes = g->dalloc<uint64_t>(16);
   return g;
@@ -2174,9 +2219,8 @@ int kc_find_components(kc_graph *g, const kc_options *opt, uint32_t *labels_out,
       else
         run_propagation(g, &o, out);
       KC_HIP(hipEventRecord(g->ev_end, g->stream));
-      d2h(g, g->h_small + 5, g->small + 5, 8 * sizeof(uint32_t));
       labels.enqueue(g->labels, g->stream);
-      sync(g);
+      fetch32(g, g->h_small + 5, g->small + 5, 8, next_signal(g));
       if (!out.tail) break;
       const uint32_t *info = g->h_small + 9;
       if (info[0] == kTailFull) {  // (not seen: a hash part of the tail outgrew its table) every level the general way
@@ -2196,9 +2240,10 @@ int kc_find_components(kc_graph *g, const kc_options *opt, uint32_t *labels_out,
     if (o.variant == KC_VARIANT_EXP || o.variant == KC_VARIANT_LOCAL)
       g->components += static_cast<uint32_t>(g->n - g->n0);  // degree-0 vertices
     g->have_labels = true;
+    labels.finish(g->labels, g->stream, true);
     float ms = 0.f;
+    KC_HIP(hipEventSynchronize(g->ev_end));
     KC_HIP(hipEventElapsedTime(&ms, g->ev_begin, g->ev_end));
-    labels.finish(g->labels, g->stream);
     const auto t1 = std::chrono::steady_clock::now();
     if (stats) {
       std::memset(stats, 0, sizeof(*stats));

@@ -92,10 +92,18 @@ void init_keys_uniform(uint64_t n, const uint32_t *gid, const uint32_t *idx, int
                        hipStream_t s);
 void deviates_only(uint32_t gid0, uint32_t count, DeviateArgs d, uint32_t *out, hipStream_t s);
 
-// Up to two words of device memory to the host's pinned memory.
+// What a launch ahead of a wait of the host leaves in pinned memory: up to two
+// 64-bit words, up to 64 32-bit ones, and then, if signal is set, its value
+// there, which the host may poll for (9 us from enqueueing the launch to the
+// host's next step, against 15 for a copy and a stream synchronisation).
 struct HostWords {
-  const uint64_t *from[2];
-  uint64_t *to[2];
+  const uint64_t *from[2] = {nullptr, nullptr};
+  uint64_t *to[2] = {nullptr, nullptr};
+  const uint32_t *from32 = nullptr;
+  uint32_t *to32 = nullptr;
+  uint32_t count32 = 0;
+  uint32_t *signal = nullptr;
+  uint32_t value = 0;
 };
 void publish_words(HostWords words, hipStream_t s);
 
@@ -212,13 +220,12 @@ void cluster_ranks_hot(uint64_t n, uint64_t k, const uint32_t *lab, uint32_t *us
 // (rank null: not), gid_next by next-level index, seg_off[0..n_next] bucket
 // offsets, in sum every bucket's start and the lists of medium and huge
 // buckets; and to the host (pinned) host_sizes[0] = n_next, [1] = cluster edges,
-// [3], [4] = medium, huge buckets, [9] = *ids (ids null: not) and the radius.
+// [3], [4] = medium, huge buckets, [9] = *ids (ids null: not), and words.
 void cluster_sums(uint64_t n, const uint32_t *lab, const uint32_t *deg_inter, uint32_t *sum, uint32_t *pos_of,
                   hipStream_t s);
 void sum_segments(uint64_t n, uint32_t *sum, const uint32_t *gid, const uint32_t *rank, uint32_t *newidx,
                   uint32_t *seg_of_cid, uint32_t *gid_next, uint64_t *seg_off, uint32_t *medium, uint32_t *huge,
-                  const uint32_t *radius, const uint64_t *ids, uint64_t *host_sizes, uint32_t *host_radius,
-                  uint64_t *scratch, hipStream_t s);
+                  const uint64_t *ids, uint64_t *host_sizes, HostWords words, uint64_t *scratch, hipStream_t s);
 
 // The labels lab[col[e]] of row v that differ from lab[v] (after a best-effort
 // LDS filter of repeats), packed at relab[off[v] ...] (hub chunks: at the

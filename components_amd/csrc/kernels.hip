@@ -182,18 +182,30 @@ __global__ __launch_bounds__(kBlock) void k_bin_write(uint64_t n, const uint64_t
   }
 }
 
-// The bins' sizes (to device memory or the host's pinned memory) and up to two
-// words more to the host: one launch ahead of a synchronisation in place of a
-// copy for each.
-__global__ void k_bin_totals(const uint64_t *prefix, const uint64_t *total, uint32_t nblocks, uint32_t *counters,
-                             HostWords words) {
+// words by one wave of a workgroup; the signal once every lane's own stores to
+// the host are through.
+__device__ __forceinline__ void put_words(const HostWords &w) {
+  const uint32_t t = threadIdx.x;
+  if (t < 2 && w.from[t]) *w.to[t] = *w.from[t];
+  if (t < w.count32) w.to32[t] = w.from32[t];
+  if (!w.signal) return;
+  __threadfence_system();
+  __builtin_amdgcn_wave_barrier();
+  if (t == 0) __hip_atomic_store(w.signal, w.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ __launch_bounds__(kWave) void k_put_words(HostWords w) { put_words(w); }
+
+// The bins' sizes (to device memory or the host's pinned memory), and words to
+// the host: one launch ahead of a wait in place of a copy for each.
+__global__ __launch_bounds__(kWave) void k_bin_totals(const uint64_t *prefix, const uint64_t *total, uint32_t nblocks,
+                                                     uint32_t *counters, HostWords words) {
   const int r = threadIdx.x;
-  if (r < 4 && prefix) {
+  if (r < 4) {
     const uint64_t hi = r < 3 ? prefix[static_cast<uint64_t>(r + 1) * nblocks] : *total;
     counters[r] = static_cast<uint32_t>(hi - prefix[static_cast<uint64_t>(r) * nblocks]);
-  } else if (r >= 4 && r < 6 && words.from[r - 4]) {
-    words.to[r - 4][0] = *words.from[r - 4];
   }
+  put_words(words);
 }
 
 // ---------------------------------------------------------------------------
@@ -1205,16 +1217,18 @@ struct SumStore {
     if (v.b >> kSumHuge) huge[prefix.b >> kSumHuge] = at;
   }
 };
-__global__ void k_sum_finish(const Pair64 *total, uint64_t *seg_off, const uint32_t *radius, uint64_t *host_sizes,
-                             uint32_t *host_radius, const uint64_t *ids) {
-  const uint64_t clusters = static_cast<uint32_t>(total->a), edges = sum_edges(total->b);
-  if (ids) host_sizes[9] = *ids;
-  seg_off[clusters] = edges;
-  host_sizes[0] = clusters;
-  host_sizes[1] = edges;
-  host_sizes[3] = total->a >> 32;
-  host_sizes[4] = total->b >> kSumHuge;
-  *host_radius = *radius;
+__global__ __launch_bounds__(kWave) void k_sum_finish(const Pair64 *total, uint64_t *seg_off, const uint64_t *ids,
+                                                     uint64_t *host_sizes, HostWords words) {
+  if (threadIdx.x == 0) {
+    const uint64_t clusters = static_cast<uint32_t>(total->a), edges = sum_edges(total->b);
+    if (ids) host_sizes[9] = *ids;
+    seg_off[clusters] = edges;
+    host_sizes[0] = clusters;
+    host_sizes[1] = edges;
+    host_sizes[3] = total->a >> 32;
+    host_sizes[4] = total->b >> kSumHuge;
+  }
+  put_words(words);
 }
 
 // ---------------------------------------------------------------------------
@@ -2360,9 +2374,7 @@ void bin_vertices(uint64_t n, const uint64_t *off, BinCfg cfg, uint32_t *listT, 
 }
 
 void publish_words(HostWords words, hipStream_t s) {
-  if (!words.from[0] && !words.from[1]) return;
-  hipLaunchKernelGGL(k_bin_totals, dim3(1), dim3(64), 0, s, static_cast<const uint64_t *>(nullptr),
-                     static_cast<const uint64_t *>(nullptr), 0u, static_cast<uint32_t *>(nullptr), words);
+  hipLaunchKernelGGL(k_put_words, dim3(1), dim3(kWave), 0, s, words);
   KC_LAUNCH_CHECK();
 }
 
@@ -2562,13 +2574,11 @@ void cluster_sums(uint64_t n, const uint32_t *lab, const uint32_t *deg_inter, ui
 
 void sum_segments(uint64_t n, uint32_t *sum, const uint32_t *gid, const uint32_t *rank, uint32_t *newidx,
                   uint32_t *seg_of_cid, uint32_t *gid_next, uint64_t *seg_off, uint32_t *medium, uint32_t *huge,
-                  const uint32_t *radius, const uint64_t *ids, uint64_t *host_sizes, uint32_t *host_radius,
-                  uint64_t *scratch, hipStream_t s) {
+                  const uint64_t *ids, uint64_t *host_sizes, HostWords words, uint64_t *scratch, hipStream_t s) {
   Pair64 *total = reinterpret_cast<Pair64 *>(scratch);
-  scan_exclusive<Pair64>(n, SumLoad{sum}, SumStore{sum, newidx, seg_of_cid, gid_next, medium, huge, gid, rank, seg_off}, total,
-                         scratch + 4, s);
-  hipLaunchKernelGGL(k_sum_finish, dim3(1), dim3(1), 0, s, total, seg_off, radius, host_sizes, host_radius,
-                     ids);
+  scan_exclusive<Pair64>(n, SumLoad{sum}, SumStore{sum, newidx, seg_of_cid, gid_next, medium, huge, gid, rank, seg_off},
+                         total, scratch + 4, s);
+  hipLaunchKernelGGL(k_sum_finish, dim3(1), dim3(kWave), 0, s, total, seg_off, ids, host_sizes, words);
   KC_LAUNCH_CHECK();
 }
 
