@@ -265,8 +265,9 @@ struct kc_graph {
   uint64_t *d_huge_info = nullptr;
   uint64_t huge_info_cap = 0;
   int *flags = nullptr;
-  // [4] radius, [5] roots, [6] hubs found, [7] packed keys do not fit, [8] edges of
-  // the tail, [9..12] its status, levels, sweeps, radius sum
+  // [5] roots, [6] hubs found, [7] packed keys do not fit, [8] edges of
+  // the tail, [9..12] its status, levels, sweeps, radius sum, [13] radius,
+  // [14] medium and [15] huge buckets of a level
   uint32_t *small = nullptr;
   uint64_t *sizes = nullptr;  // [0] n_next [1] P [2] m2_next [3..5] dedup counters [9] clusters
   // pinned host mirrors
@@ -1205,7 +1206,7 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
       rec.keys_copy = g->arena.alloc_n<uint64_t>(n_l);
       KC_HIP(hipMemcpyAsync(rec.keys_copy, g->key, n_l * 8, hipMemcpyDeviceToDevice, g->stream));
     }
-    fill_u32(g->small + 4, 1, 0, g->stream);
+    fill_u32(g->small + 13, 3, 0, g->stream);  // radius, medium and huge buckets
     // on a degree-ordered level 0 whose first kHotClusters positions hold a
     // large share of the edge slots, the clusters of those positions take the
     // ids below 65536, so the relabel keeps those positions' ids in LDS at 16
@@ -1221,7 +1222,7 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
     if (dense) fill_u32(g->cid, n_l, 0, g->stream);  // the used-label flags, then the ids
     {
       TimedScope ts(g->timer, KC_K_COUNT, 8 * n_l + 4 * n_l + 4 * n_l + (local ? 0 : 8 * n_l));
-      labels_radius(n_l, g->key, pos_l, rec.lab, g->small + 4, !local && !pre, g->stream, dense ? g->cid : nullptr, sum);
+      labels_radius(n_l, g->key, pos_l, rec.lab, g->small + 13, !local && !pre, g->stream, dense ? g->cid : nullptr, sum);
     }
     if (g->collect && !pre) {
       // trace of the plain method: features and the log2 size of each vertex's cluster
@@ -1290,17 +1291,17 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
     {
       TimedScope ts(g->timer, KC_K_SCAN, 2 * 4 * n_l + 4 * n_l);
       HostWords w = next_signal(g);
-      w.from32 = g->small + 4;  // the radius
-      w.to32 = g->h_small + 4;
-      w.count32 = 1;
+      w.from32 = g->small + 13;
+      w.to32 = g->h_small + 13;
+      w.count32 = 3;
       sum_segments(n_l, sum, gid_l, dense ? g->crank : nullptr, rec.newidx, g->seg_of_cid, gid_next, g->seg_off,
-                   g->dl_medium, g->dl_huge, dense ? g->sizes + 9 : nullptr, g->h_sizes, w, g->scan_scratch, g->stream);
+                   g->dl_medium, g->dl_huge, g->small + 14, dense ? g->sizes + 9 : nullptr, g->h_sizes, w, g->scan_scratch, g->stream);
     }
     await(g);
     const uint64_t label_space = dense ? g->h_sizes[9] : n_l;
     const uint64_t n_next = g->h_sizes[0], P = g->h_sizes[1];
-    const uint64_t n_medium = g->h_sizes[3], n_huge = g->h_sizes[4];
-    rec.radius = local || pre ? 0 : g->h_small[4];
+    const uint64_t n_medium = g->h_small[14], n_huge = g->h_small[15];
+    rec.radius = local || pre ? 0 : g->h_small[13];
     if (!pre) out.sweeps += sweeps;  // the block passes are not decomposition sweeps
     out.radius_sum += rec.radius;
     g->levels.push_back(rec);

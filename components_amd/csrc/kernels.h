@@ -219,13 +219,15 @@ void cluster_ranks_hot(uint64_t n, uint64_t k, const uint32_t *lab, uint32_t *us
 // (kNone: no cluster edge), seg_of_cid[rank[a]] = the same by dense cluster id
 // (rank null: not), gid_next by next-level index, seg_off[0..n_next] bucket
 // offsets, in sum every bucket's start and the lists of medium and huge
-// buckets; and to the host (pinned) host_sizes[0] = n_next, [1] = cluster edges,
-// [3], [4] = medium, huge buckets, [9] = *ids (ids null: not), and words.
+// buckets, in any order, their lengths added to counts[0] and [1]; and to the
+// host (pinned) host_sizes[0] = n_next, [1] = cluster edges, [9] = *ids (ids
+// null: not), and words.
 void cluster_sums(uint64_t n, const uint32_t *lab, const uint32_t *deg_inter, uint32_t *sum, uint32_t *pos_of,
                   hipStream_t s);
 void sum_segments(uint64_t n, uint32_t *sum, const uint32_t *gid, const uint32_t *rank, uint32_t *newidx,
                   uint32_t *seg_of_cid, uint32_t *gid_next, uint64_t *seg_off, uint32_t *medium, uint32_t *huge,
-                  const uint64_t *ids, uint64_t *host_sizes, HostWords words, uint64_t *scratch, hipStream_t s);
+                  uint32_t *counts, const uint64_t *ids, uint64_t *host_sizes, HostWords words, uint64_t *scratch,
+                  hipStream_t s);
 
 // The labels lab[col[e]] of row v that differ from lab[v] (after a best-effort
 // LDS filter of repeats), packed at relab[off[v] ...] (hub chunks: at the

@@ -945,7 +945,8 @@ __global__ __launch_bounds__(kBlock) void k_labels_radius(uint64_t n, const uint
     __syncthreads();
     if (threadIdx.x == 0) {
       for (int w = 1; w < kBlock / kWave; ++w) r = max(r, wave_max[w]);
-      if (r) atomicMax(radius, r);
+      // (skipped where a block before has met the radius)
+      if (r > __hip_atomic_load(radius, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(radius, r);
     }
   }
 }
@@ -961,54 +962,25 @@ struct Pair64 {
   __host__ __device__ Pair64 operator+(const Pair64 &o) const { return {a + o.a, b + o.b}; }
 };
 
-// Block-wide exclusive scan (Hillis-Steele in LDS); *total receives the block sum.
-template <class T>
-__device__ T block_exclusive_scan_shift(T v, T *smem, T *total) {
-  const int tid = threadIdx.x;
-  smem[tid] = v;
-  __syncthreads();
-  for (int o = 1; o < kBlock; o <<= 1) {
-    T t = tid >= o ? smem[tid - o] : T{};
-    __syncthreads();
-    if (tid >= o) smem[tid] = smem[tid] + t;
-    __syncthreads();
-  }
-  T excl = tid > 0 ? smem[tid - 1] : T{};
-  T tot = smem[kBlock - 1];
-  __syncthreads();
-  if (total) *total = tot;
-  return excl;
-}
-
-template <class T, class Load>
-__global__ __launch_bounds__(kBlock) void k_scan_reduce(uint64_t n, Load load, T *block_sums) {
-  __shared__ T smem[kBlock];
-  const uint64_t base = static_cast<uint64_t>(blockIdx.x) * kScanTile;
-  T acc{};
-  for (int j = 0; j < kScanPerThread; ++j) {
-    uint64_t i = base + static_cast<uint64_t>(j) * kBlock + threadIdx.x;
-    if (i < n) acc = acc + load(i);
-  }
-  T tot;
-  block_exclusive_scan_shift<T>(acc, smem, &tot);
-  if (threadIdx.x == 0) block_sums[blockIdx.x] = tot;
-}
-
 __device__ __forceinline__ uint64_t shfl_up_t(uint64_t x, int o) {
   return static_cast<uint64_t>(__shfl_up(static_cast<unsigned long long>(x), o));
 }
 __device__ __forceinline__ Pair64 shfl_up_t(Pair64 x, int o) { return {shfl_up_t(x.a, o), shfl_up_t(x.b, o)}; }
+__device__ __forceinline__ uint64_t last_lane(uint64_t x) {
+  return static_cast<uint64_t>(__shfl(static_cast<unsigned long long>(x), kWave - 1));
+}
+__device__ __forceinline__ Pair64 last_lane(Pair64 x) { return {last_lane(x.a), last_lane(x.b)}; }
+__device__ __forceinline__ uint64_t shfl_xor_t(uint64_t x, int o) {
+  return static_cast<uint64_t>(__shfl_xor(static_cast<unsigned long long>(x), o));
+}
+__device__ __forceinline__ Pair64 shfl_xor_t(Pair64 x, int o) { return {shfl_xor_t(x.a, o), shfl_xor_t(x.b, o)}; }
 
-// Sum of one value per thread over the block (wave scans, then the wave sums
-// through LDS); every thread receives it.
+// Sum of one value per thread over the block (wave sums through LDS); every
+// thread receives it.
 template <class T>
 __device__ T block_total(T v, T *wsum) {
-  const uint32_t ln = lane_id(), wv = threadIdx.x / kWave;
-  for (int o = 1; o < kWave; o <<= 1) {
-    const T t = shfl_up_t(v, o);
-    if (ln >= static_cast<uint32_t>(o)) v = v + t;
-  }
-  if (ln == kWave - 1) wsum[wv] = v;
+  for (int o = kWave / 2; o > 0; o >>= 1) v = v + shfl_xor_t(v, o);
+  if (lane_id() == 0) wsum[threadIdx.x / kWave] = v;
   __syncthreads();
   T tot{};
   for (uint32_t w = 0; w < kBlock / kWave; ++w) tot = tot + wsum[w];
@@ -1016,18 +988,43 @@ __device__ T block_total(T v, T *wsum) {
   return tot;
 }
 
-// A tile is kScanPerThread rounds of kBlock consecutive items (lane i of a
-// round takes item i, so loads and stores are coalesced); each round is one
-// block-wide scan (wave scans, then the wave sums through LDS), carried into
-// the next.  block_prefix: the exclusive prefix of every block's tile; or
-// block_sums (block_prefix null): every block's tile sum, the block adding up
-// those before its own (for grids of up to kScanFusedBlocks blocks, in place
-// of a scan launch over the sums).
-template <class T, class Load, class Store>
-__global__ __launch_bounds__(kBlock) void k_scan_down(uint64_t n, Load load, Store store, const T *block_prefix,
-                                                     T *total_out, const T *block_sums = nullptr) {
+// A tile is cut into one run of consecutive items per wave, and a run into
+// kScanPerThread rounds of a wave's lanes, so that loads and stores are
+// coalesced.  Both passes issue a lane's loads together, and a wave scans its
+// rounds by itself, with one barrier for the waves' totals: the scan is bound
+// by latency on the levels' sizes.  With a block-wide scan, two barriers and one
+// load a round the clusters' scan took 12 + 13 us on 2^20 labels and 32 + 98 on
+// 15 M; so 5 + 9 and 17 + 62.
+template <class T, class Load>
+__global__ __launch_bounds__(kBlock) void k_scan_reduce(uint64_t n, Load load, T *block_sums) {
   __shared__ T wsum[kBlock / kWave];
   const uint64_t base = static_cast<uint64_t>(blockIdx.x) * kScanTile;
+  T v[kScanPerThread];
+#pragma unroll
+  for (int j = 0; j < kScanPerThread; ++j) {
+    const uint64_t i = base + static_cast<uint64_t>(j) * kBlock + threadIdx.x;
+    v[j] = i < n ? load(i) : T{};
+  }
+  T acc = v[0];
+#pragma unroll
+  for (int j = 1; j < kScanPerThread; ++j) acc = acc + v[j];
+  const T tot = block_total<T>(acc, wsum);
+  if (threadIdx.x == 0) block_sums[blockIdx.x] = tot;
+}
+
+// A thread's share of a tile scanned: v, its items (base + j * kWave, j in
+// order); before, the exclusive prefix of each inside the wave's run.  Returns
+// the prefix of the run; *all is the prefix of the tile's end (last wave).
+// block_prefix: the exclusive prefix of every block's tile; or block_sums
+// (block_prefix null): every block's tile sum, the block adding up those
+// before its own (for grids of up to kScanFusedBlocks blocks, in place of a
+// scan launch over the sums).
+__device__ __forceinline__ uint64_t scan_base() {
+  return static_cast<uint64_t>(blockIdx.x) * kScanTile + threadIdx.x / kWave * (kScanTile / (kBlock / kWave)) + lane_id();
+}
+template <class T>
+__device__ __forceinline__ T scan_tile(const T (&v)[kScanPerThread], T (&before)[kScanPerThread], const T *block_prefix,
+                                       const T *block_sums, T *wsum, T *all) {
   const uint32_t ln = lane_id(), wv = threadIdx.x / kWave;
   T run{};
   if (block_prefix) {
@@ -1037,29 +1034,43 @@ __global__ __launch_bounds__(kBlock) void k_scan_down(uint64_t n, Load load, Sto
     for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kBlock) acc = acc + block_sums[b];
     run = block_total<T>(acc, wsum);
   }
+  T sum{};  // of the wave's run so far
+#pragma unroll
   for (int j = 0; j < kScanPerThread; ++j) {
-    const uint64_t i = base + static_cast<uint64_t>(j) * kBlock + threadIdx.x;
-    const T v = i < n ? load(i) : T{};
-    T inc = v;
+    T inc = v[j];
     for (int o = 1; o < kWave; o <<= 1) {
       const T t = shfl_up_t(inc, o);
       if (ln >= static_cast<uint32_t>(o)) inc = inc + t;
     }
     T ex = shfl_up_t(inc, 1);
     if (ln == 0) ex = T{};
-    if (ln == kWave - 1) wsum[wv] = inc;
-    __syncthreads();
-    T before{}, round_total{};
-    for (uint32_t w = 0; w < kBlock / kWave; ++w) {
-      const T x = wsum[w];
-      if (w < wv) before = before + x;
-      round_total = round_total + x;
-    }
-    __syncthreads();
-    if (i < n) store(i, run + before + ex, v);
-    run = run + round_total;
+    before[j] = sum + ex;
+    sum = sum + last_lane(inc);
   }
-  if (total_out && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total_out = run;
+  if (ln == 0) wsum[wv] = sum;
+  __syncthreads();
+  T tile{};
+  for (uint32_t w = 0; w < kBlock / kWave; ++w) {
+    if (w == wv) run = run + tile;
+    tile = tile + wsum[w];
+  }
+  *all = run + sum;
+  return run;
+}
+
+template <class T, class Load, class Store>
+__global__ __launch_bounds__(kBlock) void k_scan_down(uint64_t n, Load load, Store store, const T *block_prefix,
+                                                     T *total_out, const T *block_sums = nullptr) {
+  __shared__ T wsum[kBlock / kWave];
+  const uint64_t base = scan_base();
+  T v[kScanPerThread], before[kScanPerThread], all;
+#pragma unroll
+  for (int j = 0; j < kScanPerThread; ++j) v[j] = base + j * kWave < n ? load(base + j * kWave) : T{};
+  const T run = scan_tile<T>(v, before, block_prefix, block_sums, wsum, &all);
+#pragma unroll
+  for (int j = 0; j < kScanPerThread; ++j)
+    if (base + j * kWave < n) store(base + j * kWave, run + before[j], v[j]);
+  if (total_out && blockIdx.x == gridDim.x - 1 && threadIdx.x == kBlock - 1) *total_out = all;
 }
 
 template <class T>
@@ -1189,44 +1200,81 @@ __global__ __launch_bounds__(kSumBlock) void k_cluster_sums(uint64_t n, const ui
     if (d[u]) pos_of[v0 + u * B] = part[slot[u]] + at[u];
 }
 
-// (clusters, medium buckets in the upper half; cluster edges, huge buckets above
-// kSumHuge)
-constexpr int kSumHuge = 40;  // a level has fewer than 2^32 edge slots: at most 2^19 huge buckets
+// (clusters in the upper half, cluster edges, fewer than 2^32 in a level)
 struct SumLoad {
   const uint32_t *sum;
-  __device__ Pair64 operator()(uint64_t l) const {
+  __device__ uint64_t operator()(uint64_t l) const {
     const uint64_t d = sum[l];
-    const uint64_t medium = d > kDedupWaveCap && d <= kDedupBlockCap, huge = d > kDedupBlockCap;
-    return {(d != 0) | medium << 32, d | huge << kSumHuge};
+    return (d != 0 ? 1ull << 32 : 0ull) | d;
   }
 };
-__device__ __forceinline__ uint64_t sum_edges(uint64_t b) { return b & ((1ull << kSumHuge) - 1); }
-struct SumStore {
-  uint32_t *sum, *newidx, *seg_of_cid, *gid_next, *medium, *huge;
+struct SumOut {
+  uint32_t *sum, *newidx, *seg_of_cid, *gid_next, *medium, *huge, *counts;  // counts: medium, huge
   const uint32_t *gid, *rank;  // rank null: the buckets hold labels
   uint64_t *seg_off;
-  __device__ void operator()(uint64_t l, Pair64 prefix, Pair64 v) const {
-    const uint32_t at = static_cast<uint32_t>(prefix.a);
-    newidx[l] = v.a ? at : kNone;
-    if (!v.a) return;
-    sum[l] = static_cast<uint32_t>(prefix.b);
-    if (rank) seg_of_cid[rank[l]] = at;
-    gid_next[at] = gid ? gid[l] : static_cast<uint32_t>(l);
-    seg_off[at] = sum_edges(prefix.b);
-    if (v.a >> 32) medium[prefix.a >> 32] = at;
-    if (v.b >> kSumHuge) huge[prefix.b >> kSumHuge] = at;
-  }
 };
-__global__ __launch_bounds__(kWave) void k_sum_finish(const Pair64 *total, uint64_t *seg_off, const uint64_t *ids,
+// k_scan_down over the sums, everything read of a label loaded ahead of the
+// stores and the lists appended with one atomic each per wave.
+__global__ __launch_bounds__(kBlock) void k_sum_down(uint64_t n, SumOut o, const uint64_t *block_prefix,
+                                                    uint64_t *total_out, const uint64_t *block_sums) {
+  __shared__ uint64_t wsum[kBlock / kWave];
+  const uint64_t base = scan_base();
+  const SumLoad load{o.sum};
+  uint64_t v[kScanPerThread], before[kScanPerThread], all;
+  uint32_t gid[kScanPerThread], rank[kScanPerThread];
+#pragma unroll
+  for (int j = 0; j < kScanPerThread; ++j) v[j] = base + j * kWave < n ? load(base + j * kWave) : 0ull;
+#pragma unroll
+  for (int j = 0; j < kScanPerThread; ++j) {
+    const uint64_t l = base + j * kWave;
+    gid[j] = o.gid && l < n ? o.gid[l] : static_cast<uint32_t>(l);
+    rank[j] = o.rank && l < n ? o.rank[l] : 0u;
+  }
+  const uint64_t run = scan_tile<uint64_t>(v, before, block_prefix, block_sums, wsum, &all);
+  uint32_t n_medium = 0, n_huge = 0;  // of the wave
+#pragma unroll
+  for (int j = 0; j < kScanPerThread; ++j) {
+    const uint64_t l = base + j * kWave, prefix = run + before[j];
+    const uint32_t at = static_cast<uint32_t>(prefix >> 32), d = static_cast<uint32_t>(v[j]);
+    n_medium += static_cast<uint32_t>(__popcll(__ballot(d > kDedupWaveCap && d <= kDedupBlockCap)));
+    n_huge += static_cast<uint32_t>(__popcll(__ballot(d > kDedupBlockCap)));
+    if (l < n) o.newidx[l] = d ? at : kNone;
+    if (!d) continue;
+    o.sum[l] = static_cast<uint32_t>(prefix);
+    if (o.rank) o.seg_of_cid[rank[j]] = at;
+    o.gid_next[at] = gid[j];
+    o.seg_off[at] = static_cast<uint32_t>(prefix);
+  }
+  if (n_medium | n_huge) {
+    uint32_t at_medium = 0, at_huge = 0;
+    if (lane_id() == 0) {
+      if (n_medium) at_medium = atomicAdd(o.counts, n_medium);
+      if (n_huge) at_huge = atomicAdd(o.counts + 1, n_huge);
+    }
+    at_medium = __shfl(at_medium, 0);
+    at_huge = __shfl(at_huge, 0);
+#pragma unroll
+    for (int j = 0; j < kScanPerThread; ++j) {
+      const uint32_t d = static_cast<uint32_t>(v[j]), at = static_cast<uint32_t>((run + before[j]) >> 32);
+      const bool medium = d > kDedupWaveCap && d <= kDedupBlockCap, huge = d > kDedupBlockCap;
+      const uint64_t m = __ballot(medium), h = __ballot(huge);
+      if (medium) o.medium[at_medium + __popcll(m & lanes_below())] = at;
+      if (huge) o.huge[at_huge + __popcll(h & lanes_below())] = at;
+      at_medium += static_cast<uint32_t>(__popcll(m));
+      at_huge += static_cast<uint32_t>(__popcll(h));
+    }
+  }
+  if (total_out && blockIdx.x == gridDim.x - 1 && threadIdx.x == kBlock - 1) *total_out = all;
+}
+
+__global__ __launch_bounds__(kWave) void k_sum_finish(const uint64_t *total, uint64_t *seg_off, const uint64_t *ids,
                                                      uint64_t *host_sizes, HostWords words) {
   if (threadIdx.x == 0) {
-    const uint64_t clusters = static_cast<uint32_t>(total->a), edges = sum_edges(total->b);
+    const uint64_t clusters = *total >> 32, edges = static_cast<uint32_t>(*total);
     if (ids) host_sizes[9] = *ids;
     seg_off[clusters] = edges;
     host_sizes[0] = clusters;
     host_sizes[1] = edges;
-    host_sizes[3] = total->a >> 32;
-    host_sizes[4] = total->b >> kSumHuge;
   }
   put_words(words);
 }
@@ -2103,11 +2151,10 @@ __global__ __launch_bounds__(kBlock) void k_labels_from_keys(uint64_t n, const u
 
 // out = sum of partial[0..count) (one block).
 __global__ __launch_bounds__(kBlock) void k_reduce_sum(const uint32_t *partial, uint64_t count, uint32_t *out) {
-  __shared__ uint64_t smem[kBlock];
+  __shared__ uint64_t wsum[kBlock / kWave];
   uint64_t acc = 0;
   for (uint64_t i = threadIdx.x; i < count; i += kBlock) acc += partial[i];
-  uint64_t tot;
-  block_exclusive_scan_shift<uint64_t>(acc, smem, &tot);
+  const uint64_t tot = block_total<uint64_t>(acc, wsum);
   if (threadIdx.x == 0) *out = static_cast<uint32_t>(tot);
 }
 
@@ -2318,12 +2365,22 @@ __global__ __launch_bounds__(kBlock) void k_round_volumes(uint64_t n, const uint
                                                          uint32_t t, unsigned long long *out) {
   __shared__ unsigned long long part[2][kBlock / kWave];
   uint64_t at = 0, above = 0;
-  for (uint64_t v = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x; v < n;
-       v += static_cast<uint64_t>(gridDim.x) * kBlock) {
-    const uint32_t d = static_cast<uint32_t>(key[v] >> 32);
-    const uint64_t deg = off[v + 1] - off[v];
-    at += d == t ? deg : 0;
-    above += d > t ? deg : 0;
+  constexpr int kU = 4;  // vertices whose loads a lane keeps in flight
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
+  for (uint64_t v0 = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x; v0 < n; v0 += kU * stride) {
+    uint32_t d[kU];
+    uint64_t deg[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const uint64_t v = min(v0 + u * stride, n - 1);
+      d[u] = static_cast<uint32_t>(key[v] >> 32);
+      deg[u] = v0 + u * stride < n ? off[v + 1] - off[v] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      at += d[u] == t ? deg[u] : 0;
+      above += d[u] > t ? deg[u] : 0;
+    }
   }
   for (int o = 32; o > 0; o >>= 1) {
     at += static_cast<uint64_t>(__shfl_xor(static_cast<unsigned long long>(at), o));
@@ -2344,7 +2401,9 @@ __global__ __launch_bounds__(kBlock) void k_round_volumes(uint64_t n, const uint
 void round_volumes(uint64_t n, const uint64_t *off, const uint64_t *key, uint32_t t, uint64_t *out, hipStream_t s) {
   fill_u64(out, 2, 0, s);
   if (!n) return;
-  const unsigned g = static_cast<unsigned>(std::min<uint64_t>(ceil_div(n, kBlock), 2048));
+  // (a block's two atomics queue behind the others': 2048 blocks 28 us on 2^20
+  // vertices, 512 blocks 10)
+  const unsigned g = static_cast<unsigned>(std::min<uint64_t>(ceil_div(n, 4 * kBlock), 512));
   hipLaunchKernelGGL(k_round_volumes, dim3(g), dim3(kBlock), 0, s, n, off, key, t,
                      reinterpret_cast<unsigned long long *>(out));
   KC_LAUNCH_CHECK();
@@ -2574,10 +2633,21 @@ void cluster_sums(uint64_t n, const uint32_t *lab, const uint32_t *deg_inter, ui
 
 void sum_segments(uint64_t n, uint32_t *sum, const uint32_t *gid, const uint32_t *rank, uint32_t *newidx,
                   uint32_t *seg_of_cid, uint32_t *gid_next, uint64_t *seg_off, uint32_t *medium, uint32_t *huge,
-                  const uint64_t *ids, uint64_t *host_sizes, HostWords words, uint64_t *scratch, hipStream_t s) {
-  Pair64 *total = reinterpret_cast<Pair64 *>(scratch);
-  scan_exclusive<Pair64>(n, SumLoad{sum}, SumStore{sum, newidx, seg_of_cid, gid_next, medium, huge, gid, rank, seg_off},
-                         total, scratch + 4, s);
+                  uint32_t *counts, const uint64_t *ids, uint64_t *host_sizes, HostWords words, uint64_t *scratch,
+                  hipStream_t s) {
+  const SumOut out{sum, newidx, seg_of_cid, gid_next, medium, huge, counts, gid, rank, seg_off};
+  const uint64_t blocks = ceil_div(n, kScanTile);
+  uint64_t *total = scratch, *sums = scratch + 4, *prefix = sums + blocks;
+  hipLaunchKernelGGL((k_scan_reduce<uint64_t, SumLoad>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, s, n,
+                     SumLoad{sum}, sums);
+  KC_LAUNCH_CHECK();
+  const bool fused = blocks <= kScanFusedBlocks;
+  if (!fused)
+    scan_exclusive<uint64_t>(blocks, ArrayLoad<uint64_t>{sums}, ArrayStore<uint64_t>{prefix}, total, prefix + blocks + 4,
+                             s);
+  hipLaunchKernelGGL(k_sum_down, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, s, n, out,
+                     fused ? static_cast<const uint64_t *>(nullptr) : prefix, fused ? total : nullptr, sums);
+  KC_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_sum_finish, dim3(1), dim3(kWave), 0, s, total, seg_off, ids, host_sizes, words);
   KC_LAUNCH_CHECK();
 }

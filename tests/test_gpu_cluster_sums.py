@@ -1,5 +1,5 @@
 """Clusters placed by their running sums, against the oracle (labels, levels and radii): level sizes around the
-workgroups' 4096 vertices, one cluster holding nearly all of a level or thousands of small ones, buckets of every
+workgroups' 4096 vertices and the scans' tiles of 2048 (runs of 512 a wave), one cluster holding nearly all of a level or thousands of small ones, buckets of every
 dedup class, and levels on both sides of the dense cluster ids' bounds (2^20 vertices, average degree 8)."""
 import numpy as np
 import pytest
@@ -23,7 +23,7 @@ def check(g, trace=True, **kw):
     return lv
 
 
-@pytest.mark.parametrize("n", [2, 63, 4095, 4096, 4097, 8191, 12289])
+@pytest.mark.parametrize("n", [2, 63, 511, 513, 2047, 2048, 2049, 4095, 4096, 4097, 8191, 12289])
 @pytest.mark.parametrize("shape", ["path", "star", "random", "cliques"])
 def test_level_sizes(n, shape):
     rng = np.random.default_rng(n)
@@ -67,3 +67,11 @@ def test_dense_id_bounds(n, m):
     """G(n, m) with nearly no isolated vertex: the average degree lies below or above 8, n below or above 2^20."""
     g = ca.generate("gnm_undirected", n=n, m=m, seed=2)
     check(g, trace=False, variant="exp", seed=4, seq_limit=4096, stream=ca.STREAM_HASHED, use_bfs=True, input_order=True)
+
+
+@pytest.mark.parametrize("n", [1024 * 2048, 1024 * 2048 + 1])
+def test_scan_levels(n):
+    """A ring: the label scan takes two launches up to 1024 tiles, four above."""
+    v = np.arange(n)
+    g = ca.Graph.from_edges(n, np.stack([v, (v + 1) % n], 1))
+    check(g, trace=False, variant="exp", seed=8, seq_limit=4096, stream=ca.STREAM_HASHED, use_bfs=True)
