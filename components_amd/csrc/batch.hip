@@ -1252,7 +1252,7 @@ int kc_batch_run(kc_batch *b, const kc_options *opt, uint32_t *labels_out, kc_ba
     else
       kc_options_init(&o);
     const auto t0 = std::chrono::steady_clock::now();
-    CopyOut labels(labels_out, 4ull * b->n, b->device);
+    CopyOut labels(labels_out, 4ull * b->n);
     batch_params(b, o);
     const float ms = run_once(b, o);
     labels.finish(b->dev.labels, b->stream);

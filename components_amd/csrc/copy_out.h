@@ -1,4 +1,4 @@
-// Device arrays copied out to the caller's pageable memory.
+// Results to the caller's pageable host memory.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -11,32 +11,31 @@ namespace kc {
 // call; bytes are whole words and src is aligned to 16 bytes.  The constructor
 // (at the call's start; dst may be null: nothing to do) lets helper threads
 // fault in dst's pages while the GPU works, without changing what they hold.
-// enqueue() may put a small copy into the stream ahead of a wait the caller
-// makes anyway (waited: that is over); finish() copies, src final in stream
-// order, and returns when dst is written.  Destroying it without finish()
-// leaves dst as it was.  Throws Failure.
+// enqueue() puts the first transfers into the stream, ahead of a wait the
+// caller makes anyway; finish() copies, src final in stream order, and returns
+// when dst is written.  Destroying it without finish() leaves dst as it was.
+// Throws Failure.
 class CopyOut {
  public:
-  CopyOut(void *dst, size_t bytes, int device);
+  CopyOut(void *dst, size_t bytes);
   ~CopyOut();
   CopyOut(const CopyOut &) = delete;
   CopyOut &operator=(const CopyOut &) = delete;
   void enqueue(const void *src, hipStream_t stream);
-  void finish(const void *src, hipStream_t stream, bool waited = false);
+  void finish(const void *src, hipStream_t stream);
 
  private:
   struct Job;
-  Job *job_ = nullptr;     // large copies: the helpers' shared state
-  char *ring_ = nullptr;   // the borrowed pinned memory
-  bool queued_ = false;    // a small copy into it is in stream_
+  friend struct Helpers;
+  void issue();
+  Job *job_ = nullptr;
+  const char *src_ = nullptr;
   hipStream_t stream_ = nullptr;
-  void *dst_;
-  size_t bytes_;
-  int device_;
+  bool queued_ = false;  // transfers into the ring are in the stream
 };
 
-// Handles that copy out hold a reference; the pinned staging memory is given
-// back with the last one.
+// Handles whose calls copy results keep the pinned ring and the helper threads
+// alive; the last one gives them back.
 void copy_out_retain();
 void copy_out_release();
 

@@ -1,21 +1,24 @@
 // Labels to the caller's pageable memory.  hipMemcpy moved them through the
 // runtime's staging buffer on one thread, which also took the page faults of
 // a fresh buffer: 10 GB/s (16.8 M labels: 6.4 ms beside 7 to 9 ms of GPU work),
-// against 56 GB/s into pinned memory.  Here a ring of pinned slots takes the
-// transfers while helper threads move finished slots on, and the pages are faulted
-// in while the GPU still works.
+// against 56 GB/s into pinned memory.  Here kernels store them into a pinned
+// ring, helper threads move them on piece by piece as the pieces arrive, and the
+// pages are faulted in while the GPU still works.
 #include "copy_out.h"
 
+#include <sched.h>
 #include <sys/mman.h>
 #include <unistd.h>
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstdint>
 #include <cstring>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -29,63 +32,70 @@ namespace kc {
 
 namespace {
 
-// (short transfers leave gaps between them: 64 of 1 MB took 2.3 ms where 16 of
-// 4 MB take 1.6)
-constexpr size_t kSlotBytes = 4 << 20;
+constexpr size_t kSlotBytes = 4 << 20;  // of the ring: what one transfer fills once the ring has been round
 constexpr int kSlots = 4;
-constexpr size_t kPieceBytes = 512 << 10;  // moved on by one helper
-// below this one copy into pinned memory and one memcpy: a thread costs more
-constexpr size_t kThreadsMin = 1 << 20;
+constexpr size_t kRingBytes = kSlots * kSlotBytes;
+// what one thread moves on at once (a quarter of a megabyte takes it about 28 us)
+constexpr size_t kPiece = 256 << 10, kLargePiece = 512 << 10;
+// from here on with helper threads (below, waking them takes longer)
+constexpr size_t kHelpersMin = 256 << 10;
 constexpr int kMaxHelpers = 8;
-constexpr size_t kFaultBytes = 2 << 20;
+constexpr size_t kFaultBytes = 512 << 10;
 
-// The pinned ring: one for the process (16 MB, with an event per slot), lent
-// to one copy at a time and given back with the last handle.
+// A transfer by stores from the CUs: 50 GB/s always, where the copy engine that
+// hipMemcpyAsync picks runs at 57 or, for long stretches on some streams, at
+// 20 (67 MB: 3.6 instead of 1.6 ms).  What bounds it is the host link; 64
+// workgroups fill it (16: 5% slower).  Every workgroup tells of its share of
+// every piece by a word of its own in pinned memory, so that the host needs
+// neither an event nor a launch per piece.
+constexpr unsigned kTransferBlocks = 64;
+
+__global__ __launch_bounds__(kBlock) void k_transfer(uint32_t *dst, const uint32_t *src, uint64_t words,
+                                                     uint64_t piece_words, uint32_t *arrived, uint32_t value) {
+  const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
+  const uint64_t first = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
+  for (uint64_t at = 0, p = 0; at < words; at += piece_words, ++p) {
+    const uint64_t n = min(piece_words, words - at);
+    uint64_t *to = reinterpret_cast<uint64_t *>(dst + at);
+    const uint64_t *from = reinterpret_cast<const uint64_t *>(src + at);
+    for (uint64_t i = first; i < n / 2; i += stride) host_store(to + i, from[i]);
+    if (first == 0 && n % 2) host_store(dst + at + n - 1, src[at + n - 1]);
+    host_stores_done();
+    __syncthreads();
+    if (threadIdx.x == 0) host_store(arrived + p * kTransferBlocks + blockIdx.x, value);
+  }
+}
+
+constexpr size_t kArrivedBytes = kRingBytes / kPiece * kTransferBlocks * sizeof(uint32_t);
+
+// The pinned ring: one for the process (16 MB and the arrival words), lent to
+// one copy at a time and given back with the last handle.
 struct Ring {
   std::mutex m;
   int handles = 0;
   bool lent = false;
   char *mem = nullptr;
-  int device = -1;  // the events' device
-  hipEvent_t events[kSlots] = {};
+  uint32_t value = 0;  // of the last transfer (the borrower's)
 } g_ring;
 
-// (the caller holds the mutex)
-void ring_drop_events() {
-  for (hipEvent_t &e : g_ring.events) {
-    if (e) (void)hipEventDestroy(e);
-    e = nullptr;
-  }
-  g_ring.device = -1;
-}
-
 void ring_drop() {
-  ring_drop_events();
   if (g_ring.mem) (void)hipHostFree(g_ring.mem);
   g_ring.mem = nullptr;
 }
 
 // Null when another copy holds the ring or it cannot be had.
-char *ring_borrow(int device) {
+char *ring_borrow() {
   std::lock_guard<std::mutex> lock(g_ring.m);
   if (g_ring.lent) return nullptr;
   if (!g_ring.mem) {
     void *p = nullptr;
-    if (hipHostMalloc(&p, kSlotBytes * kSlots, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
+    if (hipHostMalloc(&p, kRingBytes + kArrivedBytes, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
       (void)hipGetLastError();
       return nullptr;
     }
     g_ring.mem = static_cast<char *>(p);
-  }
-  if (g_ring.device != device) {
-    ring_drop_events();
-    for (hipEvent_t &e : g_ring.events)
-      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-        (void)hipGetLastError();
-        e = nullptr;
-        return nullptr;
-      }
-    g_ring.device = device;
+    std::memset(g_ring.mem + kRingBytes, 0, kArrivedBytes);
+    g_ring.value = 0;
   }
   g_ring.lent = true;
   return g_ring.mem;
@@ -97,28 +107,6 @@ void ring_return() {
   if (g_ring.handles == 0) ring_drop();
 }
 
-// A transfer by stores from the CUs: 50 GB/s always, where the copy engine that
-// hipMemcpyAsync picks runs at 57 or, for long stretches on some streams, at
-// 20 (67 MB: 3.6 instead of 1.6 ms).  What bounds it is the host link; 64
-// workgroups fill it (16: 5% slower).
-constexpr unsigned kTransferBlocks = 64;
-
-__global__ __launch_bounds__(kBlock) void k_transfer(uint32_t *dst, const uint32_t *src, uint64_t words) {
-  const uint64_t quads = words / 4, stride = static_cast<uint64_t>(gridDim.x) * kBlock;
-  const uint64_t first = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
-  for (uint64_t i = first; i < quads; i += stride)
-    reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
-  if (first < words % 4) dst[4 * quads + first] = src[4 * quads + first];
-}
-
-// src and bytes: whole words, src aligned to 16 (device arrays and their
-// multiples of a piece).
-void transfer(void *slot, const void *src, size_t bytes, hipStream_t s) {
-  hipLaunchKernelGGL(k_transfer, dim3(kTransferBlocks), dim3(kBlock), 0, s, static_cast<uint32_t *>(slot),
-                     static_cast<const uint32_t *>(src), bytes / 4);
-  KC_LAUNCH_CHECK();
-}
-
 // Faults in the whole pages inside [p, p + bytes) for writing (their contents
 // stay); where the kernel cannot, the copy takes the faults.
 void fault_in(char *p, size_t bytes) {
@@ -128,180 +116,265 @@ void fault_in(char *p, size_t bytes) {
   if (z > a) (void)madvise(reinterpret_cast<void *>(a), z - a, MADV_POPULATE_WRITE);
 }
 
-}  // namespace
-
-// Pages and chunks are claimed one after another by whichever helper is free,
-// so the copy does not depend on how many threads there are (at least one).
-struct CopyOut::Job {
-  char *dst = nullptr;
-  size_t bytes = 0;
-  int helpers = 0;
-  std::thread first;                // starts the other helpers and joins them
-  std::mutex m;
-  std::condition_variable changed;  // some of the following moved on
-  size_t next_fault = 0;            // bytes whose pages are claimed
-  // once the copy begins: transfers of `chunk` bytes, one ring slot each, moved
-  // on in pieces
-  size_t chunk = 0;
-  size_t ready = 0;                 // bytes that have reached their slots
-  size_t claimed = 0, done = 0;     // bytes taken and moved by helpers
-  std::vector<size_t> left;         // per transfer: bytes still in its slot
-  bool stop = false;
-  const char *ring = nullptr;
-
-  void help() {
-    std::unique_lock<std::mutex> lock(m);
-    while (!stop) {
-      if (claimed < ready) {
-        const size_t at = claimed, c = at / chunk;
-        const size_t n = std::min({kPieceBytes, (c + 1) * chunk - at, bytes - at});
-        claimed += n;
-        lock.unlock();
-        std::memcpy(dst + at, ring + (c % kSlots) * kSlotBytes + (at - c * chunk), n);
-        lock.lock();
-        left[c] -= n;
-        done += n;
-        if (left[c] == 0) changed.notify_all();
-      } else if (claimed >= bytes) {
-        return;
-      } else if (next_fault < bytes) {
-        const size_t at = next_fault;
-        next_fault += kFaultBytes;
-        lock.unlock();
-        fault_in(dst + at, std::min(kFaultBytes, bytes - at));
-        lock.lock();
-      } else {
-        changed.wait(lock);
-      }
-    }
+// A spinning thread's turn: a pause, and after a while the CPU to others.
+struct Spin {
+  int turns = 0;
+  void operator()() {
+    if (++turns < 2000)
+      __builtin_ia32_pause();
+    else
+      sched_yield();
   }
-  void start() {
-    first = std::thread([this] {
-      std::vector<std::thread> others;
-      try {
-        for (int h = 1; h < helpers; ++h) others.emplace_back([this] { help(); });
-      } catch (...) {  // fewer helpers then
-      }
-      help();
-      for (auto &t : others) t.join();
-    });
-  }
-  void end() {
-    {
-      std::lock_guard<std::mutex> lock(m);
-      stop = true;
-      changed.notify_all();
-    }
-    if (first.joinable()) first.join();
-  }
-  ~Job() { end(); }
 };
 
-CopyOut::CopyOut(void *dst, size_t bytes, int device) : dst_(dst), bytes_(dst ? bytes : 0), device_(device) {
-  if (bytes_ <= kThreadsMin) return;
+}  // namespace
+
+// Pieces and pages are claimed one after another by whichever thread is free,
+// so a copy does not depend on how many helpers there are, or whether any.
+struct CopyOut::Job {
+  char *dst = nullptr;
+  size_t bytes = 0, piece = 0, pieces = 0;
+  unsigned blocks = 0;
+  // under the helpers' mutex
+  bool listed = false, hot = false;  // hot: the transfers are in the stream
+  int users = 0;                     // helpers at work on it
+  size_t next_fault = 0;             // bytes whose pages are claimed
+  // the copy itself
+  char *ring = nullptr;
+  uint32_t first_value = 0;              // of the first transfer; the later ones count on
+  size_t issued = 0;                     // bytes with a transfer in the stream (the calling thread's)
+  std::atomic<size_t> next_piece{0};     // claimed
+  std::atomic<size_t> done{0};           // bytes moved
+  std::unique_ptr<std::atomic<size_t>[]> left;  // per slot's turn: bytes still in it
+  std::atomic<bool> commit{false}, stop{false};
+
+  size_t slot_turns() const { return (bytes + kSlotBytes - 1) / kSlotBytes; }
+  // the transfer that a slot's turn belongs to: the first fills the whole ring
+  uint32_t value_of(size_t turn) const { return first_value + static_cast<uint32_t>(turn < kSlots ? 0 : turn - kSlots + 1); }
+
+  bool has_arrived(size_t p) const {
+    const size_t at = p * piece;
+    const uint32_t want = value_of(at / kSlotBytes);
+    const uint32_t *words =
+        reinterpret_cast<const uint32_t *>(ring + kRingBytes) + at % kRingBytes / piece * kTransferBlocks;
+    for (unsigned b = 0; b < blocks; ++b)
+      if (__atomic_load_n(words + b, __ATOMIC_ACQUIRE) != want) return false;
+    return true;
+  }
+  void move(size_t p) {
+    const size_t at = p * piece, n = std::min(piece, bytes - at);
+    std::memcpy(dst + at, ring + at % kRingBytes, n);
+    left[at / kSlotBytes].fetch_sub(n, std::memory_order_release);
+    done.fetch_add(n, std::memory_order_release);
+  }
+  // a helper's share: pieces until none is left
+  void help() {
+    while (true) {
+      const size_t p = next_piece.fetch_add(1);
+      if (p >= pieces) return;
+      Spin spin;
+      while (!commit.load(std::memory_order_acquire) || !has_arrived(p)) {
+        if (stop.load(std::memory_order_relaxed)) return;
+        spin();
+      }
+      move(p);
+    }
+  }
+};
+
+// The helper threads: up to eight for the process, asleep between copies,
+// started by the first copy that wants them and given back with the last
+// handle.  They serve every copy that is under way.
+struct Helpers {
+  std::mutex m;
+  std::condition_variable wake, idle;
+  std::vector<CopyOut::Job *> jobs;
+  std::vector<std::thread> threads;
+  bool quit = false;
+
+  void run() {
+    std::unique_lock<std::mutex> lock(m);
+    while (!quit) {
+      CopyOut::Job *hot = nullptr, *cold = nullptr;
+      for (CopyOut::Job *j : jobs) {
+        if (j->hot && j->next_piece.load() < j->pieces) hot = j;
+        if (j->next_fault < j->bytes) cold = j;
+      }
+      if (hot) {
+        ++hot->users;
+        lock.unlock();
+        hot->help();
+        lock.lock();
+        if (--hot->users == 0) idle.notify_all();
+      } else if (cold) {
+        const size_t at = cold->next_fault;
+        cold->next_fault += kFaultBytes;
+        ++cold->users;
+        lock.unlock();
+        fault_in(cold->dst + at, std::min(kFaultBytes, cold->bytes - at));
+        lock.lock();
+        if (--cold->users == 0) idle.notify_all();
+      } else {
+        wake.wait(lock);
+      }
+    }
+  }
+  void add(CopyOut::Job *j) {
+    const int cpus = static_cast<int>(std::thread::hardware_concurrency());
+    const size_t want = static_cast<size_t>(std::max(1, std::min(kMaxHelpers, cpus / 2)));
+    std::lock_guard<std::mutex> lock(m);
+    while (threads.size() < want) {
+      try {
+        threads.emplace_back([this] { run(); });
+      } catch (...) {  // fewer helpers then
+        break;
+      }
+    }
+    j->listed = true;
+    jobs.push_back(j);
+    wake.notify_all();
+  }
+  void heat(CopyOut::Job *j) {
+    std::lock_guard<std::mutex> lock(m);
+    j->hot = true;
+    j->next_fault = j->bytes;  // what is left of the pages the copy takes
+    wake.notify_all();
+  }
+  // returns when no helper touches the job
+  void remove(CopyOut::Job *j) {
+    std::unique_lock<std::mutex> lock(m);
+    if (!j->listed) return;
+    jobs.erase(std::find(jobs.begin(), jobs.end(), j));
+    idle.wait(lock, [&] { return j->users == 0; });
+  }
+  void end() {
+    std::vector<std::thread> mine;
+    {
+      std::lock_guard<std::mutex> lock(m);
+      quit = true;
+      wake.notify_all();
+      mine.swap(threads);
+    }
+    for (std::thread &t : mine) t.join();
+    std::lock_guard<std::mutex> lock(m);
+    quit = false;
+  }
+};
+
+namespace {
+// (never destroyed: a process may end with handles open and helpers asleep)
+Helpers &helpers() {
+  static Helpers *h = new Helpers;
+  return *h;
+}
+std::mutex g_handles;  // retain, release and the helpers' end
+}  // namespace
+
+CopyOut::CopyOut(void *dst, size_t bytes) {
+  if (!dst || !bytes) return;
   std::unique_ptr<Job> j(new Job);
   j->dst = static_cast<char *>(dst);
   j->bytes = bytes;
-  const int cpus = static_cast<int>(std::thread::hardware_concurrency());
-  j->helpers = std::max(1, std::min({kMaxHelpers, cpus / 2, static_cast<int>(bytes_ / kThreadsMin)}));
-  try {
-    j->start();
-  } catch (...) {  // no thread to be had: finish() copies the plain way
-    return;
-  }
+  j->piece = bytes > kRingBytes ? kLargePiece : kPiece;
+  j->pieces = (bytes + j->piece - 1) / j->piece;
+  j->blocks = static_cast<unsigned>(std::min<size_t>(kTransferBlocks, (bytes + 4095) / 4096));
+  j->left.reset(new std::atomic<size_t>[j->slot_turns()]);
+  for (size_t t = 0; t < j->slot_turns(); ++t) j->left[t] = std::min(kSlotBytes, bytes - t * kSlotBytes);
+  if (bytes > kHelpersMin) helpers().add(j.get());
   job_ = j.release();
 }
 
 CopyOut::~CopyOut() {
+  if (!job_) return;
+  job_->stop = true;
+  helpers().remove(job_);
+  if (queued_) (void)hipStreamSynchronize(stream_);  // no transfer into the ring is left in the stream
+  if (job_->ring) ring_return();
   delete job_;
-  if (queued_) (void)hipStreamSynchronize(stream_);
-  if (ring_) ring_return();
+}
+
+// The next transfer: the whole ring at first, then a slot at a time.
+void CopyOut::issue() {
+  Job &j = *job_;
+  const size_t n = std::min(j.issued ? kSlotBytes : kRingBytes, j.bytes - j.issued), at = j.issued % kRingBytes;
+  uint32_t *arrived = reinterpret_cast<uint32_t *>(j.ring + kRingBytes) + at / j.piece * kTransferBlocks;
+  queued_ = true;
+  hipLaunchKernelGGL(k_transfer, dim3(j.blocks), dim3(kBlock), 0, stream_, reinterpret_cast<uint32_t *>(j.ring + at),
+                     reinterpret_cast<const uint32_t *>(src_ + j.issued), n / 4, j.piece / 4, arrived,
+                     j.value_of(j.issued / kSlotBytes));
+  KC_LAUNCH_CHECK();
+  g_ring.value = j.value_of(j.issued / kSlotBytes);
+  j.issued += n;
 }
 
 void CopyOut::enqueue(const void *src, hipStream_t stream) {
-  if (!bytes_ || bytes_ > kThreadsMin) return;
-  if (!ring_) ring_ = ring_borrow(device_);
-  if (!ring_) return;
-  transfer(ring_, src, bytes_, stream);
-  queued_ = true;
+  if (!job_) return;
+  Job &j = *job_;
+  if (!j.ring) {
+    j.ring = ring_borrow();
+    if (!j.ring) return;
+    j.first_value = g_ring.value + 1;
+  } else {  // (a call that starts over)
+    j.first_value = g_ring.value + 1;
+    j.issued = 0;
+  }
+  src_ = static_cast<const char *>(src);
   stream_ = stream;
+  issue();
+  if (j.listed && !j.hot) helpers().heat(&j);
 }
 
-void CopyOut::finish(const void *src, hipStream_t stream, bool waited) {
-  if (!bytes_) return;
-  if (bytes_ <= kThreadsMin) {
-    waited = waited && queued_;
-    if (!queued_) enqueue(src, stream);
-    if (queued_) {
-      if (!waited) KC_HIP(hipStreamSynchronize(stream));
-      queued_ = false;
-      std::memcpy(dst_, ring_, bytes_);
-      return;
-    }
-  } else if (job_) {
-    ring_ = ring_borrow(device_);
-  }
-  if (!ring_ || !job_) {  // another copy holds the ring, or there is no helper
-    KC_HIP(hipMemcpyAsync(dst_, src, bytes_, hipMemcpyDeviceToHost, stream));
+void CopyOut::finish(const void *src, hipStream_t stream) {
+  if (!job_) return;
+  Job &j = *job_;
+  if (!queued_) enqueue(src, stream);
+  if (!queued_) {  // another copy holds the ring
+    KC_HIP(hipMemcpyAsync(j.dst, src, j.bytes, hipMemcpyDeviceToHost, stream));
     KC_HIP(hipStreamSynchronize(stream));
     return;
   }
-  Job &j = *job_;
-  // short copies in at least four transfers, so that moving overlaps them
-  const size_t chunk = std::min(kSlotBytes, (bytes_ / 4 + kPieceBytes - 1) / kPieceBytes * kPieceBytes);
-  const size_t chunks = (bytes_ + chunk - 1) / chunk;
-  {
-    std::lock_guard<std::mutex> lock(j.m);
-    j.chunk = chunk;
-    j.left.resize(chunks);
-    for (size_t c = 0; c < chunks; ++c) j.left[c] = std::min(chunk, bytes_ - c * chunk);
-    j.ring = ring_;
-  }
-  // however this ends, the helpers stop and no copy into the ring is left in
-  // the stream
-  struct Drain {
-    Job &j;
-    hipStream_t s;
-    ~Drain() {
-      j.end();
-      (void)hipStreamSynchronize(s);
+  j.commit.store(true, std::memory_order_release);
+  Spin spin;
+  int idle = 0;
+  auto looked = std::chrono::steady_clock::now();
+  while (j.done.load(std::memory_order_acquire) < j.bytes) {
+    // (only this thread talks to the runtime)
+    while (j.issued < j.bytes && j.left[j.issued / kSlotBytes - kSlots].load(std::memory_order_acquire) == 0) issue();
+    size_t p = j.next_piece.load();
+    if (p < j.pieces && p * j.piece < j.issued && j.has_arrived(p)) {
+      if (j.next_piece.compare_exchange_strong(p, p + 1)) j.move(p);
+      spin.turns = idle = 0;
+      continue;
     }
-  } drain{j, stream};
-  // (only this thread talks to the runtime)
-  size_t issued = 0, arrived = 0;
-  while (arrived < chunks) {
-    while (issued < chunks && issued < arrived + kSlots) {
-      if (issued >= kSlots) {  // its slot's last transfer has to be moved on first
-        std::unique_lock<std::mutex> lock(j.m);
-        if (j.left[issued - kSlots] != 0) {
-          if (issued > arrived) break;
-          j.changed.wait(lock, [&] { return j.left[issued - kSlots] == 0; });
-        }
+    spin();
+    if (spin.turns % 1024 == 0) {
+      const auto now = std::chrono::steady_clock::now();
+      if (now - looked > std::chrono::milliseconds(2)) {  // a fault ends the wait
+        const hipError_t e = hipStreamQuery(stream);
+        if (e != hipErrorNotReady) KC_HIP(e);
+        idle = e == hipSuccess ? idle + 1 : 0;
+        if (idle > 500) fail(KC_ERR_HIP, "internal: the stream is idle and labels did not arrive");
+        looked = now;
       }
-      const size_t off = issued * chunk;
-      transfer(ring_ + (issued % kSlots) * kSlotBytes, static_cast<const char *>(src) + off,
-               std::min(chunk, bytes_ - off), stream);
-      KC_HIP(hipEventRecord(g_ring.events[issued % kSlots], stream));
-      ++issued;
     }
-    KC_HIP(hipEventSynchronize(g_ring.events[arrived % kSlots]));
-    ++arrived;
-    std::lock_guard<std::mutex> lock(j.m);
-    j.ready = std::min(arrived * chunk, bytes_);
-    j.changed.notify_all();
   }
-  std::unique_lock<std::mutex> lock(j.m);
-  j.changed.wait(lock, [&] { return j.done == bytes_; });
+  queued_ = false;  // every transfer has arrived
 }
 
 void copy_out_retain() {
+  std::lock_guard<std::mutex> order(g_handles);
   std::lock_guard<std::mutex> lock(g_ring.m);
   ++g_ring.handles;
 }
 
 void copy_out_release() {
-  std::lock_guard<std::mutex> lock(g_ring.m);
-  if (--g_ring.handles == 0 && !g_ring.lent) ring_drop();
+  std::lock_guard<std::mutex> order(g_handles);
+  {
+    std::lock_guard<std::mutex> lock(g_ring.m);
+    if (--g_ring.handles > 0) return;
+    if (!g_ring.lent) ring_drop();
+  }
+  helpers().end();
 }
 
 }  // namespace kc

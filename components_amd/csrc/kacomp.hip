@@ -479,12 +479,13 @@ void enqueue_bins(kc_graph *g, uint64_t n, const uint64_t *off, const BinCfg &cf
                g->scan_scratch, g->stream, key, tmin, words);
 }
 
-void read_bins(kc_graph *g, Bins &b) {
+void read_bins(kc_graph *g, uint64_t n, Bins &b) {
   b.nT = g->h_small[0];
   b.nS = g->h_small[1];
   b.nW = g->h_small[2];
   b.nH = g->h_small[3];
   if (b.nH > g->hubs_cap) fail(KC_ERR_INVALID, "hub chunk overflow (%u > %llu)", b.nH, (unsigned long long)g->hubs_cap);
+  if (uint64_t(b.nT) + b.nS + b.nW > n) fail(KC_ERR_INVALID, "internal: a level's bins exceed it");
   finish_bins(b);
 }
 
@@ -511,7 +512,7 @@ Bins make_bins(kc_graph *g, uint64_t n, const uint64_t *off, const BinCfg &cfg, 
   enqueue_bins(g, n, off, cfg, b, key ? g->flists : level0 ? g->l0_lists : g->lists,
                key ? g->fhubs : level0 ? g->l0_hubs : g->hubs, key, tmin, next_signal(g));
   await(g);
-  read_bins(g, b);
+  read_bins(g, n, b);
   if (level0) {
     g->l0_bins = b;
     g->l0_cfg = cfg;
@@ -1301,6 +1302,9 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
     const uint64_t label_space = dense ? g->h_sizes[9] : n_l;
     const uint64_t n_next = g->h_sizes[0], P = g->h_sizes[1];
     const uint64_t n_medium = g->h_small[14], n_huge = g->h_small[15];
+    if (n_next > n_l || P > m2_l || label_space > n_l || n_medium + n_huge > n_next)
+      fail(KC_ERR_INVALID, "internal: a level's clusters exceed it (%llu of %llu)",
+           static_cast<unsigned long long>(n_next), static_cast<unsigned long long>(n_l));
     rec.radius = local || pre ? 0 : g->h_small[13];
     if (!pre) out.sweeps += sweeps;  // the block passes are not decomposition sweeps
     out.radius_sum += rec.radius;
@@ -1347,8 +1351,9 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
     else
       publish_words(words, g->stream);
     await(g);
-    if (bins_valid) read_bins(g, b);
+    if (bins_valid) read_bins(g, n_next, b);
     const uint64_t m2_next = g->h_sizes[2];
+    if (m2_next > P) fail(KC_ERR_INVALID, "internal: a level's edges exceed its buckets");
     level_hot = m2_next > 0 && static_cast<double>(g->h_sizes[15]) * n_next >=
                                    kHotShareFactor * static_cast<double>(hot_rows) * m2_next;
     // dedup: every bucket slot read once, the unique ones written, per
@@ -2205,7 +2210,7 @@ int kc_find_components(kc_graph *g, const kc_options *opt, uint32_t *labels_out,
     }
     const auto t0 = std::chrono::steady_clock::now();
     g->have_labels = false;
-    CopyOut labels(labels_out, g->n * 4, g->device);
+    CopyOut labels(labels_out, g->n * 4);
     if (o.variant == KC_VARIANT_EXP) ensure_table(g, o.beta);
     g->arena.reset();
     g->timer.begin_run(o.time_kernels != 0, g->stream, o.time_class - 1);
@@ -2241,7 +2246,7 @@ int kc_find_components(kc_graph *g, const kc_options *opt, uint32_t *labels_out,
     if (o.variant == KC_VARIANT_EXP || o.variant == KC_VARIANT_LOCAL)
       g->components += static_cast<uint32_t>(g->n - g->n0);  // degree-0 vertices
     g->have_labels = true;
-    labels.finish(g->labels, g->stream, true);
+    labels.finish(g->labels, g->stream);
     float ms = 0.f;
     KC_HIP(hipEventSynchronize(g->ev_end));
     KC_HIP(hipEventElapsedTime(&ms, g->ev_begin, g->ev_end));
@@ -2416,7 +2421,7 @@ int kc_copy_labels(kc_graph *g, uint32_t *labels_out) {
   return guarded([&] {
     if (!g || !labels_out) fail(KC_ERR_INVALID, "null argument");
     if (!g->have_labels) fail(KC_ERR_INVALID, "no labels: kc_find_components has not completed");
-    CopyOut(labels_out, g->n * 4, g->device).finish(g->labels, g->stream);
+    CopyOut(labels_out, g->n * 4).finish(g->labels, g->stream);
   });
 }
 

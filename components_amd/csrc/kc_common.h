@@ -170,6 +170,16 @@ __device__ __forceinline__ uint32_t peeled_fetch_add(uint32_t *arr, uint32_t key
   return 0;
 }
 
+// Stores to the host's pinned memory, past the caches; host_stores_done returns
+// when this wave's have arrived.  (A system-scope fence in its place also writes
+// back the whole L2 of the wave's chiplet: 67 MB to the host in 512 KB pieces
+// 1.53 ms against 1.25.)
+template <class T>
+__device__ __forceinline__ void host_store(T *p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void host_stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // atomicMin(&arr[key], val) for every lane with part set, merged for the
 // lanes sharing the first lane's key and skipped when arr[key] is already
 // smaller (values only decrease, so a stale read only costs an atomic).

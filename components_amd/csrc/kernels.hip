@@ -182,16 +182,16 @@ __global__ __launch_bounds__(kBlock) void k_bin_write(uint64_t n, const uint64_t
   }
 }
 
-// words by one wave of a workgroup; the signal once every lane's own stores to
-// the host are through.
+// words by one wave; the signal once the wave's stores to the host have arrived,
+// all of which have to be host_stores (an ordinary one may wait in the L2 until
+// the kernel ends).
 __device__ __forceinline__ void put_words(const HostWords &w) {
   const uint32_t t = threadIdx.x;
-  if (t < 2 && w.from[t]) *w.to[t] = *w.from[t];
-  if (t < w.count32) w.to32[t] = w.from32[t];
+  if (t < 2 && w.from[t]) host_store(w.to[t], *w.from[t]);
+  if (t < w.count32) host_store(w.to32 + t, w.from32[t]);
   if (!w.signal) return;
-  __threadfence_system();
-  __builtin_amdgcn_wave_barrier();
-  if (t == 0) __hip_atomic_store(w.signal, w.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  host_stores_done();
+  if (t == 0) host_store(w.signal, w.value);
 }
 
 __global__ __launch_bounds__(kWave) void k_put_words(HostWords w) { put_words(w); }
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(kWave) void k_bin_totals(const uint64_t *prefix, co
   const int r = threadIdx.x;
   if (r < 4) {
     const uint64_t hi = r < 3 ? prefix[static_cast<uint64_t>(r + 1) * nblocks] : *total;
-    counters[r] = static_cast<uint32_t>(hi - prefix[static_cast<uint64_t>(r) * nblocks]);
+    host_store(counters + r, static_cast<uint32_t>(hi - prefix[static_cast<uint64_t>(r) * nblocks]));
   }
   put_words(words);
 }
@@ -1271,10 +1271,10 @@ __global__ __launch_bounds__(kWave) void k_sum_finish(const uint64_t *total, uin
                                                      uint64_t *host_sizes, HostWords words) {
   if (threadIdx.x == 0) {
     const uint64_t clusters = *total >> 32, edges = static_cast<uint32_t>(*total);
-    if (ids) host_sizes[9] = *ids;
+    if (ids) host_store(host_sizes + 9, *ids);
     seg_off[clusters] = edges;
-    host_sizes[0] = clusters;
-    host_sizes[1] = edges;
+    host_store(host_sizes, clusters);
+    host_store(host_sizes + 1, edges);
   }
   put_words(words);
 }

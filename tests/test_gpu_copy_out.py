@@ -1,7 +1,7 @@
 """Labels copied out to pageable memory: every word written and none beside it, at the sizes where the copy
-changes its way (one pinned copy up to 1 MB, above it transfers of up to 4 MB moved on in pieces of
-512 KB by helper threads), into buffers at odd offsets, and from several threads at once (one of
-them gets the pinned ring, the others copy the plain way)."""
+changes its way (helper threads above 256 KB, pieces of 256 KB, or 512 KB above the ring's 16 MB, which
+later transfers of 4 MB go round), into buffers at odd offsets, and from several threads at once (one
+of them gets the pinned ring, the others copy the plain way)."""
 import ctypes
 import threading
 
@@ -40,8 +40,8 @@ def copy_into(fn, n, lead):
 KB = 1 << 8  # words per KB
 
 
-@pytest.mark.parametrize("n", [2, 1000, 1024 * KB, 1024 * KB + 1, 2048 * KB - 1, 2048 * KB, 2048 * KB + 1, 9000 * KB + 3,
-                               16384 * KB - 1, 16384 * KB + 1, 50000 * KB + 7])
+@pytest.mark.parametrize("n", [2, 1000, 256 * KB - 1, 256 * KB, 256 * KB + 1, 1024 * KB, 1024 * KB + 1, 2048 * KB - 1, 2048 * KB, 2048 * KB + 1, 9000 * KB + 3,
+                               16384 * KB - 1, 16384 * KB + 1, 20480 * KB, 20480 * KB + 1, 50000 * KB + 7])
 def test_every_word_and_no_other(n):
     g = graph(n)
     L = ca.lib()
