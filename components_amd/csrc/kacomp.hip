@@ -265,10 +265,14 @@ struct kc_graph {
   uint64_t *d_huge_info = nullptr;
   uint64_t huge_info_cap = 0;
   int *flags = nullptr;
-  // [5] roots, [6] hubs found, [7] packed keys do not fit, [8] edges of
+  // [5] roots, [6] hubs found, [8] edges of
   // the tail, [9..12] its status, levels, sweeps, radius sum, [13] radius,
   // [14] medium and [15] huge buckets of a level
   uint32_t *small = nullptr;
+  // what launches count in and leave at 0: [0..4] bins, [5] volumes, [6] cluster scan; sums: [0..1] volumes, [2]
+  // cluster scan
+  uint32_t *tickets = nullptr;
+  uint64_t *sums = nullptr;
   uint64_t *sizes = nullptr;  // [0] n_next [1] P [2] m2_next [3..5] dedup counters [9] clusters
   // pinned host mirrors
   uint64_t *h_sizes = nullptr;
@@ -475,8 +479,8 @@ void enqueue_bins(kc_graph *g, uint64_t n, const uint64_t *off, const BinCfg &cf
   b.listW = lists + 2 * g->cap_n;
   b.hubs = hubs;
   TimedScope ts(g->timer, KC_K_BIN, (key ? 24 : 16) * n + 8);
-  bin_vertices(n, off, cfg, b.listT, b.listS, b.listW, b.hubs, g->h_small, key ? nullptr : g->deg_inter,
-               g->scan_scratch, g->stream, key, tmin, words);
+  bin_vertices(n, off, cfg, b.listT, b.listS, b.listW, b.hubs, g->tickets, g->h_small, key ? nullptr : g->deg_inter,
+               g->stream, key, tmin, words);
 }
 
 void read_bins(kc_graph *g, uint64_t n, Bins &b) {
@@ -530,19 +534,25 @@ uint64_t sweep_bytes(uint64_t n, uint64_t m2) {
 // Sweeps are launched in speculative batches; a sweep whose predecessor
 // changed nothing returns at once.  Returns the number of sweeps that did work
 // (the last of them found no change).
-// packed (non-null): the sweeps run over these packed keys (pack_keys)
-// instead of key.
+// packed (non-null): the keys are packed into this buffer (pack_keys) and swept
+// there; 0 sweeps are returned when they do not fit, key as before.
 uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t *off, const uint32_t *col,
                            uint64_t *key, uint64_t hop, const Bins &b, uint32_t &flag_base, bool book_bytes = true,
                            uint32_t *packed = nullptr) {
   uint64_t done = 0;
   const uint32_t batch = n < (1u << 16) ? 8u : 3u;
+  uint32_t check = 0;  // 1: the flag before the first batch's tells that packed keys do not fit
   // (packed: 4-byte keys for the neighbours and the row's own)
   const uint64_t bytes = !book_bytes ? 0 : packed ? 8 * (n + 1) + 8 * m2 + 8 * n : sweep_bytes(n, m2);
   while (true) {
     if (flag_base + batch + 2 >= kMaxFlags) {
       fill_u32(reinterpret_cast<uint32_t *>(g->flags), kMaxFlags, 0, g->stream);
       flag_base = 0;
+    }
+    if (packed && done == 0) {
+      pack_keys(n, key, packed, reinterpret_cast<uint32_t *>(&g->flags[flag_base]), g->stream);
+      ++flag_base;
+      check = 1;
     }
     int slots[8];
     for (uint32_t i = 0; i < batch; ++i) {
@@ -560,9 +570,16 @@ uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t 
               g->stream, true);
       g->timer.stop(slots[i], bytes);
     }
-    fetch32(g, g->h_flags, &g->flags[flag_base], batch, next_signal(g));
+    fetch32(g, g->h_flags, &g->flags[flag_base - check], batch + check, next_signal(g));
+    if (check && g->h_flags[0]) {
+      for (uint32_t j = 0; j < batch; ++j) g->timer.retag(slots[j], KC_K_SWEEP, 0);
+      flag_base += batch;
+      return 0;
+    }
+    const int *flags = g->h_flags + check;
+    check = 0;
     uint32_t i = 0;
-    while (i < batch && g->h_flags[i] != 0) ++i;
+    while (i < batch && flags[i] != 0) ++i;
     const uint32_t worked = i < batch ? i + 1 : batch;
     // launches after the last change returned at once: they keep their class
     // (so launch counts match a kernel trace) but carry no bytes
@@ -799,15 +816,16 @@ uint64_t rounds_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t
       g->timer.stop(slots[i], 0);
       if (first_slot < 0) first_slot = slots[i];
     }
-    HostWords w = next_signal(g);
     if (deciding) {  // edge slots at and above the next round's distance, for its direction
-      round_volumes(n, off, key, t + batch, g->sizes + 12, g->stream);
-      for (int i = 0; i < 2; ++i) {
-        w.from[i] = g->sizes + 12 + i;
-        w.to[i] = g->h_sizes + 12 + i;
-      }
+      HostWords w = next_signal(g);
+      w.from32 = reinterpret_cast<const uint32_t *>(&g->flags[flag_base]);
+      w.to32 = reinterpret_cast<uint32_t *>(g->h_flags);
+      w.count32 = batch;
+      round_volumes(n, off, key, t + batch, g->sums, g->tickets + 5, g->h_sizes + 12, w, g->stream);
+      await(g);
+    } else {
+      fetch32(g, g->h_flags, &g->flags[flag_base], batch, next_signal(g));
     }
-    fetch32(g, g->h_flags, &g->flags[flag_base], batch, w);
     uint32_t i = 0;
     while (i < batch && g->h_flags[i] != 0) ++i;
     const uint32_t worked = i < batch ? i + 1 : batch;
@@ -974,7 +992,7 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
   // degree-0 vertices are their own components and take no part in the
   // contraction (the reference sets them inactive at load, graph_io.h:380)
   identity_u32(g->n, g->labels, g->stream);
-  fill_u32(g->small + 5, 4, 0, g->stream);
+  fill_u32(g->small + 5, 11, 0, g->stream);
   uint64_t n_l = g->n0, m2_l = g->m2;
   const uint64_t *off_l = g->off0c;
   const uint32_t *col_l = g->col0c;
@@ -1163,14 +1181,13 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
         // packed 32-bit keys (pack_keys; the buffer of the cluster ranks is
         // free until they are built).  A distance only falls, so a key plus
         // one hop stays within 32 bits.
+        // (Whether they fit comes back with the first sweeps' flags.)
         uint32_t *pk = n_l >= kPackedSweepsMin && n_l <= (1ull << kPackedLabelBits) ? g->crank : nullptr;
-        if (pk) {
-          pack_keys(n_l, g->key, pk, g->small + 7, g->stream);
-          fetch32(g, g->h_small + 7, g->small + 7, 1, next_signal(g));
-          if (g->h_small[7]) pk = nullptr;
-        }
-        sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, kOneHop, b, flag_base, true, pk);
-        if (pk) unpack_keys(n_l, pk, g->key, g->stream);
+        if (pk) sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, kOneHop, b, flag_base, true, pk);
+        if (pk && sweeps)
+          unpack_keys(n_l, pk, g->key, g->stream);
+        else
+          sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, kOneHop, b, flag_base);
       }
     }
     if (!pre && !local && !o->use_bfs && sweeps == 1) {
@@ -1207,7 +1224,6 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
       rec.keys_copy = g->arena.alloc_n<uint64_t>(n_l);
       KC_HIP(hipMemcpyAsync(rec.keys_copy, g->key, n_l * 8, hipMemcpyDeviceToDevice, g->stream));
     }
-    fill_u32(g->small + 13, 3, 0, g->stream);  // radius, medium and huge buckets
     // on a degree-ordered level 0 whose first kHotClusters positions hold a
     // large share of the edge slots, the clusters of those positions take the
     // ids below 65536, so the relabel keeps those positions' ids in LDS at 16
@@ -1291,12 +1307,9 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
     }
     {
       TimedScope ts(g->timer, KC_K_SCAN, 2 * 4 * n_l + 4 * n_l);
-      HostWords w = next_signal(g);
-      w.from32 = g->small + 13;
-      w.to32 = g->h_small + 13;
-      w.count32 = 3;
       sum_segments(n_l, sum, gid_l, dense ? g->crank : nullptr, rec.newidx, g->seg_of_cid, gid_next, g->seg_off,
-                   g->dl_medium, g->dl_huge, g->small + 14, dense ? g->sizes + 9 : nullptr, g->h_sizes, w, g->scan_scratch, g->stream);
+                   g->dl_medium, g->dl_huge, g->small + 13, dense ? g->sizes + 9 : nullptr, g->sums + 2, g->tickets + 6,
+                   g->h_sizes, g->h_small + 13, next_signal(g), g->scan_scratch, g->stream);
     }
     await(g);
     const uint64_t label_space = dense ? g->h_sizes[9] : n_l;
@@ -1486,6 +1499,10 @@ std::unique_ptr<kc_graph> new_handle() {
   KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_flags), 64 * sizeof(int), hipHostMallocCoherent));
   g->small = g->dalloc<uint32_t>(16);
   g->sizes = g->dalloc<uint64_t>(16);
+  g->tickets = g->dalloc<uint32_t>(8);
+  g->sums = g->dalloc<uint64_t>(4);
+  fill_u32(g->tickets, 8, 0, g->stream);
+  fill_u64(g->sums, 4, 0, g->stream);
   return g;
 }
 
@@ -1534,7 +1551,7 @@ void alloc_work(kc_graph *g, uint64_t cap_n, uint64_t cap_m2) {
   g->sort_scratch = g->walloc<uint64_t>(radix_sort_scratch_words(n));
   g->rep_a = g->walloc<uint32_t>(n);
   g->rep_b = g->walloc<uint32_t>(n);
-  g->scan_scratch = g->walloc<uint64_t>(std::max(scan_scratch_words(n + m2) + 1024, bin_scratch_words(n)));
+  g->scan_scratch = g->walloc<uint64_t>(scan_scratch_words(n + m2) + 1024);
   for (int i = 0; i < 2; ++i) {
     g->off_pp[i] = g->walloc<uint64_t>(n + 1);
     g->col_pp[i] = g->walloc<uint32_t>(m2);

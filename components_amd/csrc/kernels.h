@@ -107,17 +107,18 @@ struct HostWords {
 };
 void publish_words(HostWords words, hipStream_t s);
 
-// Bins vertices of a CSR by degree (stable, no global atomics); counters[0..3]
-// receive nT, nS, nW, nH.  deg_inter of degree-0 vertices is cleared.
-// scratch: bin_scratch_words(n) words.
-// With key != null only vertices at key distance >= tmin are binned.
-// out[0] = edge slots of the rows at distance t, out[1] = of the rows above t.
-void round_volumes(uint64_t n, const uint64_t *off, const uint64_t *key, uint32_t t, uint64_t *out, hipStream_t s);
-void bin_vertices(uint64_t n, const uint64_t *off, BinCfg cfg, uint32_t *listT, uint32_t *listS,
-                  uint32_t *listW, HubChunk *hubs, uint32_t *counters, uint32_t *deg_inter, uint64_t *scratch,
-                  hipStream_t s, const uint64_t *key = nullptr, uint32_t tmin = 0, HostWords words = {});
+// Edge slots of the rows at distance t and of the rows above t to host_out[0]
+// and [1] (pinned), with words; out (two words) and *done are 0 before and after.
+void round_volumes(uint64_t n, const uint64_t *off, const uint64_t *key, uint32_t t, uint64_t *out, uint32_t *done,
+                   uint64_t *host_out, HostWords words, hipStream_t s);
+// Bins vertices of a CSR by degree; host_counts[0..3] (pinned or device memory)
+// receive nT, nS, nW, nH.  deg_inter of degree-0 vertices is cleared.  With key
+// != null only vertices at key distance >= tmin are binned.  counts: five words,
+// 0 before and after.
+void bin_vertices(uint64_t n, const uint64_t *off, BinCfg cfg, uint32_t *listT, uint32_t *listS, uint32_t *listW,
+                  HubChunk *hubs, uint32_t *counts, uint32_t *host_counts, uint32_t *deg_inter, hipStream_t s,
+                  const uint64_t *key = nullptr, uint32_t tmin = 0, HostWords words = {});
 void finish_bins(Bins &b);  // computes block offsets from the counts
-uint64_t bin_scratch_words(uint64_t n);
 
 // One binned sweep.  flag: set to 1 when a key decreased; prev_flag (may be
 // null): when it reads 0 the launch returns at once (converged earlier).
@@ -125,7 +126,7 @@ void sweep(int mode, bool count, const uint64_t *off, const uint32_t *col, const
            uint64_t *kout, uint64_t hop, const Bins &b, uint32_t *deg_inter, uint32_t *hub_inter,
            int *flag, const int *prev_flag, hipStream_t s, bool hubs_first = false);
 // Packed keys (distance << 24 | label) for the pull sweeps of levels below
-// 2^24 vertices: pack_keys writes them and sets *bad (zeroed first) when a
+// 2^24 vertices: pack_keys writes them and sets *bad (0 before) when a
 // distance exceeds kPackedMaxDist - 1 or a label 24 bits; sweep_packed is
 // sweep(kSweepInPlace, no counts) over them; unpack_keys restores the keys.
 constexpr uint32_t kPackedLabelBits = 24;
@@ -219,15 +220,16 @@ void cluster_ranks_hot(uint64_t n, uint64_t k, const uint32_t *lab, uint32_t *us
 // (kNone: no cluster edge), seg_of_cid[rank[a]] = the same by dense cluster id
 // (rank null: not), gid_next by next-level index, seg_off[0..n_next] bucket
 // offsets, in sum every bucket's start and the lists of medium and huge
-// buckets, in any order, their lengths added to counts[0] and [1]; and to the
-// host (pinned) host_sizes[0] = n_next, [1] = cluster edges, [9] = *ids (ids
-// null: not), and words.
+// buckets, in any order; and to the host (pinned) host_sizes[0] = n_next, [1] =
+// cluster edges, [9] = *ids (ids null: not), host_counts[0..2] = the radius that
+// counts[0] holds, medium and huge buckets, and words.  counts (three words, from
+// [1] on), *total and *done are 0 before and, with counts[0], after.
 void cluster_sums(uint64_t n, const uint32_t *lab, const uint32_t *deg_inter, uint32_t *sum, uint32_t *pos_of,
                   hipStream_t s);
 void sum_segments(uint64_t n, uint32_t *sum, const uint32_t *gid, const uint32_t *rank, uint32_t *newidx,
                   uint32_t *seg_of_cid, uint32_t *gid_next, uint64_t *seg_off, uint32_t *medium, uint32_t *huge,
-                  uint32_t *counts, const uint64_t *ids, uint64_t *host_sizes, HostWords words, uint64_t *scratch,
-                  hipStream_t s);
+                  uint32_t *counts, const uint64_t *ids, uint64_t *total, uint32_t *done, uint64_t *host_sizes,
+                  uint32_t *host_counts, HostWords words, uint64_t *scratch, hipStream_t s);
 
 // The labels lab[col[e]] of row v that differ from lab[v] (after a best-effort
 // LDS filter of repeats), packed at relab[off[v] ...] (hub chunks: at the

@@ -99,23 +99,6 @@ __device__ __forceinline__ int bin_of(uint64_t deg, const BinCfg &cfg) {
   return deg == 0 ? -1 : deg <= cfg.tmax ? 0 : deg <= cfg.smax ? 1 : deg <= cfg.wmax ? 2 : 3;
 }
 
-// Per wave: rank of each lane among the lanes of its bin, and the wave's
-// per-bin totals in LDS (bins 0..2 count vertices, bin 3 counts hub chunks).
-__device__ __forceinline__ void bin_ranks(int bin, uint32_t chunks, uint32_t *rank, uint32_t wave_tot[4]) {
-  for (int r = 0; r < 3; ++r) {
-    const uint64_t m = __ballot(bin == r);
-    if (bin == r) *rank = static_cast<uint32_t>(__popcll(m & lanes_below()));
-    wave_tot[r] = static_cast<uint32_t>(__popcll(m));
-  }
-  uint32_t x = bin == 3 ? chunks : 0u, incl = x;
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t t = __shfl_up(incl, o);
-    if (static_cast<int>(lane_id()) >= o) incl += t;
-  }
-  if (bin == 3) *rank = incl - x;
-  wave_tot[3] = __shfl(incl, 63);
-}
-
 // With key != null only vertices at key distance >= tmin are binned (the
 // unsettled ones of the time-stepped schedule).
 __device__ __forceinline__ uint64_t binned_degree(uint64_t v, uint64_t n, const uint64_t *off, const uint64_t *key,
@@ -123,63 +106,6 @@ __device__ __forceinline__ uint64_t binned_degree(uint64_t v, uint64_t n, const 
   if (v >= n) return 0;
   if (key && static_cast<uint32_t>(key[v] >> 32) < tmin) return 0;
   return off[v + 1] - off[v];
-}
-
-__global__ __launch_bounds__(kBlock) void k_bin_count(uint64_t n, const uint64_t *off, BinCfg cfg, uint32_t *counts,
-                                                     uint32_t nblocks, const uint64_t *key, uint32_t tmin) {
-  __shared__ uint32_t tot[kBlock / kWave][4];
-  const uint64_t v = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
-  const uint64_t deg = binned_degree(v, n, off, key, tmin);
-  const int bin = bin_of(deg, cfg);
-  const uint32_t chunks = bin == 3 ? static_cast<uint32_t>(ceil_div(deg, cfg.wmax)) : 0u;
-  uint32_t rank = 0, wt[4];
-  bin_ranks(bin, chunks, &rank, wt);
-  const int w = threadIdx.x / kWave;
-  if (lane_id() == 0)
-    for (int r = 0; r < 4; ++r) tot[w][r] = wt[r];
-  __syncthreads();
-  if (threadIdx.x < 4)
-    counts[static_cast<uint64_t>(threadIdx.x) * nblocks + blockIdx.x] =
-        tot[0][threadIdx.x] + tot[1][threadIdx.x] + tot[2][threadIdx.x] + tot[3][threadIdx.x];
-}
-
-__global__ __launch_bounds__(kBlock) void k_bin_write(uint64_t n, const uint64_t *off, BinCfg cfg,
-                                                     const uint64_t *prefix, uint32_t nblocks, uint32_t *listT,
-                                                     uint32_t *listS, uint32_t *listW, HubChunk *hubs,
-                                                     uint32_t *deg_inter, const uint64_t *key, uint32_t tmin) {
-  __shared__ uint32_t tot[kBlock / kWave][4];
-  const uint64_t v = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
-  const uint64_t deg = binned_degree(v, n, off, key, tmin);
-  const uint64_t e0 = deg ? off[v] : 0;
-  if (v < n && deg == 0 && deg_inter) deg_inter[v] = 0;
-  const int bin = bin_of(deg, cfg);
-  const uint32_t chunks = bin == 3 ? static_cast<uint32_t>(ceil_div(deg, cfg.wmax)) : 0u;
-  uint32_t rank = 0, wt[4];
-  bin_ranks(bin, chunks, &rank, wt);
-  const int w = threadIdx.x / kWave;
-  if (lane_id() == 0)
-    for (int r = 0; r < 4; ++r) tot[w][r] = wt[r];
-  __syncthreads();
-  if (bin < 0) return;
-  uint64_t pos = prefix[static_cast<uint64_t>(bin) * nblocks + blockIdx.x] - prefix[static_cast<uint64_t>(bin) * nblocks];
-  for (int w2 = 0; w2 < w; ++w2) pos += tot[w2][bin];
-  pos += rank;
-  if (bin == 0) {
-    listT[pos] = static_cast<uint32_t>(v);
-  } else if (bin == 1) {
-    listS[pos] = static_cast<uint32_t>(v);
-  } else if (bin == 2) {
-    listW[pos] = static_cast<uint32_t>(v);
-  } else {
-    for (uint32_t c = 0; c < chunks; ++c) {
-      HubChunk h;
-      h.v = static_cast<uint32_t>(v);
-      h.k = c;
-      h.e0 = e0 + static_cast<uint64_t>(c) * cfg.wmax;
-      h.e1 = min(e0 + deg, h.e0 + cfg.wmax);
-      hubs[pos + c] = h;
-    }
-  }
 }
 
 // words by one wave; the signal once the wave's stores to the host have arrived,
@@ -196,15 +122,114 @@ __device__ __forceinline__ void put_words(const HostWords &w) {
 
 __global__ __launch_bounds__(kWave) void k_put_words(HostWords w) { put_words(w); }
 
-// The bins' sizes (to device memory or the host's pinned memory), and words to
-// the host: one launch ahead of a wait in place of a copy for each.
-__global__ __launch_bounds__(kWave) void k_bin_totals(const uint64_t *prefix, const uint64_t *total, uint32_t nblocks,
-                                                     uint32_t *counters, HostWords words) {
-  const int r = threadIdx.x;
-  if (r < 4) {
-    const uint64_t hi = r < 3 ? prefix[static_cast<uint64_t>(r + 1) * nblocks] : *total;
-    host_store(counters + r, static_cast<uint32_t>(hi - prefix[static_cast<uint64_t>(r) * nblocks]));
+// Whether the calling thread's block is the launch's last to come here (one
+// thread a block; its earlier atomics are done when their results are, so no
+// fence, which would write back the L2).  *done is 0 before and after a launch.
+__device__ __forceinline__ bool last_block(uint32_t *done) {
+  host_stores_done();
+  if (atomicAdd(done, 1u) != gridDim.x * gridDim.y - 1) return false;
+  atomicExch(done, 0u);
+  return true;
+}
+// The value of a word that other blocks of the launch add to, left at 0.
+template <class T>
+__device__ __forceinline__ T take(T *p) {
+  return atomicExch(p, T{0});
+}
+
+// Bins in one pass: a block of 4096 vertices counts and ranks them, takes its
+// places in the four lists by an atomic each and writes them; the last block
+// leaves the lists' sizes, and words, for the host.  The order inside a block's
+// share is the vertices' own, the blocks' shares come as they arrive; nothing
+// depends on it.  Bound by the offsets' read on large levels and by latency on
+// small ones, where counts, scan (two launches), lists and sizes as launches of
+// their own took 23 us on 2^20 vertices and 17 on 20 000; so 14 and 8.
+constexpr int kBinBlock = 1024, kBinPer = 4;
+__global__ __launch_bounds__(kBinBlock) void k_bins(uint64_t n, const uint64_t *off, BinCfg cfg, uint32_t *listT,
+                                                   uint32_t *listS, uint32_t *listW, HubChunk *hubs,
+                                                   uint32_t *deg_inter, const uint64_t *key, uint32_t tmin,
+                                                   uint32_t *counts, uint32_t *host_counts, HostWords words) {
+  constexpr int kWaves = kBinBlock / kWave, kRuns = kBinPer * kWaves;  // a run: one wave's 64 vertices
+  static_assert(kRuns == kWave, "a wave scans a list's runs");
+  __shared__ uint32_t start[4][kRuns];  // per list and run: its count, then its place
+  __shared__ bool last;
+  const uint32_t ln = lane_id(), wave = threadIdx.x / kWave;
+  const uint64_t v0 = blockIdx.x * static_cast<uint64_t>(kBinBlock * kBinPer) + threadIdx.x;
+  uint64_t e0[kBinPer], deg[kBinPer];
+#pragma unroll
+  for (int u = 0; u < kBinPer; ++u) {
+    const uint64_t v = v0 + u * kBinBlock;
+    e0[u] = v < n ? off[v] : 0;
+    deg[u] = binned_degree(v, n, off, key, tmin);
   }
+  int bin[kBinPer];
+  uint32_t rank[kBinPer], chunks[kBinPer];
+#pragma unroll
+  for (int u = 0; u < kBinPer; ++u) {
+    const uint64_t v = v0 + u * kBinBlock;
+    if (v < n && deg[u] == 0 && deg_inter) deg_inter[v] = 0;
+    bin[u] = bin_of(deg[u], cfg);
+    chunks[u] = bin[u] == 3 ? static_cast<uint32_t>(ceil_div(deg[u], cfg.wmax)) : 0u;
+    rank[u] = 0;
+    uint32_t total[4];
+    for (int r = 0; r < 3; ++r) {
+      const uint64_t m = __ballot(bin[u] == r);
+      if (bin[u] == r) rank[u] = static_cast<uint32_t>(__popcll(m & lanes_below()));
+      total[r] = static_cast<uint32_t>(__popcll(m));
+    }
+    total[3] = 0;
+    if (__ballot(bin[u] == 3)) {
+      uint32_t incl = chunks[u];
+      for (int o = 1; o < kWave; o <<= 1) {
+        const uint32_t t = __shfl_up(incl, o);
+        if (static_cast<int>(ln) >= o) incl += t;
+      }
+      if (bin[u] == 3) rank[u] = incl - chunks[u];
+      total[3] = __shfl(incl, kWave - 1);
+    }
+    if (ln == 0)
+      for (int r = 0; r < 4; ++r) start[r][u * kWaves + wave] = total[r];
+  }
+  __syncthreads();
+  if (wave < 4) {  // list `wave`: its runs' places
+    const uint32_t x = start[wave][ln];
+    uint32_t incl = x;
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t t = __shfl_up(incl, o);
+      if (static_cast<int>(ln) >= o) incl += t;
+    }
+    uint32_t base = 0;
+    if (ln == kWave - 1 && incl) base = atomicAdd(counts + wave, incl);
+    start[wave][ln] = __shfl(base, kWave - 1) + incl - x;
+  }
+  __syncthreads();
+  // (the places have returned, so the sizes are in)
+  if (threadIdx.x == 0) last = last_block(counts + 4);
+#pragma unroll
+  for (int u = 0; u < kBinPer; ++u) {
+    if (bin[u] < 0) continue;
+    const uint32_t v = static_cast<uint32_t>(v0 + u * kBinBlock);
+    const uint32_t pos = start[bin[u]][u * kWaves + wave] + rank[u];
+    if (bin[u] == 0) {
+      listT[pos] = v;
+    } else if (bin[u] == 1) {
+      listS[pos] = v;
+    } else if (bin[u] == 2) {
+      listW[pos] = v;
+    } else {
+      for (uint32_t c = 0; c < chunks[u]; ++c) {
+        HubChunk h;
+        h.v = v;
+        h.k = c;
+        h.e0 = e0[u] + static_cast<uint64_t>(c) * cfg.wmax;
+        h.e1 = min(e0[u] + deg[u], h.e0 + cfg.wmax);
+        hubs[pos + c] = h;
+      }
+    }
+  }
+  __syncthreads();
+  if (!last || wave != 0) return;
+  if (ln < 4) host_store(host_counts + ln, take(counts + ln));
   put_words(words);
 }
 
@@ -1209,15 +1234,18 @@ struct SumLoad {
   }
 };
 struct SumOut {
-  uint32_t *sum, *newidx, *seg_of_cid, *gid_next, *medium, *huge, *counts;  // counts: medium, huge
+  uint32_t *sum, *newidx, *seg_of_cid, *gid_next, *medium, *huge, *counts;  // counts: radius, medium, huge
   const uint32_t *gid, *rank;  // rank null: the buckets hold labels
   uint64_t *seg_off;
 };
 // k_scan_down over the sums, everything read of a label loaded ahead of the
 // stores and the lists appended with one atomic each per wave.
 __global__ __launch_bounds__(kBlock) void k_sum_down(uint64_t n, SumOut o, const uint64_t *block_prefix,
-                                                    uint64_t *total_out, const uint64_t *block_sums) {
+                                                    const uint64_t *block_sums, const uint64_t *ids,
+                                                    unsigned long long *total, uint32_t *done, uint64_t *host_sizes,
+                                                    uint32_t *host_counts, HostWords words) {
   __shared__ uint64_t wsum[kBlock / kWave];
+  __shared__ bool last;
   const uint64_t base = scan_base();
   const SumLoad load{o.sum};
   uint64_t v[kScanPerThread], before[kScanPerThread], all;
@@ -1248,8 +1276,8 @@ __global__ __launch_bounds__(kBlock) void k_sum_down(uint64_t n, SumOut o, const
   if (n_medium | n_huge) {
     uint32_t at_medium = 0, at_huge = 0;
     if (lane_id() == 0) {
-      if (n_medium) at_medium = atomicAdd(o.counts, n_medium);
-      if (n_huge) at_huge = atomicAdd(o.counts + 1, n_huge);
+      if (n_medium) at_medium = atomicAdd(o.counts + 1, n_medium);
+      if (n_huge) at_huge = atomicAdd(o.counts + 2, n_huge);
     }
     at_medium = __shfl(at_medium, 0);
     at_huge = __shfl(at_huge, 0);
@@ -1264,18 +1292,22 @@ __global__ __launch_bounds__(kBlock) void k_sum_down(uint64_t n, SumOut o, const
       at_huge += static_cast<uint32_t>(__popcll(h));
     }
   }
-  if (total_out && blockIdx.x == gridDim.x - 1 && threadIdx.x == kBlock - 1) *total_out = all;
-}
-
-__global__ __launch_bounds__(kWave) void k_sum_finish(const uint64_t *total, uint64_t *seg_off, const uint64_t *ids,
-                                                     uint64_t *host_sizes, HostWords words) {
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == kBlock - 1) {
+    atomicExch(total, static_cast<unsigned long long>(all));
+    host_stores_done();
+  }
+  __syncthreads();  // (the waves' appends have returned)
+  if (threadIdx.x == 0) last = last_block(done);
+  __syncthreads();
+  if (!last || threadIdx.x >= kWave) return;
   if (threadIdx.x == 0) {
-    const uint64_t clusters = *total >> 32, edges = static_cast<uint32_t>(*total);
+    const uint64_t t = take(total), clusters = t >> 32, edges = static_cast<uint32_t>(t);
     if (ids) host_store(host_sizes + 9, *ids);
-    seg_off[clusters] = edges;
+    o.seg_off[clusters] = edges;
     host_store(host_sizes, clusters);
     host_store(host_sizes + 1, edges);
   }
+  if (threadIdx.x < 3) host_store(host_counts + threadIdx.x, take(o.counts + threadIdx.x));
   put_words(words);
 }
 
@@ -2362,8 +2394,10 @@ void deviates_only(uint32_t gid0, uint32_t count, DeviateArgs d, uint32_t *out, 
 // rows above it: out[0] and out[1] (zeroed by the caller); one atomic pair
 // per block.
 __global__ __launch_bounds__(kBlock) void k_round_volumes(uint64_t n, const uint64_t *off, const uint64_t *key,
-                                                         uint32_t t, unsigned long long *out) {
+                                                         uint32_t t, unsigned long long *out, uint32_t *done,
+                                                         uint64_t *host_out, HostWords words) {
   __shared__ unsigned long long part[2][kBlock / kWave];
+  __shared__ bool last;
   uint64_t at = 0, above = 0;
   constexpr int kU = 4;  // vertices whose loads a lane keeps in flight
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
@@ -2396,39 +2430,30 @@ __global__ __launch_bounds__(kBlock) void k_round_volumes(uint64_t n, const uint
     for (int w = 0; w < kBlock / kWave; ++w) s += part[threadIdx.x][w];
     if (s) atomicAdd(&out[threadIdx.x], s);
   }
+  if (threadIdx.x == 0) last = last_block(done);  // (this wave's additions are in)
+  __syncthreads();
+  if (!last || threadIdx.x >= kWave) return;
+  if (threadIdx.x < 2) host_store(host_out + threadIdx.x, static_cast<uint64_t>(take(out + threadIdx.x)));
+  put_words(words);
 }
 
-void round_volumes(uint64_t n, const uint64_t *off, const uint64_t *key, uint32_t t, uint64_t *out, hipStream_t s) {
-  fill_u64(out, 2, 0, s);
-  if (!n) return;
+void round_volumes(uint64_t n, const uint64_t *off, const uint64_t *key, uint32_t t, uint64_t *out, uint32_t *done,
+                   uint64_t *host_out, HostWords words, hipStream_t s) {
   // (a block's two atomics queue behind the others': 2048 blocks 28 us on 2^20
   // vertices, 512 blocks 10)
-  const unsigned g = static_cast<unsigned>(std::min<uint64_t>(ceil_div(n, 4 * kBlock), 512));
+  const unsigned g = static_cast<unsigned>(std::max<uint64_t>(1, std::min<uint64_t>(ceil_div(n, 4 * kBlock), 512)));
   hipLaunchKernelGGL(k_round_volumes, dim3(g), dim3(kBlock), 0, s, n, off, key, t,
-                     reinterpret_cast<unsigned long long *>(out));
+                     reinterpret_cast<unsigned long long *>(out), done, host_out, words);
   KC_LAUNCH_CHECK();
 }
 
 void bin_vertices(uint64_t n, const uint64_t *off, BinCfg cfg, uint32_t *listT, uint32_t *listS, uint32_t *listW,
-                  HubChunk *hubs, uint32_t *counters, uint32_t *deg_inter, uint64_t *scratch, hipStream_t s,
+                  HubChunk *hubs, uint32_t *counts, uint32_t *host_counts, uint32_t *deg_inter, hipStream_t s,
                   const uint64_t *key, uint32_t tmin, HostWords words) {
-  if (!n) {
-    fill_u32(counters, 4, 0, s);
-    publish_words(words, s);
-    return;
-  }
-  const uint32_t nb = static_cast<uint32_t>(ceil_div(n, kBlock));
-  uint32_t *counts = reinterpret_cast<uint32_t *>(scratch);
-  uint64_t *prefix = scratch + ceil_div(4ull * nb, 2) + 8;
-  uint64_t *total = prefix + 4ull * nb + 8;
-  uint64_t *rest = total + 8;
-  hipLaunchKernelGGL(k_bin_count, dim3(nb), dim3(kBlock), 0, s, n, off, cfg, counts, nb, key, tmin);
-  KC_LAUNCH_CHECK();
-  scan_exclusive<uint64_t>(4ull * nb, ArrLoadU32{counts}, ArrayStore<uint64_t>{prefix}, total, rest, s);
-  hipLaunchKernelGGL(k_bin_write, dim3(nb), dim3(kBlock), 0, s, n, off, cfg, prefix, nb, listT, listS, listW, hubs,
-                     deg_inter, key, tmin);
-  KC_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_bin_totals, dim3(1), dim3(64), 0, s, prefix, total, nb, counters, words);
+  // (a block even for n = 0: it leaves the words)
+  const unsigned g = static_cast<unsigned>(std::max<uint64_t>(1, ceil_div(n, kBinBlock * kBinPer)));
+  hipLaunchKernelGGL(k_bins, dim3(g), dim3(kBinBlock), 0, s, n, off, cfg, listT, listS, listW, hubs, deg_inter, key, tmin,
+                     counts, host_counts, words);
   KC_LAUNCH_CHECK();
 }
 
@@ -2466,7 +2491,6 @@ void sweep(int mode, bool count, const uint64_t *off, const uint32_t *col, const
 }
 
 void pack_keys(uint64_t n, const uint64_t *key, uint32_t *pk, uint32_t *bad, hipStream_t s) {
-  fill_u32(bad, 1, 0u, s);
   if (!n) return;
   const unsigned g = static_cast<unsigned>(std::min<uint64_t>(ceil_div(n, kBlock), 4096));
   hipLaunchKernelGGL(k_pack_keys, dim3(g), dim3(kBlock), 0, s, n, key, pk, bad);
@@ -2517,11 +2541,6 @@ void block_interface(const uint64_t *off, const uint32_t *col, uint64_t n, uint6
   if (n == 0) return;
   hipLaunchKernelGGL(k_block_interface, dim3(row_wave_grid(n)), dim3(kBlock), 0, s, off, col, n, bsize, key);
   KC_LAUNCH_CHECK();
-}
-
-uint64_t bin_scratch_words(uint64_t n) {
-  const uint64_t nb = ceil_div(n, kBlock) + 1;
-  return 6 * nb + 64 + scan_words_for(4 * nb, 1) + 64;
 }
 
 void huge_sizes(uint32_t n_huge, const uint32_t *huge, const uint64_t *seg_off, uint64_t *out, hipStream_t s) {
@@ -2633,22 +2652,21 @@ void cluster_sums(uint64_t n, const uint32_t *lab, const uint32_t *deg_inter, ui
 
 void sum_segments(uint64_t n, uint32_t *sum, const uint32_t *gid, const uint32_t *rank, uint32_t *newidx,
                   uint32_t *seg_of_cid, uint32_t *gid_next, uint64_t *seg_off, uint32_t *medium, uint32_t *huge,
-                  uint32_t *counts, const uint64_t *ids, uint64_t *host_sizes, HostWords words, uint64_t *scratch,
-                  hipStream_t s) {
+                  uint32_t *counts, const uint64_t *ids, uint64_t *total, uint32_t *done, uint64_t *host_sizes,
+                  uint32_t *host_counts, HostWords words, uint64_t *scratch, hipStream_t s) {
   const SumOut out{sum, newidx, seg_of_cid, gid_next, medium, huge, counts, gid, rank, seg_off};
   const uint64_t blocks = ceil_div(n, kScanTile);
-  uint64_t *total = scratch, *sums = scratch + 4, *prefix = sums + blocks;
+  uint64_t *sums = scratch + 4, *prefix = sums + blocks;
   hipLaunchKernelGGL((k_scan_reduce<uint64_t, SumLoad>), dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, s, n,
                      SumLoad{sum}, sums);
   KC_LAUNCH_CHECK();
   const bool fused = blocks <= kScanFusedBlocks;
   if (!fused)
-    scan_exclusive<uint64_t>(blocks, ArrayLoad<uint64_t>{sums}, ArrayStore<uint64_t>{prefix}, total, prefix + blocks + 4,
-                             s);
+    scan_exclusive<uint64_t>(blocks, ArrayLoad<uint64_t>{sums}, ArrayStore<uint64_t>{prefix}, scratch,
+                             prefix + blocks + 4, s);
   hipLaunchKernelGGL(k_sum_down, dim3(static_cast<unsigned>(blocks)), dim3(kBlock), 0, s, n, out,
-                     fused ? static_cast<const uint64_t *>(nullptr) : prefix, fused ? total : nullptr, sums);
-  KC_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_sum_finish, dim3(1), dim3(kWave), 0, s, total, seg_off, ids, host_sizes, words);
+                     fused ? static_cast<const uint64_t *>(nullptr) : prefix, sums, ids,
+                     reinterpret_cast<unsigned long long *>(total), done, host_sizes, host_counts, words);
   KC_LAUNCH_CHECK();
 }
 

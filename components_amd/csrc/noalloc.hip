@@ -36,7 +36,6 @@ namespace {
 constexpr uint64_t kMaxVertices = KC_NOALLOC_MAX_VERTICES;
 constexpr uint64_t kMaxSlots = KC_NOALLOC_MAX_EDGE_SLOTS;
 constexpr uint32_t kFlagSlots = 1024;  // sweep flags, reused round-robin
-constexpr uint64_t kBinScratchBytes = 1ull << 20;
 
 constexpr uint64_t align256(uint64_t x) { return (x + 255) & ~uint64_t(255); }
 constexpr uint64_t kHubCap = kMaxSlots / (kMinWaveBin / 2) + 2;  // hub_chunk_cap(kMaxSlots)
@@ -48,10 +47,9 @@ constexpr uint64_t kDegAt = align256(kListsAt + 12 * kMaxVertices);             
 constexpr uint64_t kHubsAt = align256(kDegAt + 4 * kMaxVertices);               // HubChunk[kHubCap]
 constexpr uint64_t kHubInterAt = align256(kHubsAt + sizeof(HubChunk) * kHubCap);  // u32[kHubCap]
 constexpr uint64_t kFlagsAt = align256(kHubInterAt + 4 * kHubCap);              // int[kFlagSlots]
-constexpr uint64_t kSmallAt = align256(kFlagsAt + 4 * kFlagSlots);              // u32[16]: bin counts, roots
+constexpr uint64_t kSmallAt = align256(kFlagsAt + 4 * kFlagSlots);              // u32[16]: [0..3] bin counts, roots, [8..12] binning's counters
 constexpr uint64_t kPartialAt = align256(kSmallAt + 64);                        // u32[n/256 + 64]
-constexpr uint64_t kBinScratchAt = align256(kPartialAt + 4 * (kMaxVertices / kBlock + 64));
-constexpr uint64_t kScratchBytes = align256(kBinScratchAt + kBinScratchBytes);
+constexpr uint64_t kScratchBytes = align256(kPartialAt + 4 * (kMaxVertices / kBlock + 64));
 
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
@@ -99,8 +97,8 @@ uint64_t propagate(uint64_t n, const uint64_t *offsets, const uint32_t *targets,
   b.listS = lists + n;
   b.listW = lists + 2 * n;
   b.hubs = hubs;
-  bin_vertices(n, offsets, cfg, b.listT, b.listS, b.listW, b.hubs, small, deg_inter,
-               region<uint64_t>(base, kBinScratchAt), s);
+  fill_u32(small, 16, 0, s);
+  bin_vertices(n, offsets, cfg, b.listT, b.listS, b.listW, b.hubs, small + 8, small, deg_inter, s);
   uint32_t counts[4];
   KC_HIP(hipMemcpyAsync(counts, small, sizeof(counts), hipMemcpyDeviceToHost, s));
   KC_HIP(hipStreamSynchronize(s));
@@ -174,7 +172,6 @@ extern "C" int kc_find_components_noalloc(uint64_t n, const uint64_t *offsets, c
       fail(KC_ERR_INVALID, "kc_find_components_noalloc: 2m=%llu exceeds the scratch limit of %llu edge slots",
            static_cast<unsigned long long>(m2), static_cast<unsigned long long>(kMaxSlots));
     if (m2 && !targets) fail(KC_ERR_INVALID, "null device pointer");
-    if (bin_scratch_words(n) * 8 > kBinScratchBytes) fail(KC_ERR_INVALID, "internal: binning scratch too small");
     uint64_t sweeps = 0;
     uint32_t components = 0;
     if (n) {
