@@ -382,7 +382,7 @@ typedef struct kc_batch_gen_params {
 } kc_batch_gen_params;
 
 /* Launch shape of the persistent kernel: threads per workgroup (256, 512 or
- * 1024), workgroups per compute unit, and whether the launch sequence replays
+ * 1024), workgroups per compute unit, and whether its launch replays
  * a captured HIP graph.  Graphs of up to 8192 vertices run in workgroups of
  * their own size class instead, with their keys in LDS, whatever the shape.
  * In the persistent kernel every row of a graph is processed by one lane, so it
