@@ -855,6 +855,7 @@ struct kc_batch {
   uint64_t n = 0, m2 = 0;
   int cus = 0;
   std::vector<uint64_t> h_vtx_off, h_edge_off;
+  uint64_t largest = 0;  // vertices of the largest graph: the bound of the local labels
   std::vector<uint64_t> h_up;  // per graph: slots whose target is above their row (its edges, once each)
   std::vector<void *> owned;
   uint32_t *order_d = nullptr;
@@ -1206,6 +1207,7 @@ int kc_batch_create(const kc_batch_host *h, kc_batch **out) {
     b->n = n;
     b->m2 = m2;
     b->h_vtx_off.assign(h->vtx_off, h->vtx_off + G + 1);
+    for (uint32_t g = 0; g < G; ++g) b->largest = std::max(b->largest, h->vtx_off[g + 1] - h->vtx_off[g]);
     b->h_edge_off.assign(h->edge_off, h->edge_off + G + 1);
     b->h_up = std::move(up);
     BatchDev &d = b->dev;
@@ -1284,7 +1286,7 @@ int kc_batch_run(kc_batch *b, const kc_options *opt, uint32_t *labels_out, kc_ba
     else
       kc_options_init(&o);
     const auto t0 = std::chrono::steady_clock::now();
-    CopyOut labels(labels_out, 4ull * b->n);
+    CopyOut labels(labels_out, b->n, b->largest);
     batch_params(b, o);
     const float ms = run_once(b, o);
     labels.finish(b->dev.labels, b->stream);

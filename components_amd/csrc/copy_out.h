@@ -4,11 +4,12 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <cstdint>
 
 namespace kc {
 
-// One copy of `bytes` from device memory to the caller's `dst` at the end of a
-// call; bytes are whole words and src is aligned to 16 bytes.  The constructor
+// One copy of `count` 32-bit numbers below `bound` from device memory to the
+// caller's `dst` at the end of a call; src is aligned to 16 bytes.  The constructor
 // (at the call's start; dst may be null: nothing to do) lets helper threads
 // fault in dst's pages while the GPU works, without changing what they hold.
 // enqueue() puts the first transfers into the stream, ahead of a wait the
@@ -17,19 +18,19 @@ namespace kc {
 // Throws Failure.
 class CopyOut {
  public:
-  CopyOut(void *dst, size_t bytes);
+  CopyOut(uint32_t *dst, size_t count, uint64_t bound);
   ~CopyOut();
   CopyOut(const CopyOut &) = delete;
   CopyOut &operator=(const CopyOut &) = delete;
-  void enqueue(const void *src, hipStream_t stream);
-  void finish(const void *src, hipStream_t stream);
+  void enqueue(const uint32_t *src, hipStream_t stream);
+  void finish(const uint32_t *src, hipStream_t stream);
 
  private:
   struct Job;
   friend struct Helpers;
   void issue();
   Job *job_ = nullptr;
-  const char *src_ = nullptr;
+  const uint32_t *src_ = nullptr;
   hipStream_t stream_ = nullptr;
   bool queued_ = false;  // transfers into the ring are in the stream
 };

@@ -32,41 +32,76 @@ namespace kc {
 
 namespace {
 
-constexpr size_t kSlotBytes = 4 << 20;  // of the ring: what one transfer fills once the ring has been round
+// The ring takes 4 M numbers: four slots, each what one transfer fills once the
+// ring has been round.
+constexpr size_t kSlotCount = 1 << 20;
 constexpr int kSlots = 4;
-constexpr size_t kRingBytes = kSlots * kSlotBytes;
-// what one thread moves on at once (a quarter of a megabyte takes it about 28 us)
-constexpr size_t kPiece = 256 << 10, kLargePiece = 512 << 10;
+constexpr size_t kRingCount = kSlots * kSlotCount, kRingBytes = 4 * kRingCount;
+// what one thread moves on at once (64 k numbers take it about 28 us)
+constexpr size_t kPiece = 64 << 10, kLargePiece = 128 << 10;
 // from here on with helper threads (below, waking them takes longer)
-constexpr size_t kHelpersMin = 256 << 10;
+constexpr size_t kHelpersMin = 64 << 10;
 constexpr int kMaxHelpers = 8;
 constexpr size_t kFaultBytes = 512 << 10;
 
+// Numbers cross the link in as few bytes as the largest needs, two, three or
+// four: output word i (8 bytes) of n packed numbers.
+__device__ __forceinline__ uint64_t packed_word(int width, const uint32_t *src, uint64_t n, uint64_t i) {
+  const auto at = [&](uint64_t k) -> uint64_t { return k < n ? src[k] : 0u; };
+  if (width == 4) return at(2 * i) | at(2 * i + 1) << 32;
+  if (width == 2) return at(4 * i) | at(4 * i + 1) << 16 | at(4 * i + 2) << 32 | at(4 * i + 3) << 48;
+  const uint64_t k = 8 * i / 3;  // the number that byte 8 i belongs to, and its bytes before that one
+  const int s = static_cast<int>(8 * i - 3 * k);
+  uint64_t v = at(k) >> 8 * s | at(k + 1) << (24 - 8 * s) | at(k + 2) << (48 - 8 * s);
+  if (s == 2) v |= at(k + 3) << 56;
+  return v;
+}
+
 // A transfer by stores from the CUs: 50 GB/s always, where the copy engine that
 // hipMemcpyAsync picks runs at 57 or, for long stretches on some streams, at
-// 20 (67 MB: 3.6 instead of 1.6 ms).  What bounds it is the host link; 64
-// workgroups fill it (16: 5% slower).  Every workgroup tells of its share of
-// every piece by a word of its own in pinned memory, so that the host needs
-// neither an event nor a launch per piece.
+// 20 (67 MB: 3.6 instead of 1.6 ms).  What bounds it is the host link, so the
+// numbers are packed (16.8 M at three bytes 1.29 -> 1.06 ms, 5.9 M at two 0.42
+// -> 0.21); 64 workgroups fill it (16: 5% slower).
+// Every workgroup tells of its share of every piece by a word of its own in
+// pinned memory, so that the host needs neither an event nor a launch per piece.
 constexpr unsigned kTransferBlocks = 64;
 
-__global__ __launch_bounds__(kBlock) void k_transfer(uint32_t *dst, const uint32_t *src, uint64_t words,
-                                                     uint64_t piece_words, uint32_t *arrived, uint32_t value) {
+template <int kWidth>
+__global__ __launch_bounds__(kBlock) void k_transfer(char *dst, const uint32_t *src, uint64_t count, uint64_t piece,
+                                                     uint32_t *arrived, uint32_t value) {
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
   const uint64_t first = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
-  for (uint64_t at = 0, p = 0; at < words; at += piece_words, ++p) {
-    const uint64_t n = min(piece_words, words - at);
-    uint64_t *to = reinterpret_cast<uint64_t *>(dst + at);
-    const uint64_t *from = reinterpret_cast<const uint64_t *>(src + at);
-    for (uint64_t i = first; i < n / 2; i += stride) host_store(to + i, from[i]);
-    if (first == 0 && n % 2) host_store(dst + at + n - 1, src[at + n - 1]);
+  for (uint64_t at = 0, p = 0; at < count; at += piece, ++p) {
+    const uint64_t n = min(piece, count - at), words = (n * kWidth + 7) / 8;
+    uint64_t *to = reinterpret_cast<uint64_t *>(dst + at * kWidth);  // (a piece is a multiple of 8 numbers)
+    for (uint64_t i = first; i < words; i += stride) host_store(to + i, packed_word(kWidth, src + at, n, i));
     host_stores_done();
     __syncthreads();
     if (threadIdx.x == 0) host_store(arrived + p * kTransferBlocks + blockIdx.x, value);
   }
 }
 
-constexpr size_t kArrivedBytes = kRingBytes / kPiece * kTransferBlocks * sizeof(uint32_t);
+// The host's side: n numbers of `width` bytes each to dst (which need not be
+// aligned).
+void unpack(char *dst, const char *src, size_t n, int width) {
+  if (width == 4) {
+    std::memcpy(dst, src, 4 * n);
+    return;
+  }
+  uint32_t *to = reinterpret_cast<uint32_t *>(dst);
+  if (width == 2) {
+    const uint16_t *from = reinterpret_cast<const uint16_t *>(src);
+    for (size_t i = 0; i < n; ++i) to[i] = from[i];
+    return;
+  }
+  for (size_t i = 0; i < n; ++i) {  // (the last reads a byte past them, inside the ring's memory)
+    uint32_t x;
+    std::memcpy(&x, src + 3 * i, 4);
+    to[i] = x & 0xFFFFFFu;
+  }
+}
+
+constexpr size_t kArrivedBytes = kRingCount / kPiece * kTransferBlocks * sizeof(uint32_t);
 
 // The pinned ring: one for the process (16 MB and the arrival words), lent to
 // one copy at a time and given back with the last handle.
@@ -133,7 +168,8 @@ struct Spin {
 // so a copy does not depend on how many helpers there are, or whether any.
 struct CopyOut::Job {
   char *dst = nullptr;
-  size_t bytes = 0, piece = 0, pieces = 0;
+  size_t count = 0, bytes = 0, piece = 0, pieces = 0;  // numbers, their bytes at dst, numbers a piece, pieces
+  int width = 4;                                       // bytes of a number in the ring
   unsigned blocks = 0;
   // under the helpers' mutex
   bool listed = false, hot = false;  // hot: the transfers are in the stream
@@ -142,29 +178,31 @@ struct CopyOut::Job {
   // the copy itself
   char *ring = nullptr;
   uint32_t first_value = 0;              // of the first transfer; the later ones count on
-  size_t issued = 0;                     // bytes with a transfer in the stream (the calling thread's)
+  size_t issued = 0;                     // numbers with a transfer in the stream (the calling thread's)
   std::atomic<size_t> next_piece{0};     // claimed
-  std::atomic<size_t> done{0};           // bytes moved
-  std::unique_ptr<std::atomic<size_t>[]> left;  // per slot's turn: bytes still in it
+  std::atomic<size_t> done{0};           // numbers moved
+  std::unique_ptr<std::atomic<size_t>[]> left;  // per slot's turn: numbers still in it
   std::atomic<bool> commit{false}, stop{false};
 
-  size_t slot_turns() const { return (bytes + kSlotBytes - 1) / kSlotBytes; }
+  size_t slot_turns() const { return (count + kSlotCount - 1) / kSlotCount; }
   // the transfer that a slot's turn belongs to: the first fills the whole ring
   uint32_t value_of(size_t turn) const { return first_value + static_cast<uint32_t>(turn < kSlots ? 0 : turn - kSlots + 1); }
 
+  uint32_t *arrived_words(size_t at) const {
+    return reinterpret_cast<uint32_t *>(ring + kRingBytes) + at % kRingCount / piece * kTransferBlocks;
+  }
   bool has_arrived(size_t p) const {
     const size_t at = p * piece;
-    const uint32_t want = value_of(at / kSlotBytes);
-    const uint32_t *words =
-        reinterpret_cast<const uint32_t *>(ring + kRingBytes) + at % kRingBytes / piece * kTransferBlocks;
+    const uint32_t want = value_of(at / kSlotCount);
+    const uint32_t *words = arrived_words(at);
     for (unsigned b = 0; b < blocks; ++b)
       if (__atomic_load_n(words + b, __ATOMIC_ACQUIRE) != want) return false;
     return true;
   }
   void move(size_t p) {
-    const size_t at = p * piece, n = std::min(piece, bytes - at);
-    std::memcpy(dst + at, ring + at % kRingBytes, n);
-    left[at / kSlotBytes].fetch_sub(n, std::memory_order_release);
+    const size_t at = p * piece, n = std::min(piece, count - at);
+    unpack(dst + 4 * at, ring + at % kRingCount * width, n, width);
+    left[at / kSlotCount].fetch_sub(n, std::memory_order_release);
     done.fetch_add(n, std::memory_order_release);
   }
   // a helper's share: pieces until none is left
@@ -270,17 +308,19 @@ Helpers &helpers() {
 std::mutex g_handles;  // retain, release and the helpers' end
 }  // namespace
 
-CopyOut::CopyOut(void *dst, size_t bytes) {
-  if (!dst || !bytes) return;
+CopyOut::CopyOut(uint32_t *dst, size_t count, uint64_t bound) {
+  if (!dst || !count) return;
   std::unique_ptr<Job> j(new Job);
-  j->dst = static_cast<char *>(dst);
-  j->bytes = bytes;
-  j->piece = bytes > kRingBytes ? kLargePiece : kPiece;
-  j->pieces = (bytes + j->piece - 1) / j->piece;
-  j->blocks = static_cast<unsigned>(std::min<size_t>(kTransferBlocks, (bytes + 4095) / 4096));
+  j->dst = reinterpret_cast<char *>(dst);
+  j->count = count;
+  j->bytes = 4 * count;
+  j->width = bound <= 1ull << 16 ? 2 : bound <= 1ull << 24 ? 3 : 4;
+  j->piece = count > kRingCount ? kLargePiece : kPiece;
+  j->pieces = (count + j->piece - 1) / j->piece;
+  j->blocks = static_cast<unsigned>(std::min<size_t>(kTransferBlocks, (count + 1023) / 1024));
   j->left.reset(new std::atomic<size_t>[j->slot_turns()]);
-  for (size_t t = 0; t < j->slot_turns(); ++t) j->left[t] = std::min(kSlotBytes, bytes - t * kSlotBytes);
-  if (bytes > kHelpersMin) helpers().add(j.get());
+  for (size_t t = 0; t < j->slot_turns(); ++t) j->left[t] = std::min(kSlotCount, count - t * kSlotCount);
+  if (count > kHelpersMin) helpers().add(j.get());
   job_ = j.release();
 }
 
@@ -296,35 +336,31 @@ CopyOut::~CopyOut() {
 // The next transfer: the whole ring at first, then a slot at a time.
 void CopyOut::issue() {
   Job &j = *job_;
-  const size_t n = std::min(j.issued ? kSlotBytes : kRingBytes, j.bytes - j.issued), at = j.issued % kRingBytes;
-  uint32_t *arrived = reinterpret_cast<uint32_t *>(j.ring + kRingBytes) + at / j.piece * kTransferBlocks;
+  const size_t n = std::min(j.issued ? kSlotCount : kRingCount, j.count - j.issued);
+  const uint32_t value = j.value_of(j.issued / kSlotCount);
+  auto kernel = j.width == 2 ? k_transfer<2> : j.width == 3 ? k_transfer<3> : k_transfer<4>;
   queued_ = true;
-  hipLaunchKernelGGL(k_transfer, dim3(j.blocks), dim3(kBlock), 0, stream_, reinterpret_cast<uint32_t *>(j.ring + at),
-                     reinterpret_cast<const uint32_t *>(src_ + j.issued), n / 4, j.piece / 4, arrived,
-                     j.value_of(j.issued / kSlotBytes));
+  hipLaunchKernelGGL(kernel, dim3(j.blocks), dim3(kBlock), 0, stream_, j.ring + j.issued % kRingCount * j.width,
+                     src_ + j.issued, n, j.piece, j.arrived_words(j.issued), value);
   KC_LAUNCH_CHECK();
-  g_ring.value = j.value_of(j.issued / kSlotBytes);
+  g_ring.value = value;
   j.issued += n;
 }
 
-void CopyOut::enqueue(const void *src, hipStream_t stream) {
+void CopyOut::enqueue(const uint32_t *src, hipStream_t stream) {
   if (!job_) return;
   Job &j = *job_;
-  if (!j.ring) {
-    j.ring = ring_borrow();
-    if (!j.ring) return;
-    j.first_value = g_ring.value + 1;
-  } else {  // (a call that starts over)
-    j.first_value = g_ring.value + 1;
-    j.issued = 0;
-  }
-  src_ = static_cast<const char *>(src);
+  if (!j.ring) j.ring = ring_borrow();
+  if (!j.ring) return;
+  j.first_value = g_ring.value + 1;
+  j.issued = 0;  // (also for a call that starts over)
+  src_ = src;
   stream_ = stream;
   issue();
   if (j.listed && !j.hot) helpers().heat(&j);
 }
 
-void CopyOut::finish(const void *src, hipStream_t stream) {
+void CopyOut::finish(const uint32_t *src, hipStream_t stream) {
   if (!job_) return;
   Job &j = *job_;
   if (!queued_) enqueue(src, stream);
@@ -337,9 +373,9 @@ void CopyOut::finish(const void *src, hipStream_t stream) {
   Spin spin;
   int idle = 0;
   auto looked = std::chrono::steady_clock::now();
-  while (j.done.load(std::memory_order_acquire) < j.bytes) {
+  while (j.done.load(std::memory_order_acquire) < j.count) {
     // (only this thread talks to the runtime)
-    while (j.issued < j.bytes && j.left[j.issued / kSlotBytes - kSlots].load(std::memory_order_acquire) == 0) issue();
+    while (j.issued < j.count && j.left[j.issued / kSlotCount - kSlots].load(std::memory_order_acquire) == 0) issue();
     size_t p = j.next_piece.load();
     if (p < j.pieces && p * j.piece < j.issued && j.has_arrived(p)) {
       if (j.next_piece.compare_exchange_strong(p, p + 1)) j.move(p);

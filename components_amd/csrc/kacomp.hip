@@ -2227,7 +2227,7 @@ int kc_find_components(kc_graph *g, const kc_options *opt, uint32_t *labels_out,
     }
     const auto t0 = std::chrono::steady_clock::now();
     g->have_labels = false;
-    CopyOut labels(labels_out, g->n * 4);
+    CopyOut labels(labels_out, g->n, g->n);
     if (o.variant == KC_VARIANT_EXP) ensure_table(g, o.beta);
     g->arena.reset();
     g->timer.begin_run(o.time_kernels != 0, g->stream, o.time_class - 1);
@@ -2438,7 +2438,7 @@ int kc_copy_labels(kc_graph *g, uint32_t *labels_out) {
   return guarded([&] {
     if (!g || !labels_out) fail(KC_ERR_INVALID, "null argument");
     if (!g->have_labels) fail(KC_ERR_INVALID, "no labels: kc_find_components has not completed");
-    CopyOut(labels_out, g->n * 4).finish(g->labels, g->stream);
+    CopyOut(labels_out, g->n, g->n).finish(g->labels, g->stream);
   });
 }
 

@@ -1,6 +1,6 @@
 """Labels copied out to pageable memory: every word written and none beside it, at the sizes where the copy
-changes its way (helper threads above 256 KB, pieces of 256 KB, or 512 KB above the ring's 16 MB, which
-later transfers of 4 MB go round), into buffers at odd offsets, and from several threads at once (one
+changes its way (helper threads above 256 KB, pieces of 64 k labels, or 128 k above the ring's 4 M, which
+later transfers of 1 M go round; two, three or four bytes a label), into buffers at odd offsets, and from several threads at once (one
 of them gets the pinned ring, the others copy the plain way)."""
 import ctypes
 import threading
@@ -40,8 +40,9 @@ def copy_into(fn, n, lead):
 KB = 1 << 8  # words per KB
 
 
-@pytest.mark.parametrize("n", [2, 1000, 256 * KB - 1, 256 * KB, 256 * KB + 1, 1024 * KB, 1024 * KB + 1, 2048 * KB - 1, 2048 * KB, 2048 * KB + 1, 9000 * KB + 3,
-                               16384 * KB - 1, 16384 * KB + 1, 20480 * KB, 20480 * KB + 1, 50000 * KB + 7])
+@pytest.mark.parametrize("n", [2, 1000, 65536, 65537, 256 * KB - 1, 256 * KB, 256 * KB + 1, 1024 * KB, 1024 * KB + 1, 2048 * KB - 1, 2048 * KB, 2048 * KB + 1, 9000 * KB + 3,
+                               16384 * KB - 1, 16384 * KB + 1, 20480 * KB, 20480 * KB + 1, 50000 * KB + 7, 1 << 24,
+                               (1 << 24) + 1])
 def test_every_word_and_no_other(n):
     g = graph(n)
     L = ca.lib()
