@@ -534,11 +534,13 @@ uint64_t sweep_bytes(uint64_t n, uint64_t m2) {
 // Sweeps are launched in speculative batches; a sweep whose predecessor
 // changed nothing returns at once.  Returns the number of sweeps that did work
 // (the last of them found no change).
+// settled: the rows up to this distance are final before the first sweep (-1:
+// not known, hop = 0).
 // packed (non-null): the keys are packed into this buffer (pack_keys) and swept
 // there; 0 sweeps are returned when they do not fit, key as before.
 uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t *off, const uint32_t *col,
-                           uint64_t *key, uint64_t hop, const Bins &b, uint32_t &flag_base, bool book_bytes = true,
-                           uint32_t *packed = nullptr) {
+                           uint64_t *key, uint64_t hop, const Bins &b, uint32_t &flag_base, int settled,
+                           bool book_bytes = true, uint32_t *packed = nullptr) {
   uint64_t done = 0;
   const uint32_t batch = n < (1u << 16) ? 8u : 3u;
   uint32_t check = 0;  // 1: the flag before the first batch's tells that packed keys do not fit
@@ -560,14 +562,16 @@ uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t 
       // the first sweep of a batch always runs: the previous batch ended with a change
       const int *prev = i == 0 ? nullptr : &g->flags[f - 1];
       slots[i] = g->timer.start(KC_K_SWEEP);
+      // (one distance more is final with every sweep)
+      const int final_to = settled < 0 ? -1 : settled + static_cast<int>(done + i);
       // hub chunks first, then wave, 16-lane and one-lane rows: the many
       // short rows then read the keys the hubs lowered in the same sweep
       // (R-MAT 24, sweeps schedule: 11.8 -> 11.0 sweeps, 24.7 -> 21.9 ms)
       if (packed)
-        sweep_packed(off, col, packed, b, &g->flags[f], prev, g->stream, true);
+        sweep_packed(off, col, packed, b, &g->flags[f], prev, g->stream, true, final_to);
       else
         sweep(kSweepInPlace, false, off, col, key, key, hop, b, g->deg_inter, g->hub_inter, &g->flags[f], prev,
-              g->stream, true);
+              g->stream, true, final_to);
       g->timer.stop(slots[i], bytes);
     }
     fetch32(g, g->h_flags, &g->flags[flag_base - check], batch + check, next_signal(g));
@@ -782,7 +786,8 @@ uint64_t rounds_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t
         // reach the same fixed point in as many sweeps as the longest chain
         // of improvements among them, instead of one round per distance left.
         // (The rounds' booked bytes already cover one read of every row.)
-        done += sweep_to_fixpoint(g, n, m2, off, col, key, kOneHop, b, flag_base, false);
+        // (the keys up to distance t are final, as before a round)
+        done += sweep_to_fixpoint(g, n, m2, off, col, key, kOneHop, b, flag_base, static_cast<int>(t), false);
         break;
       }
     }
@@ -1183,11 +1188,11 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
         // one hop stays within 32 bits.
         // (Whether they fit comes back with the first sweeps' flags.)
         uint32_t *pk = n_l >= kPackedSweepsMin && n_l <= (1ull << kPackedLabelBits) ? g->crank : nullptr;
-        if (pk) sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, kOneHop, b, flag_base, true, pk);
+        if (pk) sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, kOneHop, b, flag_base, 0, true, pk);
         if (pk && sweeps)
           unpack_keys(n_l, pk, g->key, g->stream);
         else
-          sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, kOneHop, b, flag_base);
+          sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, kOneHop, b, flag_base, 0);
       }
     }
     if (!pre && !local && !o->use_bfs && sweeps == 1) {
@@ -1452,7 +1457,7 @@ void run_propagation(kc_graph *g, const kc_options *o, RunOut &out) {
     TimedScope ts(g->timer, KC_K_DEVIATES, 8 * g->n);
     init_keys_index(g->n, g->key, g->stream);
   }
-  out.sweeps = sweep_to_fixpoint(g, g->n, g->m2, g->off0, g->col0, g->key, 0, b, flag_base);
+  out.sweeps = sweep_to_fixpoint(g, g->n, g->m2, g->off0, g->col0, g->key, 0, b, flag_base, -1);
   TimedScope ts(g->timer, KC_K_CANON, 12 * g->n);
   labels_from_keys(g->n, g->key, g->labels, g->small + 5, partial, g->stream);
 }

@@ -122,9 +122,11 @@ void finish_bins(Bins &b);  // computes block offsets from the counts
 
 // One binned sweep.  flag: set to 1 when a key decreased; prev_flag (may be
 // null): when it reads 0 the launch returns at once (converged earlier).
+// settled: in-place sweeps without counts skip the rows up to this distance,
+// which the caller knows to be final (-1: none).
 void sweep(int mode, bool count, const uint64_t *off, const uint32_t *col, const uint64_t *kin,
            uint64_t *kout, uint64_t hop, const Bins &b, uint32_t *deg_inter, uint32_t *hub_inter,
-           int *flag, const int *prev_flag, hipStream_t s, bool hubs_first = false);
+           int *flag, const int *prev_flag, hipStream_t s, bool hubs_first = false, int settled = -1);
 // Packed keys (distance << 24 | label) for the pull sweeps of levels below
 // 2^24 vertices: pack_keys writes them and sets *bad (0 before) when a
 // distance exceeds kPackedMaxDist - 1 or a label 24 bits; sweep_packed is
@@ -135,7 +137,7 @@ constexpr uint32_t kPackedMaxDist = 255;
 void pack_keys(uint64_t n, const uint64_t *key, uint32_t *pk, uint32_t *bad, hipStream_t s);
 void unpack_keys(uint64_t n, const uint32_t *pk, uint64_t *key, hipStream_t s);
 void sweep_packed(const uint64_t *off, const uint32_t *col, uint32_t *pk, const Bins &b, int *flag,
-                  const int *prev_flag, hipStream_t s, bool hubs_first);
+                  const int *prev_flag, hipStream_t s, bool hubs_first, int settled);
 // Round t of the time-stepped schedule: vertices at key distance t push
 // key + hop; *pending = 1 while a vertex is still above distance t;
 // prev_pending (may be null) reading 0 makes the launch return at once.

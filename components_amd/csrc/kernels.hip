@@ -249,18 +249,31 @@ struct SweepArgs {
   int *flag;
   const int *prev_flag;
   int hubs_first = 0;  // k_sweep: sections dispatched from the hub chunks down (as k_round's)
+  int settled = -1;    // k_sweep: rows up to this distance are final and not read (-1: none)
 };
 
 // Edges whose gathers one lane keeps in flight together in the row loops.
 constexpr int kGather = 4;
 constexpr int kRelabelGather = 16;
 
+// Sweeps with one hop per edge reach the keys of distance D in D sweeps at the
+// latest: a neighbour's key of distance D - 1 is final before sweep D reads it.
+// So before sweep s every row of distance s - 1 or less is final (its distance
+// can only be its final one or more), and its edges are not read again: on
+// graphs of small diameter most of the work of the sweeps after the third
+// (calls in sweeps: R-MAT 24 19.6 -> 11.5 ms, R-MAT 20 1.71 -> 1.29, 256^3 grid
+// 5.48 -> 4.70, random geometric 2 M 1.24 -> 1.03).
 template <int MODE, bool COUNT, int W>
 __device__ __forceinline__ bool sweep_group(const SweepArgs &a, bool active, uint32_t v, uint64_t e0,
                                             uint64_t e1, int gl, bool hub, uint32_t chunk) {
   uint64_t kv = active ? a.kin[v] : ~0ull;
   uint64_t best = kv;
   uint32_t cnt = 0;
+  if (MODE == kSweepInPlace && !COUNT) active = active && static_cast<int>(kv >> 32) > a.settled;
+  if (active && !hub) {
+    e0 = a.off[v];
+    e1 = a.off[v + 1];
+  }
   if (active) {
     const uint32_t lv = static_cast<uint32_t>(kv);
     uint64_t e = e0 + gl;
@@ -326,20 +339,17 @@ __global__ __launch_bounds__(kBlock) void k_sweep(SweepArgs a) {
     const uint32_t i = blk * kBlock + tid;
     const bool act = i < a.b.nT;
     uint32_t v = act ? a.b.listT[i] : 0;
-    uint64_t e0 = act ? a.off[v] : 0, e1 = act ? a.off[v + 1] : 0;
-    changed = sweep_group<MODE, COUNT, 1>(a, act, v, e0, e1, 0, false, 0);
+    changed = sweep_group<MODE, COUNT, 1>(a, act, v, 0, 0, 0, false, 0);
   } else if (blk < a.b.bW) {
     const uint32_t i = (blk - a.b.bS) * (kBlock / 16) + tid / 16;
     const bool act = i < a.b.nS;
     uint32_t v = act ? a.b.listS[i] : 0;
-    uint64_t e0 = act ? a.off[v] : 0, e1 = act ? a.off[v + 1] : 0;
-    changed = sweep_group<MODE, COUNT, 16>(a, act, v, e0, e1, tid & 15, false, 0);
+    changed = sweep_group<MODE, COUNT, 16>(a, act, v, 0, 0, tid & 15, false, 0);
   } else if (blk < a.b.bH) {
     const uint32_t i = (blk - a.b.bW) * (kBlock / kWave) + tid / kWave;
     const bool act = i < a.b.nW;
     uint32_t v = act ? a.b.listW[i] : 0;
-    uint64_t e0 = act ? a.off[v] : 0, e1 = act ? a.off[v + 1] : 0;
-    changed = sweep_group<MODE, COUNT, kWave>(a, act, v, e0, e1, tid & 63, false, 0);
+    changed = sweep_group<MODE, COUNT, kWave>(a, act, v, 0, 0, tid & 63, false, 0);
   } else {
     const uint32_t i = (blk - a.b.bH) * (kBlock / kWave) + tid / kWave;
     const bool act = i < a.b.nH;
@@ -386,7 +396,7 @@ struct PackedSweepArgs {
   Bins b;
   int *flag;
   const int *prev_flag;
-  int hubs_first;
+  int hubs_first, settled;
 };
 
 template <int W>
@@ -394,6 +404,11 @@ __device__ __forceinline__ bool packed_group(const PackedSweepArgs &a, bool acti
                                              uint64_t e1, int gl, bool hub) {
   const uint32_t kv = active ? a.key[v] : ~0u;
   uint32_t best = kv;
+  active = active && static_cast<int>(kv >> kPackedLabelBits) > a.settled;
+  if (active && !hub) {
+    e0 = a.off[v];
+    e1 = a.off[v + 1];
+  }
   if (active) {
     uint64_t e = e0 + gl;
     for (; e + (kGather - 1) * W < e1; e += kGather * W) {
@@ -435,17 +450,17 @@ __global__ __launch_bounds__(kBlock) void k_sweep_packed(PackedSweepArgs a) {
     const uint32_t i = blk * kBlock + tid;
     const bool act = i < a.b.nT;
     const uint32_t v = act ? a.b.listT[i] : 0;
-    changed = packed_group<1>(a, act, v, act ? a.off[v] : 0, act ? a.off[v + 1] : 0, 0, false);
+    changed = packed_group<1>(a, act, v, 0, 0, 0, false);
   } else if (blk < a.b.bW) {
     const uint32_t i = (blk - a.b.bS) * (kBlock / 16) + tid / 16;
     const bool act = i < a.b.nS;
     const uint32_t v = act ? a.b.listS[i] : 0;
-    changed = packed_group<16>(a, act, v, act ? a.off[v] : 0, act ? a.off[v + 1] : 0, tid & 15, false);
+    changed = packed_group<16>(a, act, v, 0, 0, tid & 15, false);
   } else if (blk < a.b.bH) {
     const uint32_t i = (blk - a.b.bW) * (kBlock / kWave) + tid / kWave;
     const bool act = i < a.b.nW;
     const uint32_t v = act ? a.b.listW[i] : 0;
-    changed = packed_group<kWave>(a, act, v, act ? a.off[v] : 0, act ? a.off[v + 1] : 0, tid & 63, false);
+    changed = packed_group<kWave>(a, act, v, 0, 0, tid & 63, false);
   } else {
     const uint32_t i = (blk - a.b.bH) * (kBlock / kWave) + tid / kWave;
     const bool act = i < a.b.nH;
@@ -2475,9 +2490,9 @@ void finish_bins(Bins &b) {
 
 void sweep(int mode, bool count, const uint64_t *off, const uint32_t *col, const uint64_t *kin, uint64_t *kout,
            uint64_t hop, const Bins &b, uint32_t *deg_inter, uint32_t *hub_inter, int *flag, const int *prev_flag,
-           hipStream_t s, bool hubs_first) {
+           hipStream_t s, bool hubs_first, int settled) {
   if (b.blocks == 0) return;
-  SweepArgs a{off, col, kin, kout, hop, b, deg_inter, hub_inter, flag, prev_flag, hubs_first ? 1 : 0};
+  SweepArgs a{off, col, kin, kout, hop, b, deg_inter, hub_inter, flag, prev_flag, hubs_first ? 1 : 0, settled};
   dim3 g(b.blocks), t(kBlock);
   if (mode == kSweepInPlace && count)
     hipLaunchKernelGGL((k_sweep<kSweepInPlace, true>), g, t, 0, s, a);
@@ -2504,9 +2519,9 @@ void unpack_keys(uint64_t n, const uint32_t *pk, uint64_t *key, hipStream_t s) {
 }
 
 void sweep_packed(const uint64_t *off, const uint32_t *col, uint32_t *pk, const Bins &b, int *flag,
-                  const int *prev_flag, hipStream_t s, bool hubs_first) {
+                  const int *prev_flag, hipStream_t s, bool hubs_first, int settled) {
   if (b.blocks == 0) return;
-  PackedSweepArgs a{off, col, pk, b, flag, prev_flag, hubs_first ? 1 : 0};
+  PackedSweepArgs a{off, col, pk, b, flag, prev_flag, hubs_first ? 1 : 0, settled};
   hipLaunchKernelGGL(k_sweep_packed, dim3(b.blocks), dim3(kBlock), 0, s, a);
   KC_LAUNCH_CHECK();
 }
