@@ -398,6 +398,12 @@ constexpr uint64_t kLevelHotRows = 28672;  // labels the one-pass relabel serves
 // against n/32; n/4 took 7.22, R-MAT 24 and the others alike)
 constexpr int kTailShift = 3;
 constexpr uint64_t kPackedSweepsMin = 1u << 16;  // levels at least this large sweep packed keys
+// -bfs: rounds on skewed levels at least this large, elsewhere the sweeps that
+// a level's rounds end with from its start.  A call in rounds everywhere, so, and
+// in sweeps everywhere: R-MAT 24 8.66, 8.63 and 10.8 ms, R-MAT 22 2.70, 2.57, 3.02,
+// R-MAT 20 1.25, 1.05, 1.05, 256^3 grid 5.22, 4.73, 4.71, G(2^20, 2^22) 1.35, 1.22,
+// 1.21.
+constexpr uint64_t kRoundsMin = 1u << 20;
 constexpr uint64_t kPullRoundsMin = 1u << 16;  // -bfs: levels at least this large choose round directions
 constexpr uint32_t kDirectionRounds = 6;        // rounds 1 .. this may be pulled
 constexpr uint64_t kDirectionMinDegree = 8;     // ... on levels of this average degree or more (sparse,
@@ -1175,7 +1181,8 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
                 &g->flags[kMaxFlags - 1], nullptr, g->stream);
         }
         sweeps = 2;
-      } else if (o->use_bfs) {
+      } else if (o->use_bfs && (o->tail_sweeps || o->pull_rounds ||
+                                (n_l >= kRoundsMin && (input_level0 ? g->l0_hot_skewed : level_hot)))) {
         const bool choose = o->pull_rounds > 0 || (o->pull_rounds == 0 && n_l >= kPullRoundsMin &&
                                                    m2_l >= kDirectionMinDegree * n_l);
         sweeps = rounds_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, b, cfg, flag_base,
