@@ -404,6 +404,7 @@ constexpr uint64_t kPackedSweepsMin = 1u << 16;  // levels at least this large s
 // R-MAT 20 1.25, 1.05, 1.05, 256^3 grid 5.22, 4.73, 4.71, G(2^20, 2^22) 1.35, 1.22,
 // 1.21.
 constexpr uint64_t kRoundsMin = 1u << 20;
+constexpr uint32_t kLongBatchBlocks = 1u << 15;  // sweeps of up to this many blocks go eight to a wait, others three
 constexpr uint64_t kPullRoundsMin = 1u << 16;  // -bfs: levels at least this large choose round directions
 constexpr uint32_t kDirectionRounds = 6;        // rounds 1 .. this may be pulled
 constexpr uint64_t kDirectionMinDegree = 8;     // ... on levels of this average degree or more (sparse,
@@ -548,7 +549,9 @@ uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t 
                            uint64_t *key, uint64_t hop, const Bins &b, uint32_t &flag_base, int settled,
                            bool book_bytes = true, uint32_t *packed = nullptr) {
   uint64_t done = 0;
-  const uint32_t batch = n < (1u << 16) ? 8u : 3u;
+  // once most rows are settled a sweep costs less than a wait of the host, and one
+  // after the last change returns at once (2 us, but 14 with 58 000 blocks)
+  const uint32_t batch = b.blocks <= kLongBatchBlocks ? 8u : 3u;
   uint32_t check = 0;  // 1: the flag before the first batch's tells that packed keys do not fit
   // (packed: 4-byte keys for the neighbours and the row's own)
   const uint64_t bytes = !book_bytes ? 0 : packed ? 8 * (n + 1) + 8 * m2 + 8 * n : sweep_bytes(n, m2);
