@@ -1104,7 +1104,6 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
       t.cur = g->crank;
       t.gid = g->seg_of_cid;
       t.key0 = g->uniq;
-      t.nidx = reinterpret_cast<uint16_t *>(g->pos_of);
       t.rep = g->rep_a;
       t.count = g->small + 8;
       t.info = g->small + 9;

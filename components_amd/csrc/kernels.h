@@ -170,10 +170,10 @@ void union_labels(uint64_t n, const uint32_t *parent, uint32_t *labels, uint32_t
 // edgeless graph or the base case, rep[v] = the id (gid_in; null: identity) of
 // v's last centre.  m: the level's undirected edges as the cut-off counts
 // them; stall_rule: the default schedule's rule for levels that change no key.
-// cur, gid, key0: n words of scratch each, nidx: n half-words, edge: m2 words,
+// cur, gid, key0: n words of scratch each, edge: m2 words,
 // count: a zeroed word; info = {status, levels, sweeps, radius sum}.
 constexpr uint64_t kTailVertices = 32768;     // 128 KB of LDS: a key per vertex
-constexpr uint64_t kTailSmall = 16128;        // ... two keys and a 16-bit index per vertex in 160 KB
+constexpr uint64_t kTailSmall = 16128;        // ... two keys per vertex (the local variant's)
 constexpr uint64_t kTailSlots = 1u << 19;     // edge slots of up to kTailSmall vertices
 constexpr uint64_t kTailBigSlots = 1u << 18;  // ... of more
 constexpr uint32_t kTailMaxDeviate = (1u << 17) - 3;  // distances share a word with 15 label bits
@@ -186,7 +186,6 @@ struct TailArgs {
   DeviateArgs d;
   const uint32_t *gid_in;
   uint32_t *edge, *cur, *gid, *key0, *rep, *count, *info;
-  uint16_t *nidx;
 };
 void tail_levels(const TailArgs &a, uint64_t m2, const uint64_t *off, const uint32_t *col, hipStream_t s);
 

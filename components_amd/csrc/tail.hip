@@ -113,25 +113,32 @@ __device__ __forceinline__ uint4 load4(const uint32_t *edge, uint32_t i, uint32_
   return i < n4 ? reinterpret_cast<const uint4 *>(edge)[i] : make_uint4(0u, 0u, 0u, 0u);
 }
 
-// kBig: more than kTailSmall vertices; the index per label then lives in
-// global memory until a level is that small, and the local variant's second
-// copy of the keys has no room.
-template <bool kBig>
+// The next level's index of a label is its rank among the marked ones: a bit
+// and a count per 32 labels in LDS, where an index per label had to be written
+// for all of them, above kTailSmall vertices to global memory: 32 008 vertices 300
+// -> 232 us, 26 157 with 16 levels that hardly contract 4.5 -> 3.4 ms.
 __global__ __launch_bounds__(kTailBlock) void k_tail(TailArgs a) {
-  constexpr int kPer = (kBig ? kTailVertices : kTailSmall + 256) / kTailBlock;  // level indices per thread
-  static_assert(kPer * kTailBlock >= (kBig ? kTailVertices : kTailSmall), "every index has a thread");
-  __shared__ uint32_t lds[kTable];  // the keys, up to kTailSmall of them with a copy; all of it the edge table
-  __shared__ uint16_t nidx_lds[kTailSmall];  // per label: the next level's index (kNoIndex: none)
+  static_assert(kTailVertices == 32 * kTailBlock, "a thread per word of marks");
+  __shared__ __align__(16) uint32_t lds[kTable];  // the keys, up to kTailSmall of them with a copy; all of it the edge table
+  __shared__ uint2 rank[kTailBlock];              // 32 labels: those of clusters with an edge, and their number before
   __shared__ uint32_t wave[kTailBlock / kWave];
   __shared__ uint32_t s_radius, s_full;
   uint32_t *key = lds, *key2 = lds + kTable / 2;
-  bool wide = kBig;  // the level's indices are in a.nidx
-  const auto index_of = [&](uint32_t l) -> uint32_t { return kBig && wide ? a.nidx[l] : nidx_lds[l]; };
-  const auto set_index = [&](uint32_t l, uint32_t x) {
-    if (kBig && wide)
-      a.nidx[l] = static_cast<uint16_t>(x);
-    else
-      nidx_lds[l] = static_cast<uint16_t>(x);
+  const auto set_mark = [&](uint32_t l) {
+    if (!(rank[l >> 5].x >> (l & 31) & 1u)) atomicOr(&rank[l >> 5].x, 1u << (l & 31));
+  };
+  const auto index_of = [&](uint32_t l) -> uint32_t {
+    const uint2 w = rank[l >> 5];
+    const uint32_t bit = 1u << (l & 31);
+    return w.x & bit ? w.y + static_cast<uint32_t>(__popc(w.x & (bit - 1))) : kNoIndex;
+  };
+  const auto marked_index = [&](uint32_t l) -> uint32_t {  // of a marked label
+    const uint2 w = rank[l >> 5];
+    return w.y + static_cast<uint32_t>(__popc(w.x & ((1u << (l & 31)) - 1)));
+  };
+  const auto clear_table = [&] {
+    for (uint32_t j = threadIdx.x; j < kTable / 4; j += kTailBlock)
+      reinterpret_cast<uint4 *>(lds)[j] = make_uint4(kNone, kNone, kNone, kNone);
   };
   const uint32_t tid = threadIdx.x;
   const uint32_t n0 = a.n;
@@ -145,7 +152,6 @@ __global__ __launch_bounds__(kTailBlock) void k_tail(TailArgs a) {
   __syncthreads();
   while (true) {
     const bool base = a.seq_limit > 0 && m <= a.seq_limit;
-    wide = kBig && nl > kTailSmall;
     if (!base && levels >= a.max_levels) {
       status = kTailLevels;
       break;
@@ -243,8 +249,8 @@ __global__ __launch_bounds__(kTailBlock) void k_tail(TailArgs a) {
       const uint32_t k = key[v];
       const uint32_t h = a.local ? 0u : (k >> kLabelBits) - (key[k & kLabelMask] >> kLabelBits);
       r = h > r ? h : r;
-      set_index(v, 0);
     }
+    rank[tid].x = 0;
     for (int o = 32; o > 0; o >>= 1) {
       const uint32_t t = static_cast<uint32_t>(__shfl_xor(static_cast<int>(r), o));
       r = t > r ? t : r;
@@ -260,8 +266,8 @@ __global__ __launch_bounds__(kTailBlock) void k_tail(TailArgs a) {
       for (int j = 0; j < 8; ++j) {  // (the zeros past the end become kNone too)
         const uint32_t x = key[e[j] & 0xFFFFu] & kLabelMask, y = key[e[j] >> 16] & kLabelMask;
         if (x != y) {
-          set_index(x, 1);
-          set_index(y, 1);
+          set_mark(x);
+          set_mark(y);
         }
         e[j] = x == y ? kNone : x < y ? x | (y << 16) : y | (x << 16);
       }
@@ -269,26 +275,15 @@ __global__ __launch_bounds__(kTailBlock) void k_tail(TailArgs a) {
       if (i0 + kTailBlock < n4) edge4[i0 + kTailBlock] = make_uint4(e[4], e[5], e[6], e[7]);
     }
     __syncthreads();
-    // next-level indices in label order: each thread numbers kPer consecutive labels
-    static_assert(kPer <= 32, "a bit per label");
-    uint32_t marks = 0;
-#pragma unroll 8
-    for (int j = 0; j < kPer; ++j) {
-      const uint32_t v = tid * kPer + j;
-      marks |= (v < nl && index_of(v) ? 1u : 0u) << j;
-    }
+    // next-level indices in label order
     uint32_t n_next = 0;
-    const uint32_t first = tail_scan(static_cast<uint32_t>(__popc(marks)), wave, n_next);
-    uint32_t next = first;
-#pragma unroll 4
-    for (int j = 0; j < kPer; ++j) {
-      const uint32_t v = tid * kPer + j;
-      if (v >= nl) break;
-      const bool mark = marks >> j & 1u;
-      if (mark) gid_next[next] = gid[v];
-      set_index(v, mark ? next++ : kNoIndex);
-    }
+    rank[tid].y = tail_scan(static_cast<uint32_t>(__popc(rank[tid].x)), wave, n_next);
     __syncthreads();
+#pragma unroll 4
+    for (uint32_t v = tid; v < nl; v += kTailBlock) {
+      const uint32_t x = index_of(v);
+      if (x != kNoIndex) gid_next[x] = gid[v];
+    }
     for (uint32_t v = tid; v < n0; v += kTailBlock) {
       const uint32_t c = a.cur[v];
       if (c == kNone) continue;
@@ -306,7 +301,7 @@ __global__ __launch_bounds__(kTailBlock) void k_tail(TailArgs a) {
     // The pairs renumbered and moved to the front, repeats dropped where the
     // filter meets them: of equal edges the first to reach their slot is kept
     // (a repeat that stays changes no key).
-    for (uint32_t j = tid; j < kTable; j += kTailBlock) lds[j] = kNone;
+    clear_table();
     __syncthreads();
     uint32_t out = 0;
     const uint4 none = make_uint4(kNone, kNone, kNone, kNone);
@@ -318,7 +313,7 @@ __global__ __launch_bounds__(kTailBlock) void k_tail(TailArgs a) {
       c1 = ahead + kTailBlock < n4 ? edge4[ahead + kTailBlock] : none;
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        if (x[j] != kNone) x[j] = index_of(x[j] & 0xFFFFu) | (index_of(x[j] >> 16) << 16);
+        if (x[j] != kNone) x[j] = marked_index(x[j] & 0xFFFFu) | (marked_index(x[j] >> 16) << 16);
 #pragma unroll
       for (int j = 0; j < 8; ++j)
         if (x[j] != kNone && atomicExch(&lds[edge_hash(x[j]) & (kTable - 1)], x[j]) == x[j]) x[j] = kNone;
@@ -345,16 +340,18 @@ __global__ __launch_bounds__(kTailBlock) void k_tail(TailArgs a) {
     if (a.seq_limit > 0 && ne > a.seq_limit) {
       // The cut-off compares the distinct edges: they are counted by hash
       // parts, each in a table of its own, until there are more than the
-      // bound; where a table of one part holds the bound and a step, one
-      // part does whatever their number.
-      const uint32_t step_edges = 4 * kTailBlock;
-      const uint32_t parts = a.seq_limit + step_edges <= kTableLoad ? 1 : (ne + kTableLoad - 1) / kTableLoad;
+      // bound; where a table of one part holds the bound and the steps between
+      // two looks at the count, one part does whatever their number.
+      constexpr uint32_t step_edges = 4 * kTailBlock, look_steps = 2;
+      const uint32_t parts =
+          a.seq_limit + look_steps * step_edges <= kTableLoad ? 1 : (ne + kTableLoad - 1) / kTableLoad;
       uint64_t distinct = 0;
       for (uint32_t part = 0; part < parts && distinct <= a.seq_limit; ++part) {
-        for (uint32_t j = tid; j < kTable; j += kTailBlock) lds[j] = kNone;
+        clear_table();
         __syncthreads();
+        uint32_t added = 0, steps = 0, total = 0;
         for (uint32_t b = 0; b < ne && distinct <= a.seq_limit; b += step_edges) {
-          uint32_t e[4], slot[4], jump[4], open = 0, added = 0;  // bit j of open: edge j still probing
+          uint32_t e[4], slot[4], jump[4], open = 0;  // bit j of open: edge j still probing
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const uint32_t i = b + j * kTailBlock + tid;
@@ -394,11 +391,14 @@ __global__ __launch_bounds__(kTailBlock) void k_tail(TailArgs a) {
               break;
             }
           }
-          uint32_t total = 0;
-          tail_scan(added, wave, total);
-          distinct += total;
+          if (parts == 1 && ++steps % look_steps == 0) {
+            tail_scan(added, wave, total);
+            distinct += total;
+            added = 0;
+          }
         }
-        __syncthreads();
+        tail_scan(added, wave, total);
+        distinct += total;
       }
       if (s_full) {
         status = kTailFull;
@@ -429,10 +429,7 @@ void tail_levels(const TailArgs &a, uint64_t m2, const uint64_t *off, const uint
                               ceil_div(a.n, static_cast<uint64_t>(kBlock)));
   hipLaunchKernelGGL(k_tail_edges, dim3(static_cast<unsigned>(g)), dim3(kBlock), 0, s, a, m2, off, col);
   KC_LAUNCH_CHECK();
-  if (a.n > kTailSmall)
-    hipLaunchKernelGGL(k_tail<true>, dim3(1), dim3(kTailBlock), 0, s, a);
-  else
-    hipLaunchKernelGGL(k_tail<false>, dim3(1), dim3(kTailBlock), 0, s, a);
+  hipLaunchKernelGGL(k_tail, dim3(1), dim3(kTailBlock), 0, s, a);
   KC_LAUNCH_CHECK();
 }
 
