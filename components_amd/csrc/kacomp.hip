@@ -543,8 +543,8 @@ uint64_t sweep_bytes(uint64_t n, uint64_t m2) {
 // (the last of them found no change).
 // settled: the rows up to this distance are final before the first sweep (-1:
 // not known, hop = 0).
-// packed (non-null): the keys are packed into this buffer (pack_keys) and swept
-// there; 0 sweeps are returned when they do not fit, key as before.
+// packed (non-null): the sweeps run over these packed keys, whose check went to
+// the flag before flag_base; 0 sweeps are returned when they do not fit.
 uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t *off, const uint32_t *col,
                            uint64_t *key, uint64_t hop, const Bins &b, uint32_t &flag_base, int settled,
                            bool book_bytes = true, uint32_t *packed = nullptr) {
@@ -552,18 +552,13 @@ uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t 
   // once most rows are settled a sweep costs less than a wait of the host, and one
   // after the last change returns at once (2 us, but 14 with 58 000 blocks)
   const uint32_t batch = b.blocks <= kLongBatchBlocks ? 8u : 3u;
-  uint32_t check = 0;  // 1: the flag before the first batch's tells that packed keys do not fit
+  uint32_t check = packed ? 1 : 0;  // the flag before the first batch's tells that packed keys do not fit
   // (packed: 4-byte keys for the neighbours and the row's own)
   const uint64_t bytes = !book_bytes ? 0 : packed ? 8 * (n + 1) + 8 * m2 + 8 * n : sweep_bytes(n, m2);
   while (true) {
     if (flag_base + batch + 2 >= kMaxFlags) {
       fill_u32(reinterpret_cast<uint32_t *>(g->flags), kMaxFlags, 0, g->stream);
       flag_base = 0;
-    }
-    if (packed && done == 0) {
-      pack_keys(n, key, packed, reinterpret_cast<uint32_t *>(&g->flags[flag_base]), g->stream);
-      ++flag_base;
-      check = 1;
     }
     int slots[8];
     for (uint32_t i = 0; i < batch; ++i) {
@@ -1124,6 +1119,7 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
       bins_valid = true;
     }
     uint64_t sweeps = 0;
+    uint32_t *pk = nullptr;  // the level's packed keys
     if (pre) {
       // components inside the blocks: union-find over the edges inside a block
       const uint64_t bsize = ceil_div(n_l, static_cast<uint64_t>(o->pre_blocks));
@@ -1162,15 +1158,32 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
         }
         la.delay = g->delay;
       }
-      {
-        TimedScope ts(g->timer, KC_K_DEVIATES, 8 * n_l + (gid_l ? 4 * n_l : 0) + (la.delay ? n_l : 0));
+      const bool rounds = !local && o->use_bfs &&
+                          (o->tail_sweeps || o->pull_rounds ||
+                           (n_l >= kRoundsMin && (input_level0 ? g->l0_hot_skewed : level_hot)));
+      // Levels below 2^24 vertices whose key distances stay below 255 sweep
+      // packed 32-bit keys (the buffer of the cluster ranks is free until they
+      // are built).  A distance only falls, so a key plus one hop stays within
+      // 32 bits.  Whether they fit comes back with the first sweeps' flags.
+      if (!local && !rounds && n_l >= kPackedSweepsMin && n_l <= (1ull << kPackedLabelBits)) pk = g->crank;
+      const auto draw_keys = [&](bool packed) {
+        TimedScope ts(g->timer, KC_K_DEVIATES, (packed ? 4 : 8) * n_l + (gid_l ? 4 * n_l : 0) + (la.delay ? n_l : 0));
+        da.iteration = iteration;
         if (local) {
           init_keys_uniform(n_l, dev_gid_l, idx_l, o->seed, iteration, g->key, g->stream);
+        } else if (packed) {
+          if (flag_base + 12 >= kMaxFlags) {  // (its flag and the first batch's stay together)
+            fill_u32(reinterpret_cast<uint32_t *>(g->flags), kMaxFlags, 0, g->stream);
+            flag_base = 0;
+          }
+          init_keys_packed(n_l, dev_gid_l, idx_l, da, la, pk, reinterpret_cast<uint32_t *>(&g->flags[flag_base]),
+                           g->stream);
+          ++flag_base;
         } else {
-          da.iteration = iteration;
           init_keys_exp(n_l, dev_gid_l, idx_l, da, la, g->key, g->stream);
         }
-      }
+      };
+      draw_keys(pk != nullptr);
       if (local) {
         // two synchronous min passes over the closed neighbourhood
         // (local_contraction.h:195-274), then a counting pass on the final keys
@@ -1183,25 +1196,20 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
                 &g->flags[kMaxFlags - 1], nullptr, g->stream);
         }
         sweeps = 2;
-      } else if (o->use_bfs && (o->tail_sweeps || o->pull_rounds ||
-                                (n_l >= kRoundsMin && (input_level0 ? g->l0_hot_skewed : level_hot)))) {
+      } else if (rounds) {
         const bool choose = o->pull_rounds > 0 || (o->pull_rounds == 0 && n_l >= kPullRoundsMin &&
                                                    m2_l >= kDirectionMinDegree * n_l);
         sweeps = rounds_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, b, cfg, flag_base,
                                     o->tail_sweeps < 0 ? -1 : o->tail_sweeps == 0 ? kTailShift : o->tail_sweeps,
                                     choose, pos_l != nullptr && off_l == g->off0p && g->l0_hot_skewed);
       } else {
-        // Levels below 2^24 vertices whose key distances stay below 255 sweep
-        // packed 32-bit keys (pack_keys; the buffer of the cluster ranks is
-        // free until they are built).  A distance only falls, so a key plus
-        // one hop stays within 32 bits.
-        // (Whether they fit comes back with the first sweeps' flags.)
-        uint32_t *pk = n_l >= kPackedSweepsMin && n_l <= (1ull << kPackedLabelBits) ? g->crank : nullptr;
         if (pk) sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, kOneHop, b, flag_base, 0, true, pk);
-        if (pk && sweeps)
-          unpack_keys(n_l, pk, g->key, g->stream);
-        else
+        if (!sweeps) {
+          if (pk) draw_keys(false);
+          pk = nullptr;
           sweeps = sweep_to_fixpoint(g, n_l, m2_l, off_l, col_l, g->key, kOneHop, b, flag_base, 0);
+        }
+        if (pk && o->record_trace) unpack_keys(n_l, pk, g->key, g->stream);
       }
     }
     if (!pre && !local && !o->use_bfs && sweeps == 1) {
@@ -1253,7 +1261,7 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
     if (dense) fill_u32(g->cid, n_l, 0, g->stream);  // the used-label flags, then the ids
     {
       TimedScope ts(g->timer, KC_K_COUNT, 8 * n_l + 4 * n_l + 4 * n_l + (local ? 0 : 8 * n_l));
-      labels_radius(n_l, g->key, pos_l, rec.lab, g->small + 13, !local && !pre, g->stream, dense ? g->cid : nullptr, sum);
+      labels_radius(n_l, g->key, pk, pos_l, rec.lab, g->small + 13, !local && !pre, g->stream, dense ? g->cid : nullptr, sum);
     }
     if (g->collect && !pre) {
       // trace of the plain method: features and the log2 size of each vertex's cluster

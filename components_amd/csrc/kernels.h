@@ -128,13 +128,14 @@ void sweep(int mode, bool count, const uint64_t *off, const uint32_t *col, const
            uint64_t *kout, uint64_t hop, const Bins &b, uint32_t *deg_inter, uint32_t *hub_inter,
            int *flag, const int *prev_flag, hipStream_t s, bool hubs_first = false, int settled = -1);
 // Packed keys (distance << 24 | label) for the pull sweeps of levels below
-// 2^24 vertices: pack_keys writes them and sets *bad (0 before) when a
+// 2^24 vertices: init_keys_packed writes init_keys_exp's and sets *bad (0 before) when a
 // distance exceeds kPackedMaxDist - 1 or a label 24 bits; sweep_packed is
-// sweep(kSweepInPlace, no counts) over them; unpack_keys restores the keys.
+// sweep(kSweepInPlace, no counts) over them; unpack_keys gives the 64-bit ones.
 constexpr uint32_t kPackedLabelBits = 24;
 constexpr uint32_t kPackedHop = 1u << kPackedLabelBits;
 constexpr uint32_t kPackedMaxDist = 255;
-void pack_keys(uint64_t n, const uint64_t *key, uint32_t *pk, uint32_t *bad, hipStream_t s);
+void init_keys_packed(uint64_t n, const uint32_t *gid, const uint32_t *idx, DeviateArgs d, LearnedArgs la, uint32_t *pk,
+                      uint32_t *bad, hipStream_t s);
 void unpack_keys(uint64_t n, const uint32_t *pk, uint64_t *key, hipStream_t s);
 void sweep_packed(const uint64_t *off, const uint32_t *col, uint32_t *pk, const Bins &b, int *flag,
                   const int *prev_flag, hipStream_t s, bool hubs_first, int settled);
@@ -194,11 +195,11 @@ void tail_levels(const TailArgs &a, uint64_t m2, const uint64_t *off, const uint
 void block_interface(const uint64_t *off, const uint32_t *col, uint64_t n, uint64_t bsize, uint64_t *key,
                      hipStream_t s);
 
-// lab[v] = low half of key[v]; max cluster radius (atomicMax into *radius);
+// lab[v] = low half of key[v], or of its packed form (null: key); max cluster radius (atomicMax into *radius);
 // used (may be null, pre-zeroed): used[lab[v]] = 1, the used-label flags of
 // cluster_ranks.
-void labels_radius(uint64_t n, const uint64_t *key, const uint32_t *pos, uint32_t *lab, uint32_t *radius,
-                   bool with_radius, hipStream_t s, uint32_t *used = nullptr, uint32_t *zero = nullptr);
+void labels_radius(uint64_t n, const uint64_t *key, const uint32_t *packed, const uint32_t *pos, uint32_t *lab,
+                   uint32_t *radius, bool with_radius, hipStream_t s, uint32_t *used, uint32_t *zero);
 // Dense cluster ids in label order from the used-label flags (labels_radius):
 // rank[a] = number of used labels below a, written for the used ones, and
 // *count (device) = number of clusters C; then cid[v] = rank[lab[v]] in [0, C).

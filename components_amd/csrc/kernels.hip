@@ -63,14 +63,17 @@ __global__ void k_fill(T *p, uint64_t n, T v) {
 // Keys.
 // Key of the vertex stored at v: (deviate << 32) | level index, where the
 // level index is idx[v] when the level is stored in another order (null: v).
+__device__ __forceinline__ uint32_t first_distance(uint64_t v, const uint32_t *gid, const DeviateArgs &d,
+                                                   const LearnedArgs &la) {
+  const uint32_t g = gid ? gid[v] : static_cast<uint32_t>(v);
+  const uint32_t dev = exp_deviate(g, d.seed, d.iteration, d.rng_offset, d.fused != 0, d.stream, d.table, d.k_max);
+  return la.delay ? dev + la.delay[v] : dev;
+}
 __global__ void k_init_keys_exp(uint64_t n, const uint32_t *gid, const uint32_t *idx, DeviateArgs d, LearnedArgs la,
                                 uint64_t *key) {
   uint64_t v = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
   if (v >= n) return;
-  uint32_t g = gid ? gid[v] : static_cast<uint32_t>(v);
-  uint32_t dev = exp_deviate(g, d.seed, d.iteration, d.rng_offset, d.fused != 0, d.stream, d.table, d.k_max);
-  if (la.delay) dev += la.delay[v];
-  key[v] = (static_cast<uint64_t>(dev) << 32) | (idx ? idx[v] : static_cast<uint32_t>(v));
+  key[v] = (static_cast<uint64_t>(first_distance(v, gid, d, la)) << 32) | (idx ? idx[v] : static_cast<uint32_t>(v));
 }
 
 __global__ void k_init_keys_index(uint64_t n, uint64_t *key) {
@@ -366,16 +369,18 @@ __global__ __launch_bounds__(kBlock) void k_sweep(SweepArgs a) {
 // the same order in half the bytes, so that a 128-byte line brings 32 keys to
 // the gathers instead of 16.  *bad receives a nonzero value when a key does
 // not fit (the caller then sweeps the 64-bit keys).
-__global__ __launch_bounds__(kBlock) void k_pack_keys(uint64_t n, const uint64_t *key, uint32_t *pk, uint32_t *bad) {
+// (written so from the start: 64-bit keys packed here and unpacked again for the
+// labels took 60 us more on a level of 15 M vertices, and two launches)
+__global__ __launch_bounds__(kBlock) void k_init_keys_packed(uint64_t n, const uint32_t *gid, const uint32_t *idx,
+                                                            DeviateArgs d, LearnedArgs la, uint32_t *pk,
+                                                            uint32_t *bad) {
+  const uint64_t v = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
   bool over = false;
-  for (uint64_t v = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x; v < n;
-       v += static_cast<uint64_t>(gridDim.x) * kBlock) {
-    const uint64_t k = key[v];
-    const uint32_t d = static_cast<uint32_t>(k >> 32), l = static_cast<uint32_t>(k);
+  if (v < n) {
+    const uint32_t dist = first_distance(v, gid, d, la), l = idx ? idx[v] : static_cast<uint32_t>(v);
     // a neighbour's key plus one hop must fit as well: distances up to 254
-    const bool fits = d < kPackedMaxDist && l < (1u << kPackedLabelBits);
-    over |= !fits;
-    pk[v] = fits ? (d << kPackedLabelBits) | l : ~0u;
+    over = dist >= kPackedMaxDist || l >= (1u << kPackedLabelBits);
+    pk[v] = over ? ~0u : (dist << kPackedLabelBits) | l;
   }
   if (__ballot(over) != 0 && lane_id() == 0) *bad = 1;
 }
@@ -944,7 +949,13 @@ __global__ __launch_bounds__(kBlock) void k_block_interface(const uint64_t *off,
 // level is stored in another order (null: l).
 // Grid-stride, with one atomic per workgroup: atomics on one address are
 // serialised by the device, so one per wave cost more than the pass itself.
-__global__ __launch_bounds__(kBlock) void k_labels_radius(uint64_t n, const uint64_t *key, const uint32_t *pos,
+__device__ __forceinline__ uint32_t key_label(uint64_t k) { return static_cast<uint32_t>(k); }
+__device__ __forceinline__ uint32_t key_distance(uint64_t k) { return static_cast<uint32_t>(k >> 32); }
+__device__ __forceinline__ uint32_t key_label(uint32_t k) { return k & ((1u << kPackedLabelBits) - 1); }
+__device__ __forceinline__ uint32_t key_distance(uint32_t k) { return k >> kPackedLabelBits; }
+
+template <class Key>
+__global__ __launch_bounds__(kBlock) void k_labels_radius(uint64_t n, const Key *key, const uint32_t *pos,
                                                          uint32_t *lab, uint32_t *used, uint32_t *zero,
                                                          uint32_t *radius, int with_radius) {
   __shared__ uint32_t wave_max[kBlock / kWave];
@@ -954,15 +965,15 @@ __global__ __launch_bounds__(kBlock) void k_labels_radius(uint64_t n, const uint
   constexpr int kU = 4;
   const uint64_t stride = static_cast<uint64_t>(gridDim.x) * kBlock;
   for (uint64_t v0 = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x; v0 < n; v0 += kU * stride) {
-    uint64_t k[kU];
+    Key k[kU];
     uint32_t c[kU];
 #pragma unroll
-    for (int u = 0; u < kU; ++u) k[u] = v0 + u * stride < n ? key[v0 + u * stride] : 0ull;
+    for (int u = 0; u < kU; ++u) k[u] = v0 + u * stride < n ? key[v0 + u * stride] : Key{0};
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       const uint64_t v = v0 + u * stride;
       if (v >= n) continue;
-      const uint32_t l = static_cast<uint32_t>(k[u]);
+      const uint32_t l = key_label(k[u]);
       lab[v] = l;
       if (used) used[l] = 1;
       if (zero) zero[v] = 0;
@@ -970,13 +981,13 @@ __global__ __launch_bounds__(kBlock) void k_labels_radius(uint64_t n, const uint
     if (with_radius) {
 #pragma unroll
       for (int u = 0; u < kU; ++u) {
-        const uint32_t l = static_cast<uint32_t>(k[u]);
+        const uint32_t l = key_label(k[u]);
         c[u] = v0 + u * stride < n ? (pos ? pos[l] : l) : 0u;
       }
 #pragma unroll
       for (int u = 0; u < kU; ++u)
         if (v0 + u * stride < n)
-          r = max(r, static_cast<uint32_t>(k[u] >> 32) - static_cast<uint32_t>(key[c[u]] >> 32));
+          r = max(r, key_distance(k[u]) - key_distance(key[c[u]]));
     }
   }
   if (with_radius) {
@@ -2505,10 +2516,10 @@ void sweep(int mode, bool count, const uint64_t *off, const uint32_t *col, const
   KC_LAUNCH_CHECK();
 }
 
-void pack_keys(uint64_t n, const uint64_t *key, uint32_t *pk, uint32_t *bad, hipStream_t s) {
+void init_keys_packed(uint64_t n, const uint32_t *gid, const uint32_t *idx, DeviateArgs d, LearnedArgs la, uint32_t *pk,
+                      uint32_t *bad, hipStream_t s) {
   if (!n) return;
-  const unsigned g = static_cast<unsigned>(std::min<uint64_t>(ceil_div(n, kBlock), 4096));
-  hipLaunchKernelGGL(k_pack_keys, dim3(g), dim3(kBlock), 0, s, n, key, pk, bad);
+  hipLaunchKernelGGL(k_init_keys_packed, dim3(grid_for(n)), dim3(kBlock), 0, s, n, gid, idx, d, la, pk, bad);
   KC_LAUNCH_CHECK();
 }
 
@@ -2565,12 +2576,16 @@ void huge_sizes(uint32_t n_huge, const uint32_t *huge, const uint64_t *seg_off, 
   KC_LAUNCH_CHECK();
 }
 
-void labels_radius(uint64_t n, const uint64_t *key, const uint32_t *pos, uint32_t *lab, uint32_t *radius,
-                   bool with_radius, hipStream_t s, uint32_t *used, uint32_t *zero) {
+void labels_radius(uint64_t n, const uint64_t *key, const uint32_t *packed, const uint32_t *pos, uint32_t *lab,
+                   uint32_t *radius, bool with_radius, hipStream_t s, uint32_t *used, uint32_t *zero) {
   if (!n) return;
   const unsigned g = static_cast<unsigned>(std::min<uint64_t>(ceil_div(n, kBlock), 2048));
-  hipLaunchKernelGGL(k_labels_radius, dim3(g), dim3(kBlock), 0, s, n, key, pos, lab, used, zero, radius,
-                     with_radius ? 1 : 0);
+  if (packed)
+    hipLaunchKernelGGL(k_labels_radius<uint32_t>, dim3(g), dim3(kBlock), 0, s, n, packed, pos, lab, used, zero, radius,
+                       with_radius ? 1 : 0);
+  else
+    hipLaunchKernelGGL(k_labels_radius<uint64_t>, dim3(g), dim3(kBlock), 0, s, n, key, pos, lab, used, zero, radius,
+                       with_radius ? 1 : 0);
   KC_LAUNCH_CHECK();
 }
 
