@@ -1339,7 +1339,8 @@ int kc_batch_autotune(kc_batch *b, const kc_options *opt, kc_batch_tuning *chose
     best.use_graph = 0;
     float best_ms = 0.f;
     bool have = false;
-    const uint32_t splits[] = {0u, 1u << 12, 1u << 14, 1u << 16};
+    // (the largest size class among the splits: with it nothing is left for the queue)
+    const uint32_t splits[] = {0u, 1u << 12, kLdsClass[kLdsClasses - 1].n, 1u << 14, 1u << 16};
     for (uint32_t sp : splits) {
       kc_batch_tuning t = best;
       t.split_vertices = sp;
@@ -1350,18 +1351,23 @@ int kc_batch_autotune(kc_batch *b, const kc_options *opt, kc_batch_tuning *chose
         have = true;
       }
     }
-    const int blocks[] = {256, 512, 1024};
-    const int gpcs[] = {1, 2, 4, 8};
-    for (int blk : blocks)
-      for (int gpc : gpcs) {
-        if (blk * gpc > 2048) continue;  // at most 32 waves per compute unit
-        kc_batch_tuning t{blk, gpc, 0, best.split_vertices};
-        const float ms = time_of(t);
-        if (ms < best_ms) {
-          best_ms = ms;
-          best = t;
+    // The shape is the persistent kernel's alone: where the size classes and the
+    // device-wide path take every graph the caller's stands.
+    prepare_split(b, best.split_vertices);
+    if (b->dev.queued) {
+      const int blocks[] = {256, 512, 1024};
+      const int gpcs[] = {1, 2, 4, 8};
+      for (int blk : blocks)
+        for (int gpc : gpcs) {
+          if (blk * gpc > 2048) continue;  // at most 32 waves per compute unit
+          kc_batch_tuning t{blk, gpc, 0, best.split_vertices};
+          const float ms = time_of(t);
+          if (ms < best_ms) {
+            best_ms = ms;
+            best = t;
+          }
         }
-      }
+    }
     best.use_graph = keep.use_graph;
     b->tuning = best;
     if (chosen) *chosen = best;

@@ -123,6 +123,34 @@ def test_small_rate_queues_every_graph():
         db.close()
 
 
+def test_autotune_leaves_a_shape_that_nothing_uses():
+    b = ca.batch_generate(graphs=64, log_n_min=5, log_n_max=10, seed=3)
+    want = references(b, 5, stream=ca.STREAM_HASHED)
+    db = ca.DeviceBatch(b)
+    try:
+        db.set_tuning(block=512, groups_per_cu=3, use_graph=False)  # three groups are no candidate of the search
+        t = db.autotune(seed=5, stream=ca.STREAM_HASHED)
+        assert (t["block"], t["groups_per_cu"]) == (512, 3)
+        compare(b, db, want, seed=5, stream=ca.STREAM_HASHED)
+    finally:
+        db.close()
+
+
+def test_autotune_of_queued_graphs():
+    b = queued_batch()
+    want = references(b, 5, stream=ca.STREAM_HASHED)
+    db = ca.DeviceBatch(b)
+    try:
+        t = db.autotune(seed=5, stream=ca.STREAM_HASHED)
+        assert t["block"] in (256, 512, 1024) and t["groups_per_cu"] in (1, 2, 4, 8)
+        lab, st = db.run(seed=5, stream=ca.STREAM_HASHED)
+        assert st["tuning"]["split_vertices"] == t["split_vertices"]
+        for k, w in enumerate(want):
+            assert np.array_equal(lab[int(b.vtx_off[k]):int(b.vtx_off[k + 1])], w[0]), k
+    finally:
+        db.close()
+
+
 def test_classes_run_beside_the_queue():
     def gnm(n, seed):
         return ca.generate("gnm_undirected", n=n, m=3 * n, seed=seed)
