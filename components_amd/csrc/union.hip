@@ -3,12 +3,17 @@
 // 908-922), the shortcuts variant and the components inside the blocks of the
 // pre-contraction.
 //
-// parent[v] <= v always; a root is its own parent, and only roots are hooked,
-// under a smaller root, by compare-and-swap.  So the forest has no cycles and
-// a finished tree's root is its component's smallest index.  Any parent value
-// ever read stays an ancestor, so loads may be stale (the chiplets' L2s are
+// parent[v] <= v always, so the forest has no cycles, and a root is its own parent.
+// The last pass over the edges (link) hooks roots alone, each under a smaller root
+// by compare-and-swap as in Anderson and Woll 1991, so that a finished tree's
+// root is its component's smallest index.  Any parent value ever read in that
+// pass stays an ancestor, so loads may be stale (the chiplets' L2s are
 // not coherent within a launch): a hook with a stale root fails and returns
-// the current parent, from which the search goes on downward.
+// the current parent, from which the search goes on downward.  The passes
+// ahead of it only have to keep parents within the component and below their
+// children: they start every vertex at a neighbour, as in the connected-components
+// code ECL-CC (Jaiganesh and Burtscher 2018), and replace the links of
+// vertices that may be no roots any more (hook); the last pass links every edge again.
 //
 // A few passes over the edges replace min-label sweeps with a pointer jump
 // after each, whose number grows with the diameter (2D grid 1500 x 1100, p =
@@ -70,17 +75,17 @@ __global__ __launch_bounds__(kBlock) void k_union_shorten(uint64_t n, uint32_t *
   if (p != first) parent[v] = p;
 }
 
-// Root of v; every vertex passed is pointed at its grandparent.
+// Root of v, by path halving (van Leeuwen and van der Weide 1977): two hops a
+// step, and the vertex that the step began at gets the second as its parent.
+// The store needs no atomic: it goes to a vertex that has been hooked already, so
+// no compare-and-swap on it can succeed any more, and leaves it an ancestor.
 __device__ __forceinline__ uint32_t find_root(uint32_t *parent, uint32_t v) {
-  uint32_t cur = parent[v];
-  if (cur == v) return cur;
-  uint32_t prev = v, next;
-  while (cur > (next = parent[cur])) {
-    parent[prev] = next;
-    prev = cur;
-    cur = next;
+  while (true) {
+    const uint32_t p = parent[v], q = parent[p];
+    if (p == q) return p;
+    parent[v] = q;
+    v = q;
   }
-  return cur;
 }
 
 __device__ __forceinline__ void link(uint32_t *parent, uint32_t u, uint32_t w) {
