@@ -2268,7 +2268,7 @@ int kc_find_components(kc_graph *g, const kc_options *opt, uint32_t *labels_out,
       fetch32(g, g->h_small + 5, g->small + 5, 8, next_signal(g));
       if (!out.tail) break;
       const uint32_t *info = g->h_small + 9;
-      if (info[0] == kTailFull) {  // (not seen: a hash part of the tail outgrew its table) every level the general way
+      if (info[0] == kTailFull) {  // a hash part outgrew its table (graphs made for it only): every level the general way
         use_tail = false;
         out = RunOut();
         g->arena.reset();

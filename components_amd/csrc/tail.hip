@@ -386,7 +386,7 @@ __global__ __launch_bounds__(kTailBlock) void k_tail(TailArgs a) {
                 if (seen[j] == e[j]) open &= ~(1u << j);
                 slot[j] = (slot[j] + jump[j]) & (kTable - 1);
               }
-            if (probe >= kTable) {  // cannot happen at this load
+            if (probe >= kTable) {  // the part's table is full: its hash took more than kTable of the edges
               s_full = 1;
               break;
             }
