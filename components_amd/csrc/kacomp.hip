@@ -574,8 +574,7 @@ uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t 
       if (packed)
         sweep_packed(off, col, packed, b, &g->flags[f], prev, g->stream, true, final_to);
       else
-        sweep(kSweepInPlace, false, off, col, key, key, hop, b, g->deg_inter, g->hub_inter, &g->flags[f], prev,
-              g->stream, true, final_to);
+        sweep(kSweepInPlace, off, col, key, key, hop, b, &g->flags[f], prev, g->stream, true, final_to);
       g->timer.stop(slots[i], bytes);
     }
     fetch32(g, g->h_flags, &g->flags[flag_base - check], batch + check, next_signal(g));
@@ -728,9 +727,8 @@ int dedup_buckets(kc_graph *g, uint64_t nb, const uint64_t *seg_off, const uint3
 // Level 0's cached bins in level-index order (see l0i_bins).
 Bins round0_bins(kc_graph *g, const Bins &b);
 
-// Time-stepped schedule until no vertex lies above the current round, then
-// one counting pass for the cluster-edge counts.  Returns the rounds that did
-// work (the reported "sweeps" of this schedule).
+// Time-stepped schedule until no vertex lies above the current round.  Returns
+// the rounds that did work (the reported "sweeps" of this schedule).
 uint64_t rounds_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t *off, const uint32_t *col,
                             uint64_t *key, const Bins &level_bins, const BinCfg &cfg, uint32_t &flag_base,
                             int tail_shift, bool choose_direction, bool index_round0) {
@@ -760,8 +758,7 @@ uint64_t rounds_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t
         }
         {
           TimedScope ts(g->timer, KC_K_SWEEP, 0);
-          sweep(kSweepInPlace, false, off, col, key, key, kOneHop, b, g->deg_inter, g->hub_inter,
-                &g->flags[flag_base], nullptr, g->stream);
+          sweep(kSweepInPlace, off, col, key, key, kOneHop, b, &g->flags[flag_base], nullptr, g->stream);
         }
         ++flag_base;
         ++done;
@@ -1186,14 +1183,13 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
       draw_keys(pk != nullptr);
       if (local) {
         // two synchronous min passes over the closed neighbourhood
-        // (local_contraction.h:195-274), then a counting pass on the final keys
+        // (local_contraction.h:195-274)
         for (int pass = 0; pass < 2; ++pass) {
           uint64_t *kin = pass == 0 ? g->key : g->key2;
           uint64_t *kout = pass == 0 ? g->key2 : g->key;
           KC_HIP(hipMemcpyAsync(kout, kin, n_l * 8, hipMemcpyDeviceToDevice, g->stream));
           TimedScope ts(g->timer, KC_K_SWEEP, sweep_bytes(n_l, m2_l));
-          sweep(kSweepJacobi, false, off_l, col_l, kin, kout, 0, b, g->deg_inter, g->hub_inter,
-                &g->flags[kMaxFlags - 1], nullptr, g->stream);
+          sweep(kSweepJacobi, off_l, col_l, kin, kout, 0, b, &g->flags[kMaxFlags - 1], nullptr, g->stream);
         }
         sweeps = 2;
       } else if (rounds) {

@@ -57,8 +57,7 @@ struct Bins {
 
 enum SweepMode : int {
   kSweepInPlace = 0,  // key[v] <- min(key[v], key[w] + hop), updates visible at once
-  kSweepJacobi = 1,   // kout[v] <- min over closed neighbourhood of kin (kout pre-copied)
-  kSweepCountOnly = 2  // no update: count neighbours with a different label
+  kSweepJacobi = 1    // kout[v] <- min over closed neighbourhood of kin (kout pre-copied)
 };
 
 struct DeviateArgs {
@@ -122,15 +121,14 @@ void finish_bins(Bins &b);  // computes block offsets from the counts
 
 // One binned sweep.  flag: set to 1 when a key decreased; prev_flag (may be
 // null): when it reads 0 the launch returns at once (converged earlier).
-// settled: in-place sweeps without counts skip the rows up to this distance,
+// settled: in-place sweeps skip the rows up to this distance,
 // which the caller knows to be final (-1: none).
-void sweep(int mode, bool count, const uint64_t *off, const uint32_t *col, const uint64_t *kin,
-           uint64_t *kout, uint64_t hop, const Bins &b, uint32_t *deg_inter, uint32_t *hub_inter,
-           int *flag, const int *prev_flag, hipStream_t s, bool hubs_first = false, int settled = -1);
+void sweep(int mode, const uint64_t *off, const uint32_t *col, const uint64_t *kin, uint64_t *kout, uint64_t hop,
+           const Bins &b, int *flag, const int *prev_flag, hipStream_t s, bool hubs_first = false, int settled = -1);
 // Packed keys (distance << 24 | label) for the pull sweeps of levels below
 // 2^24 vertices: init_keys_packed writes init_keys_exp's and sets *bad (0 before) when a
 // distance exceeds kPackedMaxDist - 1 or a label 24 bits; sweep_packed is
-// sweep(kSweepInPlace, no counts) over them; unpack_keys gives the 64-bit ones.
+// sweep(kSweepInPlace) over them; unpack_keys gives the 64-bit ones.
 constexpr uint32_t kPackedLabelBits = 24;
 constexpr uint32_t kPackedHop = 1u << kPackedLabelBits;
 constexpr uint32_t kPackedMaxDist = 255;

@@ -266,19 +266,17 @@ constexpr int kRelabelGather = 16;
 // graphs of small diameter most of the work of the sweeps after the third
 // (calls in sweeps: R-MAT 24 19.6 -> 11.5 ms, R-MAT 20 1.71 -> 1.29, 256^3 grid
 // 5.48 -> 4.70, random geometric 2 M 1.24 -> 1.03).
-template <int MODE, bool COUNT, int W>
+template <int MODE, int W>
 __device__ __forceinline__ bool sweep_group(const SweepArgs &a, bool active, uint32_t v, uint64_t e0,
-                                            uint64_t e1, int gl, bool hub, uint32_t chunk) {
+                                            uint64_t e1, int gl, bool hub) {
   uint64_t kv = active ? a.kin[v] : ~0ull;
   uint64_t best = kv;
-  uint32_t cnt = 0;
-  if (MODE == kSweepInPlace && !COUNT) active = active && static_cast<int>(kv >> 32) > a.settled;
+  if (MODE == kSweepInPlace) active = active && static_cast<int>(kv >> 32) > a.settled;
   if (active && !hub) {
     e0 = a.off[v];
     e1 = a.off[v + 1];
   }
   if (active) {
-    const uint32_t lv = static_cast<uint32_t>(kv);
     uint64_t e = e0 + gl;
     // kGather edges per lane per step: their neighbour ids, then their keys,
     // are all in flight together
@@ -290,44 +288,26 @@ __device__ __forceinline__ bool sweep_group(const SweepArgs &a, bool active, uin
 #pragma unroll
       for (int j = 0; j < kGather; ++j) k[j] = a.kin[c[j]];
 #pragma unroll
-      for (int j = 0; j < kGather; ++j) {
-        best = min_u64(best, k[j] + a.hop);
-        if (COUNT) cnt += static_cast<uint32_t>(k[j]) != lv;
-      }
+      for (int j = 0; j < kGather; ++j) best = min_u64(best, k[j] + a.hop);
     }
-    for (; e < e1; e += W) {
-      const uint64_t kw = a.kin[a.col[e]];
-      best = min_u64(best, kw + a.hop);
-      if (COUNT) cnt += static_cast<uint32_t>(kw) != lv;
-    }
+    for (; e < e1; e += W) best = min_u64(best, a.kin[a.col[e]] + a.hop);
   }
-  if (W > 1) {
-    best = group_min_u64(best, W);
-    if (COUNT) cnt = group_sum_u32(cnt, W);
-  }
+  if (W > 1) best = group_min_u64(best, W);
   bool changed = false;
-  if (active && gl == 0) {
-    if (MODE != kSweepCountOnly && best < kv) {
-      if (hub) {
-        uint64_t old = atomicMin(reinterpret_cast<unsigned long long *>(&a.kout[v]),
-                                 static_cast<unsigned long long>(best));
-        changed = old > best;
-      } else {
-        a.kout[v] = best;
-        changed = true;
-      }
-    }
-    if (COUNT) {
-      if (hub)
-        a.hub_inter[chunk] = cnt;
-      else
-        a.deg_inter[v] = cnt;
+  if (active && gl == 0 && best < kv) {
+    if (hub) {
+      uint64_t old = atomicMin(reinterpret_cast<unsigned long long *>(&a.kout[v]),
+                               static_cast<unsigned long long>(best));
+      changed = old > best;
+    } else {
+      a.kout[v] = best;
+      changed = true;
     }
   }
   return changed;
 }
 
-template <int MODE, bool COUNT>
+template <int MODE>
 __global__ __launch_bounds__(kBlock) void k_sweep(SweepArgs a) {
   if (a.prev_flag && *a.prev_flag == 0) return;
   uint32_t blk = blockIdx.x;
@@ -342,26 +322,24 @@ __global__ __launch_bounds__(kBlock) void k_sweep(SweepArgs a) {
     const uint32_t i = blk * kBlock + tid;
     const bool act = i < a.b.nT;
     uint32_t v = act ? a.b.listT[i] : 0;
-    changed = sweep_group<MODE, COUNT, 1>(a, act, v, 0, 0, 0, false, 0);
+    changed = sweep_group<MODE, 1>(a, act, v, 0, 0, 0, false);
   } else if (blk < a.b.bW) {
     const uint32_t i = (blk - a.b.bS) * (kBlock / 16) + tid / 16;
     const bool act = i < a.b.nS;
     uint32_t v = act ? a.b.listS[i] : 0;
-    changed = sweep_group<MODE, COUNT, 16>(a, act, v, 0, 0, tid & 15, false, 0);
+    changed = sweep_group<MODE, 16>(a, act, v, 0, 0, tid & 15, false);
   } else if (blk < a.b.bH) {
     const uint32_t i = (blk - a.b.bW) * (kBlock / kWave) + tid / kWave;
     const bool act = i < a.b.nW;
     uint32_t v = act ? a.b.listW[i] : 0;
-    changed = sweep_group<MODE, COUNT, kWave>(a, act, v, 0, 0, tid & 63, false, 0);
+    changed = sweep_group<MODE, kWave>(a, act, v, 0, 0, tid & 63, false);
   } else {
     const uint32_t i = (blk - a.b.bH) * (kBlock / kWave) + tid / kWave;
     const bool act = i < a.b.nH;
     HubChunk h = act ? a.b.hubs[i] : HubChunk{0, 0, 0, 0};
-    changed = sweep_group<MODE, COUNT, kWave>(a, act, h.v, h.e0, h.e1, tid & 63, true, i);
+    changed = sweep_group<MODE, kWave>(a, act, h.v, h.e0, h.e1, tid & 63, true);
   }
-  if (MODE != kSweepCountOnly) {
-    if (__ballot(changed) != 0 && lane_id() == 0) *a.flag = 1;
-  }
+  if (__ballot(changed) != 0 && lane_id() == 0) *a.flag = 1;
 }
 
 // Packed keys for the pull sweeps of levels below 2^24 vertices whose key
@@ -2499,20 +2477,14 @@ void finish_bins(Bins &b) {
   b.blocks = b.bH + blocksH;
 }
 
-void sweep(int mode, bool count, const uint64_t *off, const uint32_t *col, const uint64_t *kin, uint64_t *kout,
-           uint64_t hop, const Bins &b, uint32_t *deg_inter, uint32_t *hub_inter, int *flag, const int *prev_flag,
-           hipStream_t s, bool hubs_first, int settled) {
+void sweep(int mode, const uint64_t *off, const uint32_t *col, const uint64_t *kin, uint64_t *kout, uint64_t hop,
+           const Bins &b, int *flag, const int *prev_flag, hipStream_t s, bool hubs_first, int settled) {
   if (b.blocks == 0) return;
-  SweepArgs a{off, col, kin, kout, hop, b, deg_inter, hub_inter, flag, prev_flag, hubs_first ? 1 : 0, settled};
-  dim3 g(b.blocks), t(kBlock);
-  if (mode == kSweepInPlace && count)
-    hipLaunchKernelGGL((k_sweep<kSweepInPlace, true>), g, t, 0, s, a);
-  else if (mode == kSweepInPlace)
-    hipLaunchKernelGGL((k_sweep<kSweepInPlace, false>), g, t, 0, s, a);
-  else if (mode == kSweepJacobi)
-    hipLaunchKernelGGL((k_sweep<kSweepJacobi, false>), g, t, 0, s, a);
+  SweepArgs a{off, col, kin, kout, hop, b, nullptr, nullptr, flag, prev_flag, hubs_first ? 1 : 0, settled};
+  if (mode == kSweepInPlace)
+    hipLaunchKernelGGL(k_sweep<kSweepInPlace>, dim3(b.blocks), dim3(kBlock), 0, s, a);
   else
-    hipLaunchKernelGGL((k_sweep<kSweepCountOnly, true>), g, t, 0, s, a);
+    hipLaunchKernelGGL(k_sweep<kSweepJacobi>, dim3(b.blocks), dim3(kBlock), 0, s, a);
   KC_LAUNCH_CHECK();
 }
 

@@ -43,10 +43,8 @@ constexpr uint64_t kHubCap = kMaxSlots / (kMinWaveBin / 2) + 2;  // hub_chunk_ca
 // Byte offsets of the regions inside `scratch`.
 constexpr uint64_t kKeyAt = 0;                                                  // u64[n]
 constexpr uint64_t kListsAt = align256(kKeyAt + 8 * kMaxVertices);              // u32[3n]
-constexpr uint64_t kDegAt = align256(kListsAt + 12 * kMaxVertices);             // u32[n]
-constexpr uint64_t kHubsAt = align256(kDegAt + 4 * kMaxVertices);               // HubChunk[kHubCap]
-constexpr uint64_t kHubInterAt = align256(kHubsAt + sizeof(HubChunk) * kHubCap);  // u32[kHubCap]
-constexpr uint64_t kFlagsAt = align256(kHubInterAt + 4 * kHubCap);              // int[kFlagSlots]
+constexpr uint64_t kHubsAt = align256(kListsAt + 12 * kMaxVertices);            // HubChunk[kHubCap]
+constexpr uint64_t kFlagsAt = align256(kHubsAt + sizeof(HubChunk) * kHubCap);   // int[kFlagSlots]
 constexpr uint64_t kSmallAt = align256(kFlagsAt + 4 * kFlagSlots);              // u32[16]: [0..3] bin counts, roots, [8..12] binning's counters
 constexpr uint64_t kPartialAt = align256(kSmallAt + 64);                        // u32[n/256 + 64]
 constexpr uint64_t kScratchBytes = align256(kPartialAt + 4 * (kMaxVertices / kBlock + 64));
@@ -85,9 +83,7 @@ uint64_t propagate(uint64_t n, const uint64_t *offsets, const uint32_t *targets,
                    uint32_t *labels, hipStream_t s) {
   uint64_t *key = region<uint64_t>(base, kKeyAt);
   uint32_t *lists = region<uint32_t>(base, kListsAt);
-  uint32_t *deg_inter = region<uint32_t>(base, kDegAt);
   HubChunk *hubs = region<HubChunk>(base, kHubsAt);
-  uint32_t *hub_inter = region<uint32_t>(base, kHubInterAt);
   int *flags = region<int>(base, kFlagsAt);
   uint32_t *small = region<uint32_t>(base, kSmallAt);
   // degree bins of the graph (as make_bins does for this variant)
@@ -98,7 +94,7 @@ uint64_t propagate(uint64_t n, const uint64_t *offsets, const uint32_t *targets,
   b.listW = lists + 2 * n;
   b.hubs = hubs;
   fill_u32(small, 16, 0, s);
-  bin_vertices(n, offsets, cfg, b.listT, b.listS, b.listW, b.hubs, small + 8, small, deg_inter, s);
+  bin_vertices(n, offsets, cfg, b.listT, b.listS, b.listW, b.hubs, small + 8, small, nullptr, s);
   uint32_t counts[4];
   KC_HIP(hipMemcpyAsync(counts, small, sizeof(counts), hipMemcpyDeviceToHost, s));
   KC_HIP(hipStreamSynchronize(s));
@@ -123,7 +119,7 @@ uint64_t propagate(uint64_t n, const uint64_t *offsets, const uint32_t *targets,
     for (uint32_t i = 0; i < batch; ++i) {
       const uint32_t f = flag_base + i;
       const int *prev = i == 0 ? nullptr : &flags[f - 1];
-      sweep(kSweepInPlace, false, offsets, targets, key, key, 0, b, deg_inter, hub_inter, &flags[f], prev, s);
+      sweep(kSweepInPlace, offsets, targets, key, key, 0, b, &flags[f], prev, s);
     }
     int h_flags[8];
     KC_HIP(hipMemcpyAsync(h_flags, &flags[flag_base], batch * sizeof(int), hipMemcpyDeviceToHost, s));
