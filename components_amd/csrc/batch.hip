@@ -819,6 +819,13 @@ struct LdsClass {
 };
 constexpr int kLdsClasses = 4;
 constexpr LdsClass kLdsClass[kLdsClasses] = {{1024, 4096}, {2048, 12288}, {4096, 30592}, {8192, ~0u}};
+// The smallest class that holds a graph of n vertices and `edges` edges; kLdsClasses:
+// none does.
+int lds_class(uint64_t n, uint64_t edges) {
+  int cls = 0;
+  while (cls < kLdsClasses && (n > kLdsClass[cls].n || edges > kLdsClass[cls].edges)) ++cls;
+  return cls;
+}
 // packed keys: the distances (at most k_max + 1) and 13 label bits share 32
 constexpr uint32_t kLdsMaxDeviate = (1u << 19) - 2;
 
@@ -848,6 +855,8 @@ void batch_table_clear(uint64_t n, uint64_t *tab, hipStream_t s) {
 // Host side.
 using namespace kc;
 
+constexpr size_t kFiguresAt = (sizeof(BatchParams) + 127) / 128 * 128;  // in the pinned memory of a batch
+
 struct kc_batch {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -872,7 +881,8 @@ struct kc_batch {
   uint64_t *d_uoff = nullptr, *d_ueoff = nullptr;
   BatchDev dev{};
   BatchParams *d_params = nullptr, *h_params = nullptr;
-  uint32_t *h_figures = nullptr;  // pinned: the last run's gstatus, glevels, gsweeps, gradius, gcomp (graphs each)
+  // pinned, behind h_params: the last run's gstatus, glevels, gsweeps, gradius, gcomp (graphs each)
+  uint32_t *h_figures = nullptr;
   uint64_t *table = nullptr;
   uint64_t table_words = 0;
   uint32_t *queue = nullptr;
@@ -884,7 +894,7 @@ struct kc_batch {
   hipGraphExec_t exec = nullptr;
   kc_batch_tuning exec_tuning{0, 0, 0, 0};
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  hipStream_t side = nullptr;  // for every other class of small graphs
+  hipStream_t side = nullptr;  // for size classes, where the graphs are of more than one kind
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   bool ran = false;
 
@@ -905,7 +915,6 @@ struct kc_batch {
     if (exec) (void)hipGraphExecDestroy(exec);
     for (void *p : owned) (void)hipFree(p);
     if (h_params) (void)hipHostFree(h_params);
-    if (h_figures) (void)hipHostFree(h_figures);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (ev_fork) (void)hipEventDestroy(ev_fork);
@@ -962,8 +971,7 @@ void prepare_split(kc_batch *b, uint32_t split) {
   std::vector<uint32_t> small, bigs, fits[kLdsClasses];
   for (uint32_t g = 0; g < b->graphs; ++g) {
     const uint64_t ng = b->h_vtx_off[g + 1] - b->h_vtx_off[g];
-    int cls = 0;
-    while (cls < kLdsClasses && (ng > kLdsClass[cls].n || b->h_up[g] > kLdsClass[cls].edges)) ++cls;
+    const int cls = lds_class(ng, b->h_up[g]);
     (split && ng > split ? bigs : lds && cls < kLdsClasses ? fits[cls] : small).push_back(g);
   }
   const auto larger = [&](uint32_t x, uint32_t y) {
@@ -1206,10 +1214,10 @@ int kc_batch_create(const kc_batch_host *h, kc_batch **out) {
     KC_HIP(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
     KC_HIP(hipEventCreate(&b->ev0));
     KC_HIP(hipEventCreate(&b->ev1));
-    KC_HIP(hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking));
-    KC_HIP(hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming));
-    KC_HIP(hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming));
-    KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&b->h_params), sizeof(BatchParams), hipHostMallocDefault));
+    void *pinned = nullptr;
+    KC_HIP(hipHostMalloc(&pinned, kFiguresAt + 20ull * G, hipHostMallocDefault));
+    b->h_params = static_cast<BatchParams *>(pinned);
+    b->h_figures = reinterpret_cast<uint32_t *>(static_cast<char *>(pinned) + kFiguresAt);
     b->graphs = G;
     b->n = n;
     b->m2 = m2;
@@ -1217,6 +1225,15 @@ int kc_batch_create(const kc_batch_host *h, kc_batch **out) {
     for (uint32_t g = 0; g < G; ++g) b->largest = std::max(b->largest, h->vtx_off[g + 1] - h->vtx_off[g]);
     b->h_edge_off.assign(h->edge_off, h->edge_off + G + 1);
     b->h_up = std::move(up);
+    // What a run launches side by side is at most these kinds, whatever the
+    // split and the rate.  (A stream and two events: 40 us of a small batch's 900.)
+    uint32_t kinds = 0;
+    for (uint32_t g = 0; g < G; ++g) kinds |= 1u << lds_class(h->vtx_off[g + 1] - h->vtx_off[g], b->h_up[g]);
+    if (kinds & (kinds - 1)) {
+      KC_HIP(hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking));
+      KC_HIP(hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming));
+      KC_HIP(hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming));
+    }
     BatchDev &d = b->dev;
     d.graphs = G;
     uint32_t *order_d = b->dalloc<uint32_t>(G);
@@ -1260,7 +1277,6 @@ int kc_batch_create(const kc_batch_host *h, kc_batch **out) {
     d.gsweeps = d.glevels + G;
     d.gradius = d.gsweeps + G;
     d.gcomp = d.gradius + G;
-    KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&b->h_figures), 20ull * G + 64, hipHostMallocDefault));
     b->queue = b->dalloc<uint32_t>(1);
     d.queue = b->queue;
     b->d_params = b->dalloc<BatchParams>(1);

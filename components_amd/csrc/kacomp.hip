@@ -275,6 +275,14 @@ struct kc_graph {
   uint64_t *sums = nullptr;
   uint64_t *sizes = nullptr;  // [0] n_next [1] P [2] m2_next [3..5] dedup counters [9] clusters
   // pinned host mirrors
+  // (one allocation: giving four back took some 80 us more of a tiny graph's 750)
+  struct HostWordsArea {
+    uint64_t sizes[16];
+    uint32_t small[16];
+    int flags[64];
+    alignas(128) uint32_t signal;
+  };
+  HostWordsArea *h_area = nullptr;
   uint64_t *h_sizes = nullptr;
   uint32_t *h_small = nullptr;
   uint32_t *h_signal = nullptr;  // the last signal that arrived (next_signal, await)
@@ -369,10 +377,7 @@ struct kc_graph {
     if (stream) (void)hipStreamSynchronize(stream);
     for (void *p : work_owned) (void)hipFree(p);
     for (void *p : owned) (void)hipFree(p);
-    if (h_sizes) (void)hipHostFree(h_sizes);
-    if (h_small) (void)hipHostFree(h_small);
-    if (h_signal) (void)hipHostFree(h_signal);
-    if (h_flags) (void)hipHostFree(h_flags);
+    if (h_area) (void)hipHostFree(h_area);
     if (ev_begin) (void)hipEventDestroy(ev_begin);
     if (ev_end) (void)hipEventDestroy(ev_end);
     if (stream) (void)hipStreamDestroy(stream);
@@ -1510,15 +1515,16 @@ std::unique_ptr<kc_graph> new_handle() {
   KC_HIP(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
   KC_HIP(hipEventCreate(&g->ev_begin));
   KC_HIP(hipEventCreate(&g->ev_end));
-  KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_sizes), 16 * sizeof(uint64_t), hipHostMallocCoherent));
-  KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_small), 16 * sizeof(uint32_t), hipHostMallocCoherent));
-  KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_signal), sizeof(uint32_t), hipHostMallocCoherent));
+  KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_area), sizeof(*g->h_area), hipHostMallocCoherent));
+  g->h_sizes = g->h_area->sizes;
+  g->h_small = g->h_area->small;
+  g->h_flags = g->h_area->flags;
+  g->h_signal = &g->h_area->signal;
   *g->h_signal = 0;
-  KC_HIP(hipHostMalloc(reinterpret_cast<void **>(&g->h_flags), 64 * sizeof(int), hipHostMallocCoherent));
-  g->small = g->dalloc<uint32_t>(16);
-  g->sizes = g->dalloc<uint64_t>(16);
-  g->tickets = g->dalloc<uint32_t>(8);
-  g->sums = g->dalloc<uint64_t>(4);
+  g->sizes = g->dalloc<uint64_t>(4 * 32);  // 256 bytes each
+  g->small = reinterpret_cast<uint32_t *>(g->sizes + 32);
+  g->tickets = reinterpret_cast<uint32_t *>(g->sizes + 64);
+  g->sums = g->sizes + 96;
   fill_u32(g->tickets, 8, 0, g->stream);
   fill_u64(g->sums, 4, 0, g->stream);
   return g;
