@@ -2341,6 +2341,7 @@ int kc_graph_autotune(kc_graph *g, const kc_options *opt, kc_bin_tuning *chosen)
     // one lane, 16 lanes, one wave (and the hub chunk size): the defaults and
     // their neighbours by factors of 2 to 4
     const int32_t smalls[] = {8, 16, 32}, mids[] = {128, 256, 512}, larges[] = {1024, 4096, 16384};
+    bool binned = false;  // some launch of the calls went over bins
     auto time_of = [&](int32_t a, int32_t b, int32_t c) {
       kc_options t = o;
       t.sweep_group_small = a;
@@ -2353,6 +2354,7 @@ int kc_graph_autotune(kc_graph *g, const kc_options *opt, kc_bin_tuning *chosen)
         const int rc = kc_find_components(g, &t, nullptr, &st);
         if (rc != KC_OK) throw Failure{rc};
         if (rep) sum += st.time_ms;  // the first call warms the bins and buffers
+        for (int cls : {KC_K_SWEEP, KC_K_ROUND, KC_K_RELABEL, KC_K_SCATTER}) binned |= st.kernel_launches[cls] != 0;
       }
       return sum / 2;
     };
@@ -2372,8 +2374,10 @@ int kc_graph_autotune(kc_graph *g, const kc_options *opt, kc_bin_tuning *chosen)
             bl = c;
           }
         }
-    // a choice within 2% of the defaults is run-to-run noise: keep the defaults
-    if (best > 0.98 * def_ms) {
+    // a choice within 2% of the defaults is run-to-run noise, and any choice is
+    // where the thresholds served no launch (a level small enough for one
+    // workgroup, shortcuts): keep the defaults
+    if (!binned || best > 0.98 * def_ms) {
       best = def_ms;
       bs = 16;
       bm = 256;
