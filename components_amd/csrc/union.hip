@@ -75,17 +75,21 @@ __global__ __launch_bounds__(kBlock) void k_union_shorten(uint64_t n, uint32_t *
   if (p != first) parent[v] = p;
 }
 
-// Root of v, by path halving (van Leeuwen and van der Weide 1977): two hops a
-// step, and the vertex that the step began at gets the second as its parent.
-// The store needs no atomic: it goes to a vertex that has been hooked already, so
-// no compare-and-swap on it can succeed any more, and leaves it an ancestor.
+// Root of v, by path splitting (Tarjan and van Leeuwen 1984): every vertex on the
+// way gets its parent's parent for its own.  The store needs no atomic: it goes to
+// a vertex that has been hooked already, so no compare-and-swap on it can succeed
+// any more, and leaves it an ancestor.  (Path halving, a store every other
+// vertex: a path of 10 000 in index order 180 -> 130 us, G(1000, 2000) 34 -> 37,
+// G(10 000, 10 000) 60 -> 64.)
 __device__ __forceinline__ uint32_t find_root(uint32_t *parent, uint32_t v) {
-  while (true) {
-    const uint32_t p = parent[v], q = parent[p];
-    if (p == q) return p;
-    parent[v] = q;
-    v = q;
+  uint32_t p = parent[v];
+  if (p == v) return v;
+  for (uint32_t above = parent[p]; above != p; above = parent[p]) {
+    parent[v] = above;
+    v = p;
+    p = above;
   }
+  return p;
 }
 
 __device__ __forceinline__ void link(uint32_t *parent, uint32_t u, uint32_t w) {
