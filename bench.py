@@ -41,7 +41,8 @@ def parse():
     ap.add_argument("--edge-factor", type=int, default=16)
     ap.add_argument("--stream", choices=["hashed", "reference"], default="hashed")
     ap.add_argument("--schedule", choices=["rounds", "sweeps"], default="rounds",
-                    help="rounds: time-stepped push (each edge pushed once); sweeps: in-place pull sweeps")
+                    help="rounds: time-stepped push (each edge pushed once) on large skewed levels, or with "
+                         "--tail-sweeps or --pull-rounds on all; sweeps: in-place pull sweeps")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline and the label check")
     ap.add_argument("--cpu-scale", type=int, default=24,
                     help="R-MAT scale of the CPU baseline's graph (the bench workload's scale by default)")
@@ -284,8 +285,10 @@ def forms_leg(a, dg, run_kw, m):
 def configs_leg(a, stream, run_kw):
     """The plain form on the other workloads: G(n,m) n = 2^20, m = 2^22, seed 1;
     3D grid 256^3 with every bond kept with probability 0.3, seed 2; 2D random
-    geometric graph n = 2^24 at average degree 8, seed 2.  Labels are checked
-    against the oracle's union-find."""
+    geometric graph n = 2^24 at average degree 8, seed 2.  In the schedule that
+    use_bfs picks by itself (rounds on large skewed levels alone), in rounds on
+    every level (tail_sweeps given: 3 is the default cut-over) and in sweeps.
+    Labels are checked against the oracle's union-find."""
     import numpy as np
 
     import components_amd as ca
@@ -307,8 +310,11 @@ def configs_leg(a, stream, run_kw):
         m = dg.m
         seq = max(m // 256, 4096)
         res = {"n": dg.n, "m": m}
-        for sched, bfs in (("rounds", True), ("sweeps", False)):
-            kw2 = dict(run_kw, seq_limit=seq, use_bfs=bfs)
+        for sched, opts in (("bfs", dict(use_bfs=True)),
+                            ("rounds", dict(use_bfs=True, tail_sweeps=a.tail_sweeps or 3)),
+                            ("sweeps", dict(use_bfs=False))):
+            kw2 = dict(run_kw, seq_limit=seq)
+            kw2.update(opts)
             for i in range(a.warmup):
                 dg.find_components(copy_labels=False, seed=1 + i + 1000, **kw2)
             sts = []
@@ -327,8 +333,8 @@ def configs_leg(a, stream, run_kw):
         dg.close()
         del host
         out[label] = res
-        print(f"[bench] {label}: rounds {res['rounds']['ms_per_step']:.2f} ms, sweeps {res['sweeps']['ms_per_step']:.2f} ms,"
-              f" exact {res['labels_bit_exact']} ({time.time() - t0:.1f}s)", file=sys.stderr, flush=True)
+        print(f"[bench] {label}: -bfs {res['bfs']['ms_per_step']:.2f} ms, rounds {res['rounds']['ms_per_step']:.2f} ms, "
+              f"sweeps {res['sweeps']['ms_per_step']:.2f} ms, exact {res['labels_bit_exact']} ({time.time() - t0:.1f}s)", file=sys.stderr, flush=True)
     return out
 
 

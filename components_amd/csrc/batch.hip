@@ -428,7 +428,7 @@ __global__ __launch_bounds__(B) void k_batch(BatchDev d) {
 // (a repeated edge changes no key, label or level).  What bounds it: LDS
 // accesses and the barriers between the phases; the general kernel above pays
 // a chain of L2 or HBM round trips per phase instead (4096 graphs of 2^8 to
-// 2^12 vertices: 4.53 ms, here 0.81).
+// 2^12 vertices: 4.53 ms, here 0.69).
 template <int B, uint32_t CapN, uint32_t CapE>
 struct LdsGraph {
   uint32_t key[CapN];  // packed keys; the filter while the edges contract
@@ -811,9 +811,10 @@ void batch_launch(int block, uint32_t grid, const BatchDev &d, hipStream_t s) {
   KC_LAUNCH_CHECK();
 }
 
-// Size classes of the LDS kernel: (threads, vertices, undirected edges).  The
-// LDS of one class is what bounds its workgroups per CU: 6, 2, 1 and 2
-// (the last streams its edges: any number).
+// Size classes of the LDS kernel: (vertices, undirected edges).  LDS bounds the
+// workgroups per CU: 27, 70, 164 and 82 KB leave 6, 2, 1 and 1 of 4, 8, 16 and 16
+// waves.  The last streams its edges, any number, and misses a second workgroup
+// by its registers too: 112 a lane let 4 waves share a SIMD, which are its own.
 struct LdsClass {
   uint32_t n, edges;
 };
@@ -961,7 +962,7 @@ void batch_params(kc_batch *b, const kc_options &o) {
 
 // Routes the graphs with more than `split` vertices (none when 0) to the
 // device-wide path; of the others, those that fit an LDS class go to the
-// smallest one (4096 graphs of 2^8 to 2^12 vertices: 4.5 -> 0.81 ms),
+// smallest one (4096 graphs of 2^8 to 2^12 vertices: 4.5 -> 0.69 ms),
 // the rest to the persistent kernel's queue, each list largest first.  The
 // large ones are copied into one union handle.
 void prepare_split(kc_batch *b, uint32_t split) {

@@ -219,7 +219,9 @@ typedef struct kc_stats {
   uint64_t n, m;        /* vertices, undirected edges of the input */
   uint32_t levels;      /* contraction levels (decompositions) executed */
   uint32_t components;  /* number of connected components (isolated vertices count) */
-  uint64_t sweeps;      /* sum over levels of sweeps executed */
+  uint64_t sweeps;      /* sum over levels of sweeps or rounds executed (in-place sweeps: varies from call to
+                           call); the last, small levels count their passes over the edges, a base case by
+                           union-find and the shortcuts variant one */
   uint64_t radius_sum;  /* sum over levels of the maximum cluster radius */
   uint64_t alg_bytes;   /* algorithmic bytes of all launched kernels */
   double kernel_ms[KC_KERNEL_CLASSES];        /* valid with time_kernels */
