@@ -103,30 +103,54 @@ __device__ __forceinline__ void link(uint32_t *parent, uint32_t u, uint32_t w) {
   }
 }
 
-// Hooks the larger of the two ends' parents under the smaller one without a
+// Hooks the larger of two ends' parents, a and b, under the smaller one without a
 // search: trees that are stars (or nearly) merge in one step each.  Where the
 // larger is no root any more its link is replaced; every edge is linked again
 // by the last pass, so nothing is lost.
-__device__ __forceinline__ void hook(uint32_t *parent, uint32_t u, uint32_t w) {
-  const uint32_t a = parent[u], b = parent[w];
+__device__ __forceinline__ void hook(uint32_t *parent, uint32_t a, uint32_t b) {
   if (a == b) return;
   const uint32_t hi = a > b ? a : b, lo = a > b ? b : a;
   if (parent[hi] > lo) atomicMin(&parent[hi], lo);
 }
 
+// Hooks along four edges of every row, other ones in either round (a shorter row:
+// all).
+__global__ __launch_bounds__(kBlock) void k_union_hook_rows(uint64_t n, const uint64_t *off, const uint32_t *col,
+                                                           uint64_t block, uint32_t *parent, uint32_t round) {
+  constexpr uint64_t kSamples = 4;
+  const uint64_t v = blockIdx.x * static_cast<uint64_t>(kBlock) + threadIdx.x;
+  if (v >= n) return;
+  const uint32_t self = static_cast<uint32_t>(v);
+  const uint64_t e0 = off[v], len = off[v + 1] - e0;
+  uint32_t c[kSamples], p[kSamples];
+#pragma unroll
+  for (uint64_t j = 0; j < kSamples; ++j) {
+    const uint64_t i = len <= kSamples ? j : len * (2 * j + 1 + round) / (2 * kSamples + 2);
+    c[j] = i < len ? col[e0 + i] : self;
+  }
+  const uint32_t own = parent[v];
+#pragma unroll
+  for (uint64_t j = 0; j < kSamples; ++j) p[j] = same_block(c[j], self, block) ? parent[c[j]] : own;
+#pragma unroll
+  for (uint64_t j = 0; j < kSamples; ++j) hook(parent, own, p[j]);
+}
+
 // Links (or, with kHook, hooks) the two ends of every edge, from its larger
-// end's row.
+// end's row; with every > 1, of the edges in each every-th share of a wave's slots,
+// from share `first` on.
 template <bool kHook>
 __global__ __launch_bounds__(kBlock) void k_union_link(uint64_t n, uint64_t m2, const uint64_t *off,
-                                                      const uint32_t *col, uint64_t block, uint32_t *parent) {
+                                                      const uint32_t *col, uint64_t block, uint32_t *parent,
+                                                      uint32_t every, uint32_t first) {
   __shared__ uint32_t row_lds[kBlock / kWave][kWaveSlots];
-  const uint64_t c0 = (blockIdx.x * static_cast<uint64_t>(kBlock / kWave) + threadIdx.x / kWave) * kWaveSlots;
+  const uint64_t share = blockIdx.x * static_cast<uint64_t>(kBlock / kWave) + threadIdx.x / kWave;
+  const uint64_t c0 = (share * every + first) * kWaveSlots;
   if (c0 >= m2) return;
   const uint64_t c1 = c0 + kWaveSlots < m2 ? c0 + kWaveSlots : m2;
   for_wave_slots(n, off, col, c0, c1, row_lds[threadIdx.x / kWave], [&](uint32_t, uint32_t v, uint32_t w) {
     if (w < v && same_block(w, v, block)) {
       if (kHook)
-        hook(parent, v, w);
+        hook(parent, parent[v], parent[w]);
       else
         link(parent, v, w);
     }
@@ -170,24 +194,38 @@ __global__ __launch_bounds__(kBlock) void k_union_labels(uint64_t n, const uint3
 
 unsigned blocks_for(uint64_t n) { return static_cast<unsigned>(ceil_div(n, static_cast<uint64_t>(kBlock))); }
 
-void shorten(uint64_t n, uint32_t *parent, hipStream_t s) {
+void shorten(uint64_t n, uint32_t *parent, hipStream_t s, bool again = true) {
   // (a path of 2^20 vertices in index order is the worst case: two passes
   // before the links and two after leave about a thousand hops to the search)
-  for (int pass = 0; pass < (n >= kShortenTwiceMin ? 2 : 1); ++pass) {
+  for (int pass = 0; pass < (again && n >= kShortenTwiceMin ? 2 : 1); ++pass) {
     hipLaunchKernelGGL(k_union_shorten, dim3(blocks_for(n)), dim3(kBlock), 0, s, n, parent);
     KC_LAUNCH_CHECK();
   }
 }
 
-// Rounds of hooks before the links.  The links of many neighbouring trees wait
-// for one another along chains of roots (2D grid 1500 x 1100, p = 0.6: 940 us
-// in all with no hooks, 641, 692, 214 and 236 with 1 to 4 rounds; G(n, 3n) of
-// 200 K vertices: 787, 970, 143, 156); small graphs are done sooner without
-// (10 K vertices: 56 against 63 us), and on dense ones the first neighbours'
-// minima have left few trees (R-MAT 20, 30 slots a vertex: 330, 392, 516 us).
-int hook_rounds(uint64_t n, uint64_t m2) {
-  if (n < (1u << 14) || m2 > 16 * n) return 0;
-  return n < (1u << 20) ? 2 : 3;
+// Rounds of hooks before the links: along four edges of every row (rows), or
+// along the edges of each every-th share (shares).  The links of many
+// neighbouring trees wait for one another along chains of roots, so the hooks
+// have to leave few trees; and a round costs its launches, which counts on small
+// graphs.  Shortcuts calls on the device in us:
+//   below 2^14 vertices, with no round and with two of rows (two full ones take
+//   as long or longer): G(16 000, 10 n) 168 -> 64, G(4000, 4 n) 54 -> 51, a path of
+//   16 000 in index order 222 -> 46, 2D grid 60^2 49 -> 45, R-MAT 13 31 -> 34, a clique
+//   of 1500 21 -> 29;
+//   above 16 slots a vertex, with no round, one and two full ones, and two of an
+//   eighth: G(n, 10 n) of 60 000 vertices 413, 81, 84, 89; of 200 000 1468, 146, 157,
+//   122; G(n, 20 n) of 10^6 940, 528, 677, 441; R-MAT 20 328, 394, 526, 322; random
+//   geometric 10^6 328, 201, -, 172;
+//   elsewhere by the number of full rounds, from none: 2D grid 1500 x 1100, p = 0.6:
+//   940, 641, 692, 214, 236; G(n, 3n) of 200 000 vertices 787, 970, 143, 156.
+struct HookRounds {
+  int rows, shares;
+  uint32_t every;
+};
+HookRounds hook_rounds(uint64_t n, uint64_t m2) {
+  if (n < (1u << 14)) return {2, 0, 1};
+  if (m2 > 16 * n) return {0, 2, 8};
+  return {0, n < (1u << 19) ? 2 : 3, 1};
 }
 
 }  // namespace
@@ -198,14 +236,24 @@ void union_components(uint64_t n, uint64_t m2, const uint64_t *off, const uint32
   hipLaunchKernelGGL(k_union_init, dim3(blocks_for(n)), dim3(kBlock), 0, s, n, off, col, block, parent);
   KC_LAUNCH_CHECK();
   if (!m2) return;
-  const unsigned g = static_cast<unsigned>(ceil_div(m2, static_cast<uint64_t>(kWaveSlots) * (kBlock / kWave)));
+  const auto share_blocks = [&](uint32_t every) {
+    return dim3(static_cast<unsigned>(ceil_div(m2, static_cast<uint64_t>(kWaveSlots) * (kBlock / kWave) * every)));
+  };
+  const HookRounds rounds = hook_rounds(n, m2);
   shorten(n, parent, s);
-  for (int r = 0; r < hook_rounds(n, m2); ++r) {
-    hipLaunchKernelGGL(k_union_link<true>, dim3(g), dim3(kBlock), 0, s, n, m2, off, col, block, parent);
+  for (int r = 0; r < rounds.rows; ++r) {
+    hipLaunchKernelGGL(k_union_hook_rows, dim3(blocks_for(n)), dim3(kBlock), 0, s, n, off, col, block, parent,
+                       static_cast<uint32_t>(r));
     KC_LAUNCH_CHECK();
     shorten(n, parent, s);
   }
-  hipLaunchKernelGGL(k_union_link<false>, dim3(g), dim3(kBlock), 0, s, n, m2, off, col, block, parent);
+  for (int r = 0; r < rounds.shares; ++r) {
+    hipLaunchKernelGGL(k_union_link<true>, share_blocks(rounds.every), dim3(kBlock), 0, s, n, m2, off, col, block,
+                       parent, rounds.every, rounds.every > 1 ? static_cast<uint32_t>(r) : 0u);
+    KC_LAUNCH_CHECK();
+    shorten(n, parent, s, rounds.every == 1);  // (dense graphs' trees are shallow)
+  }
+  hipLaunchKernelGGL(k_union_link<false>, share_blocks(1), dim3(kBlock), 0, s, n, m2, off, col, block, parent, 1u, 0u);
   KC_LAUNCH_CHECK();
   shorten(n, parent, s);
 }
