@@ -983,7 +983,6 @@ bool build_replicated(kc_graph *g, const kc_options *o, uint64_t n0, uint64_t m2
   return true;
 }
 
-// Exponential (or local) contraction down to an edgeless graph or the base case.
 // Levels whose rest runs in one workgroup.  A pass over the edges takes one CU
 // about 0.14 us per thousand, the general path some 0.3 ms per level whatever
 // its size.  Whole calls, default schedule / rounds, general path and this (us):
@@ -991,11 +990,19 @@ bool build_replicated(kc_graph *g, const kc_options *o, uint64_t n0, uint64_t m2
 // 914 -> 206; 16 K, 120 K 1180 -> 453 / 838 -> 384; 16 K, 240 K 1428 -> 771 /
 // 638 -> 599; 32 K, 40 K 1556 -> 439 / 1104 -> 356; 32 K, 125 K 2392 -> 903 /
 // 910 -> 624.  With 250 K edges at 32 K vertices the rounds lost (1065 -> 1148).
-bool tail_fits(uint64_t n, uint64_t m2, bool local) {
-  if (n <= kTailSmall) return m2 <= kTailSlots;
-  return !local && n <= kTailVertices && m2 <= kTailBigSlots;
+// Above 2^18 slots two kinds of graph stay out, which the general path is done
+// with sooner: the local variant's where two passes merge nearly everything (1000
+// vertices, 262 K edges 150 against 228; 2000 152, 252; but 8000 435, 423), and,
+// above 4096 vertices, cut-offs that take several hash parts to count against
+// (seq_limit m / 3, 8000 vertices, 220 K edges 763 against 1097; 16 K 785, 1290).
+bool tail_fits(uint64_t n, uint64_t m2, bool local, uint64_t seq_limit) {
+  if (n > kTailSmall) return !local && n <= kTailVertices && m2 <= kTailBigSlots;
+  if (m2 <= kTailBigSlots) return true;
+  if (m2 > kTailSlots || (local && m2 > 128 * n)) return false;
+  return n <= 4096 || seq_limit <= kTailCountOnce;
 }
 
+// Exponential (or local) contraction down to an edgeless graph or the base case.
 // use_tail: the last levels, where small enough, in one workgroup.
 void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tail) {
   const bool local = o->variant == KC_VARIANT_LOCAL;
@@ -1084,7 +1091,7 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
       top_from_keys = true;
       break;
     }
-    if (use_tail && !pre && pre_left == 0 && !idx_l && tail_fits(n_l, m2_l, local) &&
+    if (use_tail && !pre && pre_left == 0 && !idx_l && tail_fits(n_l, m2_l, local, o->seq_limit) &&
         (local || g->table_k <= kTailMaxDeviate)) {
       TailArgs t{};
       t.n = static_cast<uint32_t>(n_l);

@@ -175,6 +175,7 @@ constexpr uint64_t kTailVertices = 32768;     // 128 KB of LDS: a key per vertex
 constexpr uint64_t kTailSmall = 16128;        // ... two keys per vertex (the local variant's)
 constexpr uint64_t kTailSlots = 1u << 19;     // edge slots of up to kTailSmall vertices
 constexpr uint64_t kTailBigSlots = 1u << 18;  // ... of more
+constexpr uint64_t kTailCountOnce = 11808;    // cut-offs up to here are counted against in one table
 constexpr uint32_t kTailMaxDeviate = (1u << 17) - 3;  // distances share a word with 15 label bits
 constexpr uint32_t kTailDone = 0, kTailLevels = 1, kTailFull = 2;
 struct TailArgs {

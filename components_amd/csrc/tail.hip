@@ -343,8 +343,8 @@ __global__ __launch_bounds__(kTailBlock) void k_tail(TailArgs a) {
       // bound; where a table of one part holds the bound and the steps between
       // two looks at the count, one part does whatever their number.
       constexpr uint32_t step_edges = 4 * kTailBlock, look_steps = 2;
-      const uint32_t parts =
-          a.seq_limit + look_steps * step_edges <= kTableLoad ? 1 : (ne + kTableLoad - 1) / kTableLoad;
+      static_assert(kTailCountOnce + look_steps * step_edges == kTableLoad, "cut-offs of one part");
+      const uint32_t parts = a.seq_limit <= kTailCountOnce ? 1 : (ne + kTableLoad - 1) / kTableLoad;
       uint64_t distinct = 0;
       for (uint32_t part = 0; part < parts && distinct <= a.seq_limit; ++part) {
         clear_table();
