@@ -555,12 +555,17 @@ uint64_t sweep_to_fixpoint(kc_graph *g, uint64_t n, uint64_t m2, const uint64_t 
                            bool book_bytes = true, uint32_t *packed = nullptr) {
   uint64_t done = 0;
   // once most rows are settled a sweep costs less than a wait of the host, and one
-  // after the last change returns at once (2 us, but 14 with 58 000 blocks)
-  const uint32_t batch = b.blocks <= kLongBatchBlocks ? 8u : 3u;
+  // after the last change returns at once (2 us, but 14 with 58 000 blocks); where
+  // none settle, the first two waits see three (min labels on 2^20 pairs, two
+  // sweeps: 304 us a call so, 331 in eights; 100 000 points, 380 sweeps: 2590 in
+  // eights, 3180 in threes)
+  const bool long_batches = b.blocks <= kLongBatchBlocks;
+  const bool short_first = settled < 0 && n >= (1u << 16);
   uint32_t check = packed ? 1 : 0;  // the flag before the first batch's tells that packed keys do not fit
   // (packed: 4-byte keys for the neighbours and the row's own)
   const uint64_t bytes = !book_bytes ? 0 : packed ? 8 * (n + 1) + 8 * m2 + 8 * n : sweep_bytes(n, m2);
   while (true) {
+    const uint32_t batch = !long_batches || (short_first && done < 6) ? 3u : 8u;
     if (flag_base + batch + 2 >= kMaxFlags) {
       fill_u32(reinterpret_cast<uint32_t *>(g->flags), kMaxFlags, 0, g->stream);
       flag_base = 0;

@@ -271,8 +271,14 @@ __device__ __forceinline__ bool sweep_group(const SweepArgs &a, bool active, uin
                                             uint64_t e1, int gl, bool hub) {
   uint64_t kv = active ? a.kin[v] : ~0ull;
   uint64_t best = kv;
-  if (MODE == kSweepInPlace) active = active && static_cast<int>(kv >> 32) > a.settled;
-  if (active && !hub) {
+  // (the row's bounds do not wait for its key where no row is settled)
+  const bool look = MODE == kSweepInPlace && a.settled >= 0;
+  if (!look && active && !hub) {
+    e0 = a.off[v];
+    e1 = a.off[v + 1];
+  }
+  if (look) active = active && static_cast<int>(kv >> 32) > a.settled;
+  if (look && active && !hub) {
     e0 = a.off[v];
     e1 = a.off[v + 1];
   }
