@@ -403,11 +403,11 @@ constexpr uint64_t kLevelHotRows = 28672;  // labels the one-pass relabel serves
 // against n/32; n/4 took 7.22, R-MAT 24 and the others alike)
 constexpr int kTailShift = 3;
 constexpr uint64_t kPackedSweepsMin = 1u << 16;  // levels at least this large sweep packed keys
-// -bfs: rounds on skewed levels at least this large, elsewhere the sweeps that
-// a level's rounds end with from its start.  A call in rounds everywhere, so, and
-// in sweeps everywhere: R-MAT 24 8.66, 8.63 and 10.8 ms, R-MAT 22 2.70, 2.57, 3.02,
-// R-MAT 20 1.25, 1.05, 1.05, 256^3 grid 5.22, 4.73, 4.71, G(2^20, 2^22) 1.35, 1.22,
-// 1.21.
+// -bfs: rounds on levels at least this large that are skewed or that
+// rounds_pay finds; elsewhere the sweeps that a level's rounds end with from
+// its start.  A call in rounds everywhere, so, and in sweeps everywhere, ms: R-MAT 24
+// 8.66, 8.63, 10.8; R-MAT 22 2.70, 2.57, 3.02; R-MAT 20 1.25, 1.05, 1.05; 256^3 grid 5.22,
+// 4.73, 4.71; G(2^20, 2^22) 1.35, 1.22, 1.21.
 constexpr uint64_t kRoundsMin = 1u << 20;
 constexpr uint32_t kLongBatchBlocks = 1u << 15;  // sweeps of up to this many blocks go eight to a wait, others three
 constexpr uint64_t kPullRoundsMin = 1u << 16;  // -bfs: levels at least this large choose round directions
@@ -988,6 +988,19 @@ bool build_replicated(kc_graph *g, const kc_options *o, uint64_t n0, uint64_t m2
   return true;
 }
 
+// Whether a large level that is not skewed is done sooner in rounds.  At small
+// rates its sweeps run over 64-bit keys (the largest of n deviates is about
+// ln(n) / beta; rounds and sweeps at beta = 0.02, ms: G(4 M, 16 M) 3.02, 4.68, G(8 M,
+// 16 M) 4.46, 6.54, the 200^3 grid 2.58, 3.02, random geometric 4 M of degree 16
+// 2.42, 3.51).  Above 2^24 vertices they do too, and on many long rows the rounds
+// read less (beta = 0.1: G(20 M, 160 M) 31.3, 38.2, G(4 M, 32 M) 5.79, 6.38; but G(4 M,
+// 16 M) 4.13, 4.17, G(1.2 M, 9.6 M) 1.87, 1.83, the 280^3 grid 6.42, 6.07, 2^24 points of
+// degree 8 6.51, 5.53).
+bool rounds_pay(uint64_t n, uint64_t m2, double beta) {
+  if (std::log(static_cast<double>(n)) >= kPackedMaxDist * beta) return true;
+  return (n > (1ull << kPackedLabelBits) && m2 >= kDirectionMinDegree * n) || (m2 >= (1ull << 25) && m2 >= 12 * n);
+}
+
 // Levels whose rest runs in one workgroup.  A pass over the edges takes one CU
 // about 0.14 us per thousand, the general path some 0.3 ms per level whatever
 // its size.  Whole calls, default schedule / rounds, general path and this (us):
@@ -1174,7 +1187,8 @@ void run_contraction(kc_graph *g, const kc_options *o, RunOut &out, bool use_tai
       }
       const bool rounds = !local && o->use_bfs &&
                           (o->tail_sweeps || o->pull_rounds ||
-                           (n_l >= kRoundsMin && (input_level0 ? g->l0_hot_skewed : level_hot)));
+                           (n_l >= kRoundsMin && ((input_level0 ? g->l0_hot_skewed : level_hot) ||
+                                                  rounds_pay(n_l, m2_l, o->beta))));
       // Levels below 2^24 vertices whose key distances stay below 255 sweep
       // packed 32-bit keys (the buffer of the cluster ranks is free until they
       // are built).  A distance only falls, so a key plus one hop stays within

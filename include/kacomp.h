@@ -110,8 +110,10 @@ typedef struct kc_options {
   double beta;          /* -beta (default 0.1), rate of the exponential deviates */
   uint64_t seq_limit;   /* base case once remaining undirected edges <= seq_limit
                            (default 4096; 0 = contract until no edge is left) */
-  int32_t use_bfs;      /* -bfs: time-stepped frontier schedule of the decomposition, on the levels where it
-                           pays (large and skewed) or with tail_sweeps or pull_rounds set on all; else sweeps */
+  int32_t use_bfs;      /* -bfs: time-stepped frontier schedule of the decomposition, on the levels of 2^20
+                           vertices and more where it pays (skewed ones, small rates, many long rows),
+                           with tail_sweeps or pull_rounds set on all; else sweeps (same results but
+                           for the count of sweeps) */
   int32_t deviate_fma;  /* 1: canonical draw summed with a fused multiply-add, as
                            libstdc++ compiled with -O3 -march=native on FMA hardware;
                            0: separate multiply and add */

@@ -1,7 +1,8 @@
 """The time-stepped rounds of -bfs against the oracle: sizes, radius, ids and keys of every level, and the labels.  By
-default only skewed levels of 2^20 vertices and more run in rounds, so the small graphs ask for them with the options
-that have every level run so (the default cut-over to sweeps given outright, other cut-overs, pushes only, directions
-chosen on every level), and a large skewed graph takes the default.  Each run's launches say that it did run rounds."""
+default only levels of 2^20 vertices and more that are skewed, or whose deviates do not fit packed keys, run in rounds,
+so the small graphs ask for them with the options that have every level run so (the default cut-over to sweeps given
+outright, other cut-overs, pushes only, directions chosen on every level), and large graphs take the default.  Each
+run's launches say which schedule it ran."""
 import numpy as np
 import pytest
 
@@ -91,3 +92,16 @@ def test_default_rounds_on_a_large_skewed_level():
     run = oracle.Run(g.offsets, g.targets, variant="exp", keep_keys=True, **okw)
     check(g, run, **okw)
     check(g, run, **okw, tail_sweeps=-1)
+
+
+@pytest.mark.parametrize("beta,rounds", [(0.1, False), (0.02, True)])
+def test_default_schedule_by_rate(beta, rounds):
+    g = ca.generate("gnm_undirected", n=1100000, m=2500000, seed=3)
+    assert int((np.diff(g.offsets.astype(np.int64)) > 0).sum()) >= 1 << 20
+    kw = dict(variant="exp", seed=5, seq_limit=1 << 14, stream=ca.STREAM_HASHED, beta=beta)
+    run = oracle.Run(g.offsets, g.targets, **kw)
+    lv = run.levels()
+    lab, st = ca.find_components(g, use_bfs=True, **kw)
+    assert np.array_equal(lab, run.labels())
+    assert (st["levels"], st["radius_sum"]) == (len(lv), sum(x[3] for x in lv))
+    assert (st["kernel_launches"]["round"] > 0) == rounds
