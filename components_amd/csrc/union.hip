@@ -92,13 +92,27 @@ __device__ __forceinline__ uint32_t find_root(uint32_t *parent, uint32_t v) {
   return p;
 }
 
+// Joins the trees of u and w.  A large tree whose root hi was hooked a moment
+// ago still looks a root to the other chiplets, and each of its edges to another
+// tree would send its own compare-and-swap there, 4 ns apart: 1 ms where two large
+// trees were left (the base case of a contracted R-MAT 25, some seeds, of 70 us).  So
+// where many of a wave's lanes share the first one's hi, that lane's swap serves them.
+constexpr int kCrowd = 8;
 __device__ __forceinline__ void link(uint32_t *parent, uint32_t u, uint32_t w) {
   uint32_t a = find_root(parent, u), b = find_root(parent, w);
   while (a != b) {
     const uint32_t hi = a > b ? a : b, lo = a > b ? b : a;
-    const uint32_t old = atomicCAS(&parent[hi], hi, lo);
-    if (old == hi) break;
-    a = find_root(parent, old);  // hi was hooked meanwhile: old < hi
+    const bool like_first = hi == static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(hi)));
+    const uint64_t crowd = __ballot(like_first);
+    const bool served = like_first && __popcll(crowd) >= kCrowd;
+    const uint32_t first_lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(lo)));
+    const uint32_t under = served ? first_lo : lo;
+    uint32_t old = 0;
+    if (!served || lane_id() == static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(crowd)) - 1))
+      old = atomicCAS(&parent[hi], hi, under);
+    const uint32_t firsts = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(old)));
+    if (served) old = firsts;
+    a = old == hi ? under : find_root(parent, old);  // hi is hooked now, by this swap or another: under < hi
     b = lo;
   }
 }

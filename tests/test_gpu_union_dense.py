@@ -47,6 +47,22 @@ def test_dense_graphs_of_many_components():
         check(ca.Graph.from_edges(n, rng.permutation(n)[np.concatenate([e, hub])]))
 
 
+def test_two_large_trees():
+    # stars around the lowest ids (so that every leaf starts in its hub's tree) and many edges between their leaves,
+    # which all find the same two roots; as many again in a third tree of its own
+    rng = np.random.default_rng(8)
+    n = 60000
+    hub = rng.integers(0, 2, n)
+    leaves = np.arange(3, n)
+    stars = np.stack([hub[3:], leaves], 1)
+    a, b = leaves[hub[3:] == 0], leaves[hub[3:] == 1]
+    for cross in (1, 500, 400000):
+        between = np.stack([rng.choice(a, cross), rng.choice(b, cross)], 1)
+        check(ca.Graph.from_edges(n, np.concatenate([stars, between])))
+        alone = np.stack([np.full(1000, n), n + 1 + np.arange(1000)], 1)
+        check(ca.Graph.from_edges(n + 1001, np.concatenate([stars, alone, between])))
+
+
 @pytest.mark.parametrize("blocks", [3, 64])
 def test_blocks(blocks):
     for n, m in ((9000, 200000), (40000, 500000)):
