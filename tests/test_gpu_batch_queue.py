@@ -161,7 +161,7 @@ def test_classes_run_beside_the_queue():
     for graphs in (large, small, large + small):
         db = ca.DeviceBatch(ca.BatchGraphs.pack(graphs))
         db.set_tuning(block=256, groups_per_cu=4, use_graph=False)
-        ms.append(sorted(db.run(seed=5, stream=ca.STREAM_HASHED, copy_labels=False)[1]["time_ms"] for _ in range(7))[3])
+        ms.append(min(db.run(seed=5, stream=ca.STREAM_HASHED, copy_labels=False)[1]["time_ms"] for _ in range(9)))
         db.close()
     print(f"queue {ms[0]:.2f} ms, classes {ms[1]:.2f} ms, both {ms[2]:.2f} ms", flush=True)
     assert ms[1] < ms[0]  # else the queue hides nothing
